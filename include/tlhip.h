@@ -430,7 +430,10 @@ int tlhip_topk(const float* logits, int64_t offset, int64_t length, int k, float
  * with a group size that is a multiple of 64, on 256x256 2x4, 256x128 2x4, 128x256
  * 2x4, 128x128 2x2; p5 = 2, 4, 8 or 16: that many workgroups share a tile, each walking a
  * slice of K, and a second launch adds their partial sums in slice order - for
- * launches of far fewer tiles than the chip has CUs),
+ * launches of far fewer tiles than the chip has CUs; with tile K 64 its eight-wave form, the
+ * default above 64 rows, in which the weights are dequantised once per workgroup: tiles
+ * (M, N, waves M, waves N) 256x256 2x4, 256x192 2x4, 256x128 4x2, 128x128 2x4, 64x128 2x4, K a
+ * multiple of 64, every format with groups of 32 (int4) or 64 (int8) times a power of two),
  * 4 = "gemv_mfma_xreg" (skinny MFMA for int4 g32 with the activations held in
  * registers: p0 waves per workgroup, p1 iterations in flight, p2 workgroups per
  * CU, p3 K slices across workgroups, p4 = 1: every weight load of a wave issued

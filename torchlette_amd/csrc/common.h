@@ -115,6 +115,11 @@ bool epilogue_tail_applicable(const void* y, int64_t n);
 int launch_epilogue_tail(void* y, int y_dtype, int64_t m, int64_t n, const DevEpilogue& ep, hipStream_t stream);
 bool gemm_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
 int launch_gemm(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
+// The tiled_direct variant's form with tile K 64 (gemm_pipe.hip): eight waves, weights packed up
+// to the registers, dequantised once per workgroup.
+bool is_pipe_config(const tlhip_kernel_config_t& c);
+bool gemm_pipe_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
+int launch_gemm_pipe(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 bool gemm_direct_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
 int launch_gemm_direct(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 
@@ -163,6 +168,7 @@ int prepare_gemv_xreg_kernels();  // gemv_mfma_xreg.hip
 int prepare_gemv_wave_kernels();  // gemv_wave.hip
 int prepare_gemm_kernels();       // gemm_prefill.hip
 int prepare_gemm_direct_kernels();  // gemm_direct.hip
+int prepare_gemm_pipe_kernels();  // gemm_pipe.hip
 
 // Counters.
 void count_gemv_dispatch();
@@ -171,5 +177,7 @@ void count_dequant_dispatch();
 void count_autotune_run();
 
 enum { VARIANT_GEMV = 0, VARIANT_GEMV_MFMA = 1, VARIANT_TILED = 2, VARIANT_TILED_DIRECT = 3, VARIANT_GEMV_XREG = 4, VARIANT_GEMV_WAVE = 5 };
+
+inline bool is_pipe_config(const tlhip_kernel_config_t& c) { return c.variant == VARIANT_TILED_DIRECT && c.p2 == 64; }
 
 }  // namespace tlhip

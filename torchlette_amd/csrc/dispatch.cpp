@@ -286,9 +286,77 @@ int direct_k_split(const Problem& p) {
   return best;
 }
 
+// The tiles of the eight-wave tiled kernel (gemm_pipe.hip) and what a launch of them costs, in
+// microseconds, as measured at 1024..151936 x 1024..12288, M = 17..8192 on int4-32 and int8-64
+// (218 problems: the choice by this table is 0.3 % behind the best of the tiles and slices):
+// `fixed` (launch, first operands, epilogue), and per step of 64 k the time `light` while at
+// most 70 % of the CUs have a workgroup, `full` with one on every CU (the chip clocks down) and,
+// where two fit a CU, from `shared` (some CU has two) to `twice`.
+struct PipeTileCost {
+  int bm, bn, wm, wn, per_cu;
+  double fixed, light, full, shared, twice;
+};
+const PipeTileCost kPipeTileCosts[] = {
+    {256, 256, 2, 4, 1, 7.0, 1.27, 1.65, 0, 0},   {256, 192, 2, 4, 1, 6.5, 1.28, 1.48, 0, 0},
+    {256, 128, 4, 2, 1, 5.5, 0.80, 0.96, 0, 0},   {128, 128, 2, 4, 2, 5.0, 0.62, 0.67, 1.00, 1.22},
+    {64, 128, 2, 4, 2, 4.5, 0.46, 0.48, 0.56, 0.92},
+};
+
+tlhip_kernel_config_t pipe_cfg(const PipeTileCost& t, int ks) {
+  tlhip_kernel_config_t c = direct_cfg(t.bm, t.bn, t.wm, t.wn);
+  c.p2 = 64;
+  c.p5 = ks > 1 ? ks : 0;
+  return c;
+}
+
+double pipe_launch_us(const Problem& p, const PipeTileCost& t, int ks) {
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int64_t wgs = ((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn) * ks;
+  const int64_t cap = (int64_t)cus * t.per_cu, rounds = wgs / cap, rest = wgs % cap;
+  auto step_us = [&](double fill) {
+    if (fill <= 0.7) return t.light;
+    if (fill <= 1.0) return t.light + (t.full - t.light) * (fill - 0.7) / 0.3;
+    return t.shared + (t.twice - t.shared) * (fill - 1.0);
+  };
+  double us = t.fixed + (double)p.k / 64.0 / ks *
+                            ((double)rounds * step_us((double)t.per_cu) + (rest ? step_us((double)rest / cus) : 0.0));
+  // the launch that adds the slices' planes
+  if (ks > 1) us += 2.6 + 0.2 * ks + 0.40 * (double)ks * (double)p.m * (double)p.n * 4.0 / 1e6;
+  return us;
+}
+
+// The cheapest tile and number of K slices (each at least four steps) for p, or false.
+bool pipe_config(const Problem& p, tlhip_kernel_config_t* out, double* out_us) {
+  bool found = false;
+  for (const PipeTileCost& t : kPipeTileCosts)
+    for (int ks = 1; ks <= 16; ks *= 2) {
+      if (ks > 1 && p.k / 64 / ks < 4) break;
+      const double us = pipe_launch_us(p, t, ks);
+      if (found && us >= *out_us) continue;
+      tlhip_kernel_config_t c = pipe_cfg(t, ks);
+      if (!gemm_pipe_config_applicable(p, c, nullptr)) continue;
+      *out = c;
+      *out_us = us;
+      found = true;
+    }
+  return found;
+}
+
 // Heuristic default, used when nothing is tuned.
 tlhip_kernel_config_t default_config(const Problem& p) {
   if (p.m > 16 && p.x_dtype == TLHIP_F16) {
+    // the eight-wave kernel wherever it takes the problem (K a multiple of 64, groups of 32 or
+    // 64 times a power of two): ahead of the kernels below at every one of 196 problems from 64
+    // rows up, by 11 % in the geometric mean, 16-35 % on launches that fill the chip
+    // Not for an f32 output with a cast to f16 inside its chain: there a last bit of a sum
+    // decides over a whole step of f16, and such a chain keeps the sums (their order) of the
+    // kernel below, so that the default and an explicit configuration of it agree to 2e-6
+    // (4.6e-6 between the two kernels).
+    bool cast_inside = false;
+    for (int i = 0; i < p.epi.n_ops; ++i) cast_inside = cast_inside || (p.epi.kind[i] == TLHIP_EPI_CAST_F16 && p.y_dtype == TLHIP_F32);
+    tlhip_kernel_config_t pipe;
+    double pipe_us = 0.0;
+    if (!cast_inside && pipe_config(p, &pipe, &pipe_us)) return pipe;
     const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
     // int4: the kernel that keeps the weights packed up to the operand registers.
     // Tiles by how many there are (best of every tile at 2048..28672 x 2048..12288, M =
@@ -548,6 +616,12 @@ std::vector<tlhip_kernel_config_t> candidates(const Problem& p) {
           if (gemm_config_applicable(p, c, nullptr)) out.push_back(c);
         }
     }
+    for (const PipeTileCost& t : kPipeTileCosts)
+      for (int ks = 1; ks <= 16; ks *= 2) {
+        const tlhip_kernel_config_t c = pipe_cfg(t, ks);
+        if (ks > 1 && (((p.m + t.bm - 1) / t.bm) * ((p.n + t.bn - 1) / t.bn) >= (device_cu_count() > 0 ? device_cu_count() : 256) || p.k / 64 / ks < 4)) break;
+        if (gemm_pipe_config_applicable(p, c, nullptr)) out.push_back(c);
+      }
     static const int direct[][4] = {{256, 256, 2, 4}, {256, 128, 2, 4}, {128, 256, 2, 4}, {256, 128, 4, 2}, {128, 128, 2, 2}, {256, 256, 2, 2}, {128, 256, 1, 4}, {128, 192, 2, 2}};
     for (auto& t : direct) {
       tlhip_kernel_config_t c = direct_cfg(t[0], t[1], t[2], t[3]);
@@ -615,6 +689,11 @@ tlhip_kernel_config_t select_config(const Problem& p) {
     if (it != g_tuned.end() && config_applicable(p, it->second, nullptr)) return it->second;
   }
   tlhip_kernel_config_t c;
+  // Above 64 rows a neighbour's winner knows less than the launch model of the eight-wave
+  // kernel, which counts this problem's own tiles (0.3 % behind the best; the 512-row winner
+  // of 12288 x 4096, 256 x 128 tiles, is 30 % behind at 24576 x 4096).
+  double us = 0.0;
+  if (p.m > 64 && pipe_config(p, &c, &us)) return default_config(p);
   if (class_config(p, &c)) return c;
   return default_config(p);
 }
@@ -658,37 +737,60 @@ Problem as_f16_activations(const Problem& p) {
   return q;
 }
 
+// How the rows of such a problem go: `rows` at a time, rounded to f16 into the first `used`
+// floats of the stream's workspace, each chunk with configuration `c` of the f16 problem, whose
+// K slices (eight-wave kernel) leave their planes in what the workspace has left.  False: no
+// tiled kernel for the shape, or K too long for the workspace.
+struct F32Rows {
+  int64_t rows;
+  size_t used;
+  tlhip_kernel_config_t c;
+};
+bool plan_f32_rows(const Problem& p, F32Rows* r) {
+  if (p.x_dtype != TLHIP_F32 || p.m < kF32TiledFromRows || p.pro.kind != TLHIP_PRO_NONE) return false;
+  const int64_t capacity = (int64_t)(kSplitWorkspaceFloats * sizeof(float) / sizeof(_Float16));
+  r->rows = capacity / std::max<int64_t>(p.k, 1);
+  if (r->rows >= 256) r->rows -= r->rows % 256;  // whole tiles per chunk
+  if (r->rows < 32) return false;
+  r->rows = std::min<int64_t>(r->rows, p.m);
+  r->used = ((size_t)r->rows * (size_t)p.k / 2 + 63) / 64 * 64;
+  const SplitScratch rest = {nullptr, nullptr, kSplitWorkspaceFloats - r->used, kSplitCounters};
+  Problem q = as_f16_activations(p);
+  q.m = r->rows;
+  q.scratch = &rest;
+  auto tiled = [](const tlhip_kernel_config_t& c) { return c.variant == VARIANT_TILED || c.variant == VARIANT_TILED_DIRECT; };
+  r->c = select_config(q);
+  // (a tuned winner of the f16 problem may be the skinny kernel, which keeps its K-slice
+  // tiles where the rounded rows are: the heuristic tile then)
+  if (!tiled(r->c)) r->c = default_config(q);
+  if (!tiled(r->c)) return false;
+  if (!is_pipe_config(r->c)) r->c.p5 = 0;  // the other tiled kernels keep their planes where the rounded rows are
+  return true;
+}
+
 // f32 activations, many rows: the matrix cores take f16 operands, so the rows are
 // rounded to f16 once (a cast launch into the stream's workspace, as many rows at a time
 // as it holds) and go through the tiled kernel selected for the f16 problem.  Returns
-// false when this route does not apply (no tiled kernel for the shape, K too long for
-// the workspace) and nothing was launched.
+// false when this route does not apply and nothing was launched.
 bool f32_rows_through_tiled(const Problem& p, hipStream_t stream, int* rc) {
-  if (p.x_dtype != TLHIP_F32 || p.m < kF32TiledFromRows || p.pro.kind != TLHIP_PRO_NONE) return false;
-  Problem q = as_f16_activations(p);
-  tlhip_kernel_config_t c = select_config(q);
-  // (a tuned winner of the f16 problem may be the skinny kernel, which keeps its K-slice
-  // tiles where the rounded rows are: the heuristic tile then)
-  if (c.variant != VARIANT_TILED && c.variant != VARIANT_TILED_DIRECT) c = default_config(q);
-  if (c.variant != VARIANT_TILED && c.variant != VARIANT_TILED_DIRECT) return false;
-  c.p5 = 0;  // no K split across workgroups: its partial sums live in the workspace too
-  const int64_t capacity = (int64_t)(kSplitWorkspaceFloats * sizeof(float) / sizeof(_Float16));
-  int64_t rows = capacity / std::max<int64_t>(p.k, 1);
-  if (rows >= 256) rows -= rows % 256;  // whole tiles per chunk
-  if (rows < 32) return false;
+  F32Rows r;
+  if (!plan_f32_rows(p, &r)) return false;
   float* workspace = nullptr;
   int* counters = nullptr;
   *rc = split_workspace(stream, &workspace, &counters);
   if (*rc) return true;
+  const SplitScratch rest = {workspace + r.used, counters, kSplitWorkspaceFloats - r.used, kSplitCounters};
   const int yb = p.y_dtype == TLHIP_F16 ? 2 : 4;
-  for (int64_t m0 = 0; m0 < p.m; m0 += rows) {
-    q.m = std::min<int64_t>(rows, p.m - m0);
+  Problem q = as_f16_activations(p);
+  q.scratch = r.c.p5 > 1 ? &rest : nullptr;
+  for (int64_t m0 = 0; m0 < p.m; m0 += r.rows) {
+    q.m = std::min<int64_t>(r.rows, p.m - m0);
     *rc = tlhip_cast((const float*)p.x + m0 * p.k, TLHIP_F32, workspace, TLHIP_F16, q.m * p.k, (tlhip_stream_t)stream);
     if (*rc) return true;
     q.x = workspace;
     q.y = (char*)p.y + m0 * p.n * yb;
     q.epi = epilogue_from_row(p.epi, m0, p.n);
-    *rc = run_config(q, c, stream);
+    *rc = run_config(q, r.c, stream);
     if (*rc) return true;
   }
   return true;
@@ -784,11 +886,15 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     const int64_t passes = (p.m + 15) / 16;
     const int64_t tiles = ((p.m + 127) / 128) * ((p.n + 127) / 128);
     const double rounds = (double)tiles <= g_model.resident_tiles ? 1.0 : (double)tiles / g_model.resident_tiles;
-    const double tiled_us =
-        direct_round_us(p, c.p5 > 1 ? c.p5 : 1,
-                        c.variant == VARIANT_TILED_DIRECT ? g_model.walk_direct_us
-                                                          : (c.p0 <= 64 ? g_model.walk_staged64_us : g_model.walk_staged128_us)) *
-        rounds;
+    double tiled_us = 0.0;
+    for (const PipeTileCost& t : kPipeTileCosts)
+      if (is_pipe_config(c) && c.p0 == t.bm && c.p1 == t.bn)
+        tiled_us = pipe_launch_us(p, t, c.p5 > 1 ? c.p5 : 1);
+    if (tiled_us == 0.0)
+      tiled_us = rounds * direct_round_us(p, c.p5 > 1 ? c.p5 : 1,
+                                          c.variant == VARIANT_TILED_DIRECT ? g_model.walk_direct_us
+                                          : c.p0 <= 64                      ? g_model.walk_staged64_us
+                                                                            : g_model.walk_staged128_us);
     // Up to 64 rows per launch of the decode kernel: 1.2-1.6 times a 16-row pass for two
     // tiles of rows, 2.3-3.2 times for four (the activations a workgroup stages grow with
     // the rows, and their K slices are combined across workgroups).  More rows go 64 at a
@@ -1564,13 +1670,8 @@ int tlhip_selected_config(const tlhip_qweight_t* w, int x_dtype, int64_t m, int 
   if (rc) return rc;
   if (!out) return set_error(TLHIP_ERR_INVALID, "selected_config: null output");
   *out = plan_route(p, select_config(p)).first;  // of the first launch, where the rows go in chunks
-  if (p.x_dtype == TLHIP_F32 && p.m >= kF32TiledFromRows) {
-    // what tlhip_matmul_quantized launches for these rows: the f16 problem's tiled kernel
-    tlhip_kernel_config_t c = select_config(as_f16_activations(p));
-    if (c.variant != VARIANT_TILED && c.variant != VARIANT_TILED_DIRECT) c = default_config(as_f16_activations(p));
-    c.p5 = 0;  // as f32_rows_through_tiled launches it
-    if (c.variant == VARIANT_TILED || c.variant == VARIANT_TILED_DIRECT) *out = c;
-  }
+  F32Rows r;
+  if (plan_f32_rows(p, &r)) *out = r.c;  // what tlhip_matmul_quantized launches for these rows
   return TLHIP_OK;
 }
 

@@ -528,6 +528,7 @@ bool gemm_direct_config_applicable(const Problem& p, const tlhip_kernel_config_t
     return false;
   };
   if (c.variant != VARIANT_TILED_DIRECT) return fail(0);
+  if (is_pipe_config(c)) return gemm_pipe_config_applicable(p, c, why);
   const bool row = p.format == TLHIP_FMT_INT8_ROW;
   const bool int8 = p.format == TLHIP_FMT_INT8_GROUPED || row;
   if (p.format != TLHIP_FMT_INT4_GROUPED && !int8) return fail(1);
@@ -556,6 +557,7 @@ int launch_gemm_direct(const Problem& p, const tlhip_kernel_config_t& c, hipStre
   const char* why = nullptr;
   if (!gemm_direct_config_applicable(p, c, &why))
     return set_error(TLHIP_ERR_INVALID, "gemm_direct: config not applicable: %s", why);
+  if (is_pipe_config(c)) return launch_gemm_pipe(p, c, stream);
   if (p.m == 0 || p.n == 0) return TLHIP_OK;
   DirectArgs a;
   a.packed = (const uint8_t*)p.packed;

@@ -193,6 +193,7 @@ int prepare_all_kernels() {
   if (!rc) rc = prepare_gemv_seq_kernels();
   if (!rc) rc = prepare_gemm_kernels();
   if (!rc) rc = prepare_gemm_direct_kernels();
+  if (!rc) rc = prepare_gemm_pipe_kernels();
   t_prepare_mode = false;
   return rc;
 }
