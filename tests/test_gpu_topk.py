@@ -97,6 +97,23 @@ def test_topk_after_the_lm_head_gemv(be):
     assert np.allclose(vals, np.sort(want)[::-1][:8], rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("n", [1000, 4096, 8193, 256001, 600001])
+@pytest.mark.parametrize("k", [1, 64, 65, 256, 257])
+def test_topk_selection_on_unfavourable_orders(be, n, k):
+    """Both group counts of the selection and the sort behind it; one workgroup, the last
+    workgroup's level, a level of its own; orders in which a group holds all of the largest."""
+    i = np.arange(n)
+    rng = np.random.default_rng(n + k)
+    few = np.where(rng.random(n) < 0.002, rng.standard_normal(n), -np.inf)  # nearly all masked
+    for v in (i, -i, 0 * i, -(i % 512), (i % 128 == 5) * 1.0 + i % 3, few, np.where(i < n - 3, np.nan, i)):
+        v = v.astype(np.float32)
+        t = be.ops.tensorFromArray(v, [n], "f32")
+        vals, idx = be.readTopK(t, k)
+        want_v, want_i = reference_topk(v, k)
+        assert np.array_equal(idx, want_i)
+        assert np.array_equal(vals, want_v, equal_nan=True)
+
+
 def test_topk_errors(be):
     t = be.ops.tensorFromArray(np.zeros(10, np.float32), [10], "f32")
     with pytest.raises(L.TlhipError, match="k="):

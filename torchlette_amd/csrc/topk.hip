@@ -7,11 +7,14 @@
 //
 // Every element becomes a 64-bit key, (order-preserving bits of the value) << 32 |
 // (0xffffffff - index), so that "larger key" is exactly "larger value, then smaller
-// index"; NaN maps below every number.  A workgroup sorts up to 4096 keys in LDS
-// (bitonic, descending) and keeps the first k; levels repeat (chunk -> k per
-// workgroup) until one workgroup holds the answer.  Chunks of 1024 keys for
-// k <= 256 (many small sorts, every CU busy: 250 + 16 + 1 workgroups for 256 000
-// logits at k = 64), of 4096 above.  HBM traffic: the row once.
+// index"; NaN maps below every number.  A workgroup reduces up to 4096 keys to their k
+// largest; levels repeat (chunk -> k per workgroup) until one workgroup holds the answer.
+//
+// What bounds it: latency.  A row is 1 MB (0.2 us of HBM), the rest is dependent steps and
+// launches.  Up to k = 256 a workgroup therefore selects instead of sorting
+// (topk_select_kernel), and up to 8192 surviving keys the workgroup that arrives last does
+// the last level in the same launch: 256 000 logits at k = 64 are 63 workgroups and one
+// launch.  Above k = 256 a bitonic sort in LDS (topk_sort_kernel).
 #include "device_utils.h"
 
 namespace tlhip {
@@ -32,11 +35,168 @@ __device__ __forceinline__ float topk_value(uint64_t key) {
   return __builtin_bit_cast(float, b);
 }
 
+constexpr int kTopkChunk = 4096;        // keys a workgroup reduces
+constexpr int kSelectThreads = 512;
+constexpr int kSelectMaxK = 256;
+constexpr int kSelectFused = 8192;      // keys the last workgroup reduces in the same launch
+
+__device__ __forceinline__ uint64_t max_key(uint64_t a, uint64_t b) { return a > b ? a : b; }
+
+// The largest bound (of those tried) that at least `k` of the wave's 64 * R values reach.
+// One bit per step; a step that leaves exactly k values ends the search.
+template <int R>
+__device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool (&in)[R], int k, bool* exact) {
+  uint32_t bound = 0;
+  *exact = false;
+  for (int bit = 31; bit >= 0; --bit) {
+    const uint32_t trial = bound | (1u << bit);
+    int count = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) count += __popcll(__ballot(in[r] && v[r] >= trial));
+    if (count >= k) bound = trial;
+    if (count == k) {
+      *exact = true;
+      break;
+    }
+  }
+  return bound;
+}
+
+// The k largest of the keys the workgroup's threads hold (E each; 0 = none), in order, to
+// emit(rank, key); ranks without a key get 0.  Returns with every thread past its LDS reads.
+//   1. the maximum of every group of 4 threads (G = 128) or thread (G = 512);
+//   2. a bound that k of the G maxima reach, hence at least k keys: for k = 64 of 4096
+//      random keys about 90 do, at worst k groups' whole contents (4096);
+//   3. the keys from the bound on, collected in LDS; the rank of each is the number of
+//      larger ones.
+template <int G, int E, typename Emit>
+__device__ __forceinline__ void select_keys(const uint64_t (&key)[E], int k, uint64_t* maxima, uint64_t* found, int* n_found, Emit emit) {
+  constexpr int R = G / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  uint64_t best = key[0];
+#pragma unroll
+  for (int e = 1; e < E; ++e) best = max_key(best, key[e]);
+  if (G == kSelectThreads / 4) {
+    best = max_key(best, __shfl_xor(best, 1));
+    best = max_key(best, __shfl_xor(best, 2));
+    if ((tid & 3) == 0) maxima[tid >> 2] = best;
+  } else {
+    maxima[tid] = best;
+  }
+  if (tid == 0) *n_found = 0;
+  __syncthreads();
+  uint32_t hi[R], lo[R];
+  bool in[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint64_t m = maxima[r * 64 + lane];
+    hi[r] = (uint32_t)(m >> 32);
+    lo[r] = (uint32_t)m;
+    in[r] = true;
+  }
+  bool exact;
+  const uint32_t bound_hi = bound_of<R>(hi, in, k, &exact);
+  uint32_t bound_lo = 0;
+  if (!exact) {  // equal values around the bound: the index decides
+    int larger = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      larger += __popcll(__ballot(hi[r] > bound_hi));
+      in[r] = hi[r] == bound_hi;
+    }
+    bound_lo = bound_of<R>(lo, in, k - larger, &exact);
+  }
+  const uint64_t bound = ((uint64_t)bound_hi << 32) | bound_lo;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (key[e] != 0 && key[e] >= bound) found[atomicAdd(n_found, 1)] = key[e];
+  __syncthreads();
+  const int c = *n_found;
+  for (int i = tid; i < c; i += kSelectThreads) {
+    const uint64_t mine = found[i];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < c; ++j) rank += found[j] > mine ? 1 : 0;
+    if (rank < k) emit(rank, mine);
+  }
+  for (int i = c + tid; i < k; i += kSelectThreads) emit(i, (uint64_t)0);
+  __syncthreads();
+}
+
+__device__ __forceinline__ void write_result(int i, uint64_t key, float* out_values, void* out_indices, int index_dtype) {
+  const bool real = key != 0;
+  out_values[i] = real ? topk_value(key) : kTopkNegInf;
+  const int32_t idx = real ? (int32_t)(0xffffffffu - (uint32_t)key) : -1;
+  if (index_dtype == TLHIP_F32) ((float*)out_indices)[i] = (float)idx;  // token ids as f32 (deviceTopK)
+  else ((int32_t*)out_indices)[i] = idx;
+}
+
 // FROM_FLOAT: keys are made from `logits[offset + i]` with index i; else read from `keys_in`.
-// The first `k` keys of the sorted chunk go to keys_out[block * k ..]; with `final`
-// they are decoded into values / indices instead.
-template <bool FROM_FLOAT, int kTopkChunk>
-__global__ __launch_bounds__(kTopkChunk / 4) void topk_level_kernel(const float* __restrict__ logits, int64_t offset,
+// The chunk's k keys go to keys_out[rank * gridDim.x + block].  With `counter` the workgroup that arrives
+// last reduces all of them to the result (gridDim.x * k <= kSelectFused); a launch of one
+// workgroup writes the result at once.
+// 256 000 logits, k = 64, 8 rows behind each other: 35 us a row with three launches of sorted
+// chunks of 1024 before, SELECT_US us now.
+template <bool FROM_FLOAT, int G>
+__global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(const float* __restrict__ logits, int64_t offset,
+                                                                     const uint64_t* __restrict__ keys_in, int64_t count, int k,
+                                                                     uint64_t* keys_out, int* counter,
+                                                                     float* __restrict__ out_values,
+                                                                     void* __restrict__ out_indices, int index_dtype) {
+  __shared__ uint64_t maxima[G];
+  __shared__ uint64_t found[kTopkChunk];
+  __shared__ int n_found, arrived;
+  constexpr int E = kTopkChunk / kSelectThreads;
+  const int64_t base = (int64_t)blockIdx.x * kTopkChunk + threadIdx.x;
+  uint64_t key[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) key[e] = 0;  // padding is below every key: the index part of a real key is at least 1
+  if (count > 0) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int64_t at = base + e * kSelectThreads, clamped = at < count ? at : count - 1;
+      const uint64_t v = FROM_FLOAT ? topk_key(logits[offset + clamped], (uint32_t)at) : keys_in[clamped];
+      key[e] = at < count ? v : 0;
+    }
+  }
+  if (gridDim.x == 1) {
+    select_keys<G, E>(key, k, maxima, found, &n_found, [&](int i, uint64_t v) { write_result(i, v, out_values, out_indices, index_dtype); });
+    return;
+  }
+  // Device-scope accesses only, as for the K slices of the matrix-core GEMV: coherent between
+  // the L2 caches by themselves, without a fence that writes back and invalidates them.
+  // Largest first over all chunks: the next selection's groups of neighbours then hold keys of
+  // one rank.  (Chunk after chunk a few groups held every chunk's largest, so that its bound
+  // let thousands of keys pass: 68 us a row.)
+  uint64_t* mine = keys_out + blockIdx.x;
+  select_keys<G, E>(key, k, maxima, found, &n_found,
+                    [&](int i, uint64_t v) { __hip_atomic_store(mine + (size_t)i * gridDim.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
+  if (!counter) return;
+  // select_keys ends with a barrier, but a wave's stores are complete only once they are acknowledged
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+  if (threadIdx.x == 0) arrived = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  if (arrived != (int)gridDim.x - 1) return;
+  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+  constexpr int E2 = kSelectFused / kSelectThreads;
+  const int total = (int)gridDim.x * k;
+  uint64_t all[E2];
+#pragma unroll
+  for (int e = 0; e < E2; ++e) {
+    const int at = e * kSelectThreads + (int)threadIdx.x;
+    const uint64_t v = __hip_atomic_load(keys_out + (at < total ? at : total - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    all[e] = at < total ? v : 0;
+  }
+  select_keys<G, E2>(all, k, maxima, found, &n_found, [&](int i, uint64_t v) { write_result(i, v, out_values, out_indices, index_dtype); });
+}
+
+// k above kSelectMaxK: the chunk sorted in LDS, its first k keys to keys_out[block * k ..] or,
+// with `final`, decoded to the result.
+template <bool FROM_FLOAT>
+__global__ __launch_bounds__(kTopkChunk / 4) void topk_sort_kernel(const float* __restrict__ logits, int64_t offset,
                                                         const uint64_t* __restrict__ keys_in, int64_t count, int k,
                                                         uint64_t* __restrict__ keys_out, int final,
                                                         float* __restrict__ out_values,
@@ -70,11 +230,7 @@ __global__ __launch_bounds__(kTopkChunk / 4) void topk_level_kernel(const float*
   for (int i = threadIdx.x; i < k; i += THREADS) {
     const uint64_t key = keys[i];
     if (final) {
-      const bool real = key != 0;
-      out_values[i] = real ? topk_value(key) : kTopkNegInf;
-      const int32_t idx = real ? (int32_t)(0xffffffffu - (uint32_t)key) : -1;
-      if (index_dtype == TLHIP_F32) ((float*)out_indices)[i] = (float)idx;  // token ids as f32 (deviceTopK)
-      else ((int32_t*)out_indices)[i] = idx;
+      write_result(i, key, out_values, out_indices, index_dtype);
     } else {
       keys_out[(int64_t)blockIdx.x * k + i] = key;
     }
@@ -98,46 +254,48 @@ extern "C" int tlhip_topk(const float* logits, int64_t offset, int64_t length, i
   hipStream_t s = resolve_stream(stream);
   // level 0 reads the floats; later levels read the keys the level before wrote
   // into the stream's workspace, alternating between its two halves
-  const int chunk = k <= 256 ? 1024 : 4096;
-  int64_t count = length;
-  int64_t blocks = (count + chunk - 1) / chunk;
-  if (blocks < 1) blocks = 1;
+  const bool select = k <= kSelectMaxK;
   float* ws = nullptr;
   int* counters = nullptr;
   const size_t half = kSplitWorkspaceFloats / 4;  // uint64 keys per half
-  if (blocks > 1) {
-    if ((size_t)blocks * k > half)
+  // the lengths a call takes, and from which it works through the workspace: one row of k
+  // keys per 1024 logits (k <= 256; the levels below need a quarter of it) or per 4096
+  const int64_t limit_chunk = select ? 1024 : kTopkChunk;
+  const int64_t limit_blocks = (length + limit_chunk - 1) / limit_chunk;
+  if (limit_blocks > 1) {
+    if ((size_t)limit_blocks * k > half)
       return set_error(TLHIP_ERR_INVALID, "topk: length %lld with k=%d needs more workspace than the library holds",
                        (long long)length, k);
     const int rc = split_workspace(s, &ws, &counters);
     if (rc) return rc;
   }
   uint64_t* bufs[2] = {(uint64_t*)ws, (uint64_t*)ws + half};
-  int level = 0;
+  int64_t count = length;
   const uint64_t* keys_in = nullptr;
-  while (true) {
-    const int final = blocks == 1;
-    uint64_t* keys_out = final ? nullptr : bufs[level & 1];
-    const dim3 grid((unsigned)blocks), threads(chunk / 4);
-    const int64_t zero = 0;
-    if (level == 0 && chunk == 1024)
-      hipLaunchKernelGGL((topk_level_kernel<true, 1024>), grid, threads, 0, s, logits, offset, nullptr, count, k,
-                         keys_out, final, out_values, out_indices, index_dtype);
-    else if (level == 0)
-      hipLaunchKernelGGL((topk_level_kernel<true, 4096>), grid, threads, 0, s, logits, offset, nullptr, count, k,
-                         keys_out, final, out_values, out_indices, index_dtype);
-    else if (chunk == 1024)
-      hipLaunchKernelGGL((topk_level_kernel<false, 1024>), grid, threads, 0, s, nullptr, zero, keys_in, count, k,
-                         keys_out, final, out_values, out_indices, index_dtype);
-    else
-      hipLaunchKernelGGL((topk_level_kernel<false, 4096>), grid, threads, 0, s, nullptr, zero, keys_in, count, k,
-                         keys_out, final, out_values, out_indices, index_dtype);
+  for (int level = 0;; ++level) {
+    int64_t blocks = (count + kTopkChunk - 1) / kTopkChunk;
+    if (blocks < 1) blocks = 1;
+    const int64_t survivors = blocks * k;
+    uint64_t* keys_out = blocks == 1 ? nullptr : bufs[level & 1];
+    const dim3 grid((unsigned)blocks);
+    bool final = blocks == 1;
+    if (select) {
+      int* counter = !final && survivors <= kSelectFused ? counters : nullptr;
+      final = final || counter;
+      // groups of 4 threads are enough maxima up to k = 64
+      auto kernel = level == 0 ? (k <= 64 ? topk_select_kernel<true, 128> : topk_select_kernel<true, 512>)
+                               : (k <= 64 ? topk_select_kernel<false, 128> : topk_select_kernel<false, 512>);
+      hipLaunchKernelGGL(kernel, grid, dim3(kSelectThreads), 0, s, logits, offset, keys_in, count, k, keys_out, counter,
+                         out_values, out_indices, index_dtype);
+    } else {
+      auto kernel = level == 0 ? topk_sort_kernel<true> : topk_sort_kernel<false>;
+      hipLaunchKernelGGL(kernel, grid, dim3(kTopkChunk / 4), 0, s, logits, offset, keys_in, count, k, keys_out, (int)final,
+                         out_values, out_indices, index_dtype);
+    }
     TLHIP_CHECK_HIP(hipGetLastError());
     if (final) break;
     keys_in = keys_out;
-    count = blocks * k;
-    blocks = (count + chunk - 1) / chunk;
-    ++level;
+    count = survivors;
   }
   return TLHIP_OK;
 }
