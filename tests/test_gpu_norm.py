@@ -70,6 +70,28 @@ def test_rmsnorm_matches_oracle(be, m, d, xdt, ydt):
         t.destroy()
 
 
+@pytest.mark.parametrize("m,d,skip", [(3, 4104, 0), (2, 8192, 0), (2, 8200, 0), (2, 16384, 0), (1, 16392, 0), (2, 4096, 1)])
+@pytest.mark.parametrize("xdt", ["f32", "f16"])
+def test_rmsnorm_row_in_registers_and_beyond(be, m, d, skip, xdt):
+    """One, two and four pieces a lane, the lengths and the alignment (`skip` elements into a
+    buffer) that take the element-wise kernel; in place, as a caller may."""
+    rng = seeded("rmsnorm-row", m, d, skip, xdt)
+    x = make_x(m, d, xdt, rng, std=3.0)
+    w = norm_weight(d, rng)
+    flat = np.concatenate([np.zeros(skip, x.dtype), x.ravel()])
+    xt, wt = be.ops.tensorFromArray(flat, [flat.size], xdt), be.ops.tensorFromArray(w, [d], "f32")
+    at, code = xt.ptr + skip * x.dtype.itemsize, L.F16 if xdt == "f16" else L.F32
+    L.call("tlhip_rmsnorm", at, code, wt.ptr, at, code, m, d, 1e-6, None)
+    got = xt.numpy()[skip:].reshape(m, d).astype(np.float32)
+    want = O.rmsnorm(x.astype(np.float32), w, 1e-6)
+    if xdt == "f32":
+        assert max_rel(got, want) <= ELEMENTWISE_F32
+    else:
+        assert rel_l2(got, want) <= F16_BAR
+    for t in (xt, wt):
+        t.destroy()
+
+
 def test_rmsnorm_reference_spec_rows(be):
     # the rows of test/nn-rmsnorm.spec.ts:31-41, unit weight, eps 1e-6, tolerance 1e-4 there
     rows = np.array([[0.5, -1.2, 2.0, 0.1, -0.7, 1.5, -2.2, 0.9],

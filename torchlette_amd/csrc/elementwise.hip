@@ -40,6 +40,50 @@ __global__ __launch_bounds__(256) void cast_kernel(const S* __restrict__ in, D* 
   for (; i < count; i += stride) out[i] = (D)in[i];
 }
 
+// Eight consecutive elements, 16-byte aligned, as floats and back.
+template <typename T>
+__device__ __forceinline__ void load8(const T* p, float (&v)[8]) {
+  constexpr int PER = 16 / sizeof(T);
+#pragma unroll
+  for (int i = 0; i < 8 / PER; ++i) unit_to_floats<T>(((const u32x4*)p)[i], *(float(*)[PER])(v + i * PER));
+}
+template <typename T>
+__device__ __forceinline__ void store8(T* p, const float (&v)[8]) {
+  constexpr int PER = 16 / sizeof(T);
+#pragma unroll
+  for (int i = 0; i < 8 / PER; ++i) ((u32x4*)p)[i] = floats_to_unit<T>(*(const float(*)[PER])(v + i * PER));
+}
+
+// The same two ops eight elements a lane, for 16-byte aligned buffers (the last count % 8
+// elements one a lane).  Bound by latency at a decode step's sizes and by HBM at a prompt's.
+template <typename S, typename D>
+__global__ __launch_bounds__(256) void cast8_kernel(const S* __restrict__ in, D* __restrict__ out, int64_t count) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = t; i < count / 8; i += stride) {
+    float v[8];
+    load8(in + i * 8, v);
+    store8(out + i * 8, v);
+  }
+  if (t < count % 8) out[count - 1 - t] = (D)in[count - 1 - t];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void gated_mul8_kernel(int op, const T* gate, const T* up, T* out, int64_t count) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = t; i < count / 8; i += stride) {
+    float g[8], u[8];
+    load8(gate + i * 8, g);
+    load8(up + i * 8, u);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g[e] = apply_unary(op, g[e]) * u[e];
+    store8(out + i * 8, g);
+  }
+  if (t < count % 8) {
+    const int64_t i = count - 1 - t;
+    out[i] = (T)(apply_unary(op, (float)gate[i]) * (float)up[i]);
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void gated_mul_kernel(int op, const T* __restrict__ gate, const T* __restrict__ up,
                                                        T* __restrict__ out, int64_t count) {
@@ -68,6 +112,62 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const XT* __restrict__ x, 
   const float inv = 1.f / sqrtf(total / (float)d + eps);
   for (int64_t i = threadIdx.x; i < d; i += 256) yr[i] = (YT)(((float)xr[i] * inv) * weight[i]);
 }
+
+// The row in registers: up to R times 8 columns a lane of up to 8 waves, read once, in 16-byte
+// pieces, with the weights requested beside it.  Latency-bound: one trip to memory and one
+// barrier, where the kernel above walks a row of 4096 in 16 loads of one element a lane behind
+// each other, twice.  4096 f16 columns: 10.4 -> 3.2 us (16 rows), D a multiple of 8, every
+// pointer 16-byte aligned, D <= 16384.
+template <typename XT, typename YT, int R>
+__global__ __launch_bounds__(512) void rmsnorm_row_kernel(const XT* x, const float* __restrict__ weight, YT* y, int d, float eps) {
+  __shared__ float red[8];
+  const int units = d / 8, threads = blockDim.x;
+  const XT* xr = x + (int64_t)blockIdx.x * d;
+  YT* yr = y + (int64_t)blockIdx.x * d;
+  float v[R][8], w[R][8], ss = 0.f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) load8(xr + min(r * threads + (int)threadIdx.x, units - 1) * 8, v[r]);
+#pragma unroll
+  for (int r = 0; r < R; ++r) load8(weight + min(r * threads + (int)threadIdx.x, units - 1) * 8, w[r]);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float part = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) part = fmaf(v[r][e], v[r][e], part);
+    ss += r * threads + (int)threadIdx.x < units ? part : 0.f;
+  }
+  ss = group_sum(ss, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  float total = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) total += i * 64 < threads ? red[i] : 0.f;
+  const float inv = 1.f / sqrtf(total / (float)d + eps);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int u = r * threads + (int)threadIdx.x;
+    if (u < units) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[r][e] = (v[r][e] * inv) * w[r][e];
+      store8(yr + u * 8, v[r]);
+    }
+  }
+}
+
+template <typename XT, typename YT>
+void launch_rmsnorm(const XT* x, const float* weight, YT* y, int64_t m, int64_t d, float eps, hipStream_t s) {
+  const dim3 grid((unsigned)m);
+  const bool aligned = (((uintptr_t)x | (uintptr_t)weight | (uintptr_t)y) & 15) == 0;
+  if (d % 8 == 0 && d <= 16384 && aligned) {
+    const int units = (int)(d / 8), threads = std::min(512, (units + 63) / 64 * 64);
+    auto kernel = units <= 512 ? rmsnorm_row_kernel<XT, YT, 1> : (units <= 1024 ? rmsnorm_row_kernel<XT, YT, 2> : rmsnorm_row_kernel<XT, YT, 4>);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, x, weight, y, (int)d, eps);
+  } else {
+    hipLaunchKernelGGL((rmsnorm_kernel<XT, YT>), grid, dim3(256), 0, s, x, weight, y, d, eps);
+  }
+}
+
+bool aligned16(const void* a, const void* b, const void* c = nullptr) { return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0; }
 
 // The rest of an epilogue chain over a finished [M,N] output, in place: a lane takes 8
 // consecutive columns of a row (N is a multiple of 8), the output and the steps' inputs in
@@ -108,6 +208,22 @@ int grid_for(int64_t count) {
   const int64_t blocks = (count + 255) / 256;
   const int64_t cap = (int64_t)device_cu_count() * 16;
   return (int)std::max<int64_t>(1, std::min(blocks, cap));
+}
+
+template <typename T>
+void launch_gated_mul(int unary, const T* gate, const T* up, T* out, int64_t count, hipStream_t s) {
+  if (aligned16(gate, up, out))
+    hipLaunchKernelGGL(gated_mul8_kernel<T>, dim3(grid_for((count + 7) / 8)), dim3(256), 0, s, unary, gate, up, out, count);
+  else
+    hipLaunchKernelGGL(gated_mul_kernel<T>, dim3(grid_for(count)), dim3(256), 0, s, unary, gate, up, out, count);
+}
+
+template <typename S, typename D>
+void launch_cast(const S* in, D* out, int64_t count, hipStream_t s) {
+  if (aligned16(in, out))
+    hipLaunchKernelGGL((cast8_kernel<S, D>), dim3(grid_for((count + 7) / 8)), dim3(256), 0, s, in, out, count);
+  else
+    hipLaunchKernelGGL((cast_kernel<S, D>), dim3(grid_for(count)), dim3(256), 0, s, in, out, count);
 }
 
 }  // namespace
@@ -182,11 +298,9 @@ int tlhip_gated_mul(int unary, const void* gate, const void* up, int dtype, void
   if (dtype != TLHIP_F32 && dtype != TLHIP_F16) return set_error(TLHIP_ERR_INVALID, "gated_mul: bad dtype");
   hipStream_t s = resolve_stream(stream);
   if (dtype == TLHIP_F16)
-    hipLaunchKernelGGL(gated_mul_kernel<_Float16>, dim3(grid_for(count)), dim3(256), 0, s, unary,
-                       (const _Float16*)gate, (const _Float16*)up, (_Float16*)out, count);
+    launch_gated_mul(unary, (const _Float16*)gate, (const _Float16*)up, (_Float16*)out, count, s);
   else
-    hipLaunchKernelGGL(gated_mul_kernel<float>, dim3(grid_for(count)), dim3(256), 0, s, unary, (const float*)gate,
-                       (const float*)up, (float*)out, count);
+    launch_gated_mul(unary, (const float*)gate, (const float*)up, (float*)out, count, s);
   TLHIP_CHECK_HIP(hipGetLastError());
   return TLHIP_OK;
 }
@@ -202,18 +316,10 @@ int tlhip_rmsnorm(const void* x, int x_dtype, const float* weight, void* y, int 
   if (!(eps >= 0.f)) return set_error(TLHIP_ERR_INVALID, "rmsnorm: eps must be >= 0");
   if (m > 0x7fffffff) return set_error(TLHIP_ERR_INVALID, "rmsnorm: too many rows");
   hipStream_t s = resolve_stream(stream);
-  const dim3 grid((unsigned)m), block(256);
-  if (x_dtype == TLHIP_F16 && y_dtype == TLHIP_F16)
-    hipLaunchKernelGGL((rmsnorm_kernel<_Float16, _Float16>), grid, block, 0, s, (const _Float16*)x, weight,
-                       (_Float16*)y, d, eps);
-  else if (x_dtype == TLHIP_F16)
-    hipLaunchKernelGGL((rmsnorm_kernel<_Float16, float>), grid, block, 0, s, (const _Float16*)x, weight, (float*)y, d,
-                       eps);
-  else if (y_dtype == TLHIP_F16)
-    hipLaunchKernelGGL((rmsnorm_kernel<float, _Float16>), grid, block, 0, s, (const float*)x, weight, (_Float16*)y, d,
-                       eps);
-  else
-    hipLaunchKernelGGL((rmsnorm_kernel<float, float>), grid, block, 0, s, (const float*)x, weight, (float*)y, d, eps);
+  if (x_dtype == TLHIP_F16 && y_dtype == TLHIP_F16) launch_rmsnorm((const _Float16*)x, weight, (_Float16*)y, m, d, eps, s);
+  else if (x_dtype == TLHIP_F16) launch_rmsnorm((const _Float16*)x, weight, (float*)y, m, d, eps, s);
+  else if (y_dtype == TLHIP_F16) launch_rmsnorm((const float*)x, weight, (_Float16*)y, m, d, eps, s);
+  else launch_rmsnorm((const float*)x, weight, (float*)y, m, d, eps, s);
   TLHIP_CHECK_HIP(hipGetLastError());
   return TLHIP_OK;
 }
@@ -225,11 +331,9 @@ int tlhip_cast(const void* in, int in_dtype, void* out, int out_dtype, int64_t c
   if (!in || !out) return set_error(TLHIP_ERR_INVALID, "cast: null pointer");
   hipStream_t s = resolve_stream(stream);
   if (in_dtype == TLHIP_F32 && out_dtype == TLHIP_F16)
-    hipLaunchKernelGGL((cast_kernel<float, _Float16>), dim3(grid_for(count)), dim3(256), 0, s, (const float*)in,
-                       (_Float16*)out, count);
+    launch_cast((const float*)in, (_Float16*)out, count, s);
   else if (in_dtype == TLHIP_F16 && out_dtype == TLHIP_F32)
-    hipLaunchKernelGGL((cast_kernel<_Float16, float>), dim3(grid_for(count)), dim3(256), 0, s, (const _Float16*)in,
-                       (float*)out, count);
+    launch_cast((const _Float16*)in, (float*)out, count, s);
   else if (in_dtype == out_dtype && (in_dtype == TLHIP_F32 || in_dtype == TLHIP_F16))
     TLHIP_CHECK_HIP(hipMemcpyAsync(out, in, (size_t)count * (in_dtype == TLHIP_F16 ? 2 : 4), hipMemcpyDeviceToDevice, s));
   else
