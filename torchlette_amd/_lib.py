@@ -23,7 +23,7 @@ UNARY = {"none": 0, "relu": 1, "silu": 2, "gelu": 3, "gelu_tanh": 3, "gelu_erf":
 EPI_NONE, EPI_BIAS, EPI_UNARY, EPI_BINARY, EPI_CAST_F16 = 0, 1, 2, 3, 4
 BINARY = {"add": 0, "sub": 1, "mul": 2}
 MAX_EPILOGUE_OPS = 4
-VARIANT_GEMV, VARIANT_GEMV_MFMA, VARIANT_TILED, VARIANT_TILED_DIRECT, VARIANT_GEMV_XREG, VARIANT_GEMV_WAVE = 0, 1, 2, 3, 4, 5
+VARIANT_GEMV, VARIANT_GEMV_MFMA, VARIANT_TILED, VARIANT_TILED_DIRECT, VARIANT_GEMV_XREG, VARIANT_GEMV_WAVE, VARIANT_GEMV_F32 = 0, 1, 2, 3, 4, 5, 6
 
 
 class TlhipError(RuntimeError):

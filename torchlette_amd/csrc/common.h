@@ -110,6 +110,10 @@ bool gemv_xreg_group_applicable(const Problem* ps, int count, const tlhip_kernel
 int launch_gemv_xreg_group(const Problem* ps, int count, const tlhip_kernel_config_t& c, hipStream_t stream);
 bool gemv_wave_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
 int launch_gemv_wave(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
+// gemv_f32.hip: f32 activations in three bf16 pieces on the matrix cores
+bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
+bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out);
+int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 // elementwise.hip: the steps of `ep` over a finished [M,N] output, in place, 8 columns a lane
 bool epilogue_tail_applicable(const void* y, int64_t n);
 int launch_epilogue_tail(void* y, int y_dtype, int64_t m, int64_t n, const DevEpilogue& ep, hipStream_t stream);
@@ -166,6 +170,7 @@ int prepare_gemv_kernels();       // gemv.hip (+ the per-format units)
 int prepare_gemv_mfma_kernels();  // gemv_mfma.hip
 int prepare_gemv_xreg_kernels();  // gemv_mfma_xreg.hip
 int prepare_gemv_wave_kernels();  // gemv_wave.hip
+int prepare_gemv_f32_kernels();   // gemv_f32.hip
 int prepare_gemm_kernels();       // gemm_prefill.hip
 int prepare_gemm_direct_kernels();  // gemm_direct.hip
 int prepare_gemm_pipe_kernels();  // gemm_pipe.hip
@@ -176,7 +181,7 @@ void count_gemm_dispatch();
 void count_dequant_dispatch();
 void count_autotune_run();
 
-enum { VARIANT_GEMV = 0, VARIANT_GEMV_MFMA = 1, VARIANT_TILED = 2, VARIANT_TILED_DIRECT = 3, VARIANT_GEMV_XREG = 4, VARIANT_GEMV_WAVE = 5 };
+enum { VARIANT_GEMV = 0, VARIANT_GEMV_MFMA = 1, VARIANT_TILED = 2, VARIANT_TILED_DIRECT = 3, VARIANT_GEMV_XREG = 4, VARIANT_GEMV_WAVE = 5, VARIANT_GEMV_F32 = 6 };
 
 inline bool is_pipe_config(const tlhip_kernel_config_t& c) { return c.variant == VARIANT_TILED_DIRECT && c.p2 == 64; }
 

@@ -196,6 +196,7 @@ bool config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const c
   if (c.variant == VARIANT_GEMV_MFMA) return gemv_mfma_config_applicable(p, c, why);
   if (c.variant == VARIANT_GEMV_XREG) return gemv_xreg_config_applicable(p, c, why);
   if (c.variant == VARIANT_GEMV_WAVE) return gemv_wave_config_applicable(p, c, why);
+  if (c.variant == VARIANT_GEMV_F32) return gemv_f32_config_applicable(p, c, why);
   return gemv_config_applicable(p, c, why);
 }
 
@@ -436,6 +437,15 @@ tlhip_kernel_config_t default_config(const Problem& p) {
       if (have) return best_c;
     }
   }
+  // f32 rows on the matrix cores, three bf16 pieces each: ahead of the VALU kernel from five rows
+  // on at every size (1024 x 768: 7.3 against 8.6 us; 9216 x 2304: 15.7 against 34.4 us, int8-64),
+  // for three and four rows on int4 (1024 x 768: 9.4 against 23.2 us) and on int8 from 8 MB
+  // of weights (2304 x 9216: 18.4 against 21.6 us; 2304 x 2048: 8.9 against 8.2 us)
+  if (p.x_dtype == TLHIP_F32 && p.m <= 16 &&
+      (p.m >= 5 || (p.m >= 3 && (p.format == TLHIP_FMT_INT4_GROUPED || p.n * p.k >= 8000000)))) {
+    tlhip_kernel_config_t c;
+    if (gemv_f32_default(p, &c)) return c;
+  }
   // three or four rows of int4 weights with K up to 8192, from 8 MB of weights on: the
   // VALU kernel's 4x4x4 matrix-core form (tuned winner at 5120..14336 x 4096..8192:
   // 7.8-12.2 us against 9.9-15.7 us for the skinny kernel below, which is ahead for
@@ -546,6 +556,13 @@ tlhip_kernel_config_t default_valu_config(const Problem& p) {
 
 std::vector<tlhip_kernel_config_t> candidates(const Problem& p) {
   std::vector<tlhip_kernel_config_t> out;
+  for (int slices = 1; slices <= 32; slices *= 2) {
+    tlhip_kernel_config_t c;
+    memset(&c, 0, sizeof c);
+    c.variant = VARIANT_GEMV_F32;
+    c.p0 = slices;
+    if (gemv_f32_config_applicable(p, c, nullptr)) out.push_back(c);
+  }
   if (p.m <= 16) {
     for (int lpr : {16, 32, 64})
       for (int r : {1, 2, 4})
@@ -722,6 +739,7 @@ int run_config(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t str
   if (c.variant == VARIANT_GEMV_MFMA) return launch_gemv_mfma(p, c, stream);
   if (c.variant == VARIANT_GEMV_XREG) return launch_gemv_xreg(p, c, stream);
   if (c.variant == VARIANT_GEMV_WAVE) return launch_gemv_wave(p, c, stream);
+  if (c.variant == VARIANT_GEMV_F32) return launch_gemv_f32(p, c, stream);
   return launch_gemv(p, c, stream);
 }
 
@@ -1008,6 +1026,9 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       vary(2, {1, 2, 4, 8, 16});
       vary(3, {1, 2, 4, 8});
       vary(5, {0, 1});
+      break;
+    case VARIANT_GEMV_F32:
+      vary(0, {1, 2, 4, 8, 16, 32});
       break;
     case VARIANT_GEMV_WAVE:
       vary(0, {4, 8});
