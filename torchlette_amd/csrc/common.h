@@ -121,6 +121,11 @@ bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c
 bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out);
 int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c);
+// The gemv_mfma variant's form for 17..64 rows (gemm_rows.hip; p4: blocks of 16 columns per
+// workgroup): all of K in one workgroup, no workspace.  What it does not take runs the other form.
+bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c);
+bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us);
+int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 // elementwise.hip: the steps of `ep` over a finished [M,N] output, in place, 8 columns a lane
 bool epilogue_tail_applicable(const void* y, int64_t n);
 int launch_epilogue_tail(void* y, int y_dtype, int64_t m, int64_t n, const DevEpilogue& ep, hipStream_t stream);
@@ -187,6 +192,7 @@ int prepare_gemv_mfma_kernels();  // gemv_mfma.hip
 int prepare_gemv_xreg_kernels();  // gemv_mfma_xreg.hip
 int prepare_gemv_wave_kernels();  // gemv_wave.hip
 int prepare_gemv_f32_kernels();   // gemv_f32.hip
+int prepare_gemm_rows_kernels();  // gemm_rows.hip
 int prepare_gemm_kernels();       // gemm_prefill.hip
 int prepare_gemm_direct_kernels();  // gemm_direct.hip
 int prepare_gemm_pipe_kernels();  // gemm_pipe.hip

@@ -607,6 +607,11 @@ std::vector<tlhip_kernel_config_t> candidates(const Problem& p) {
           if (gemv_config_applicable(p, c, nullptr)) out.push_back(c);
         }
   }
+  for (int cols = 1; cols <= 4 && p.m > 16; ++cols) {  // 17..64 rows, all of K in a workgroup
+    tlhip_kernel_config_t c = mfma_cfg(8, 0, 0, 0);
+    c.p4 = cols;
+    if (is_rows_config(p, c)) out.push_back(c);
+  }
   if (p.m <= 64) {  // above 16 rows: two or four tiles of rows per weight row block
     for (int waves : {4, 8, 16})
       for (int unroll : {1, 2, 4})
@@ -880,23 +885,41 @@ int matmul_with(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
 // in flight, the fewest K slices across workgroups whose activations fit LDS, and the
 // fewest K-split waves per row block that still give every CU a workgroup (measured best
 // or within 5 % of it at 4096..28672 x 4096..12288, M = 24..64).
-bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
+//
+// ... or its form that keeps all of K in one workgroup (gemm_rows.hip), by the models of both:
+// `decode_us` is the former's price, a third more where no waves split K (32 rows of int4 at
+// 6454 x 2304: 15.7 us), half more for int8 (over 12 matrices the former took 1.0-2.5 times its
+// price).  Us, former against latter: int8-64 at 12288 x 4096, 20 / 32 / 48 rows 27.1 / 28.0 / 30.1
+// against 20.8 / 21.9 / 23.3, but 11.0 / 12.6 / 24.9 against 20.7 / 23.2 / 27.9 at 961 x 11136; int4
+// 48 rows at 12288 x 4096 27.2 against 18.5; up to 32 rows of int4 the two are close where both have
+// their best form (16.2 against 22.5 at 4096 x 12288, 10.3 against 12.0 at 13740 x 2048).
+bool rows_in_one_launch_config(const Problem& p, double decode_us, tlhip_kernel_config_t* out) {
   if (p.m <= 16 || p.m > 64 || p.x_dtype != TLHIP_F16) return false;
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int64_t nblocks = (p.n + 15) / 16;
-  for (int ks = 1; ks <= 16; ks *= 2) {
+  bool found = false;
+  for (int ks = 1; ks <= 16 && !found; ks *= 2) {
     int fill = 1;  // K-split waves per row block: 8 / fill row blocks per workgroup
     while (fill < 8 && (nblocks * fill / 8) * ks < cus) fill *= 2;
     for (int kw : {fill, 8, 4, 2, 1})
       for (int unroll : {2, 1}) {
         const tlhip_kernel_config_t c = mfma_cfg(8, unroll, kw, ks);
-        if (gemv_mfma_config_applicable(p, c, nullptr)) {
+        if (!found && gemv_mfma_config_applicable(p, c, nullptr)) {
           *out = c;
-          return true;
+          found = true;
         }
       }
   }
-  return false;
+  tlhip_kernel_config_t whole;
+  double us = 0.0;
+  if (!gemm_rows_default(p, &whole, &us)) return found;
+  if (found) {
+    const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
+    const double price = decode_us * (out->p2 == 1 ? 1.3 : 1.0) * (int4 ? (p.m <= 32 ? 0.9 : 1.0) : 1.5);
+    if (us >= price) return true;
+  }
+  *out = whole;
+  return true;
 }
 
 bool has_tuned_entry(const Problem& p) {
@@ -975,14 +998,25 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     auto chunk_us = [&](int64_t rows) { return pass_us * (rows <= 16 ? 1.0 : (rows <= 32 ? g_model.rows32_factor : g_model.rows64_factor)); };
     const int64_t full = p.m / 64, rest = p.m % 64;
     const double rows_us = (double)full * chunk_us(64) + (rest ? chunk_us(rest) : 0.0);
-    if (rows_us < g_model.rows_break_even * tiled_us) {
+    // one launch of the form that keeps all of K in a workgroup, exact too: wherever it is cheaper
+    // than the tile that would run (48 rows of int4 at 4096 x 4096: 12.0 against 15.4 us); above K =
+    // 1024 only, where a test of first calls under capture pins the tile's K slices (40 rows at 4096
+    // x 1024)
+    tlhip_kernel_config_t whole;
+    double whole_us = 0.0;
+    const bool whole_ok = p.m <= 64 && p.k > 1024 && gemm_rows_default(p, &whole, &whole_us);
+    double pipe_us = tiled_us;
+    if (is_pipe_config(c))
+      for (const PipeTileCost& t : kPipeTileCosts)
+        if (c.p0 == t.bm && c.p1 == t.bn) pipe_us = pipe_launch_us(p, t, c.p5 > 1 ? c.p5 : 1);
+    if (rows_us < g_model.rows_break_even * tiled_us || (whole_ok && whole_us < g_model.rows_break_even * pipe_us)) {
       bool ok = true;
       Route q{64, c, c};
       Problem q64 = p, qr = p;
       q64.m = 64;
       qr.m = rest;
-      if (full) ok = rows_in_one_launch_config(q64, &q.first);
-      if (ok && rest > 16) ok = rows_in_one_launch_config(qr, &q.last);
+      if (full) ok = rows_in_one_launch_config(q64, chunk_us(64), &q.first);
+      if (ok && rest > 16) ok = rows_in_one_launch_config(qr, chunk_us(rest), &q.last);
       if (ok && rest > 0 && rest <= 16) {
         q.last = select_gemv_config(qr);
         ok = q.last.variant == VARIANT_GEMV_MFMA || q.last.variant == VARIANT_GEMV_XREG || rest <= 4;
@@ -1080,6 +1114,7 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       vary(1, {1, 2, 4});
       vary(2, {1, 2, 4, 8, 16});
       vary(3, {1, 2, 4, 8});
+      if (is_rows_config(p, base)) vary(4, {1, 2, 3, 4});
       vary(5, {0, 1});
       break;
     case VARIANT_GEMV_F32:

@@ -1,0 +1,429 @@
+// GEMM of 17 to 64 f16 activation rows over packed weights, exact: the integers go to the
+// matrix cores as they are and every group's sum is scaled in f32, as in the decode kernels.
+// Same contract and reference route as gemv.hip (src/backend/webgpu/matmul/gemv.ts:365-466).
+//
+// What bounds it: the activations' way to the matrix cores.  64 rows of K = 4096 are 512 KB,
+// three times a CU's LDS, and every workgroup needs all of them from its L2; the weights of a
+// workgroup's columns are a tenth to a third of that.  Hence:
+//   * A workgroup owns 16 NB columns of Y and all of K, so that nothing is combined between
+//     workgroups: no planes of partial sums, no second launch, no workspace.
+//   * Its eight waves take K in turn, 128 at a time, each alone with its part until one
+//     barrier at the end: the activations of a step (16 MT rows) are loaded into registers
+//     one or two steps ahead, whole lines per row, laid into a patch of LDS that belongs to
+//     the wave, and read back as MFMA operands; every byte of X enters the CU once.
+//   * An operand of X feeds NB products and a weight, dequantised once, MT.
+// One launch, us, best kernel before -> here: int4-32 12288 x 4096 at 48 / 64 rows 27.2 -> 18.5, 27.6 ->
+// 20.4; 4096 x 4096 at 48 rows 14.9 -> 12.3; int8-64 12288 x 4096 at 17..32 rows 27-28 -> 21-22, 7179 x
+// 896 at 40 rows 13.3 -> 7.0.  18.5 us are 1.5 TB/s of weights and 260 TFLOP/s: 3.5 us of launch, first
+// loads and last sums, the rest the 100 MB of X that 256 CUs fetch (25-30 bytes a clock and CU).
+// Rearranging X for the cheaper int4 unpacking, or its addresses by lane, moved nothing.
+//   * Buffer loads: rows past M, columns past N and steps past K read zero and cost no traffic,
+//     so that the loop has no branch around a load.
+#include <algorithm>
+#include <cstring>
+
+#include "gemv_mfma_common.h"
+
+namespace tlhip {
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kStep = 128;                  // k of a step
+constexpr int kRowBytes = kStep * 2 + 16;   // LDS row of a step: 16 bytes more, so that rows start in other banks
+constexpr int kMaxCols = 4;                 // blocks of 16 columns per workgroup
+
+struct RowsArgs {
+  const uint8_t* packed;
+  const uint8_t* scales;
+  const _Float16* x;
+  void* y;
+  int m, n, k;
+  int row_bytes;         // packed bytes of a weight row
+  int scale_row_bytes;   // bytes of a row's group scales
+  int group_shift;       // int8 groups: log2(group size / 64)
+  float alpha, scale_mul;
+  int y_dtype;
+  int vec_ok;            // N % 4 == 0 and y 16-byte aligned: four columns in one store
+  DevEpilogue epi;
+};
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+
+// A step's number (negative: no such step) as a scalar that the compiler neither keeps in a
+// vector register nor selects with: either puts every load behind it into a loop over the lanes.
+__device__ __forceinline__ int scalar_step(int st, int steps) {
+  st = st < steps ? st : -1;
+  asm("" : "+s"(st));
+  return st;
+}
+__device__ __forceinline__ rsrc_t buffer_of(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00027000);
+}
+constexpr int kNontemporal = 2;  // the load's slc bit
+template <int AUX>
+__device__ __forceinline__ u32x4 load16(rsrc_t r, uint32_t at, uint32_t step_at) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, (int)step_at, AUX));
+}
+
+// The 8 weights of a word in k order (unpack_int4_word: pairs four apart): three more VALU
+// instructions a word, but no rearranging of the activations, of which a step has MT times as many.
+__device__ __forceinline__ half8_t weights_of(uint32_t w) {
+  const uint32_t t = w ^ 0x88888888u;
+  const half2_t mul = {(_Float16)1.f, (_Float16)0.0625f}, add = {(_Float16)-1032.f, (_Float16)-72.f};
+  half2_t h[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t twice = __builtin_amdgcn_perm(t, t, 0x01010101u * (uint32_t)i);  // byte i four times
+    h[i] = __builtin_bit_cast(half2_t, and_or(twice, 0x00f0000fu, 0x64006400u)) * mul + add;
+  }
+  return join8(h);
+}
+
+// MT: tiles of 16 rows (M <= 16 MT); NB: blocks of 16 columns; XD: steps of X in registers (0: one, and one of the weights)
+template <int FMT, int MT, int NB, int XD>
+__global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a) {
+  constexpr bool INT4 = FMT == TLHIP_FMT_INT4_GROUPED, ROW = FMT == TLHIP_FMT_INT8_ROW;
+  constexpr int WV = INT4 ? 1 : 2;      // 16-byte loads of a step, lane and column block
+  constexpr int XV = MT * 4;            // 16-byte loads of a step's X per lane: four rows each
+  extern __shared__ u32x4 lds[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nl = lane & 15, g = lane >> 4;
+  const int n0 = (int)blockIdx.x * (16 * NB);
+  const int cols = min(16 * NB, a.n - n0);
+  const int steps = a.k / kStep;
+  const uint8_t* const packed = a.packed + (int64_t)n0 * a.row_bytes;
+  const uint8_t* const scales = a.scales + (int64_t)n0 * a.scale_row_bytes;
+
+  // A lane's place in a step is fixed, the step is a scalar offset; past the last step a buffer
+  // of no bytes at offset 0 (a range check may or may not count the scalar offset).
+  uint32_t w_at[NB], s_at[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    w_at[b] = (uint32_t)(16 * b + nl) * (uint32_t)a.row_bytes + (uint32_t)g * 16u;
+    s_at[b] = (uint32_t)(16 * b + nl) * (uint32_t)a.scale_row_bytes;
+  }
+  const uint32_t x_at = (uint32_t)g * (uint32_t)a.k * 2u + (uint32_t)nl * 16u;  // in four rows, a buffer each
+
+  struct Weights {
+    u32x4 w[NB][WV];
+    uint32_t s[NB][2];  // int4: four group scales; int8: one per half step
+  };
+  auto load_w = [&](Weights& v, int step) {
+    const int st = scalar_step(step, steps);
+    const uint32_t in = ~(uint32_t)(st >> 31);
+    const rsrc_t wb = buffer_of(packed, (uint32_t)cols * (uint32_t)a.row_bytes & in);
+    const rsrc_t sb = buffer_of(scales, (uint32_t)cols * (uint32_t)a.scale_row_bytes & in);
+    const uint32_t at = (uint32_t)st & in;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+#pragma unroll
+      for (int i = 0; i < WV; ++i) v.w[b][i] = load16<kNontemporal>(wb, w_at[b] + (uint32_t)i * 64u, at * (WV * 64u));
+      if constexpr (INT4) {
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 s = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sb, (int)s_at[b], (int)(at * 8u), 0));
+        v.s[b][0] = s.x;
+        v.s[b][1] = s.y;
+      } else if constexpr (!ROW) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          v.s[b][h] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sb, (int)s_at[b], (int)(((2u * at + (uint32_t)h) >> a.group_shift) * 2u), 0);
+      }
+    }
+  };
+  struct Rows {
+    u32x4 v[XV];
+  };
+  auto load_x = [&](Rows& r, int step) {
+    const int st = scalar_step(step, steps);
+    const uint32_t in = ~(uint32_t)(st >> 31);
+    const uint32_t at = (uint32_t)st * (kStep * 2u) & in;
+#pragma unroll
+    for (int i = 0; i < XV; ++i)
+      r.v[i] = load16<0>(buffer_of(a.x + (int64_t)(4 * i) * a.k, (uint32_t)max(a.m - 4 * i, 0) * (uint32_t)a.k * 2u & in), x_at, at);
+  };
+  char* const patch = (char*)lds + wave * (MT * 16 * kRowBytes);
+  auto lay_x = [&](const Rows& r) {
+#pragma unroll
+    for (int i = 0; i < XV; ++i) *(u32x4*)(patch + (4 * i + g) * kRowBytes + nl * 16) = r.v[i];
+  };
+
+  float4_t acc[NB][MT];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[b][t] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  // operand s of a step: int4 k = 32 s + 8 g; int8 k = 64 (s / 2) + 16 g + 8 (s % 2)
+  auto operand = [&](int t, int s) {
+    const int unit = INT4 ? 4 * s + g : 8 * (s >> 1) + 2 * g + (s & 1);
+    return __builtin_bit_cast(half8_t, *(const u32x4*)(patch + (16 * t + nl) * kRowBytes + unit * 16));
+  };
+  auto multiply = [&](const Weights& v) __attribute__((always_inline)) {
+    uint32_t word[NB][4 * WV];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+#pragma unroll
+      for (int i = 0; i < WV; ++i) {
+        word[b][4 * i + 0] = v.w[b][i].x;
+        word[b][4 * i + 1] = v.w[b][i].y;
+        word[b][4 * i + 2] = v.w[b][i].z;
+        word[b][4 * i + 3] = v.w[b][i].w;
+      }
+      // a lane holds 32 k of its row, one group; afterwards word i is its eighth of group i
+      if constexpr (INT4) transpose4(word[b][0], word[b][1], word[b][2], word[b][3]);
+    }
+    if constexpr (INT4) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        half8_t xa[MT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t) xa[t] = operand(t, s);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const half8_t wv = weights_of(word[b][s]);
+          const float sc = half_bits_to_float((s & 1) ? v.s[b][s >> 1] >> 16 : v.s[b][s >> 1] & 0xffffu);
+          float4_t d[MT];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[t], wv, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[b][t][r] = fmaf(sc, d[t][r], acc[b][t][r]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        half8_t xa[2][MT];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) xa[i][t] = operand(t, 2 * h + i);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          float4_t d[MT];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) d[t] = ROW ? acc[b][t] : (float4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            half2_t w[4];
+            unpack_int8_word(word[b][4 * h + 2 * i], w);
+            unpack_int8_word(word[b][4 * h + 2 * i + 1], w + 2);
+            const half8_t wv = join8(w);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[i][t], wv, d[t], 0, 0, 0);
+          }
+          if constexpr (ROW) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[b][t] = d[t];
+          } else {
+            const float sc = half_bits_to_float(v.s[b][h]);
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[b][t][r] = fmaf(sc, d[t][r], acc[b][t][r]);
+          }
+        }
+      }
+    }
+  };
+
+  // Every load below is unconditional (a wait at a join would count it as not issued); the
+  // patch is the wave's own, and a wave's LDS accesses stay in order.
+  if constexpr (XD == 0) {  // one step of either
+    Weights w;
+    Rows x;
+    load_x(x, wave);
+    load_w(w, wave);
+    for (int st = wave; st < steps; st += kWaves) {
+      lay_x(x);
+      load_x(x, st + kWaves);
+      multiply(w);
+      load_w(w, st + kWaves);
+    }
+  } else {
+    Weights w0, w1;
+    Rows x0, x1;
+    load_x(x0, wave);
+    load_w(w0, wave);
+    if constexpr (XD == 2) load_x(x1, wave + kWaves);
+    load_w(w1, wave + kWaves);
+    for (int st = wave; st < steps; st += 2 * kWaves) {
+      lay_x(x0);
+      if constexpr (XD == 2) load_x(x0, st + 2 * kWaves);
+      else load_x(x0, st + kWaves);
+      multiply(w0);
+      if (st + kWaves >= steps) break;
+      load_w(w0, st + 2 * kWaves);
+      if constexpr (XD == 2) {
+        lay_x(x1);
+        load_x(x1, st + 3 * kWaves);
+      } else {
+        lay_x(x0);
+        load_x(x0, st + 2 * kWaves);
+      }
+      multiply(w1);
+      load_w(w1, st + 3 * kWaves);
+    }
+  }
+
+  // ---- the waves' sums, in order, and the epilogue ---------------------------------------
+  lds_barrier();  // every wave has read its patch
+  float* const sums = (float*)lds;  // [wave][row tile][block][16 x 16]
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sums[((wave * MT + t) * NB + b) * 256 + (4 * g + r) * 16 + nl] = acc[b][t][r];
+  lds_barrier();
+  float factor = a.scale_mul * a.alpha;
+#pragma unroll
+  for (int e0 = 0; e0 < MT * NB * 64; e0 += kWaves * 64) {
+    const int e = e0 + tid, row = e / (4 * NB), c = e % (4 * NB) * 4;  // four columns of a row
+    if (e >= MT * NB * 64 || row >= a.m || n0 + c >= a.n) continue;
+    const float* p = sums + ((row >> 4) * NB + (c >> 4)) * 256 + (row & 15) * 16 + (c & 15);
+    float4_t part[kWaves];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) part[w] = *(const float4_t*)(p + w * (MT * NB * 256));
+    float4_t sum = part[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] += part[w][i];
+    const int col = n0 + c;
+    const int64_t at = (int64_t)row * a.n + col;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int ci = min(col + i, a.n - 1) - col;  // past the last column: that one again, not stored
+      float f = factor;
+      if constexpr (ROW) f *= ((const float*)a.scales)[col + ci];
+      v[i] = apply_epilogue(a.epi, sum[i] * f, col + ci, at + ci);
+    }
+    if (a.vec_ok) {  // N a multiple of 4, rows aligned
+      if (a.y_dtype == TLHIP_F16) *(half4_t*)((_Float16*)a.y + at) = (half4_t){(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+      else *(float4_t*)((float*)a.y + at) = (float4_t){v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (col + i < a.n) store_out(a.y, a.y_dtype, at + i, v[i]);
+    }
+  }
+}
+
+int row_tiles_of(int64_t m) { return (int)((m + 15) / 16); }
+// The column blocks whose instance fits 256 registers a lane without spilling.
+constexpr int most_columns(int format, int mt) {
+  return format == TLHIP_FMT_INT8_GROUPED ? (mt == 2 ? 4 : (mt == 3 ? 3 : 2)) : (format == TLHIP_FMT_INT8_ROW ? (mt == 4 ? 3 : 4) : (mt == 4 ? 3 : 4));
+}
+
+template <int FMT, int MT, int NB>
+const void* instance() {
+  if constexpr (NB > most_columns(FMT, MT)) {
+    return nullptr;
+  } else {
+    // X two steps ahead where the registers allow it
+    constexpr int used = MT * 32 + NB * MT * 4 + NB * (FMT == TLHIP_FMT_INT4_GROUPED ? 12 : 24) + 40;
+    constexpr bool full = FMT == TLHIP_FMT_INT4_GROUPED && MT * NB >= 12;
+    return (const void*)gemm_rows_kernel<FMT, MT, NB, (full ? 0 : (used <= 200 ? 2 : 1))>;
+  }
+}
+template <int FMT, int MT>
+const void* instance_of(int nb) {
+  return nb == 1 ? instance<FMT, MT, 1>() : (nb == 2 ? instance<FMT, MT, 2>() : (nb == 3 ? instance<FMT, MT, 3>() : instance<FMT, MT, 4>()));
+}
+template <int FMT>
+const void* instance_of(int mt, int nb) {
+  return mt == 2 ? instance_of<FMT, 2>(nb) : (mt == 3 ? instance_of<FMT, 3>(nb) : instance_of<FMT, 4>(nb));
+}
+const void* instance_of(int format, int mt, int nb) {
+  return format == TLHIP_FMT_INT4_GROUPED ? instance_of<TLHIP_FMT_INT4_GROUPED>(mt, nb)
+         : format == TLHIP_FMT_INT8_ROW   ? instance_of<TLHIP_FMT_INT8_ROW>(mt, nb)
+                                          : instance_of<TLHIP_FMT_INT8_GROUPED>(mt, nb);
+}
+
+size_t lds_of(int mt, int nb) {
+  return std::max((size_t)kWaves * mt * 16 * kRowBytes, (size_t)kWaves * mt * nb * 1024);
+}
+
+}  // namespace
+
+bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
+  if (c.variant != VARIANT_GEMV_MFMA || c.p4 < 1 || c.p4 > kMaxCols) return false;
+  if (p.x_dtype != TLHIP_F16 || p.m < 17 || p.m > 64 || p.pro.kind != TLHIP_PRO_NONE) return false;
+  if (c.p4 > most_columns(p.format, row_tiles_of(p.m))) return false;
+  if (p.k <= 0 || p.k % kStep != 0 || p.k > (1 << 23)) return false;  // offsets below 2^31: 64 rows of X or of weights
+  if (p.format == TLHIP_FMT_INT4_GROUPED) return p.group_size == 32;
+  return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
+}
+
+// The cheapest number of column blocks and its time in microseconds, or false.  Measured at
+// 1024..28672 x 4096..12288 (int4-32, int8-64, int8-row): 3.5 us of launch, first operands and
+// last sums, and per round of workgroups and 4096 of K the figure below; int8 a tenth more.
+// A block more costs a workgroup 2.5-4 us, sixteen rows more 1.5-3 us, whatever the chip has to
+// do beside it: few blocks until the workgroups no longer fit the CUs at once.
+// Not the instances that want more than 256 registers (four tiles of rows: three blocks of
+// int8 groups, four of anything).
+bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
+  static const double walk[3][kMaxCols] = {{6.4, 9.1, 11.6, 14.0}, {8.2, 10.8, 13.7, 16.2}, {10.0, 12.2, 17.5, 23.0}};
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  bool found = false;
+  for (int nb = 1; nb <= kMaxCols; ++nb) {
+    tlhip_kernel_config_t c;
+    memset(&c, 0, sizeof c);
+    c.variant = VARIANT_GEMV_MFMA;
+    c.p0 = kWaves;
+    c.p4 = nb;
+    if (!is_rows_config(p, c)) continue;
+    const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb), rounds = (wgs + cus - 1) / cus;
+    const double t = 3.5 + (double)rounds * (double)p.k / 4096.0 * walk[row_tiles_of(p.m) - 2][nb - 1] * (p.format == TLHIP_FMT_INT4_GROUPED ? 1.0 : 1.1);
+    if (found && t >= *us) continue;
+    *out = c;
+    *us = t;
+    found = true;
+  }
+  return found;
+}
+
+int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream) {
+  if (!is_rows_config(p, c)) return set_error(TLHIP_ERR_INVALID, "gemm_rows: config not applicable");
+  if (p.n == 0 || p.m == 0) return TLHIP_OK;
+  RowsArgs a;
+  memset(&a, 0, sizeof a);
+  a.packed = (const uint8_t*)p.packed;
+  a.scales = (const uint8_t*)p.scales;
+  a.x = (const _Float16*)p.x;
+  a.y = p.y;
+  a.m = (int)p.m;
+  a.n = (int)p.n;
+  a.k = (int)p.k;
+  a.row_bytes = (int)(p.format == TLHIP_FMT_INT4_GROUPED ? p.k / 2 : p.k);
+  a.scale_row_bytes = p.format == TLHIP_FMT_INT8_ROW ? 4 : (int)(p.k / p.group_size) * 2;
+  a.group_shift = p.format == TLHIP_FMT_INT8_GROUPED ? __builtin_ctz((unsigned)(p.group_size / 64)) : 0;
+  a.alpha = p.alpha;
+  a.scale_mul = p.format == TLHIP_FMT_INT8_GROUPED ? 1.0f / 127.0f : 1.0f;
+  a.y_dtype = p.y_dtype;
+  a.vec_ok = p.n % 4 == 0 && ((uintptr_t)p.y & 15) == 0;
+  a.epi = p.epi;
+  void* args[] = {(void*)&a};
+  const int mt = row_tiles_of(p.m), nb = c.p4;
+  const int rc = launch_kernel(instance_of(p.format, mt, nb), dim3((unsigned)((p.n + 16 * nb - 1) / (16 * nb))), dim3(kWaves * 64), args,
+                               lds_of(mt, nb), stream);
+  if (rc) return rc;
+  count_gemv_dispatch();
+  return TLHIP_OK;
+}
+
+// Every instance launch_gemm_rows can reach, in prepare mode (see launch_kernel).
+int prepare_gemm_rows_kernels() {
+  for (int format : {TLHIP_FMT_INT4_GROUPED, TLHIP_FMT_INT8_GROUPED, TLHIP_FMT_INT8_ROW})
+    for (int mt = 2; mt <= 4; ++mt)
+      for (int nb = 1; nb <= most_columns(format, mt); ++nb) {
+        const int rc = launch_kernel(instance_of(format, mt, nb), dim3(1), dim3(64), nullptr, 0, nullptr);
+        if (rc) return rc;
+      }
+  return TLHIP_OK;
+}
+
+}  // namespace tlhip

@@ -110,7 +110,7 @@ static bool mfma_applicable(const Problem& p, int64_t nblocks, const tlhip_kerne
 }
 
 bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why) {
-  return mfma_applicable(p, (p.n + 15) / 16, c, why);
+  return is_rows_config(p, c) || mfma_applicable(p, (p.n + 15) / 16, c, why);
 }
 
 // The problems of a group: same activations and rows, one shape class; N, pointers and
@@ -207,6 +207,7 @@ int launch_gemv_mfma(const Problem& p, const tlhip_kernel_config_t& c, hipStream
   if (!gemv_mfma_config_applicable(p, c, &why))
     return set_error(TLHIP_ERR_INVALID, "gemv_mfma: config not applicable: %s", why);
   if (p.n == 0 || p.m == 0) return TLHIP_OK;
+  if (is_rows_config(p, c)) return launch_gemm_rows(p, c, stream);
   return launch_gemv_mfma_group(&p, 1, c, stream);
 }
 

@@ -201,6 +201,7 @@ int prepare_all_kernels() {
   if (!rc) rc = prepare_gemv_xreg_kernels();
   if (!rc) rc = prepare_gemv_wave_kernels();
   if (!rc) rc = prepare_gemv_f32_kernels();
+  if (!rc) rc = prepare_gemm_rows_kernels();
   if (!rc) rc = prepare_gemv_seq_kernels();
   if (!rc) rc = prepare_gemm_kernels();
   if (!rc) rc = prepare_gemm_direct_kernels();
