@@ -120,3 +120,15 @@ def test_topk_errors(be):
         be.readTopK(t, 0)
     with pytest.raises(ValueError, match="range"):
         be.readTopK(t, 2, offset=8, length=5)
+
+
+@pytest.mark.parametrize("k", [1, 3, 63, 64, 65, 255, 256])
+@pytest.mark.parametrize("n", [4097, 70001, 131072, 135169])  # 2, 18, 32 and 34 chunks: 2, 8 or 16 keys a thread at the end
+def test_topk_of_runs_that_pass_the_bound_together(be, n, k):
+    """Sorted, constant and stepped rows: whole groups of neighbours pass the bound, or none but k do."""
+    v0 = np.linspace(-3, 5, n).astype(np.float32)
+    for v in (v0, v0[::-1].copy(), np.full(n, 2.5, np.float32), np.floor(v0 * 4) / 4):
+        vals, idx = be.readTopK(be.ops.tensorFromArray(v, [n], "f32"), k)
+        want_v, want_i = reference_topk(v, k)
+        assert np.array_equal(idx, want_i)
+        assert np.array_equal(vals, want_v)

@@ -15,6 +15,8 @@
 // (topk_select_kernel), and up to 8192 surviving keys the workgroup that arrives last does
 // the last level in the same launch: 256 000 logits at k = 64 are 63 workgroups and one
 // launch.  Above k = 256 a bitonic sort in LDS (topk_sort_kernel).
+#include <type_traits>
+
 #include "device_utils.h"
 
 namespace tlhip {
@@ -42,20 +44,21 @@ constexpr int kSelectFused = 8192;      // keys the last workgroup reduces in th
 
 __device__ __forceinline__ uint64_t max_key(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-// The largest bound (of those tried) that at least `k` of the wave's 64 * R values reach.
-// One bit per step; a step that leaves exactly k values ends the search.
+// A bound that at least `k` of the wave's 64 * R values reach: the first one tried that no more
+// than `most` reach (`enough`), else the largest.  One bit per step, a chain of 60 clocks; `most`
+// a quarter above k saves about eight of twenty steps and lets a few more keys pass.
 template <int R>
-__device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool (&in)[R], int k, bool* exact) {
+__device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool (&in)[R], int k, int most, bool* enough) {
   uint32_t bound = 0;
-  *exact = false;
+  *enough = false;
   for (int bit = 31; bit >= 0; --bit) {
     const uint32_t trial = bound | (1u << bit);
     int count = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) count += __popcll(__ballot(in[r] && v[r] >= trial));
     if (count >= k) bound = trial;
-    if (count == k) {
-      *exact = true;
+    if (count >= k && count <= most) {
+      *enough = true;
       break;
     }
   }
@@ -66,9 +69,10 @@ __device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool 
 // emit(rank, key); ranks without a key get 0.  Returns with every thread past its LDS reads.
 //   1. the maximum of every group of 4 threads (G = 128) or thread (G = 512);
 //   2. a bound that k of the G maxima reach, hence at least k keys: for k = 64 of 4096
-//      random keys about 90 do, at worst k groups' whole contents (4096);
-//   3. the keys from the bound on, collected in LDS; the rank of each is the number of
-//      larger ones.
+//      random keys about 100 do, at worst the whole contents of the groups that reach it (4096);
+//   3. the keys from the bound on, collected in LDS (a wave counts its own by ballots and takes
+//      its places with one atomic: an atomic a key was a chain of E round trips to LDS); the rank
+//      of each is the number of larger ones, counted by four threads.
 template <int G, int E, typename Emit>
 __device__ __forceinline__ void select_keys(const uint64_t (&key)[E], int k, uint64_t* maxima, uint64_t* found, int* n_found, Emit emit) {
   constexpr int R = G / 64;
@@ -94,30 +98,45 @@ __device__ __forceinline__ void select_keys(const uint64_t (&key)[E], int k, uin
     lo[r] = (uint32_t)m;
     in[r] = true;
   }
-  bool exact;
-  const uint32_t bound_hi = bound_of<R>(hi, in, k, &exact);
+  constexpr int kMostGroups = kTopkChunk / (E * kSelectThreads / G);  // whose whole contents `found` holds
+  const int most = min(k + k / 4, kMostGroups) > k ? min(k + k / 4, kMostGroups) : k;
+  bool enough;
+  const uint32_t bound_hi = bound_of<R>(hi, in, k, most, &enough);
   uint32_t bound_lo = 0;
-  if (!exact) {  // equal values around the bound: the index decides
+  if (!enough) {  // equal values around the bound: the index decides
     int larger = 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       larger += __popcll(__ballot(hi[r] > bound_hi));
       in[r] = hi[r] == bound_hi;
     }
-    bound_lo = bound_of<R>(lo, in, k - larger, &exact);
+    bound_lo = bound_of<R>(lo, in, k - larger, most - larger, &enough);
   }
   const uint64_t bound = ((uint64_t)bound_hi << 32) | bound_lo;
+  int mine = 0;  // of the wave
 #pragma unroll
-  for (int e = 0; e < E; ++e)
-    if (key[e] != 0 && key[e] >= bound) found[atomicAdd(n_found, 1)] = key[e];
+  for (int e = 0; e < E; ++e) mine += __popcll(__ballot(key[e] != 0 && key[e] >= bound));
+  int at = 0;
+  if (lane == 0 && mine) at = atomicAdd(n_found, mine);
+  at = __shfl(at, 0);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const bool hit = key[e] != 0 && key[e] >= bound;
+    const uint64_t hits = __ballot(hit);
+    if (hit) found[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(hits >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u))] = key[e];
+    at += __popcll(hits);
+  }
   __syncthreads();
   const int c = *n_found;
-  for (int i = tid; i < c; i += kSelectThreads) {
-    const uint64_t mine = found[i];
+  for (int i0 = 0; i0 < c; i0 += kSelectThreads / 4) {
+    const int i = i0 + (tid >> 2);
+    const uint64_t own = found[min(i, c - 1)];
     int rank = 0;
 #pragma unroll 8
-    for (int j = 0; j < c; ++j) rank += found[j] > mine ? 1 : 0;
-    if (rank < k) emit(rank, mine);
+    for (int j = tid & 3; j < c; j += 4) rank += found[j] > own ? 1 : 0;
+    rank += __shfl_xor(rank, 1);
+    rank += __shfl_xor(rank, 2);
+    if ((tid & 3) == 0 && i < c && rank < k) emit(rank, own);
   }
   for (int i = c + tid; i < k; i += kSelectThreads) emit(i, (uint64_t)0);
   __syncthreads();
@@ -136,7 +155,9 @@ __device__ __forceinline__ void write_result(int i, uint64_t key, float* out_val
 // last reduces all of them to the result (gridDim.x * k <= kSelectFused); a launch of one
 // workgroup writes the result at once.
 // 256 000 logits, k = 64, 8 rows behind each other: 35 us a row with three launches of sorted
-// chunks of 1024 before, 14 us now.
+// chunks of 1024 at first, 14 us with this launch, 11.0 us since a bound may let a few more keys pass,
+// a wave takes its places with one atomic and four threads count a rank: what is left is the launch,
+// two loads of keys, the stores and the counter, each a round trip to memory behind the other.
 template <bool FROM_FLOAT, int G>
 __global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(const float* __restrict__ logits, int64_t offset,
                                                                      const uint64_t* __restrict__ keys_in, int64_t count, int k,
@@ -181,16 +202,22 @@ __global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(const float
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   if (arrived != (int)gridDim.x - 1) return;
   if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-  constexpr int E2 = kSelectFused / kSelectThreads;
   const int total = (int)gridDim.x * k;
-  uint64_t all[E2];
+  auto last = [&](auto per_thread) {
+    constexpr int E2 = decltype(per_thread)::value;
+    uint64_t all[E2];
 #pragma unroll
-  for (int e = 0; e < E2; ++e) {
-    const int at = e * kSelectThreads + (int)threadIdx.x;
-    const uint64_t v = __hip_atomic_load(keys_out + (at < total ? at : total - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    all[e] = at < total ? v : 0;
-  }
-  select_keys<G, E2>(all, k, maxima, found, &n_found, [&](int i, uint64_t v) { write_result(i, v, out_values, out_indices, index_dtype); });
+    for (int e = 0; e < E2; ++e) {
+      const int at = e * kSelectThreads + (int)threadIdx.x;
+      const uint64_t v = __hip_atomic_load(keys_out + (at < total ? at : total - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      all[e] = at < total ? v : 0;
+    }
+    select_keys<G, E2>(all, k, maxima, found, &n_found, [&](int i, uint64_t v) { write_result(i, v, out_values, out_indices, index_dtype); });
+  };
+  // as few keys a thread as hold them all
+  if (total <= 2 * kSelectThreads) last(std::integral_constant<int, 2>());
+  else if (total <= 8 * kSelectThreads) last(std::integral_constant<int, 8>());
+  else last(std::integral_constant<int, kSelectFused / kSelectThreads>());
 }
 
 // k above kSelectMaxK: the chunk sorted in LDS, its first k keys to keys_out[block * k ..] or,
