@@ -128,3 +128,19 @@ def test_loader_branch_quantizes_once_and_then_hits_the_cache(be, tmp_path, on_d
     # no cache at all still works
     T.loadQuantizedWeight(be, None, url, name, n, k, "int8-64", fetch, "f32", onDevice=on_device)
     assert len(fetched) == 3
+
+
+@pytest.mark.parametrize("g", [16, 32, 64, 128, 256, 512, 48])
+def test_device_quantizer_halves_of_the_maximum(be, g):
+    """w = +-max/2 is +-63.5 only after w * inv is rounded: where inv lies below 127/max the exact
+    product does not reach the half.  Every f16 significand as a maximum; rows that end in a part of
+    a workgroup's piece, and NaN and infinity beside them."""
+    n, k = 1024, 3 * g
+    s = (1.0 + np.arange(n) / 1024.0).astype(np.float32) * np.float32(2.0) ** ((np.arange(n) % 9) - 12)
+    w = np.random.default_rng(g).uniform(-0.9, 0.9, (n, k)).astype(np.float32) * s[:, None]
+    w[:, 0::g], w[:, 1::g], w[:, 2::g] = s[:, None], s[:, None] / 2, -s[:, None] / 2
+    w[5, 3], w[6, 4], w[7, g + 5] = np.nan, np.inf, -np.inf
+    _, packed, scales = device_quantize(be, w, g)
+    want_packed, want_scales = O.quantize_int8_grouped(w.ravel(), n, k, g)
+    assert np.array_equal(scales, want_scales)
+    assert np.array_equal(packed, want_packed)

@@ -4,13 +4,17 @@
 // product, Math.round ties toward +infinity, the reference's f16 encoder with
 // its round-half-up subnormals).
 //
-// One workgroup per weight row at a time.  Pass 1: each thread takes 16-byte
-// pieces (4 weights = one packed word) and folds |w| into the group's maximum in
-// LDS with an unsigned atomic max on the float bits (non-negative floats order
-// like their bit patterns; NaN is skipped, as `a > max` is false for NaN in the
-// reference).  Pass 2: scale bits from the maximum, then the packed words.
-// HBM-bound: 4 bytes read (twice; the second read hits L2) and 1 + 2/G written
-// per weight.
+// HBM-bound: 4 bytes read and 1 + 2/G written per weight, if the f64 arithmetic keeps up.
+// quantize_int8_groups_kernel (groups of 16..256, a power of two): a lane holds 4 weights of a
+// group in registers, the lanes of a group find its maximum by exchanges, and one lane of four
+// divides for each of the wave's four pieces in flight: one read, no LDS, no barrier, a quarter of
+// a division per 4 weights.  quantize_int8_grouped_kernel (any other group size): one workgroup
+// per weight row at a time, the group's maximum in LDS by an unsigned atomic max on the float bits
+// (non-negative floats order like their bit patterns; NaN is skipped, as `a > max` is false for
+// NaN in the reference), the weights read twice, a division per 4 weights.  12288 x 4096 in groups
+// of 64: 81.8 us with the latter, 45.7 us (5.5 TB/s) with the former.
+#include <type_traits>
+
 #include "device_utils.h"
 
 namespace tlhip {
@@ -43,18 +47,73 @@ __device__ __forceinline__ double decode_f16_ref(uint32_t h) {
   return ldexp((double)(1024 + f), e - 25);
 }
 
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+
 __device__ __forceinline__ uint32_t quantize_one(float w, double inv) {
+#pragma clang fp contract(off)  // t is the rounded product, in t - f as well
   const double t = (double)w * inv;
-  int q = 0;  // NaN -> 0 (NaN & 0xff in JavaScript)
-  if (t == t) {
-    double rr = t;
-    if (!__builtin_isinf(t)) {
-      const double f = floor(t);
-      rr = (t - f >= 0.5) ? f + 1.0 : f;  // Math.round
-    }
-    q = rr > 127.0 ? 127 : (rr < -127.0 ? -127 : (int)rr);
-  }
+  // Math.round: up from a half on.  f beyond the integers saturates, t - f of an infinity is NaN;
+  // the clamp before the step keeps it from overflowing.
+  const double f = floor(t);
+  int q = t == t ? (int)fmin(fmax(f, -128.0), 127.0) : 0;  // NaN -> 0 (NaN & 0xff in JavaScript)
+  q += t - f >= 0.5 ? 1 : 0;
+  q = q > 127 ? 127 : (q < -127 ? -127 : q);
   return (uint32_t)q & 0xffu;
+}
+
+// LANES: lanes of a group (4 weights each)
+template <int LANES>
+__global__ __launch_bounds__(256) void quantize_int8_groups_kernel(const float4_t* __restrict__ w, int64_t n_words,
+                                                                  uint32_t* __restrict__ packed, uint16_t* __restrict__ scales) {
+  constexpr int U = 4;
+  const int64_t stride = (int64_t)gridDim.x * (256 * U);
+  const int quad = threadIdx.x & 3;
+  for (int64_t first = (int64_t)blockIdx.x * (256 * U); first < n_words; first += stride) {
+    const int64_t base = first + threadIdx.x;
+    float4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = __builtin_nontemporal_load(w + (base + u * 256 < n_words ? base + u * 256 : n_words - 1));
+    uint32_t top = 0;  // of the piece this lane divides for
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float m = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = fabsf(v[u][e]);
+        if (a > m) m = a;  // false for NaN
+      }
+      uint32_t t = __builtin_bit_cast(uint32_t, m);  // non-negative floats order like their bits
+      t = max(t, dpp<0xB1>(t));   // quad_perm [1,0,3,2]
+      t = max(t, dpp<0x4E>(t));   // quad_perm [2,3,0,1]
+      if (LANES >= 8) t = max(t, dpp<0x141>(t));   // row_half_mirror
+      if (LANES >= 16) t = max(t, dpp<0x140>(t));  // row_mirror
+      if (LANES >= 32) t = max(t, (uint32_t)__shfl_xor((int)t, 16));
+      if (LANES >= 64) t = max(t, (uint32_t)__shfl_xor((int)t, 32));
+      top = u == quad ? t : top;
+    }
+    const uint32_t sbits = encode_f16_ref(__builtin_bit_cast(float, top));
+    const double s = (double)half_bits_to_float(sbits);  // exact, never NaN
+    const uint64_t inv_bits = __builtin_bit_cast(uint64_t, s > 0 ? 127.0 / s : 0.0);
+    const uint32_t lo = (uint32_t)inv_bits, hi = (uint32_t)(inv_bits >> 32);
+    auto piece = [&](auto which) {
+      constexpr int P = decltype(which)::value, FROM = P * 0x55;  // quad_perm [P,P,P,P]
+      const double inv = __builtin_bit_cast(double, ((uint64_t)dpp<FROM>(hi) << 32) | dpp<FROM>(lo));
+      const uint32_t scale = dpp<FROM>(sbits);
+      const int64_t i = base + P * 256;
+      if (i < n_words) {
+        packed[i] = quantize_one(v[P][0], inv) | (quantize_one(v[P][1], inv) << 8) | (quantize_one(v[P][2], inv) << 16) |
+                    (quantize_one(v[P][3], inv) << 24);
+        if ((threadIdx.x & (LANES - 1)) == 0) scales[i / LANES] = (uint16_t)scale;
+      }
+    };
+    piece(std::integral_constant<int, 0>());
+    piece(std::integral_constant<int, 1>());
+    piece(std::integral_constant<int, 2>());
+    piece(std::integral_constant<int, 3>());
+  }
 }
 
 __global__ __launch_bounds__(256) void quantize_int8_grouped_kernel(const float* __restrict__ w, int64_t n, int k,
@@ -116,6 +175,19 @@ extern "C" int tlhip_quantize_int8_grouped_device(const float* weight, int64_t n
   if (lds > 64 * 1024)
     return set_error(TLHIP_ERR_INVALID, "quantize (device): %lld groups per row do not fit LDS",
                      (long long)(k / group_size));
+  const int lanes = (int)group_size / 4;
+  if (group_size >= 16 && group_size <= 256 && (group_size & (group_size - 1)) == 0) {
+    const int64_t words = n * (k / 4), blocks = (words + 1023) / 1024;
+    auto kernel = lanes == 4    ? quantize_int8_groups_kernel<4>
+                  : lanes == 8  ? quantize_int8_groups_kernel<8>
+                  : lanes == 16 ? quantize_int8_groups_kernel<16>
+                  : lanes == 32 ? quantize_int8_groups_kernel<32>
+                                : quantize_int8_groups_kernel<64>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(blocks < (1 << 20) ? blocks : (1 << 20))), dim3(256), 0, resolve_stream(stream),
+                       (const float4_t*)weight, words, packed, scales);
+    TLHIP_CHECK_HIP(hipGetLastError());
+    return TLHIP_OK;
+  }
   const int64_t cap = (int64_t)device_cu_count() * 8;
   const int grid = (int)(n < cap ? n : cap);
   hipLaunchKernelGGL(quantize_int8_grouped_kernel, dim3(grid), dim3(256), lds, resolve_stream(stream), weight, n,
