@@ -443,7 +443,8 @@ int tlhip_topk(const float* logits, int64_t offset, int64_t length, int k, float
  * (M, N, waves M, waves N) 256x256 2x4, 256x192 2x4, 256x128 4x2, 128x128 2x4, 64x128 2x4, K a
  * multiple of 64, every format with groups of 32 (int4) or 64 (int8) times a power of two),
  * 6 = "gemv_f32" (f32 activations, 1..16 rows, each value cut into three bf16 pieces on the
- * matrix cores: p0 K slices across workgroups, 1..64),
+ * matrix cores: p0 K slices across workgroups, 1..64; with p0 = 8 and p1 = 1, 2 or 4 all of K in one
+ * workgroup of 16 p1 columns, K a multiple of 128 up to 16384, int4 in groups of 32),
  * 4 = "gemv_mfma_xreg" (skinny MFMA for int4 g32 with the activations held in
  * registers: p0 waves per workgroup, p1 iterations in flight, p2 workgroups per
  * CU, p3 K slices across workgroups, p4 = 1: every weight load of a wave issued

@@ -84,3 +84,21 @@ def test_subnormal_activations(be, fmt, g):
     want, magnitudes = x.astype(np.float64) @ deq.astype(np.float64).T, np.abs(x).astype(np.float64) @ d.T
     assert np.any(want[4] != 0)
     assert np.all(np.abs(got - want) <= 2.0**-21 * magnitudes + 2.0**-133 * d.sum(1) + 2.0**-145)
+
+
+@pytest.mark.parametrize("fmt,g", [("int4-grouped", 32), ("int8-grouped", 64), ("int8-grouped", 256), ("int8-row", 0)])
+@pytest.mark.parametrize("m", [1, 2, 5, 6, 10, 11, 16])
+@pytest.mark.parametrize("n,k", [(1, 256), (131, 1280), (300, 2304)])  # one column; ten and eighteen steps on eight waves
+def test_all_of_k_in_one_workgroup(be, fmt, g, m, n, k):
+    rng = np.random.default_rng(m * 1000 + n + k + g)
+    packed, scales, deq = make_weight(fmt, n, k, g, rng)
+    w = be.createQuantizedWeight(packed, scales, n, k, T.resolveWeightFormat(fmt_name(fmt, g), "f32"))
+    x = make_x(m, k, "f32", rng, std=0.5)
+    bias, other = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    xt, bt, ot = be.ops.tensorFromArray(x, [m, k], "f32"), be.ops.tensorFromArray(bias, [n], "f32"), be.ops.tensorFromArray(other, [m, n], "f32")
+    ep = be.makeEpilogueChain([("bias", bt), ("binary", "add", ot)])
+    want = x.astype(np.float64) @ deq.astype(np.float64).T + bias + other
+    magnitudes = np.abs(x).astype(np.float64) @ np.abs(deq).astype(np.float64).T + np.abs(bias) + np.abs(other)
+    for cols in (1, 2, 4) if m <= 10 else (1, 2):
+        got = be._matmulQuantizedB(xt, be.ops.transpose(w), ep, L.KernelConfig.of(L.VARIANT_GEMV_F32, 8, cols)).numpy()
+        assert np.all(np.abs(got - want) <= 2.0**-21 * magnitudes), cols  # the bound of the K slices above

@@ -584,6 +584,9 @@ std::vector<tlhip_kernel_config_t> candidates(const Problem& p) {
     c.variant = VARIANT_GEMV_F32;
     c.p0 = slices;
     if (gemv_f32_config_applicable(p, c, nullptr)) out.push_back(c);
+    c.p0 = 8;
+    c.p1 = slices;  // all of K in one workgroup: 1, 2 or 4 blocks of 16 columns
+    if (slices <= 4 && gemv_f32_config_applicable(p, c, nullptr)) out.push_back(c);
   }
   if (p.m <= 16) {
     for (int lpr : {16, 32, 64})
@@ -851,7 +854,7 @@ bool f32_rows_through_tiled(const Problem& p, hipStream_t stream, int* rc) {
 // or the VALU kernel (f32 rows) without K slices, where the kernels that these two stand in for
 // needed no workspace: a first call under capture that such a problem may make goes through.
 tlhip_kernel_config_t config_at_hand(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream) {
-  const bool f32 = c.variant == VARIANT_GEMV_F32 && c.p0 > 1;
+  const bool f32 = c.variant == VARIANT_GEMV_F32 && c.p0 > 1 && !c.p1;
   if (p.scratch || !(f32 || (is_pipe_config(c) && c.p5 > 1)) || split_workspace_at_hand(stream)) return c;
   if (f32) return default_valu_config(p);
   tlhip_kernel_config_t wave, whole;
@@ -1119,6 +1122,7 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       break;
     case VARIANT_GEMV_F32:
       vary(0, {1, 2, 4, 8, 16, 32});
+      vary(1, {0, 1, 2, 4});
       break;
     case VARIANT_GEMV_WAVE:
       vary(0, {4, 8});

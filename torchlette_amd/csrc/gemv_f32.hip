@@ -285,6 +285,230 @@ __global__ __launch_bounds__(kThreads, 4) void gemv_f32_kernel(const F32Args a) 
     if (m_first + 4 * i < a.m) store_out(a.y, a.y_dtype, (int64_t)(m_first + 4 * i) * a.n + col, v[i]);
 }
 
+// ---- all of K in one workgroup ------------------------------------------------------------------
+// The same products where K slices across workgroups cost more than they give (the pieces of a
+// slice behind a barrier, then planes of partial sums through memory and a counter: 4-5 us of 9-17):
+// a workgroup owns 16 NB columns and all of K, which its eight waves take in turn, 128 at a time,
+// each cutting its own rows of X into pieces in a patch of LDS that belongs to it; they meet once.
+// No workspace.  What bounds it: the VALU, in cutting X (45 instructions for 4 values of a row, in
+// every workgroup: more columns share them) and in converting the weights.
+// One launch, us, K slices -> here: 5 rows of int8-64 at 9216 x 2304 13.0 -> 11.2, at 2304 x 9216 16.8 ->
+// 15.3, at 2048 x 2304 10.8 -> 5.8; 10 rows of int4 at 4096 x 4096 16.3 -> 11.3 (0.8 TB/s of weights).
+constexpr int kWhole = 8;                     // waves; the config's p0, with p1 blocks of 16 columns
+constexpr int kWholeStep = 128;
+constexpr int kWholeRow = kWholeStep * 2 + 16;  // bytes of a piece row in LDS
+constexpr int kWholeMaxCols = 4;
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t buffer_of(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ u32x4 load16(rsrc_t r, uint32_t at, uint32_t step_at) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, (int)step_at, 0));
+}
+
+template <int FMT, int T, int NB>
+__global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Args a) {
+  constexpr bool INT4 = FMT == TLHIP_FMT_INT4_GROUPED, ROW = FMT == TLHIP_FMT_INT8_ROW;
+  constexpr int WV = INT4 ? 1 : 2;         // 16-byte loads of a step, lane and column block
+  constexpr int XV = (16 * T / 3 + 1) / 2; // loads of X: two rows each
+  extern __shared__ u32x4 lds[];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int n0 = (int)blockIdx.x * (16 * NB);
+  const int cols = min(16 * NB, a.n - n0);
+  const int steps = a.k / kWholeStep;
+  const uint32_t row_bytes = (uint32_t)a.row_chunks * 16u, scale_row_bytes = ROW ? 4u : (uint32_t)a.groups_per_row * 2u;
+  const uint8_t* const packed = (const uint8_t*)a.packed + (int64_t)n0 * row_bytes;
+  const uint8_t* const scales = (const uint8_t*)a.scales + (int64_t)n0 * scale_row_bytes;
+
+  // Buffer loads: rows past M, columns past N and steps past K read zero and cost no traffic, so
+  // that no load stands under a branch.  A lane's place in a step is fixed, the step is a scalar
+  // offset (opaque, or the compiler keeps it in a vector register and loops over the lanes); past
+  // the last step a buffer of no bytes at offset 0.
+  struct Weights {
+    u32x4 w[NB][WV];
+    uint32_t s[NB][2];
+  };
+  auto scalar_step = [&](int st) {
+    st = st < steps ? st : -1;
+    asm("" : "+s"(st));
+    return st;
+  };
+  auto load_w = [&](Weights& v, int step) {
+    const int st = scalar_step(step);
+    const uint32_t in = ~(uint32_t)(st >> 31), at = (uint32_t)st & in;
+    const rsrc_t wb = buffer_of(packed, (uint32_t)cols * row_bytes & in), sb = buffer_of(scales, (uint32_t)cols * scale_row_bytes & in);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const uint32_t row = (uint32_t)(16 * b + l16);
+#pragma unroll
+      for (int i = 0; i < WV; ++i) v.w[b][i] = load16(wb, row * row_bytes + (uint32_t)lg * 16u + (uint32_t)i * 64u, at * (WV * 64u));
+      if constexpr (INT4) {
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 s = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sb, (int)(row * scale_row_bytes), (int)(at * 8u), 0));
+        v.s[b][0] = s.x;
+        v.s[b][1] = s.y;
+      } else if constexpr (!ROW) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          v.s[b][h] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sb, (int)(row * scale_row_bytes), (int)(((2u * at + (uint32_t)h) >> a.group_shift) * 2u), 0);
+      }
+    }
+  };
+  struct Rows {
+    u32x4 v[XV];
+  };
+  const int half = lane >> 5, unit = lane & 31;
+  auto load_x = [&](Rows& r, int step) {
+    const int st = scalar_step(step);
+    const uint32_t in = ~(uint32_t)(st >> 31), at = (uint32_t)st * (kWholeStep * 4u) & in;
+#pragma unroll
+    for (int i = 0; i < XV; ++i)
+      r.v[i] = load16(buffer_of(a.x + (int64_t)(2 * i) * a.k, (uint32_t)max(a.m - 2 * i, 0) * (uint32_t)a.k * 4u & in),
+                      (uint32_t)half * (uint32_t)a.k * 4u + (uint32_t)unit * 16u, at);
+  };
+  char* const patch = (char*)lds + wave * (16 * T * kWholeRow);
+  auto cut = [&](const Rows& r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+      const int row = 2 * i + half;
+      uint32_t p[4][3];
+      pieces_of(r.v[i].x, p[0]);
+      pieces_of(r.v[i].y, p[1]);
+      pieces_of(r.v[i].z, p[2]);
+      pieces_of(r.v[i].w, p[3]);
+      if (row < a.m) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const uint64_t v = (uint64_t)upper_halves(p[0][q], p[1][q]) | ((uint64_t)upper_halves(p[2][q], p[3][q]) << 32);
+          *(uint64_t*)(patch + (row * 3 + q) * kWholeRow + unit * 8) = v;
+        }
+      }
+    }
+  };
+  float4_t acc[NB][T];
+  const char* arow[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    arow[t] = patch + min(t * 16 + l16, a.m * 3 - 1) * kWholeRow + lg * (INT4 ? 16 : 32);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b][t] = (float4_t){0.f, 0.f, 0.f, 0.f};
+  }
+  auto multiply = [&](const Weights& v) __attribute__((always_inline)) {
+    bf16x8 xa[4][T];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < T; ++t) xa[i][t] = __builtin_bit_cast(bf16x8, *(const u32x4*)(arow[t] + (INT4 ? 64 * i : 128 * (i >> 1) + 16 * (i & 1))));
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      uint32_t words[4 * WV];
+#pragma unroll
+      for (int i = 0; i < WV; ++i) {
+        words[4 * i + 0] = v.w[b][i].x;
+        words[4 * i + 1] = v.w[b][i].y;
+        words[4 * i + 2] = v.w[b][i].z;
+        words[4 * i + 3] = v.w[b][i].w;
+      }
+      if constexpr (INT4) transpose4(words[0], words[1], words[2], words[3]);
+      float4_t chain[T], sum[T];  // a step's own sum first: the long one takes a step at a time
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t wb[4];
+        if constexpr (INT4) {
+          weight_bf16<FMT>(words[i], wb);
+        } else {
+          weight_bf16<FMT>(words[2 * i], wb);
+          weight_bf16<FMT>(words[2 * i + 1], wb + 2);
+        }
+        const bf16x8 wv = __builtin_bit_cast(bf16x8, (u32x4){wb[0], wb[1], wb[2], wb[3]});
+        constexpr int GROUP = INT4 ? 1 : (ROW ? 4 : 2);  // products of one scale
+        const bool first = i % GROUP == 0, last = i % GROUP == GROUP - 1;
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          chain[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][t], wv, first ? (float4_t){0.f, 0.f, 0.f, 0.f} : chain[t], 0, 0, 0);
+        if (last) {
+          const float s = ROW ? 1.f : half_bits_to_float(INT4 ? ((i & 1) ? v.s[b][i >> 1] >> 16 : v.s[b][i >> 1] & 0xffffu) : v.s[b][i >> 1]);
+#pragma unroll
+          for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[t][e] = ROW ? chain[t][e] : (i < GROUP ? s * chain[t][e] : fmaf(s, chain[t][e], sum[t][e]));
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[b][t][e] += sum[t][e];
+    }
+  };
+
+  Weights w0, w1;
+  Rows x0, x1;
+  load_x(x0, wave);
+  load_w(w0, wave);
+  load_x(x1, wave + kWhole);
+  load_w(w1, wave + kWhole);
+  for (int st = wave; st < steps; st += 2 * kWhole) {
+    cut(x0);
+    load_x(x0, st + 2 * kWhole);
+    multiply(w0);
+    if (st + kWhole >= steps) break;
+    load_w(w0, st + 2 * kWhole);
+    cut(x1);
+    load_x(x1, st + 3 * kWhole);
+    multiply(w1);
+    load_w(w1, st + 3 * kWhole);
+  }
+
+  lds_barrier();  // every wave has read its patch
+  float* const sums = (float*)lds;  // [wave][tile][block][16 x 16]
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sums[((wave * T + t) * NB + b) * 256 + (4 * lg + e) * 16 + l16] = acc[b][t][e];
+  lds_barrier();
+  for (int e = tid; e < a.m * (16 * NB); e += kWhole * 64) {
+    const int row = e / (16 * NB), c = e % (16 * NB), col = n0 + c;
+    if (col >= a.n) continue;
+    float part[kWhole];
+#pragma unroll
+    for (int w = 0; w < kWhole; ++w) {
+      float p[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int r = row * 3 + q;
+        p[q] = sums[((w * T + (r >> 4)) * NB + (c >> 4)) * 256 + (r & 15) * 16 + (c & 15)];
+      }
+      part[w] = p[0] + (p[1] + p[2]);
+    }
+    const float v = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    const float factor = ROW ? ((const float*)a.scales)[col] * a.scale_mul : a.scale_mul;
+    const int64_t at = (int64_t)row * a.n + col;
+    store_out(a.y, a.y_dtype, at, apply_epilogue(a.epi, v * factor * a.alpha, col, at));
+  }
+}
+
+template <int FMT, int T>
+const void* whole_fn(int nb) {
+  return nb == 1   ? (const void*)gemv_f32_whole_kernel<FMT, T, 1>
+         : nb == 2 ? (const void*)gemv_f32_whole_kernel<FMT, T, 2>
+                   : (const void*)gemv_f32_whole_kernel<FMT, T, (T < 3 ? 4 : 2)>;  // three tiles of pieces and four blocks: more registers than a lane has
+}
+template <int FMT>
+const void* whole_fn(int tiles, int nb) {
+  return tiles == 1 ? whole_fn<FMT, 1>(nb) : (tiles == 2 ? whole_fn<FMT, 2>(nb) : whole_fn<FMT, 3>(nb));
+}
+const void* whole_fn(int format, int tiles, int nb) {
+  return format == TLHIP_FMT_INT4_GROUPED ? whole_fn<TLHIP_FMT_INT4_GROUPED>(tiles, nb)
+         : format == TLHIP_FMT_INT8_ROW   ? whole_fn<TLHIP_FMT_INT8_ROW>(tiles, nb)
+                                          : whole_fn<TLHIP_FMT_INT8_GROUPED>(tiles, nb);
+}
+size_t whole_lds(int tiles, int nb) { return std::max((size_t)kWhole * 16 * tiles * kWholeRow, (size_t)kWhole * tiles * nb * 1024); }
+
 template <int FMT>
 const void* fn_of(int tiles) {
   return tiles == 1 ? (const void*)gemv_f32_kernel<FMT, 1> : (tiles == 2 ? (const void*)gemv_f32_kernel<FMT, 2> : (const void*)gemv_f32_kernel<FMT, 3>);
@@ -311,7 +535,7 @@ bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c
       "not the gemv_f32 variant",
       "built for f32 activations, 1..16 rows, without a prologue",
       "K must be a multiple of 32 (int4) or 16 (int8), groups at least 32 (int4) or 64 (int8)",
-      "K slices (p0) must be 1..64 and no more than K holds blocks of 128 (int4) or 64 (int8); p1..p6 must be 0",
+      "K slices (p0) must be 1..64 and no more than K holds blocks of 128 (int4) or 64 (int8), p1..p6 0; or p0 8 and p1 (blocks of 16 columns) 1, 2 or 4: K a multiple of 128 up to 16384, int4 in groups of 32; 4 blocks up to 10 rows",
       "the pieces of a K slice do not fit LDS: more slices",
       "the slices' partial sums do not fit the library's workspace",
   };
@@ -323,6 +547,12 @@ bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c
   if (p.x_dtype != TLHIP_F32 || p.m < 1 || p.m > 16 || p.pro.kind != TLHIP_PRO_NONE) return fail(1);
   const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
   if (p.k <= 0 || p.k % (int4 ? 32 : 16) != 0 || (p.format != TLHIP_FMT_INT8_ROW && p.group_size < (int4 ? 32 : 64))) return fail(2);
+  if (c.p1 != 0) {  // chains of at most 2048 in a wave: see gemv_f32_default
+    return c.p0 == kWhole && (c.p1 == 1 || c.p1 == 2 || c.p1 == 4) && p.k % kWholeStep == 0 && p.k <= 2048 * kWhole &&
+                   (!int4 || p.group_size == 32) && (c.p1 < 4 || p.m <= 10) && !c.p2 && !c.p3 && !c.p4 && !c.p5 && !c.p6
+               ? true
+               : fail(3);
+  }
   if (c.p0 < 1 || c.p0 > kMaxSlices || c.p0 > blocks_of(p) || c.p1 || c.p2 || c.p3 || c.p4 || c.p5 || c.p6) return fail(3);
   if (lds_of(p, c.p0) > kLdsPerWorkgroup) return fail(4);
   const ScratchNeed need = gemv_f32_scratch(p, c);
@@ -331,12 +561,54 @@ bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c
 }
 
 ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c) {
-  if (c.p0 <= 1) return ScratchNeed{0, 0};
+  if (c.p0 <= 1 || c.p1) return ScratchNeed{0, 0};
   return ScratchNeed{(size_t)column_tiles(p) * (size_t)c.p0 * (size_t)p.m * kCols, column_tiles(p)};
+}
+
+// Time of a launch that keeps all of K in a workgroup, in microseconds: fitted at 1024..13838 x
+// 768..12288, 3..16 rows, three formats.  x: workgroups / CUs; a second one to a CU costs as much
+// as the first (the VALU is what they share), three tiles of pieces fill its LDS alone.
+static double whole_us(const Problem& p, int nb) {
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const double x = (double)((p.n + 16 * nb - 1) / (16 * nb)) / cus, m = (double)p.m;
+  const double c = nb == 1 ? 0.75 + 0.125 * m : (nb == 2 ? 1.35 + 0.135 * m : 2.7 + 0.16 * m);
+  const double rounds = x <= 1.0 ? 1.0 : (p.m > 10 ? 1.15 * (double)(int64_t)(x + 0.999) : (x <= 2.0 ? 2.0 : 0.4 + 0.95 * x));
+  return 2.9 + (double)p.k / 1000.0 * c * rounds;
+}
+
+// All of K in one workgroup, at the cheapest number of columns, or false where K slices are ahead.
+// Us, slices against here, over 24 matrices of 512..16246 x 768..12288 at 3..16 rows:
+//   up to five rows at every one (int8-64 9216 x 2304: 13.0 -> 11.2, 2304 x 9216: 16.8 -> 15.3; int4 at
+//   4096 x 4096 15.4 -> 8.6, at 12288 x 4096 28.8 -> 17.2);
+//   more rows of int4 with K up to 4096 or enough columns for every CU (16 rows at 12288 x 4096 50.8 ->
+//   33.8, at 4096 x 12288 39.7 -> 36.0; but 12 rows at 789 x 9984: 17.9 against 24.0);
+//   more rows of int8 with K up to 4096 where one round of double blocks holds the columns (10 rows
+//   at 2048 x 2304: 12.7 -> 7.1, at 7869 x 768 9.7 -> 6.1; but 16 rows at 9216 x 2304: 16.0 against 21.9).
+static bool whole_default(const Problem& p, tlhip_kernel_config_t* out) {
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  if (p.n > 16384) return false;
+  if (p.m > 5) {
+    if (p.format == TLHIP_FMT_INT4_GROUPED ? p.k > 4096 && p.n < (int64_t)cus * 16 : p.k > 4096 || p.n > (int64_t)cus * 32) return false;
+  }
+  bool found = false;
+  double best = 0.0;
+  for (int nb = 1; nb <= kWholeMaxCols; nb *= 2) {
+    tlhip_kernel_config_t c;
+    memset(&c, 0, sizeof c);
+    c.variant = VARIANT_GEMV_F32;
+    c.p0 = kWhole;
+    c.p1 = nb;
+    if (!gemv_f32_config_applicable(p, c, nullptr) || (found && whole_us(p, nb) >= best)) continue;
+    *out = c;
+    best = whole_us(p, nb);
+    found = true;
+  }
+  return found;
 }
 
 // The K slices of the default: see the rule's figures at its caller.
 bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out) {
+  if (whole_default(p, out)) return true;
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   memset(out, 0, sizeof *out);
   out->variant = VARIANT_GEMV_F32;
@@ -372,7 +644,7 @@ int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_
   a.group_shift = row ? 0 : __builtin_ctz((unsigned)(p.group_size / (int4 ? 32 : 64)));
   a.groups_per_row = row ? 0 : (int)(p.k / p.group_size);
   a.blocks = (int)blocks_of(p);
-  a.slices = c.p0;
+  a.slices = c.p1 ? 1 : c.p0;
   if (a.slices > 1) {
     const int rc = problem_scratch(p, stream, &a.workspace, &a.counters);
     if (rc) return rc;
@@ -382,8 +654,11 @@ int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_
   a.y_dtype = p.y_dtype;
   a.epi = p.epi;
   void* args[] = {(void*)&a};
-  const int rc = launch_kernel(fn_of(p.format, tiles_of(p.m)), dim3((unsigned)(column_tiles(p) * a.slices)), dim3(kThreads), args,
-                               lds_of(p, a.slices), stream);
+  const int tiles = tiles_of(p.m);
+  const int rc = c.p1 ? launch_kernel(whole_fn(p.format, tiles, c.p1), dim3((unsigned)((p.n + 16 * c.p1 - 1) / (16 * c.p1))), dim3(kWhole * 64), args,
+                                      whole_lds(tiles, c.p1), stream)
+                      : launch_kernel(fn_of(p.format, tiles), dim3((unsigned)(column_tiles(p) * a.slices)), dim3(kThreads), args,
+                                      lds_of(p, a.slices), stream);
   if (rc) return rc;
   count_gemv_dispatch();
   return TLHIP_OK;
@@ -393,7 +668,9 @@ int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_
 int prepare_gemv_f32_kernels() {
   for (int format : {TLHIP_FMT_INT4_GROUPED, TLHIP_FMT_INT8_GROUPED, TLHIP_FMT_INT8_ROW})
     for (int tiles = 1; tiles <= 3; ++tiles) {
-      const int rc = launch_kernel(fn_of(format, tiles), dim3(1), dim3(64), nullptr, 0, nullptr);
+      int rc = launch_kernel(fn_of(format, tiles), dim3(1), dim3(64), nullptr, 0, nullptr);
+      for (int nb = 1; nb <= kWholeMaxCols && !rc; nb *= 2)
+        if (nb < 4 || tiles < 3) rc = launch_kernel(whole_fn(format, tiles, nb), dim3(1), dim3(64), nullptr, 0, nullptr);
       if (rc) return rc;
     }
   return TLHIP_OK;
