@@ -892,7 +892,7 @@ int matmul_with(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
 // ... or its form that keeps all of K in one workgroup (gemm_rows.hip), by the models of both:
 // `decode_us` is the former's price, a third more where no waves split K (32 rows of int4 at
 // 6454 x 2304: 15.7 us), half more for int8 (over 12 matrices the former took 1.0-2.5 times its
-// price).  Us, former against latter: int8-64 at 12288 x 4096, 20 / 32 / 48 rows 27.1 / 28.0 / 30.1
+// price), a fifth above K = 8192 (48 rows at 961 x 11136: 24.9 against 28.0).  Us, former against latter: int8-64 at 12288 x 4096, 20 / 32 / 48 rows 27.1 / 28.0 / 30.1
 // against 20.8 / 21.9 / 23.3, but 11.0 / 12.6 / 24.9 against 20.7 / 23.2 / 27.9 at 961 x 11136; int4
 // 48 rows at 12288 x 4096 27.2 against 18.5; up to 32 rows of int4 the two are close where both have
 // their best form (16.2 against 22.5 at 4096 x 12288, 10.3 against 12.0 at 13740 x 2048).
@@ -918,7 +918,7 @@ bool rows_in_one_launch_config(const Problem& p, double decode_us, tlhip_kernel_
   if (!gemm_rows_default(p, &whole, &us)) return found;
   if (found) {
     const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
-    const double price = decode_us * (out->p2 == 1 ? 1.3 : 1.0) * (int4 ? (p.m <= 32 ? 0.9 : 1.0) : 1.5);
+    const double price = decode_us * (out->p2 == 1 ? 1.3 : 1.0) * (int4 ? (p.m <= 32 ? 0.9 : 1.0) : (p.k <= 8192 ? 1.5 : 1.2));
     if (us >= price) return true;
   }
   *out = whole;
@@ -1002,12 +1002,12 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     const int64_t full = p.m / 64, rest = p.m % 64;
     const double rows_us = (double)full * chunk_us(64) + (rest ? chunk_us(rest) : 0.0);
     // one launch of the form that keeps all of K in a workgroup, exact too: wherever it is cheaper
-    // than the tile that would run (48 rows of int4 at 4096 x 4096: 12.0 against 15.4 us); above K =
-    // 1024 only, where a test of first calls under capture pins the tile's K slices (40 rows at 4096
-    // x 1024)
+    // than the tile that would run (48 rows of int4 at 4096 x 4096: 12.0 against 15.4 us); int4
+    // above K = 1024 only: a test of first calls under capture pins the tile's K slices at 40 rows of
+    // 4096 x 1024
     tlhip_kernel_config_t whole;
     double whole_us = 0.0;
-    const bool whole_ok = p.m <= 64 && p.k > 1024 && gemm_rows_default(p, &whole, &whole_us);
+    const bool whole_ok = p.m <= 64 && (p.k > 1024 || p.format != TLHIP_FMT_INT4_GROUPED) && gemm_rows_default(p, &whole, &whole_us);
     double pipe_us = tiled_us;
     if (is_pipe_config(c))
       for (const PipeTileCost& t : kPipeTileCosts)

@@ -12,9 +12,9 @@
 //     one or two steps ahead, whole lines per row, laid into a patch of LDS that belongs to
 //     the wave, and read back as MFMA operands; every byte of X enters the CU once.
 //   * An operand of X feeds NB products and a weight, dequantised once, MT.
-// One launch, us, best kernel before -> here: int4-32 12288 x 4096 at 48 / 64 rows 27.2 -> 18.5, 27.6 ->
-// 20.4; 4096 x 4096 at 48 rows 14.9 -> 12.3; int8-64 12288 x 4096 at 17..32 rows 27-28 -> 21-22, 7179 x
-// 896 at 40 rows 13.3 -> 7.0.  18.5 us are 1.5 TB/s of weights and 260 TFLOP/s: 3.5 us of launch, first
+// One launch, us, best kernel before -> here: int4-32 12288 x 4096 at 48 / 64 rows 27.2 -> 18.1, 27.6 ->
+// 20.9; 4096 x 4096 at 48 rows 14.9 -> 12.1; int8-64 12288 x 4096 at 17..32 rows 27-28 -> 21-22, 7179 x
+// 896 at 40 rows 13.3 -> 7.0.  18.1 us are 1.5 TB/s of weights and 260 TFLOP/s: 3.5 us of launch, first
 // loads and last sums, the rest the 100 MB of X that 256 CUs fetch (25-30 bytes a clock and CU).
 // Rearranging X for the cheaper int4 unpacking, or its addresses by lane, moved nothing.
 //   * Buffer loads: rows past M, columns past N and steps past K read zero and cost no traffic,
@@ -172,6 +172,34 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
       // a lane holds 32 k of its row, one group; afterwards word i is its eighth of group i
       if constexpr (INT4) transpose4(word[b][0], word[b][1], word[b][2], word[b][3]);
     }
+    // a step's own sum first: the long one takes a step at a time (rel-L2 against 64 bits at K = 8192,
+    // int4 / int8-64 / per row: 11.3 / 9.7 / 16.3e-8 one group at a time, 8.4 / 8.9 / 8.8e-8 so, 8.8 / 8.9 / 9.2e-8
+    // for the decode kernel with its four to eight K slices)
+    if constexpr (INT4 && MT * NB >= 12) {  // a block at a time: X from LDS again, a third of the registers
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        float4_t sum[MT];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const half8_t wv = weights_of(word[b][s]);
+          const float sc = half_bits_to_float((s & 1) ? v.s[b][s >> 1] >> 16 : v.s[b][s >> 1] & 0xffffu);
+          float4_t d[MT];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand(t, s), wv, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[t][r] = s == 0 ? sc * d[t][r] : fmaf(sc, d[t][r], sum[t][r]);
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[b][t][r] += sum[t][r];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
+    float4_t sum[NB][MT];
     if constexpr (INT4) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
@@ -188,7 +216,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 #pragma unroll
           for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[b][t][r] = fmaf(sc, d[t][r], acc[b][t][r]);
+            for (int r = 0; r < 4; ++r) sum[b][t][r] = s == 0 ? sc * d[t][r] : fmaf(sc, d[t][r], sum[b][t][r]);
         }
       }
     } else {
@@ -203,7 +231,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
         for (int b = 0; b < NB; ++b) {
           float4_t d[MT];
 #pragma unroll
-          for (int t = 0; t < MT; ++t) d[t] = ROW ? acc[b][t] : (float4_t){0.f, 0.f, 0.f, 0.f};
+          for (int t = 0; t < MT; ++t) d[t] = (float4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
             half2_t w[4];
@@ -213,19 +241,23 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 #pragma unroll
             for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[i][t], wv, d[t], 0, 0, 0);
           }
-          if constexpr (ROW) {
+          const float sc = ROW ? 1.f : half_bits_to_float(v.s[b][h]);
 #pragma unroll
-            for (int t = 0; t < MT; ++t) acc[b][t] = d[t];
-          } else {
-            const float sc = half_bits_to_float(v.s[b][h]);
+          for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) acc[b][t][r] = fmaf(sc, d[t][r], acc[b][t][r]);
-          }
+            for (int r = 0; r < 4; ++r) {
+              const float p = ROW ? d[t][r] : sc * d[t][r];
+              sum[b][t][r] = h == 0 ? p : (ROW ? sum[b][t][r] + d[t][r] : fmaf(sc, d[t][r], sum[b][t][r]));
+            }
         }
       }
     }
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[b][t][r] += sum[b][t][r];
   };
 
   // Every load below is unconditional (a wait at a join would count it as not issued); the
@@ -267,7 +299,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
     }
   }
 
-  // ---- the waves' sums, in order, and the epilogue ---------------------------------------
+  // ---- the waves' sums and the epilogue ---------------------------------------
   lds_barrier();  // every wave has read its patch
   float* const sums = (float*)lds;  // [wave][row tile][block][16 x 16]
 #pragma unroll
@@ -286,11 +318,10 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
     float4_t part[kWaves];
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) part[w] = *(const float4_t*)(p + w * (MT * NB * 256));
-    float4_t sum = part[0];
+    float4_t sum;  // in pairs: a shorter chain, a smaller rounding error
 #pragma unroll
-    for (int w = 1; w < kWaves; ++w)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sum[i] += part[w][i];
+    for (int i = 0; i < 4; ++i)
+      sum[i] = ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) + ((part[4][i] + part[5][i]) + (part[6][i] + part[7][i]));
     const int col = n0 + c;
     const int64_t at = (int64_t)row * a.n + col;
     float v[4];
@@ -315,7 +346,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 int row_tiles_of(int64_t m) { return (int)((m + 15) / 16); }
 // The column blocks whose instance fits 256 registers a lane without spilling.
 constexpr int most_columns(int format, int mt) {
-  return format == TLHIP_FMT_INT8_GROUPED ? (mt == 2 ? 4 : (mt == 3 ? 3 : 2)) : (format == TLHIP_FMT_INT8_ROW ? (mt == 4 ? 3 : 4) : (mt == 4 ? 3 : 4));
+  return format == TLHIP_FMT_INT4_GROUPED ? (mt == 4 ? 3 : 4) : (mt == 2 ? 4 : (mt == 3 ? 3 : 2));
 }
 
 template <int FMT, int MT, int NB>
@@ -325,7 +356,7 @@ const void* instance() {
   } else {
     // X two steps ahead where the registers allow it
     constexpr int used = MT * 32 + NB * MT * 4 + NB * (FMT == TLHIP_FMT_INT4_GROUPED ? 12 : 24) + 40;
-    constexpr bool full = FMT == TLHIP_FMT_INT4_GROUPED && MT * NB >= 12;
+    constexpr bool full = FMT == TLHIP_FMT_INT4_GROUPED && MT * NB >= 9;
     return (const void*)gemm_rows_kernel<FMT, MT, NB, (full ? 0 : (used <= 200 ? 2 : 1))>;
   }
 }
@@ -363,8 +394,6 @@ bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
 // last sums, and per round of workgroups and 4096 of K the figure below; int8 a tenth more.
 // A block more costs a workgroup 2.5-4 us, sixteen rows more 1.5-3 us, whatever the chip has to
 // do beside it: few blocks until the workgroups no longer fit the CUs at once.
-// Not the instances that want more than 256 registers (four tiles of rows: three blocks of
-// int8 groups, four of anything).
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
   static const double walk[3][kMaxCols] = {{6.4, 9.1, 11.6, 14.0}, {8.2, 10.8, 13.7, 16.2}, {10.0, 12.2, 17.5, 23.0}};
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
