@@ -647,7 +647,9 @@ int launch_mfma_u(int unroll, const MfmaArgs& a, int grid, int threads, size_t l
     switch (unroll) {
       case 1: fn = (const void*)gemv_mfma_kernel<FMT, 1, WIDE, 512, false, GROUP, MT>; break;
       case 2: fn = (const void*)gemv_mfma_kernel<FMT, 2, WIDE, 512, false, GROUP, MT>; break;
-      default: fn = (const void*)gemv_mfma_kernel<FMT, 4, WIDE, 512, false, GROUP, MT>; break;
+      // four tiles of rows and four iterations in flight are refused before this (mfma_applicable);
+      // their instances took most of the compile time
+      default: fn = (const void*)gemv_mfma_kernel<FMT, MT == 4 ? 2 : 4, WIDE, 512, false, GROUP, MT>; break;
     }
   }
   void* args[] = {(void*)&a};
@@ -667,7 +669,7 @@ int launch_mfma_line(int unroll, const MfmaArgs& a, int grid, int threads, size_
   } else if (unroll == 2) {
     fn = (const void*)gemv_mfma_kernel<FMT, 2, WIDE, 512, true, GROUP, MT>;
   } else {
-    fn = (const void*)gemv_mfma_kernel<FMT, 4, WIDE, 512, true, GROUP, MT>;
+    fn = (const void*)gemv_mfma_kernel<FMT, MT == 4 ? 2 : 4, WIDE, 512, true, GROUP, MT>;
   }
   void* args[] = {(void*)&a};
   return launch_kernel(fn, dim3(grid), dim3(threads), args, lds_bytes, stream);
@@ -735,5 +737,9 @@ int prepare_mfma_grouped();
 int launch_mfma_rows(int tiles, int format, int group_size, int64_t k, int unroll, int line, const MfmaArgs& a, int grid,
                      int threads, size_t lds_bytes, hipStream_t stream);
 int prepare_mfma_rows();
+// ... those of four tiles: gemv_mfma_rows4.hip.
+int launch_mfma_rows4(int format, int group_size, int64_t k, int unroll, int line, const MfmaArgs& a, int grid, int threads,
+                      size_t lds_bytes, hipStream_t stream);
+int prepare_mfma_rows4();
 
 }  // namespace tlhip
