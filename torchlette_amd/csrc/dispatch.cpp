@@ -894,7 +894,9 @@ int matmul_with(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
 // 6454 x 2304: 15.7 us), half more for int8 (over 12 matrices the former took 1.0-2.5 times its
 // price), a fifth above K = 8192 (48 rows at 961 x 11136: 24.9 against 28.0).  Us, former against latter: int8-64 at 12288 x 4096, 20 / 32 / 48 rows 27.1 / 28.0 / 30.1
 // against 20.8 / 21.9 / 23.3, but 11.0 / 12.6 / 24.9 against 20.7 / 23.2 / 27.9 at 961 x 11136; int4
-// 48 rows at 12288 x 4096 27.2 against 18.5; up to 32 rows of int4 the two are close where both have
+// 48 rows at 12288 x 4096 27.2 against 18.1, at 1024 x 4096 12.1 against 11.4 (64 rows: 15.9 against
+// 13.1; a fifth more is what its price lacks there up to K = 4096, but 64 rows at 2048 x 8192 18.6
+// against 22.2); up to 32 rows of int4 the two are close where both have
 // their best form (16.2 against 22.5 at 4096 x 12288, 10.3 against 12.0 at 13740 x 2048).
 bool rows_in_one_launch_config(const Problem& p, double decode_us, tlhip_kernel_config_t* out) {
   if (p.m <= 16 || p.m > 64 || p.x_dtype != TLHIP_F16) return false;
@@ -918,7 +920,7 @@ bool rows_in_one_launch_config(const Problem& p, double decode_us, tlhip_kernel_
   if (!gemm_rows_default(p, &whole, &us)) return found;
   if (found) {
     const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
-    const double price = decode_us * (out->p2 == 1 ? 1.3 : 1.0) * (int4 ? (p.m <= 32 ? 0.9 : 1.0) : (p.k <= 8192 ? 1.5 : 1.2));
+    const double price = decode_us * (out->p2 == 1 ? 1.3 : 1.0) * (int4 ? (p.m <= 32 ? 0.9 : (p.k <= 4096 ? 1.2 : 1.0)) : (p.k <= 8192 ? 1.5 : 1.2));
     if (us >= price) return true;
   }
   *out = whole;
