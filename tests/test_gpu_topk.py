@@ -122,7 +122,7 @@ def test_topk_errors(be):
         be.readTopK(t, 2, offset=8, length=5)
 
 
-@pytest.mark.parametrize("k", [1, 3, 63, 64, 65, 255, 256])
+@pytest.mark.parametrize("k", [1, 3, 63, 64, 65, 160, 200, 255, 256])
 @pytest.mark.parametrize("n", [4097, 70001, 131072, 135169])  # 2, 18, 32 and 34 chunks: 2, 8 or 16 keys a thread at the end
 def test_topk_of_runs_that_pass_the_bound_together(be, n, k):
     """Sorted, constant and stepped rows: whole groups of neighbours pass the bound, or none but k do."""

@@ -45,10 +45,9 @@ constexpr int kSelectFused = 8192;      // keys the last workgroup reduces in th
 __device__ __forceinline__ uint64_t max_key(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
 // A bound that at least `k` of the wave's 64 * R values reach: the first one tried that no more
-// than `most` reach (`enough`), else the largest.  One bit per step, a chain of 60 clocks; `most`
-// a quarter above k saves about eight of twenty steps and lets a few more keys pass.
+// than k + slack reach (`enough`), else the largest.  One bit per step, a chain of 60 clocks.
 template <int R>
-__device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool (&in)[R], int k, int most, bool* enough) {
+__device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool (&in)[R], int k, int slack, bool* enough) {
   uint32_t bound = 0;
   *enough = false;
   for (int bit = 31; bit >= 0; --bit) {
@@ -57,7 +56,7 @@ __device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool 
 #pragma unroll
     for (int r = 0; r < R; ++r) count += __popcll(__ballot(in[r] && v[r] >= trial));
     if (count >= k) bound = trial;
-    if (count >= k && count <= most) {
+    if ((uint32_t)(count - k) <= (uint32_t)slack) {
       *enough = true;
       break;
     }
@@ -72,7 +71,11 @@ __device__ __forceinline__ uint32_t bound_of(const uint32_t (&v)[R], const bool 
 //      random keys about 100 do, at worst the whole contents of the groups that reach it (4096);
 //   3. the keys from the bound on, collected in LDS (a wave counts its own by ballots and takes
 //      its places with one atomic: an atomic a key was a chain of E round trips to LDS); the rank
-//      of each is the number of larger ones, counted by four threads.
+//      of each is the number of larger ones, counted by as many threads as there are for a key.
+// The slack of the bound: a quarter of k saves about eight of twenty steps, but the more of the G
+// maxima pass the more keys each of them brings, and a rank's time grows with the keys.  Of 512, up
+// to 224 (k = 256, us: no slack / a sixteenth / a quarter 10.6 / 10.2 / 11.0 of 4096 logits, 32.6 /
+// 30.6 / 31.8 of 256 000; k = 160 7.8 / 7.3 / 7.0 and 21.8 / 20.9 / 20.0).
 template <int G, int E, typename Emit>
 __device__ __forceinline__ void select_keys(const uint64_t (&key)[E], int k, uint64_t* maxima, uint64_t* found, int* n_found, Emit emit) {
   constexpr int R = G / 64;
@@ -99,9 +102,9 @@ __device__ __forceinline__ void select_keys(const uint64_t (&key)[E], int k, uin
     in[r] = true;
   }
   constexpr int kMostGroups = kTopkChunk / (E * kSelectThreads / G);  // whose whole contents `found` holds
-  const int most = min(k + k / 4, kMostGroups) > k ? min(k + k / 4, kMostGroups) : k;
+  const int slack = max(0, min(max(min(k / 4, 224 - k), k / 16), kMostGroups - k));
   bool enough;
-  const uint32_t bound_hi = bound_of<R>(hi, in, k, most, &enough);
+  const uint32_t bound_hi = bound_of<R>(hi, in, k, slack, &enough);
   uint32_t bound_lo = 0;
   if (!enough) {  // equal values around the bound: the index decides
     int larger = 0;
@@ -110,34 +113,46 @@ __device__ __forceinline__ void select_keys(const uint64_t (&key)[E], int k, uin
       larger += __popcll(__ballot(hi[r] > bound_hi));
       in[r] = hi[r] == bound_hi;
     }
-    bound_lo = bound_of<R>(lo, in, k - larger, most - larger, &enough);
+    bound_lo = bound_of<R>(lo, in, k - larger, slack, &enough);
   }
   const uint64_t bound = ((uint64_t)bound_hi << 32) | bound_lo;
-  int mine = 0;  // of the wave
-#pragma unroll
-  for (int e = 0; e < E; ++e) mine += __popcll(__ballot(key[e] != 0 && key[e] >= bound));
-  int at = 0;
-  if (lane == 0 && mine) at = atomicAdd(n_found, mine);
-  at = __shfl(at, 0);
+  uint64_t hits[E];  // of the wave
+  int mine = 0;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const bool hit = key[e] != 0 && key[e] >= bound;
-    const uint64_t hits = __ballot(hit);
-    if (hit) found[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(hits >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u))] = key[e];
-    at += __popcll(hits);
+    hits[e] = __ballot(key[e] != 0 && key[e] >= bound);
+    mine += __popcll(hits[e]);
+  }
+  if (mine) {
+    int at = 0;
+    if (lane == 0) at = atomicAdd(n_found, mine);
+    at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (hits[e]) {
+        if (key[e] != 0 && key[e] >= bound)
+          found[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(hits[e] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hits[e], 0u))] = key[e];
+        at += __popcll(hits[e]);
+      }
   }
   __syncthreads();
   const int c = *n_found;
-  for (int i0 = 0; i0 < c; i0 += kSelectThreads / 4) {
-    const int i = i0 + (tid >> 2);
-    const uint64_t own = found[min(i, c - 1)];
-    int rank = 0;
+  auto rank_keys = [&](auto threads) {
+    constexpr int T = decltype(threads)::value;  // of a key, neighbours in a wave
+    for (int i0 = 0; i0 < c; i0 += kSelectThreads / T) {
+      const int i = i0 + tid / T;
+      const uint64_t own = found[min(i, c - 1)];
+      int rank = 0;
 #pragma unroll 8
-    for (int j = tid & 3; j < c; j += 4) rank += found[j] > own ? 1 : 0;
-    rank += __shfl_xor(rank, 1);
-    rank += __shfl_xor(rank, 2);
-    if ((tid & 3) == 0 && i < c && rank < k) emit(rank, own);
-  }
+      for (int j = tid % T; j < c; j += T) rank += found[j] > own ? 1 : 0;
+      if (T > 1) rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xf, 0xf, true);  // quad_perm [1,0,3,2]
+      if (T > 2) rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xf, 0xf, true);  // quad_perm [2,3,0,1]
+      if (tid % T == 0 && i < c && rank < k) emit(rank, own);
+    }
+  };
+  if (c <= kSelectThreads / 4) rank_keys(std::integral_constant<int, 4>());
+  else if (c <= kSelectThreads / 2) rank_keys(std::integral_constant<int, 2>());
+  else rank_keys(std::integral_constant<int, 1>());
   for (int i = c + tid; i < k; i += kSelectThreads) emit(i, (uint64_t)0);
   __syncthreads();
 }
@@ -155,9 +170,10 @@ __device__ __forceinline__ void write_result(int i, uint64_t key, float* out_val
 // last reduces all of them to the result (gridDim.x * k <= kSelectFused); a launch of one
 // workgroup writes the result at once.
 // 256 000 logits, k = 64, 8 rows behind each other: 35 us a row with three launches of sorted
-// chunks of 1024 at first, 14 us with this launch, 11.0 us since a bound may let a few more keys pass,
-// a wave takes its places with one atomic and four threads count a rank: what is left is the launch,
-// two loads of keys, the stores and the counter, each a round trip to memory behind the other.
+// chunks of 1024 at first, 14 us with this launch, 9.6 us since a bound may let a few more keys pass,
+// a wave takes its places with one atomic and up to four threads count a rank (k = 256: 33.6 -> 30.2):
+// what is left is the launch, two loads of keys, the stores and the counter, each a round trip to
+// memory behind the other.
 template <bool FROM_FLOAT, int G>
 __global__ __launch_bounds__(kSelectThreads) void topk_select_kernel(const float* __restrict__ logits, int64_t offset,
                                                                      const uint64_t* __restrict__ keys_in, int64_t count, int k,
