@@ -427,9 +427,9 @@ int tlhip_topk(const float* logits, int64_t offset, int64_t length, int k, float
 /* A launch configuration.  variant 0 = "gemv" (VALU dot), 1 = "gemv_mfma"
  * (skinny MFMA: up to 16 rows, and 17..64 rows for one problem with at most 8
  * waves per workgroup and, above 32 rows, at most 2 iterations in flight; 17..64 rows with
- * p4 = 1..4 keep all of K in one workgroup of 16 p4 columns: K a multiple of 128, int4 in
- * groups of 32, int8 in groups of 64 or more or per row, and few enough columns for its
- * registers),
+ * p0 = 8, p4 = 1..4 and every other field 0 keep all of K in one workgroup of 16 p4 columns: K a
+ * multiple of 128, int4 in groups of 32, int8 in groups of 64 or more or per row, and few enough
+ * columns for its registers: up to 4 / 4 / 3 for int4 and 4 / 3 / 2 for int8 at 32 / 48 / 64 rows),
  * 2 = "tiled" (prefill MFMA GEMM, both operands through LDS),
  * 3 = "tiled_direct" (prefill MFMA GEMM whose weights stay packed up to the
  * operand registers; fields as "tiled" with tile K 128; int4-grouped on the tiles
@@ -457,7 +457,7 @@ typedef struct {
   int32_t p1; /* gemv: rows per lane-group        gemv_mfma: iterations in flight  tiled: tile N */
   int32_t p2; /* gemv: waves per workgroup        gemv_mfma: K-split waves (0 = all)  tiled: tile K */
   int32_t p3; /* gemv: K-split waves (LDS combine) gemv_mfma: K slices across workgroups (0/1 = none)  tiled: waves M */
-  int32_t p4; /* gemv: chunks in flight (2/4/8)    gemv_mfma, 17..64 rows: blocks of 16 columns (0 = the other form)  tiled: waves N */
+  int32_t p4; /* gemv: chunks in flight (2/4/8)    gemv_mfma, 17..64 rows, p1 = 0: blocks of 16 columns (else not read)  tiled: waves N */
   int32_t p5; /* gemv: 1 = dot products on the 4x4x4 matrix-core instruction (int4, f16 x, m <= 4, p0 = 16, p1 = 1)
                * gemv_mfma: 1 = whole-line weight loads through a wave-private LDS patch (int8 with
                * K % 128 == 0 or int4-g32 with K % 256 == 0; p1 = 2 or 4)

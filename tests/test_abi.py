@@ -274,6 +274,29 @@ def test_a_faster_tile_does_not_take_rows_from_the_exact_kernel(fmt, g, n, k, m)
     assert chunk.value == 64 and first.variant == last.variant == L.VARIANT_GEMV_MFMA, (chunk.value, first.as_tuple(), last.as_tuple())
 
 
+@pytest.mark.parametrize("fields,runs", [
+    ((8, 0, 0, 0, 3), True), ((8, 0, 0, 0, 4), False),                     # four blocks of 64 rows: more registers than a lane has
+    ((5, 0, 0, 0, 3), False), ((16, 0, 0, 0, 3), False), ((8, 0, 3, 0, 3), False), ((8, 0, 0, 3, 3), False),
+    ((8, 0, 0, 0, 3, 1), False), ((8, 0, 0, 0, 3, 0, 1), False), ((8, 0, 0, 0, 0), False),
+    ((8, 2, 1, 4, 0), True), ((8, 2, 1, 4, 3), True), ((8, 2, 3, 4, 3), False),  # the other form has never read p4
+])
+def test_a_rows_configuration_is_told_by_all_its_fields(fields, runs):
+    """All of K in one workgroup: its width, eight waves and nothing else; a geometry that was refused
+    before the form was there stays refused."""
+    lib = L.load()
+    before = T.exportTuningCache()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    w, c = L.QWeight(L.FMT_INT4_GROUPED, 32, 12288, 4096, ptr, ptr), L.KernelConfig.of(L.VARIANT_GEMV_MFMA, *fields)
+    try:
+        rc = lib.tlhip_tune_cache_seed(ctypes.byref(w), L.F16, 64, L.F16, ctypes.byref(c))
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(before)
+    assert (rc == 0) == runs, L.last_error()
+    assert runs or fields[1] or not fields[4] or "p4 blocks of 16 columns" in L.last_error()
+
+
 @pytest.mark.parametrize("m", [1, 3, 5, 16])
 def test_f32_rows_have_one_limit_of_k(m):
     """K up to 28672 (one f32 row in LDS), however many rows a call has: longer K selects the

@@ -42,3 +42,13 @@ def test_rows_match_the_oracle(be, fmt, g, n, k, m):
         ran += 1
         assert rel_l2(got, want) <= 2e-6, cols  # exact products, f32 sums: order noise only
     assert ran >= 2
+
+
+def test_the_width_is_not_read_with_the_other_forms_fields(be):
+    fmt, g, n, k, m = "int4-grouped", 32, 512, 2048, 40
+    rng = np.random.default_rng(7)
+    packed, scales, _ = make_weight(fmt, n, k, g, rng)
+    x = make_x(m, k, "f16", rng)
+    plain, with_width = (run_linear(be, fmt, packed, scales, n, k, g, x, "f32", config=L.KernelConfig.of(L.VARIANT_GEMV_MFMA, 8, 2, 8, 2, p4))
+                         for p4 in (0, 2))
+    assert np.array_equal(plain.view(np.uint32), with_width.view(np.uint32))

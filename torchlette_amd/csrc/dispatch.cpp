@@ -888,8 +888,23 @@ int matmul_with(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
 // in flight, the fewest K slices across workgroups whose activations fit LDS, and the
 // fewest K-split waves per row block that still give every CU a workgroup (measured best
 // or within 5 % of it at 4096..28672 x 4096..12288, M = 24..64).
-//
-// ... or its form that keeps all of K in one workgroup (gemm_rows.hip), by the models of both:
+bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
+  if (p.m <= 16 || p.m > 64 || p.x_dtype != TLHIP_F16) return false;
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int64_t nblocks = (p.n + 15) / 16;
+  for (int ks = 1; ks <= 16; ks *= 2) {
+    int fill = 1;  // K-split waves per row block: 8 / fill row blocks per workgroup
+    while (fill < 8 && (nblocks * fill / 8) * ks < cus) fill *= 2;
+    for (int kw : {fill, 8, 4, 2, 1})
+      for (int unroll : {2, 1}) {
+        const tlhip_kernel_config_t c = mfma_cfg(8, unroll, kw, ks);
+        if (gemv_mfma_config_applicable(p, c, nullptr)) return *out = c, true;
+      }
+  }
+  return false;
+}
+
+// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip), by the models of both:
 // `decode_us` is the former's price, a third more where no waves split K (32 rows of int4 at
 // 6454 x 2304: 15.7 us), half more for int8 (over 12 matrices the former took 1.0-2.5 times its
 // price), a fifth above K = 8192 (48 rows at 961 x 11136: 24.9 against 28.0).  Us, former against latter: int8-64 at 12288 x 4096, 20 / 32 / 48 rows 27.1 / 28.0 / 30.1
@@ -899,22 +914,7 @@ int matmul_with(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
 // against 22.2); up to 32 rows of int4 the two are close where both have
 // their best form (16.2 against 22.5 at 4096 x 12288, 10.3 against 12.0 at 13740 x 2048).
 bool rows_in_one_launch_config(const Problem& p, double decode_us, tlhip_kernel_config_t* out) {
-  if (p.m <= 16 || p.m > 64 || p.x_dtype != TLHIP_F16) return false;
-  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const int64_t nblocks = (p.n + 15) / 16;
-  bool found = false;
-  for (int ks = 1; ks <= 16 && !found; ks *= 2) {
-    int fill = 1;  // K-split waves per row block: 8 / fill row blocks per workgroup
-    while (fill < 8 && (nblocks * fill / 8) * ks < cus) fill *= 2;
-    for (int kw : {fill, 8, 4, 2, 1})
-      for (int unroll : {2, 1}) {
-        const tlhip_kernel_config_t c = mfma_cfg(8, unroll, kw, ks);
-        if (!found && gemv_mfma_config_applicable(p, c, nullptr)) {
-          *out = c;
-          found = true;
-        }
-      }
-  }
+  const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
   if (!gemm_rows_default(p, &whole, &us)) return found;
@@ -1115,11 +1115,16 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       vary(5, {0, 1});
       break;
     case VARIANT_GEMV_MFMA:
+      if (is_rows_config(p, base)) {  // its width is its only field
+        vary(4, {1, 2, 3, 4});
+        tlhip_kernel_config_t sliced;
+        if (decode_rows_config(p, &sliced)) push(sliced);
+        break;
+      }
       vary(0, {4, 8, 16});
       vary(1, {1, 2, 4});
       vary(2, {1, 2, 4, 8, 16});
       vary(3, {1, 2, 4, 8});
-      if (is_rows_config(p, base)) vary(4, {1, 2, 3, 4});
       vary(5, {0, 1});
       break;
     case VARIANT_GEMV_F32:

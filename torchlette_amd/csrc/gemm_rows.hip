@@ -381,7 +381,8 @@ size_t lds_of(int mt, int nb) {
 }  // namespace
 
 bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
-  if (c.variant != VARIANT_GEMV_MFMA || c.p4 < 1 || c.p4 > kMaxCols) return false;
+  if (c.variant != VARIANT_GEMV_MFMA || c.p0 != kWaves || c.p4 < 1 || c.p4 > kMaxCols) return false;
+  if (c.p1 || c.p2 || c.p3 || c.p5 || c.p6) return false;  // the other form's fields: p4 is not read there
   if (p.x_dtype != TLHIP_F16 || p.m < 17 || p.m > 64 || p.pro.kind != TLHIP_PRO_NONE) return false;
   if (c.p4 > most_columns(p.format, row_tiles_of(p.m))) return false;
   if (p.k <= 0 || p.k % kStep != 0 || p.k > (1 << 23)) return false;  // offsets below 2^31: 64 rows of X or of weights

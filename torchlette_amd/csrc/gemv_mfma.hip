@@ -110,7 +110,14 @@ static bool mfma_applicable(const Problem& p, int64_t nblocks, const tlhip_kerne
 }
 
 bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why) {
-  return is_rows_config(p, c) || mfma_applicable(p, (p.n + 15) / 16, c, why);
+  if (is_rows_config(p, c)) return true;
+  if (c.variant == VARIANT_GEMV_MFMA && c.p1 == 0 && c.p4 != 0) {  // no geometry of the other form has p1 = 0
+    if (why)
+      *why = "all of K in one workgroup (p1 = 0, p4 blocks of 16 columns): 17..64 f16 rows, p0 8, p1..p3, p5 and p6 0, K a multiple "
+             "of 128, int4 in groups of 32, int8 in groups of 64 or more or per row, p4 1..4 and no more than its registers hold";
+    return false;
+  }
+  return mfma_applicable(p, (p.n + 15) / 16, c, why);
 }
 
 // The problems of a group: same activations and rows, one shape class; N, pointers and
