@@ -297,6 +297,42 @@ def test_a_rows_configuration_is_told_by_all_its_fields(fields, runs):
     assert runs or fields[1] or not fields[4] or "p4 blocks of 16 columns" in L.last_error()
 
 
+@pytest.mark.parametrize("fmt,g,n,k,m,width", [
+    # measured, us: K slices across workgroups / all of K in one workgroup at the best width
+    (L.FMT_INT8_GROUPED, 64, 2008, 8192, 32, 0),     # 12.1 / 18.2
+    (L.FMT_INT8_GROUPED, 64, 2008, 8192, 17, 0),     # 12.7 / 16.4
+    (L.FMT_INT8_ROW, 0, 2451, 8192, 32, 0),          # 12.7 / 16.5
+    (L.FMT_INT8_ROW, 0, 1253, 6528, 33, 0),          # 12.6 / 16.2
+    (L.FMT_INT8_ROW, 0, 796, 3840, 64, 0),           # 10.6 / 12.4
+    (L.FMT_INT8_GROUPED, 64, 971, 3072, 64, 0),      # 10.6 / 11.8
+    (L.FMT_INT4_GROUPED, 32, 16384, 4096, 17, 0),    # 15.7 / 19.0
+    (L.FMT_INT4_GROUPED, 32, 3312, 8960, 56, 0),     # 20.4 / 23.4
+    (L.FMT_INT4_GROUPED, 32, 3312, 8960, 128, 0),    # 43.2 / 47.6, 64 rows at a time
+    (L.FMT_INT8_ROW, 0, 2193, 3584, 17, 0),          # 7.7 / 8.7
+    (L.FMT_INT8_GROUPED, 64, 12288, 4096, 32, 3),    # 28.0 / 22.2
+    (L.FMT_INT8_ROW, 0, 3371, 3712, 20, 1),          # 20.7 / 9.6
+    (L.FMT_INT4_GROUPED, 32, 12288, 4096, 48, 3),    # 27.2 / 18.1
+    (L.FMT_INT4_GROUPED, 32, 4096, 4096, 18, 1),     # 21.8 / 8.8
+    (L.FMT_INT4_GROUPED, 32, 6144, 4096, 64, 2),     # 16.9 / 15.5
+])
+def test_rows_take_the_form_that_measured_faster(fmt, g, n, k, m, width):
+    """17..64 rows, nothing tuned: the width of the form that keeps all of K in a workgroup, or 0."""
+    lib = L.load()
+    before = T.exportTuningCache()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    w = L.QWeight(fmt, g, n, k, ptr, ptr)
+    chunk, first, last = ctypes.c_int64(), L.KernelConfig(), L.KernelConfig()
+    try:
+        T.clearTuningCache()
+        assert lib.tlhip_selected_route(ctypes.byref(w), L.F16, m, L.F16, ctypes.byref(chunk), ctypes.byref(first), ctypes.byref(last)) == 0
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(before)
+    c = (first if m >= 64 else last).as_tuple()
+    assert chunk.value == 64 and c[0] == L.VARIANT_GEMV_MFMA and c[5] == width and (c[2] == 0) == (width > 0), (chunk.value, c)
+
+
 @pytest.mark.parametrize("m", [1, 3, 5, 16])
 def test_f32_rows_have_one_limit_of_k(m):
     """K up to 28672 (one f32 row in LDS), however many rows a call has: longer K selects the

@@ -126,6 +126,8 @@ ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c);
 bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c);
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us);
 int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
+// Time of a launch of the decode kernel at 17..64 rows, in microseconds (gemv_mfma.hip); c applicable.
+double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c);
 // elementwise.hip: the steps of `ep` over a finished [M,N] output, in place, 8 columns a lane
 bool epilogue_tail_applicable(const void* y, int64_t n);
 int launch_epilogue_tail(void* y, int y_dtype, int64_t m, int64_t n, const DevEpilogue& ep, hipStream_t stream);

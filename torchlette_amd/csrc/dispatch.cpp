@@ -904,25 +904,17 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return false;
 }
 
-// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip), by the models of both:
-// `decode_us` is the former's price, a third more where no waves split K (32 rows of int4 at
-// 6454 x 2304: 15.7 us), half more for int8 (over 12 matrices the former took 1.0-2.5 times its
-// price), a fifth above K = 8192 (48 rows at 961 x 11136: 24.9 against 28.0).  Us, former against latter: int8-64 at 12288 x 4096, 20 / 32 / 48 rows 27.1 / 28.0 / 30.1
-// against 20.8 / 21.9 / 23.3, but 11.0 / 12.6 / 24.9 against 20.7 / 23.2 / 27.9 at 961 x 11136; int4
-// 48 rows at 12288 x 4096 27.2 against 18.1, at 1024 x 4096 12.1 against 11.4 (64 rows: 15.9 against
-// 13.1; a fifth more is what its price lacks there up to K = 4096, but 64 rows at 2048 x 8192 18.6
-// against 22.2); up to 32 rows of int4 the two are close where both have
-// their best form (16.2 against 22.5 at 4096 x 12288, 10.3 against 12.0 at 13740 x 2048).
-bool rows_in_one_launch_config(const Problem& p, double decode_us, tlhip_kernel_config_t* out) {
+// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip) where it is under nine
+// tenths of the former's price: of 1834 problems timed with both, five are more than 3 % behind the
+// former (the furthest, 48 rows of int4 at 20403 x 512: 11.3 against 9.9 us) and all are 1.4 % behind
+// the faster one in the mean.  Us, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0
+// against 22.2, but 2008 x 8192 12.1 against 18.2; int4 12288 x 4096, 48 rows 27.2 against 18.1, but
+// 2610 x 11520 23.0 against 25.1.
+bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
   const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
-  if (!gemm_rows_default(p, &whole, &us)) return found;
-  if (found) {
-    const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
-    const double price = decode_us * (out->p2 == 1 ? 1.3 : 1.0) * (int4 ? (p.m <= 32 ? 0.9 : (p.k <= 4096 ? 1.2 : 1.0)) : (p.k <= 8192 ? 1.5 : 1.2));
-    if (us >= price) return true;
-  }
+  if (!gemm_rows_default(p, &whole, &us) || (found && us >= 0.9 * gemv_mfma_rows_us(p, *out))) return found;
   *out = whole;
   return true;
 }
@@ -1020,8 +1012,8 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
       Problem q64 = p, qr = p;
       q64.m = 64;
       qr.m = rest;
-      if (full) ok = rows_in_one_launch_config(q64, chunk_us(64), &q.first);
-      if (ok && rest > 16) ok = rows_in_one_launch_config(qr, chunk_us(rest), &q.last);
+      if (full) ok = rows_in_one_launch_config(q64, &q.first);
+      if (ok && rest > 16) ok = rows_in_one_launch_config(qr, &q.last);
       if (ok && rest > 0 && rest <= 16) {
         q.last = select_gemv_config(qr);
         ok = q.last.variant == VARIANT_GEMV_MFMA || q.last.variant == VARIANT_GEMV_XREG || rest <= 4;

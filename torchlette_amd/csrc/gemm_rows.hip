@@ -390,14 +390,18 @@ bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
   return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
 }
 
-// The cheapest number of column blocks and its time in microseconds, or false.  Measured at
-// 1024..28672 x 4096..12288 (int4-32, int8-64, int8-row): 3.5 us of launch, first operands and
-// last sums, and per round of workgroups and 4096 of K the figure below; int8 a tenth more.
-// A block more costs a workgroup 2.5-4 us, sixteen rows more 1.5-3 us, whatever the chip has to
-// do beside it: few blocks until the workgroups no longer fit the CUs at once.
+// The cheapest number of column blocks and its time in microseconds, or false.  Fitted at 1200
+// problems (150 matrices of 400..24576 x 512..12288, 17..64 rows, four formats): 2.1 us of launch, and
+// per round of workgroups 1.1 us, 0.17 for every block of 16 x 16 sums and, per 4096 of K, the
+// figure below.  98 % of the launches take 0.89-1.12 times that; the width it picks is 0.02 % slower
+// than the best one in the mean.
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
-  static const double walk[3][kMaxCols] = {{6.4, 9.1, 11.6, 14.0}, {8.2, 10.8, 13.7, 16.2}, {10.0, 12.2, 17.5, 23.0}};
+  static const double walk[3][3][kMaxCols] = {  // format, row tiles, column blocks
+      {{4.9, 7.9, 10.6, 13.0}, {7.7, 10.1, 11.0, 15.3}, {9.4, 10.7, 14.2, 0.0}},    // int4
+      {{6.7, 10.6, 14.8, 18.0}, {9.2, 11.9, 16.1, 0.0}, {9.8, 14.0, 0.0, 0.0}},     // int8 in groups
+      {{6.0, 8.9, 11.8, 14.1}, {8.5, 9.8, 13.6, 0.0}, {9.1, 11.9, 0.0, 0.0}}};      // int8 per row
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int format = p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1), mt = row_tiles_of(p.m);
   bool found = false;
   for (int nb = 1; nb <= kMaxCols; ++nb) {
     tlhip_kernel_config_t c;
@@ -407,7 +411,7 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
     c.p4 = nb;
     if (!is_rows_config(p, c)) continue;
     const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb), rounds = (wgs + cus - 1) / cus;
-    const double t = 3.5 + (double)rounds * (double)p.k / 4096.0 * walk[row_tiles_of(p.m) - 2][nb - 1] * (p.format == TLHIP_FMT_INT4_GROUPED ? 1.0 : 1.1);
+    const double t = 2.1 + (double)rounds * (1.1 + 0.17 * mt * nb + (double)p.k / 4096.0 * walk[format][mt - 2][nb - 1]);
     if (found && t >= *us) continue;
     *out = c;
     *us = t;

@@ -120,6 +120,32 @@ bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& 
   return mfma_applicable(p, (p.n + 15) / 16, c, why);
 }
 
+// What a launch of 17..64 rows costs: fitted at 2004 launches of decode_rows_config's geometries (400
+// matrices of 400..24576 x 512..12288, four formats).  An iteration of a wave takes its time once for
+// every one that runs before it, in its round, the rounds of its workgroup and the workgroups that
+// share its CU; K slices add the arrival of the last one and the planes it adds.  96 % of the launches
+// take 0.81-1.18 times that; the furthest off are 16 slices of a few columns (dearer here than they
+// are, by up to 1.4) and eight of long int8 rows (cheaper, 0.76).
+double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
+  struct Cost {
+    double base, sliced, iteration, round, plane;
+  };
+  static const Cost costs[3][2] = {
+      {{5.59, 1.00, 0.59, 0.31, 0.30}, {6.51, 0.72, 0.84, 0.72, 0.63}},   // int4, up to 32 rows and up to 64
+      {{4.89, 1.73, 0.55, 0.21, 0.27}, {5.52, 1.61, 0.55, 0.49, 0.57}},   // int8 in groups
+      {{4.93, 1.73, 0.33, 0.35, 0.29}, {5.46, 1.76, 0.39, 0.62, 0.54}}};  // int8 per row
+  const Cost& t = costs[p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)][p.m <= 32 ? 0 : 1];
+  const int kper = p.format == TLHIP_FMT_INT4_GROUPED ? 128 : 64;
+  const int kw = c.p2 == 0 ? c.p0 : c.p2, ks = c.p3 < 1 ? 1 : c.p3, per_wg = c.p0 / kw;
+  const int64_t nblocks = (p.n + 15) / 16, wgblocks = (nblocks + per_wg - 1) / per_wg, slice = (p.k / kper + ks - 1) / ks;
+  MfmaGeometry geo;
+  if (!mfma_geometry(nblocks, slice * kper, p.m, c.p0, kw, ks, line_patch_bytes(c), &geo)) return 1e9;
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int64_t sets = geo.grid / ks, rounds = (wgblocks + sets - 1) / sets, shared = (geo.grid + cus - 1) / cus;
+  return t.base + (double)(rounds * shared) * (t.iteration * (double)slice / kw + t.round) +
+         (ks > 1 ? t.sliced + t.plane * (double)ks * (double)wgblocks / (double)sets : 0.0);
+}
+
 // The problems of a group: same activations and rows, one shape class; N, pointers and
 // epilogues per problem.  The configuration is checked against the group's total rows.
 bool gemv_mfma_group_applicable(const Problem* ps, int count, const tlhip_kernel_config_t& c, const char** why) {
