@@ -333,6 +333,29 @@ def test_rows_take_the_form_that_measured_faster(fmt, g, n, k, m, width):
     assert chunk.value == 64 and c[0] == L.VARIANT_GEMV_MFMA and c[5] == width and (c[2] == 0) == (width > 0), (chunk.value, c)
 
 
+@pytest.mark.parametrize("n,k,width", [
+    (12288, 4096, 3), (4096, 4096, 1),  # in the file: 20.7 and 14.2 us
+    (5120, 4096, 2), (6144, 4096, 2), (8192, 4096, 2),  # the nearer one's width / two blocks: 24.5 / 15.3, 24.5 / 15.5, 19.7 / 16.1
+    (12800, 4096, 0), (13312, 4096, 0), (14336, 4096, 0), (16384, 4096, 0),  # ... / K slices: 36.8 / 27.1 up to 37.3 / 28.0
+    (7010, 3328, 2),  # 21.8 / 13.3
+])
+def test_a_tuned_width_stays_with_its_own_columns(n, k, width):
+    """64 rows of int4 beside the shipped file's winners that keep all of K in a workgroup."""
+    lib = L.load()
+    before = T.exportTuningCache()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    w, c = L.QWeight(L.FMT_INT4_GROUPED, 32, n, k, ptr, ptr), L.KernelConfig()
+    try:
+        T.clearTuningCache()
+        T.importTuningCache(open(os.path.join(os.path.dirname(T.__file__), "tuning", "mi355x.json")).read())
+        assert lib.tlhip_selected_config(ctypes.byref(w), L.F16, 64, L.F16, ctypes.byref(c)) == 0
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(before)
+    assert c.variant == L.VARIANT_GEMV_MFMA and c.p4 == width, c.as_tuple()
+
+
 @pytest.mark.parametrize("m", [1, 3, 5, 16])
 def test_f32_rows_have_one_limit_of_k(m):
     """K up to 28672 (one f32 row in LDS), however many rows a call has: longer K selects the

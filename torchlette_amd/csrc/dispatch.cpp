@@ -201,6 +201,7 @@ bool config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const c
 }
 
 tlhip_kernel_config_t default_valu_config(const Problem& p);
+bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out);
 
 // The numbers the default routing was fitted with on MI355X: measurements, not structure.
 // They live next to the tuned entries: the tuning file may carry a "model" object that
@@ -707,10 +708,19 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     // at M = 16; a prefill winner is fitted to its number of tiles: the 256 x 128 tile
     // that wins M = 512 at 12288 x 4096 took 71 us at M = 256 against 54 us for the default)
     if (e.m != p.m) continue;
+    // The form that keeps all of K in a workgroup is fitted to its number of workgroups (the
+    // winner's three blocks of columns are 256 workgroups at 12288 x 4096, 64 rows, and two rounds of
+    // them at 14336 x 4096: 37.1 us against 27.4 for K slices).  What carries over is that the rows go
+    // in one launch; the form and its width are the problem's own.
+    tlhip_kernel_config_t c = e.config;
+    Problem there = p;
+    there.n = e.n;
+    there.k = e.k;
+    if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     const double d = dn + 2.0 * dk + dm;  // K decides whether the activations fit LDS: weigh it
-    if (d < best && config_applicable(p, e.config, nullptr)) {
+    if (d < best && config_applicable(p, c, nullptr)) {
       best = d;
-      *out = e.config;
+      *out = c;
       found = true;
     }
   }
