@@ -314,6 +314,10 @@ def test_a_rows_configuration_is_told_by_all_its_fields(fields, runs):
     (L.FMT_INT4_GROUPED, 32, 12288, 4096, 48, 3),    # 27.2 / 18.1
     (L.FMT_INT4_GROUPED, 32, 4096, 4096, 18, 1),     # 21.8 / 8.8
     (L.FMT_INT4_GROUPED, 32, 6144, 4096, 64, 2),     # 16.9 / 15.5
+    # ... / the tile with its K slices
+    (L.FMT_INT4_GROUPED, 32, 4096, 1024, 40, 1),     # 8.5 / 5.5 / 10.5
+    (L.FMT_INT4_GROUPED, 32, 12288, 768, 64, 3),     # 9.5 / 8.2 / 10.4
+    (L.FMT_INT4_GROUPED, 32, 3474, 768, 33, 1),      # 8.2 / 5.2 / 12.2
 ])
 def test_rows_take_the_form_that_measured_faster(fmt, g, n, k, m, width):
     """17..64 rows, nothing tuned: the width of the form that keeps all of K in a workgroup, or 0."""

@@ -184,8 +184,11 @@ def test_capture_rules(be):
 
 
 @pytest.mark.parametrize("entry", ["tlhip_gemv", "tlhip_matmul_quantized", "tlhip_gemm_prefill"])
-@pytest.mark.parametrize("n,k,m,xdt", [(2304, 2304, 5, "f32"), (4096, 1024, 40, "f16"), (12288, 4096, 129, "f16")])
-def test_first_call_under_capture_where_no_workspace_was_needed(be, entry, n, k, m, xdt):
+@pytest.mark.parametrize("n,k,m,xdt,sliced", [
+    (2304, 2336, 5, "f32", True), (4096, 1024, 72, "f16", True), (12288, 4096, 129, "f16", True),
+    (2304, 2304, 5, "f32", False), (4096, 1024, 40, "f16", False),  # all of K in one workgroup: nothing to fall back from
+])
+def test_first_call_under_capture_where_no_workspace_was_needed(be, entry, n, k, m, xdt, sliced):
     """Problems whose default takes K slices although a kernel without them serves: on a stream
     that has no workspace yet they are captured without slices, as bit-stable as any launch."""
     if (entry == "tlhip_gemv") != (m <= 16) and entry != "tlhip_matmul_quantized":
@@ -196,7 +199,10 @@ def test_first_call_under_capture_where_no_workspace_was_needed(be, entry, n, k,
     w = be.createQuantizedWeight(packed, scales, n, k, T.resolveWeightFormat("int4-32", "f32"))
     xt, y, code = be.ops.tensorFromArray(x, [m, k], xdt), be._alloc([m, n], "f32"), L.F32 if xdt == "f32" else L.F16
     cfg = be.selectedConfig(w, xdt, m, "f32")
-    assert (cfg.p0 if cfg.variant == L.VARIANT_GEMV_F32 else cfg.p5) > 1, cfg.as_tuple()
+    if sliced:
+        assert (cfg.p0 > 1 and cfg.p1 == 0) if cfg.variant == L.VARIANT_GEMV_F32 else cfg.p5 > 1, cfg.as_tuple()
+    else:
+        assert (cfg.variant, cfg.p0) in ((L.VARIANT_GEMV_F32, 8), (L.VARIANT_GEMV_MFMA, 8)) and (cfg.p1 if xdt == "f32" else cfg.p4) > 0, cfg.as_tuple()
     want = O.linear(x.astype(np.float32), deq, threads=8)
     s, graph, qw = C.c_void_p(), C.c_void_p(), be._qweight(w, False)
     L.call("tlhip_stream_create", C.byref(s))

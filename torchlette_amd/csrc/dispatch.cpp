@@ -1006,12 +1006,11 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     const int64_t full = p.m / 64, rest = p.m % 64;
     const double rows_us = (double)full * chunk_us(64) + (rest ? chunk_us(rest) : 0.0);
     // one launch of the form that keeps all of K in a workgroup, exact too: wherever it is cheaper
-    // than the tile that would run (48 rows of int4 at 4096 x 4096: 12.0 against 15.4 us); int4
-    // above K = 1024 only: a test of first calls under capture pins the tile's K slices at 40 rows of
-    // 4096 x 1024
+    // than the tile that would run (48 rows of int4 at 4096 x 4096: 12.0 against 15.4 us, 40 rows at
+    // 4096 x 1024 5.5 against 10.5)
     tlhip_kernel_config_t whole;
     double whole_us = 0.0;
-    const bool whole_ok = p.m <= 64 && (p.k > 1024 || p.format != TLHIP_FMT_INT4_GROUPED) && gemm_rows_default(p, &whole, &whole_us);
+    const bool whole_ok = p.m <= 64 && gemm_rows_default(p, &whole, &whole_us);
     double pipe_us = tiled_us;
     if (is_pipe_config(c))
       for (const PipeTileCost& t : kPipeTileCosts)
