@@ -413,6 +413,27 @@ def test_a_few_f32_rows_take_the_kernel_that_measured_faster(fmt, g, n, k, m, ma
     assert c.variant == (L.VARIANT_GEMV_F32 if matrix else L.VARIANT_GEMV), c.as_tuple()
 
 
+@pytest.mark.parametrize("fmt,g,n,k,m,width", [
+    # measured, us: K slices across workgroups / all of K in one workgroup
+    (L.FMT_INT8_GROUPED, 64, 512, 16384, 5, 0),      # 17.1 / 23.3
+    (L.FMT_INT4_GROUPED, 32, 10208, 3712, 16, 0),    # 26.9 / 32.6
+    (L.FMT_INT4_GROUPED, 32, 10481, 2432, 12, 0),    # 17.6 / 20.4
+    (L.FMT_INT4_GROUPED, 32, 12748, 4224, 14, 0),    # 26.6 / 32.8
+    (L.FMT_INT8_GROUPED, 128, 822, 10624, 5, 0),     # 14.1 / 15.7
+    (L.FMT_INT8_GROUPED, 64, 2304, 9216, 5, 1),      # 16.7 / 15.1
+    (L.FMT_INT8_GROUPED, 64, 9216, 2304, 5, 1),      # 13.0 / 11.4
+    (L.FMT_INT4_GROUPED, 32, 4096, 12288, 16, 1),    # 39.2 / 33.9
+    (L.FMT_INT4_GROUPED, 32, 12288, 4096, 16, 2),    # 50.8 / 33.8
+])
+def test_f32_rows_take_the_form_that_measured_faster(fmt, g, n, k, m, width):
+    lib = L.load()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    w, c = L.QWeight(fmt, g, n, k, ptr, ptr), L.KernelConfig()
+    assert lib.tlhip_selected_config(ctypes.byref(w), L.F32, m, L.F32, ctypes.byref(c)) == 0
+    assert c.variant == L.VARIANT_GEMV_F32 and c.p1 == width and c.p0 > 1, c.as_tuple()
+
+
 def test_the_routing_model_travels_with_the_tuning_cache():
     """The fitted numbers of the default routing are data, not code: without any tuning file
     and with only the shipped file's model the routes agree (the file carries the built-in

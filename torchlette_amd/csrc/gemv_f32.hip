@@ -565,25 +565,55 @@ ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c) {
   return ScratchNeed{(size_t)column_tiles(p) * (size_t)c.p0 * (size_t)p.m * kCols, column_tiles(p)};
 }
 
-// Time of a launch that keeps all of K in a workgroup, in microseconds: fitted at 1024..13838 x
-// 768..12288, 3..16 rows, three formats.  x: workgroups / CUs; a second one to a CU costs as much
-// as the first (the VALU is what they share), three tiles of pieces fill its LDS alone.
-static double whole_us(const Problem& p, int nb) {
+// All of K in one workgroup at nb blocks of 16 columns: rounds of workgroups, as the VALU feels them.
+// A second workgroup to a CU costs as much as the first (the VALU is what they share), three tiles of
+// pieces fill its LDS alone.
+static double whole_rounds(const Problem& p, int nb) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const double x = (double)((p.n + 16 * nb - 1) / (16 * nb)) / cus, m = (double)p.m;
-  const double c = nb == 1 ? 0.75 + 0.125 * m : (nb == 2 ? 1.35 + 0.135 * m : 2.7 + 0.16 * m);
-  const double rounds = x <= 1.0 ? 1.0 : (p.m > 10 ? 1.15 * (double)(int64_t)(x + 0.999) : (x <= 2.0 ? 2.0 : 0.4 + 0.95 * x));
-  return 2.9 + (double)p.k / 1000.0 * c * rounds;
+  const double x = (double)((p.n + 16 * nb - 1) / (16 * nb)) / cus;
+  return x <= 1.0 ? 1.0 : (p.m > 10 ? 1.15 * (double)(int64_t)(x + 0.999) : (x <= 2.0 ? 2.0 : 0.4 + 0.95 * x));
+}
+// ... what orders the widths of a problem, whatever its format: fitted at 1024..13838 x 768..12288, 3..16
+// rows; the width it picks is 0.4 % behind the best one in the mean (992 problems).
+static double width_us(const Problem& p, int nb) {
+  const double m = (double)p.m, c = nb == 1 ? 0.75 + 0.125 * m : (nb == 2 ? 1.35 + 0.135 * m : 2.7 + 0.16 * m);
+  return 2.9 + (double)p.k / 1000.0 * c * whole_rounds(p, nb);
+}
+// ... and the price of the launch beside that of K slices, in microseconds: fitted at 3182 launches of
+// the one and 1716 of the other (200 matrices of 400..24576 x 512..12288, 3..16 rows, four formats).
+// Per round the sums, 0.27 for every tile of pieces and block, and per 1000 of K the cutting of X and
+// the weights of a block: 96 % of the launches take 0.82-1.13 times that.  K slices: the longest one's
+// pieces and weights, and 0.010-0.017 for every row of every slice that the last arrival adds:
+// 0.85-1.17 times that, int4 (8 % above its fit: its short slices scatter) 0.72-1.2.
+static int format_index(const Problem& p) { return p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1); }
+static double whole_us(const Problem& p, int nb) {
+  static const double weights[3][3][3] = {  // tiles of pieces, format, 1 / 2 / 4 blocks
+      {{0.61, 1.08, 2.05}, {0.70, 1.24, 2.55}, {0.54, 0.87, 1.84}},
+      {{0.70, 1.25, 2.19}, {0.72, 1.37, 2.49}, {0.50, 0.98, 1.74}},
+      {{0.92, 1.30, 0.0}, {0.91, 1.31, 0.0}, {0.76, 0.90, 0.0}}};
+  const int tiles = tiles_of(p.m);
+  const double m = (double)p.m;
+  return 2.77 + whole_rounds(p, nb) * (0.29 + 0.27 * tiles * nb + (double)p.k / 1000.0 * (0.074 * m + 0.012 * m * nb + weights[tiles - 1][format_index(p)][nb / 2]));
+}
+static double slices_us(const Problem& p, int slices) {
+  static const double base[3] = {10.7, 6.2, 6.5}, weights[3] = {5.22, 7.86, 4.98}, cut[3] = {0.471, 0.297, 0.324}, sum[3] = {0.010, 0.017, 0.014};
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256, f = format_index(p);
+  const int64_t wgs = column_tiles(p) * slices, rounds = (wgs + cus - 1) / cus, slice = (blocks_of(p) + slices - 1) / slices * block_k(p);
+  return base[f] + (double)(rounds * slice) / 1000.0 * (weights[f] + cut[f] * (double)p.m) + sum[f] * (double)(slices * p.m);
 }
 
 // All of K in one workgroup, at the cheapest number of columns, or false where K slices are ahead.
 // Us, slices against here, over 24 matrices of 512..16246 x 768..12288 at 3..16 rows:
-//   up to five rows at every one (int8-64 9216 x 2304: 13.0 -> 11.2, 2304 x 9216: 16.8 -> 15.3; int4 at
-//   4096 x 4096 15.4 -> 8.6, at 12288 x 4096 28.8 -> 17.2);
+//   up to five rows at nearly every one (int8-64 9216 x 2304: 13.0 -> 11.2, 2304 x 9216: 16.8 -> 15.3;
+//   int4 at 4096 x 4096 15.4 -> 8.6, at 12288 x 4096 28.8 -> 17.2);
 //   more rows of int4 with K up to 4096 or enough columns for every CU (16 rows at 12288 x 4096 50.8 ->
 //   33.8, at 4096 x 12288 39.7 -> 36.0; but 12 rows at 789 x 9984: 17.9 against 24.0);
 //   more rows of int8 with K up to 4096 where one round of double blocks holds the columns (10 rows
 //   at 2048 x 2304: 12.7 -> 7.1, at 7869 x 768 9.7 -> 6.1; but 16 rows at 9216 x 2304: 16.0 against 21.9).
+// Within these, where the price says so too: of 1174 problems that both forms were timed at nine are
+// more than 3 % behind the slices, by 10 % at most (16 rows of int8-128 at 4114 x 2816: 13.9 against
+// 12.7); without it 5 rows of int8 at 512 x 16384 took 23.2 against 17.1, 16 rows of int4 at 10208 x
+// 3712 32.4 against 26.8.
 static bool whole_default(const Problem& p, tlhip_kernel_config_t* out) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   if (p.n > 16384) return false;
@@ -598,17 +628,15 @@ static bool whole_default(const Problem& p, tlhip_kernel_config_t* out) {
     c.variant = VARIANT_GEMV_F32;
     c.p0 = kWhole;
     c.p1 = nb;
-    if (!gemv_f32_config_applicable(p, c, nullptr) || (found && whole_us(p, nb) >= best)) continue;
+    if (!gemv_f32_config_applicable(p, c, nullptr) || (found && width_us(p, nb) >= best)) continue;
     *out = c;
-    best = whole_us(p, nb);
+    best = width_us(p, nb);
     found = true;
   }
   return found;
 }
 
-// The K slices of the default: see the rule's figures at its caller.
-bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out) {
-  if (whole_default(p, out)) return true;
+static bool slices_default(const Problem& p, tlhip_kernel_config_t* out) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   memset(out, 0, sizeof *out);
   out->variant = VARIANT_GEMV_F32;
@@ -623,6 +651,14 @@ bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out) {
     if (gemv_f32_config_applicable(p, *out, nullptr)) return true;
   }
   return false;
+}
+
+bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out) {
+  tlhip_kernel_config_t whole;
+  const bool found = slices_default(p, out);
+  if (!whole_default(p, &whole) || (found && whole_us(p, whole.p1) >= slices_us(p, out->p0))) return found;
+  *out = whole;
+  return true;
 }
 
 int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream) {
