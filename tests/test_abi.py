@@ -360,6 +360,29 @@ def test_a_tuned_width_stays_with_its_own_columns(n, k, width):
     assert c.variant == L.VARIANT_GEMV_MFMA and c.p4 == width, c.as_tuple()
 
 
+@pytest.mark.parametrize("n,k", [(8192, 4096), (6144, 4096), (4224, 2304)])
+def test_a_tuned_width_of_f32_rows_stays_with_its_own_columns(n, k):
+    """Five rows of int8 beside a winner that keeps all of K in workgroups of 16 columns: a neighbour
+    has the form and the width of its own default (us, the winner's width / the default: 15.8 / 14.0, 14.9 /
+    13.2, 8.6 / 7.7)."""
+    lib = L.load()
+    before = T.exportTuningCache()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    tuned, w, c = L.QWeight(L.FMT_INT8_GROUPED, 64, 4096, 4096, ptr, ptr), L.QWeight(L.FMT_INT8_GROUPED, 64, n, k, ptr, ptr), L.KernelConfig()
+    try:
+        T.clearTuningCache()
+        assert lib.tlhip_selected_config(ctypes.byref(w), L.F32, 5, L.F32, ctypes.byref(c)) == 0
+        own, winner = c.as_tuple(), L.KernelConfig.of(L.VARIANT_GEMV_F32, 8, 1)
+        assert lib.tlhip_tune_cache_seed(ctypes.byref(tuned), L.F32, 5, L.F32, ctypes.byref(winner)) == 0
+        assert lib.tlhip_selected_config(ctypes.byref(tuned), L.F32, 5, L.F32, ctypes.byref(c)) == 0 and c.as_tuple() == winner.as_tuple()
+        assert lib.tlhip_selected_config(ctypes.byref(w), L.F32, 5, L.F32, ctypes.byref(c)) == 0
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(before)
+    assert c.as_tuple() == own
+
+
 @pytest.mark.parametrize("m", [1, 3, 5, 16])
 def test_f32_rows_have_one_limit_of_k(m):
     """K up to 28672 (one f32 row in LDS), however many rows a call has: longer K selects the

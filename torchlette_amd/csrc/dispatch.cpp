@@ -708,15 +708,18 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     // at M = 16; a prefill winner is fitted to its number of tiles: the 256 x 128 tile
     // that wins M = 512 at 12288 x 4096 took 71 us at M = 256 against 54 us for the default)
     if (e.m != p.m) continue;
-    // The form that keeps all of K in a workgroup is fitted to its number of workgroups (the
+    // The forms that keep all of K in a workgroup are fitted to their number of workgroups (the
     // winner's three blocks of columns are 256 workgroups at 12288 x 4096, 64 rows, and two rounds of
-    // them at 14336 x 4096: 37.1 us against 27.4 for K slices).  What carries over is that the rows go
-    // in one launch; the form and its width are the problem's own.
+    // them at 14336 x 4096: 37.1 us against 27.4 for K slices; f32 rows of 4096 x 4096, one block, at 8192
+    // x 4096: 15.8 against 14.0 for two, 5 rows of int8-64, and 28.0 against 18.5, 16 of int4).  What
+    // carries over is that the rows go in one launch, or to the kernel of f32 rows; the form and its
+    // width are the problem's own.
     tlhip_kernel_config_t c = e.config;
     Problem there = p;
     there.n = e.n;
     there.k = e.k;
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
+    if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
     const double d = dn + 2.0 * dk + dm;  // K decides whether the activations fit LDS: weigh it
     if (d < best && config_applicable(p, c, nullptr)) {
       best = d;
