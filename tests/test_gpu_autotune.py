@@ -173,3 +173,32 @@ def test_lazy_tuning_at_first_dispatch_then_cached(be):
         T.setAutotuneEnabled(False)
         T.clearTuningCache()
         T.importTuningCache(open(TUNING).read())
+
+
+@pytest.mark.parametrize("base", [(8, 1), (5, 0)])
+def test_the_quick_search_of_f32_rows_times_slices_and_widths(be, base, capfd, monkeypatch):
+    """Both forms of the f32 kernel are neighbours of either: every number of slices and every width
+    that the problem takes, the choice itself, its default and the VALU kernel."""
+    n, k, m = 1024, 2304, 5
+    rng = np.random.default_rng(9)
+    packed, scales, _ = make_weight("int8-grouped", n, k, 64, rng)
+    w = be.createQuantizedWeight(packed, scales, n, k, T.resolveWeightFormat("int8-64", "f32"))
+    xt, out, qw = be.ops.tensorFromArray(make_x(m, k, "f32", rng), [m, k], "f32"), be._alloc([m, n], "f32"), be._qweight(w, False)
+    T.clearTuningCache()
+    try:
+        own = be.selectedConfig(w, "f32", m, "f32").as_tuple()
+        fields = {(s, 0) for s in (1, 2, 4, 8, 16, 32)} | {(8, c) for c in (1, 2, 4)} | {base}
+        want = {own}
+        for f in fields:
+            cfg = L.KernelConfig.of(L.VARIANT_GEMV_F32, *f)
+            if L.load().tlhip_tune_cache_seed(C.byref(qw), L.F32, m, L.F32, C.byref(cfg)) == 0:
+                want.add(cfg.as_tuple())
+        be.seedPerShapeMatmulChoice(w, "f32", m, "f32", L.KernelConfig.of(L.VARIANT_GEMV_F32, *base))
+        monkeypatch.setenv("TORCHLETTE_DEBUG_AUTOTUNE", "1")
+        options = L.AutotuneOptions(3, 1, 1, 1, 0.0, 0)
+        L.call("tlhip_autotune_pool", C.byref(qw), 1, xt.ptr, L.F32, m, out.ptr, L.F32, None, C.byref(options), None, None)
+        said = capfd.readouterr().err
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(open(TUNING).read())
+    assert f" {len(want) + 1} candidates" in said and len(want) >= 9, (want, said)

@@ -1132,8 +1132,19 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       vary(5, {0, 1});
       break;
     case VARIANT_GEMV_F32:
-      vary(0, {1, 2, 4, 8, 16, 32});
-      vary(1, {0, 1, 2, 4});
+      // slices, and the widths of the form that keeps all of K in a workgroup, whichever the base is
+      for (int slices : {1, 2, 4, 8, 16, 32}) {
+        tlhip_kernel_config_t c = base;
+        c.p0 = slices;
+        c.p1 = 0;
+        push(c);
+      }
+      for (int cols : {1, 2, 4}) {
+        tlhip_kernel_config_t c = base;
+        c.p0 = 8;
+        c.p1 = cols;
+        push(c);
+      }
       break;
     case VARIANT_GEMV_WAVE:
       vary(0, {4, 8});
