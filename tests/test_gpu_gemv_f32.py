@@ -53,13 +53,14 @@ def test_edges(be, fmt, g, m, n, k, slices):
         assert rel_l2(got[r], want[r]) <= 2e-6, r
 
 
-def test_default_route_and_values_that_are_not_finite(be):
+@pytest.mark.parametrize("slices", [0, 3])  # the default, all of K in one workgroup; and K slices
+def test_default_route_and_values_that_are_not_finite(be, slices):
     n, k, m = 1024, 2304, 5
     rng = np.random.default_rng(3)
     x = make_x(m, k, "f32", rng, std=0.5)
     x[1] *= np.float32(1e-30)
     x[2, 7], x[3, 9] = np.inf, np.nan
-    got, want, magnitudes = product(be, "int8-grouped", 64, n, k, x, 0, rng)
+    got, want, magnitudes = product(be, "int8-grouped", 64, n, k, x, slices, rng)
     for r in (0, 1, 4):
         assert rel_l2(got[r], want[r]) <= 2e-6, r
     assert np.array_equal(np.isnan(got[2]), np.isnan(want[2])) and np.array_equal(np.sign(got[2]), np.sign(want[2]), equal_nan=True)

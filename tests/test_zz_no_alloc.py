@@ -97,9 +97,13 @@ def test_noalloc_takes_the_route_gemv_takes(be, n, k, m):
     assert np.array_equal(again.view(np.uint32), got.view(np.uint32))
 
 
-@pytest.mark.parametrize("n,k,m", [(2304, 9216, 5), (2304, 768, 3), (300, 4096, 16), (12288, 4096, 16), (16384, 4096, 16)])
-def test_noalloc_takes_f32_activations_through_the_kernel_gemv_takes(be, n, k, m):
-    """K slices of the f32 kernel, the last two with more partial sums than 4 MiB: the same bits as
+@pytest.mark.parametrize("n,k,m,sliced", [
+    (2304, 9248, 5, True), (2304, 800, 3, True), (300, 4128, 16, True), (512, 12288, 16, True),
+    (12288, 4128, 16, True), (20000, 4096, 16, True),  # more partial sums than 4 MiB
+    (2304, 9216, 5, False), (2304, 768, 3, False), (300, 4096, 16, False), (12288, 4096, 16, False), (16384, 4096, 16, False),
+])
+def test_noalloc_takes_f32_activations_through_the_kernel_gemv_takes(be, n, k, m, sliced):
+    """K slices of the f32 kernel, and the form that keeps all of K in a workgroup: the same bits as
     tlhip_gemv, and again behind a call of f16 activations that used the same counters."""
     rng = np.random.default_rng(n + k + m)
     packed = rng.integers(0, 2 ** 32, n * k // 8, dtype=np.uint64).astype(np.uint32)
@@ -107,7 +111,8 @@ def test_noalloc_takes_f32_activations_through_the_kernel_gemv_takes(be, n, k, m
     w = be.createQuantizedWeight(packed, scales, n, k, T.resolveWeightFormat("int4-32", "f32"))
     xt = be.ops.tensorFromArray(make_x(m, k, "f32", rng), [m, k], "f32")
     cfg = be.selectedConfig(w, "f32", m, "f32")
-    assert cfg.variant == L.VARIANT_GEMV_F32 and cfg.p0 > 1, cfg.as_tuple()
+    assert cfg.variant == L.VARIANT_GEMV_F32 and (cfg.p0 > 1 and cfg.p1 == 0 if sliced else cfg.p1 > 0), cfg.as_tuple()
+    assert not sliced or n < 12288 or cfg.p0 * m * n * 4 > 4 << 20
     out = be._alloc([m, n], "f32")
     qw = be._qweight(w, False)
 
