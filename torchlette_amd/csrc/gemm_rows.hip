@@ -2,9 +2,12 @@
 // matrix cores as they are and every group's sum is scaled in f32, as in the decode kernels.
 // Same contract and reference route as gemv.hip (src/backend/webgpu/matmul/gemv.ts:365-466).
 //
-// What bounds it: the activations' way to the matrix cores.  64 rows of K = 4096 are 512 KB,
-// three times a CU's LDS, and every workgroup needs all of them from its L2; the weights of a
-// workgroup's columns are a tenth to a third of that.  Hence:
+// What bounds it: its own instructions (X into LDS and out of it as operands, the dequantising, the
+// products), then the weights' way from memory, one or two steps ahead of a wave; the activations' way
+// comes last, although every workgroup needs all of X (64 rows of K = 4096 are 512 KB, three times a
+// CU's LDS) from its L2.  Int4, K = 4096, one round of 256 workgroups, us as it is / X from a buffer of no bytes
+// / the weights so / both: 48 rows at one block of columns 11.9 / 10.9 / 9.1 / 8.3, at two 15.5 / 14.4 / 10.6 / 10.2,
+// at three 18.1 / 15.1 / 12.1 / 12.8; 64 rows at three 20.9 / 18.3 / 16.6 / 15.7.  Hence:
 //   * A workgroup owns 16 NB columns of Y and all of K, so that nothing is combined between
 //     workgroups: no planes of partial sums, no second launch, no workspace.
 //   * Its eight waves take K in turn, 128 at a time, each alone with its part until one
@@ -14,8 +17,7 @@
 //   * An operand of X feeds NB products and a weight, dequantised once, MT.
 // One launch, us, best kernel before -> here: int4-32 12288 x 4096 at 48 / 64 rows 27.2 -> 18.1, 27.6 ->
 // 20.9; 4096 x 4096 at 48 rows 14.9 -> 12.1; int8-64 12288 x 4096 at 17..32 rows 27-28 -> 21-22, 7179 x
-// 896 at 40 rows 13.3 -> 7.0.  18.1 us are 1.5 TB/s of weights and 260 TFLOP/s: 3.5 us of launch, first
-// loads and last sums, the rest the 100 MB of X that 256 CUs fetch (25-30 bytes a clock and CU).
+// 896 at 40 rows 13.3 -> 7.0.  18.1 us are 1.5 TB/s of weights and 260 TFLOP/s.
 // Rearranging X for the cheaper int4 unpacking, or its addresses by lane, moved nothing.
 //   * Buffer loads: rows past M, columns past N and steps past K read zero and cost no traffic,
 //     so that the loop has no branch around a load.
@@ -344,7 +346,9 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 }
 
 int row_tiles_of(int64_t m) { return (int)((m + 15) / 16); }
-// The column blocks whose instance fits 256 registers a lane without spilling.
+// The column blocks whose instance fits 256 vector registers a lane without spilling one; the fullest
+// (int4, three blocks of 48 rows) uses all of them, three more 249 to 253.  Four row tiles need 16
+// buffer descriptors a step and spill up to 20 scalar registers, to lanes of a vector register.
 constexpr int most_columns(int format, int mt) {
   return format == TLHIP_FMT_INT4_GROUPED ? (mt == 4 ? 3 : 4) : (mt == 2 ? 4 : (mt == 3 ? 3 : 2));
 }
