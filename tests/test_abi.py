@@ -314,6 +314,15 @@ def test_a_rows_configuration_is_told_by_all_its_fields(fields, runs):
     (L.FMT_INT4_GROUPED, 32, 12288, 4096, 48, 3),    # 27.2 / 18.1
     (L.FMT_INT4_GROUPED, 32, 4096, 4096, 18, 1),     # 21.8 / 8.8
     (L.FMT_INT4_GROUPED, 32, 6144, 4096, 64, 2),     # 16.9 / 15.5
+    (L.FMT_INT8_ROW, 0, 4491, 6272, 56, 2),          # 31.5 / 20.8
+    (L.FMT_INT8_GROUPED, 128, 4816, 6528, 51, 2),    # 33.9 / 26.3
+    (L.FMT_INT8_GROUPED, 64, 3520, 1152, 55, 1),     # 8.3 / 6.1
+    (L.FMT_INT8_ROW, 0, 2112, 10496, 63, 1),         # 35.3 / 24.3
+    (L.FMT_INT4_GROUPED, 32, 4608, 9472, 54, 2),     # 38.5 / 29.8
+    # the tile with its K slices / all of K
+    (L.FMT_INT8_GROUPED, 64, 12288, 4096, 40, 3),    # 28.5 / 23.3
+    (L.FMT_INT8_GROUPED, 64, 3072, 7424, 43, 1),     # 27.8 / 17.9
+    (L.FMT_INT4_GROUPED, 32, 19513, 2432, 43, 3),    # 30.9 / 20.2
     # ... / the tile with its K slices
     (L.FMT_INT4_GROUPED, 32, 4096, 1024, 40, 1),     # 8.5 / 5.5 / 10.5
     (L.FMT_INT4_GROUPED, 32, 12288, 768, 64, 3),     # 9.5 / 8.2 / 10.4

@@ -917,17 +917,17 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return false;
 }
 
-// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip) where it is under nine
-// tenths of the former's price: of 1834 problems timed with both, five are more than 3 % behind the
-// former (the furthest, 48 rows of int4 at 20403 x 512: 11.3 against 9.9 us) and all are 1.4 % behind
-// the faster one in the mean.  Us, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0
-// against 22.2, but 2008 x 8192 12.1 against 18.2; int4 12288 x 4096, 48 rows 27.2 against 18.1, but
-// 2610 x 11520 23.0 against 25.1.
+// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip), whichever price is
+// lower: of 1936 problems timed with both, most of them close, the choice is 0.5 % behind the faster
+// one in the mean and at 49 more than 3 % behind the former (a bar of nine tenths instead: 5 %
+// behind in the mean).  Us, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0 against 22.2,
+// per row 4491 x 6272, 56 rows 31.5 against 20.8, but int8-64 2008 x 8192, 32 rows 12.1 against 18.2; int4
+// 12288 x 4096, 48 rows 27.2 against 18.1, but 2610 x 11520 23.0 against 25.1.
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
   const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
-  if (!gemm_rows_default(p, &whole, &us) || (found && us >= 0.9 * gemv_mfma_rows_us(p, *out))) return found;
+  if (!gemm_rows_default(p, &whole, &us) || (found && us >= gemv_mfma_rows_us(p, *out))) return found;
   *out = whole;
   return true;
 }
@@ -1014,10 +1014,12 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     tlhip_kernel_config_t whole;
     double whole_us = 0.0;
     const bool whole_ok = p.m <= 64 && gemm_rows_default(p, &whole, &whole_us);
+    // (up to 64 rows the eight-wave tiles take 1.14 times their price in the median: 4/3 and the
+    // model's 0.9 are the line that was ahead of 1.05 .. 1.4 at 1116 problems timed with both)
     double pipe_us = tiled_us;
     if (is_pipe_config(c))
       for (const PipeTileCost& t : kPipeTileCosts)
-        if (c.p0 == t.bm && c.p1 == t.bn) pipe_us = pipe_launch_us(p, t, c.p5 > 1 ? c.p5 : 1);
+        if (c.p0 == t.bm && c.p1 == t.bn) pipe_us = 4.0 / 3.0 * pipe_launch_us(p, t, c.p5 > 1 ? c.p5 : 1);
     if (rows_us < g_model.rows_break_even * tiled_us || (whole_ok && whole_us < g_model.rows_break_even * pipe_us)) {
       bool ok = true;
       Route q{64, c, c};

@@ -394,16 +394,21 @@ bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
   return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
 }
 
-// The cheapest number of column blocks and its time in microseconds, or false.  Fitted at 1200
-// problems (150 matrices of 400..24576 x 512..12288, 17..64 rows, four formats): 2.1 us of launch, and
-// per round of workgroups 1.1 us, 0.17 for every block of 16 x 16 sums and, per 4096 of K, the
-// figure below.  98 % of the launches take 0.89-1.12 times that; the width it picks is 0.02 % slower
-// than the best one in the mean.
+// The cheapest number of column blocks and its time in microseconds, or false.  Fitted at 9165
+// launches of 2811 problems (400..24576 x 512..12288, 17..64 rows, four formats, most of them where
+// another kernel is close): launch, and per round of workgroups a constant, the sums of a block and
+// per 4096 of K the figure of the width, a little more for every row above the middle of its tile.
+// One block a workgroup: a second round overlaps the first (two fit a CU up to 32 rows).  96 % of
+// the launches take 0.87-1.12 times that; the width it picks is 0.08 % slower than the best one in the mean.
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
-  static const double walk[3][3][kMaxCols] = {  // format, row tiles, column blocks
-      {{4.9, 7.9, 10.6, 13.0}, {7.7, 10.1, 11.0, 15.3}, {9.4, 10.7, 14.2, 0.0}},    // int4
-      {{6.7, 10.6, 14.8, 18.0}, {9.2, 11.9, 16.1, 0.0}, {9.8, 14.0, 0.0, 0.0}},     // int8 in groups
-      {{6.0, 8.9, 11.8, 14.1}, {8.5, 9.8, 13.6, 0.0}, {9.1, 11.9, 0.0, 0.0}}};      // int8 per row
+  struct Cost {
+    double launch, round, block, walk[kMaxCols];
+  };
+  static const Cost costs[3][3] = {  // format, row tiles
+      {{1.89, 0.66, 0.42, {5.92, 8.13, 10.83, 12.95}}, {1.22, 1.64, 0.51, {7.53, 10.07, 10.61, 15.13}}, {1.07, 1.90, 0.59, {9.17, 10.59, 14.22, 0.0}}},  // int4
+      {{2.01, 0.77, 0.46, {7.34, 10.67, 14.65, 17.53}}, {1.37, 1.98, 0.32, {8.88, 11.56, 15.96, 0.0}}, {1.33, 1.37, 0.61, {9.83, 14.12, 0.0, 0.0}}},    // int8 in groups
+      {{1.29, 1.04, 0.57, {6.29, 8.79, 11.95, 13.84}}, {0.96, 2.01, 0.47, {8.12, 8.56, 13.30, 0.0}}, {1.03, 1.55, 0.68, {8.60, 11.37, 0.0, 0.0}}}};     // int8 per row
+  static const double per_row[3] = {0.008, 0.005, 0.004}, second[3] = {0.80, 0.96, 0.96};
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int format = p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1), mt = row_tiles_of(p.m);
   bool found = false;
@@ -414,8 +419,11 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
     c.p0 = kWaves;
     c.p4 = nb;
     if (!is_rows_config(p, c)) continue;
-    const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb), rounds = (wgs + cus - 1) / cus;
-    const double t = 2.1 + (double)rounds * (1.1 + 0.17 * mt * nb + (double)p.k / 4096.0 * walk[format][mt - 2][nb - 1]);
+    const Cost& cost = costs[format][mt - 2];
+    const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb);
+    const double rounds = 1.0 + (double)((wgs + cus - 1) / cus - 1) * (nb == 1 ? second[mt - 2] : 1.0);
+    const double t = cost.launch + rounds * (cost.round + cost.block * nb +
+                                             (double)p.k / 4096.0 * cost.walk[nb - 1] * (1.0 + per_row[mt - 2] * (double)(p.m - 16 * mt + 8)));
     if (found && t >= *us) continue;
     *out = c;
     *us = t;
