@@ -918,8 +918,8 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
 }
 
 // That form, or the one that keeps all of K in one workgroup (gemm_rows.hip), whichever price is
-// lower: of 1936 problems timed with both, most of them close, the choice is 0.5 % behind the faster
-// one in the mean and at 49 more than 3 % behind the former (a bar of nine tenths instead: 5 %
+// lower: of 1980 problems timed with both, most of them close, the choice is 0.4 % behind the faster
+// one in the mean and at 23 more than 3 % behind the former (a bar of nine tenths instead: 5 %
 // behind in the mean).  Us, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0 against 22.2,
 // per row 4491 x 6272, 56 rows 31.5 against 20.8, but int8-64 2008 x 8192, 32 rows 12.1 against 18.2; int4
 // 12288 x 4096, 48 rows 27.2 against 18.1, but 2610 x 11520 23.0 against 25.1.
@@ -1014,8 +1014,10 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     tlhip_kernel_config_t whole;
     double whole_us = 0.0;
     const bool whole_ok = p.m <= 64 && gemm_rows_default(p, &whole, &whole_us);
-    // (up to 64 rows the eight-wave tiles take 1.14 times their price in the median: 4/3 and the
-    // model's 0.9 are the line that was ahead of 1.05 .. 1.4 at 1116 problems timed with both)
+    // (up to 64 rows the eight-wave tiles take 1.11 times their price in the median, and among other
+    // launches a second one for the K slices costs a little more: 4/3 and the model's 0.9 are 0.5 %
+    // behind the faster one in the mean of 1200 problems timed with both; 48 rows of int4 at 4096 x
+    // 12288, a near draw behind themselves, are 0.9 us ahead of the tile in a decoder layer)
     double pipe_us = tiled_us;
     if (is_pipe_config(c))
       for (const PipeTileCost& t : kPipeTileCosts)

@@ -120,19 +120,20 @@ bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& 
   return mfma_applicable(p, (p.n + 15) / 16, c, why);
 }
 
-// What a launch of 17..64 rows costs: fitted at 1936 launches of decode_rows_config's geometries
-// (400..24576 x 512..12288, four formats).  An iteration of a wave takes its time (more where only one
-// is in flight, 0.6 % more a row) once for every one that runs before it, in its round, the rounds of
-// its workgroup and the workgroups that share its CU; K slices add the arrival of the last one and
-// the planes it adds.  96 % of the launches take 0.85-1.24 times that.
+// What a launch of 17..64 rows costs: fitted at 1980 launches of decode_rows_config's geometries
+// (400..24576 x 512..12288, four formats).  An iteration of a wave, in whole sets of those in flight,
+// takes its time (more where only one is in flight, 0.6 % more a row) once for every one that runs
+// before it, in its round, the rounds of its workgroup and the workgroups that share its CU; K slices
+// add the arrival of the last one and the planes it adds.  96 % of the launches take 0.85-1.25 times
+// that, 80 % 0.93-1.09.
 double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
   struct Cost {
     double base, sliced, iteration, round, plane, alone;
   };
   static const Cost costs[3][2] = {
-      {{5.11, 0.80, 0.62, 0.19, 0.44, 0.03}, {6.06, 0.56, 0.86, 0.64, 0.51, 0.10}},   // int4, up to 32 rows and up to 64
-      {{5.03, 1.81, 0.54, 0.00, 0.08, 0.08}, {6.31, 1.48, 0.51, 0.00, 0.31, 0.14}},   // int8 in groups
-      {{5.05, 2.01, 0.35, 0.22, 0.12, 0.08}, {6.01, 1.80, 0.43, 0.00, 0.41, 0.11}}};  // int8 per row
+      {{4.65, 0.80, 0.64, 0.39, 0.34, 0.03}, {5.58, 1.27, 0.92, 0.43, 0.59, 0.04}},   // int4, up to 32 rows and up to 64
+      {{4.56, 1.57, 0.49, 0.21, 0.17, 0.12}, {5.83, 1.71, 0.49, 0.11, 0.41, 0.11}},   // int8 in groups
+      {{4.51, 1.86, 0.30, 0.47, 0.21, 0.12}, {5.34, 1.76, 0.36, 0.54, 0.53, 0.12}}};  // int8 per row
   const bool few = p.m <= 32;
   const Cost& t = costs[p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)][few ? 0 : 1];
   const int kper = p.format == TLHIP_FMT_INT4_GROUPED ? 128 : 64;
@@ -142,7 +143,8 @@ double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
   if (!mfma_geometry(nblocks, slice * kper, p.m, c.p0, kw, ks, line_patch_bytes(c), &geo)) return 1e9;
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int64_t sets = geo.grid / ks, rounds = (wgblocks + sets - 1) / sets, shared = (geo.grid + cus - 1) / cus;
-  const double iterations = (double)((slice + kw - 1) / kw) * (1.0 + 0.006 * (double)(p.m - (few ? 24 : 48)));
+  const int64_t own = (slice + kw - 1) / kw, in_flight = c.p1 < 1 ? 1 : c.p1;
+  const double iterations = (double)((own + in_flight - 1) / in_flight * in_flight) * (1.0 + 0.006 * (double)(p.m - (few ? 24 : 48)));
   return t.base + (double)(rounds * shared) * (iterations * (t.iteration + (c.p1 == 1 ? t.alone : 0.0)) + t.round) +
          (ks > 1 ? t.sliced + t.plane * (double)ks * (double)wgblocks / (double)sets : 0.0);
 }
