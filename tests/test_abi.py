@@ -303,12 +303,12 @@ def test_a_rows_configuration_is_told_by_all_its_fields(fields, runs):
     (L.FMT_INT8_GROUPED, 64, 2008, 8192, 17, 0),     # 12.7 / 16.4
     (L.FMT_INT8_ROW, 0, 2451, 8192, 32, 0),          # 12.7 / 16.5
     (L.FMT_INT8_ROW, 0, 1253, 6528, 33, 0),          # 12.6 / 16.2
-    (L.FMT_INT8_ROW, 0, 796, 3840, 64, 0),           # 10.6 / 12.4
-    (L.FMT_INT8_GROUPED, 64, 971, 3072, 64, 0),      # 10.6 / 11.8
+    (L.FMT_INT8_ROW, 0, 796, 3840, 64, 1),           # 9.7 / 10.0, with a residual 16.3 / 11.6
+    (L.FMT_INT8_GROUPED, 64, 971, 3072, 64, 1),      # 9.3 / 10.8, 15.9 / 12.2
     (L.FMT_INT4_GROUPED, 32, 16384, 4096, 17, 0),    # 15.7 / 19.0
-    (L.FMT_INT4_GROUPED, 32, 3312, 8960, 56, 0),     # 20.4 / 23.4
+    (L.FMT_INT4_GROUPED, 32, 3312, 8960, 56, 1),     # 21.2 / 23.8, 27.3 / 24.7
     (L.FMT_INT4_GROUPED, 32, 3312, 8960, 128, 0),    # 43.2 / 47.6, 64 rows at a time
-    (L.FMT_INT8_ROW, 0, 2193, 3584, 17, 0),          # 7.7 / 8.7
+    (L.FMT_INT8_ROW, 0, 2193, 3584, 17, 1),          # 7.2 / 6.8, 8.8 / 8.0
     (L.FMT_INT8_GROUPED, 64, 12288, 4096, 32, 3),    # 28.0 / 22.2
     (L.FMT_INT8_ROW, 0, 3371, 3712, 20, 1),          # 20.7 / 9.6
     (L.FMT_INT4_GROUPED, 32, 12288, 4096, 48, 3),    # 27.2 / 18.1
@@ -349,7 +349,9 @@ def test_rows_take_the_form_that_measured_faster(fmt, g, n, k, m, width):
 @pytest.mark.parametrize("n,k,width", [
     (12288, 4096, 3), (4096, 4096, 1),  # in the file: 20.7 and 14.2 us
     (5120, 4096, 2), (6144, 4096, 2), (8192, 4096, 2),  # the nearer one's width / two blocks: 24.5 / 15.3, 24.5 / 15.5, 19.7 / 16.1
-    (12800, 4096, 0), (13312, 4096, 0), (14336, 4096, 0), (16384, 4096, 0),  # ... / K slices: 36.8 / 27.1 up to 37.3 / 28.0
+    # the winner's width / two blocks / K slices: 36.3 / 27.8 / 26.4 at 12800, 36.6 / 29.0 / 27.0 at 16384; with a
+    # residual 40.4 / 29.9 / 39.6 and 40.7 / 31.3 / 40.0
+    (12800, 4096, 2), (13312, 4096, 2), (14336, 4096, 2), (16384, 4096, 2),
     (7010, 3328, 2),  # 21.8 / 13.3
 ])
 def test_a_tuned_width_stays_with_its_own_columns(n, k, width):

@@ -710,7 +710,7 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     if (e.m != p.m) continue;
     // The forms that keep all of K in a workgroup are fitted to their number of workgroups (the
     // winner's three blocks of columns are 256 workgroups at 12288 x 4096, 64 rows, and two rounds of
-    // them at 14336 x 4096: 37.1 us against 27.4 for K slices; f32 rows of 4096 x 4096, one block, at 8192
+    // them at 14336 x 4096: 36.3 us against 28.0 for two blocks; f32 rows of 4096 x 4096, one block, at 8192
     // x 4096: 15.8 against 14.0 for two, 5 rows of int8-64, and 28.0 against 18.5, 16 of int4).  What
     // carries over is that the rows go in one launch, or to the kernel of f32 rows; the form and its
     // width are the problem's own.
@@ -917,17 +917,17 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return false;
 }
 
-// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip), whichever price is
-// lower: of 1980 problems timed with both, most of them close, the choice is 0.4 % behind the faster
-// one in the mean and at 23 more than 3 % behind the former (a bar of nine tenths instead: 5 %
-// behind in the mean).  Us, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0 against 22.2,
+// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip) unless its price is a
+// twentieth above the former's: 0.5 % behind the faster one in the mean of 1299 problems timed with
+// both (level with no margin; over 66 decoder steps and Linears it lost less where the two are
+// close).  Us of plain launches, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0 against 22.2,
 // per row 4491 x 6272, 56 rows 31.5 against 20.8, but int8-64 2008 x 8192, 32 rows 12.1 against 18.2; int4
 // 12288 x 4096, 48 rows 27.2 against 18.1, but 2610 x 11520 23.0 against 25.1.
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
   const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
-  if (!gemm_rows_default(p, &whole, &us) || (found && us >= gemv_mfma_rows_us(p, *out))) return found;
+  if (!gemm_rows_default(p, &whole, &us) || (found && us >= 1.05 * gemv_mfma_rows_us(p, *out))) return found;
   *out = whole;
   return true;
 }
@@ -1014,14 +1014,14 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     tlhip_kernel_config_t whole;
     double whole_us = 0.0;
     const bool whole_ok = p.m <= 64 && gemm_rows_default(p, &whole, &whole_us);
-    // (up to 64 rows the eight-wave tiles take 1.11 times their price in the median, and among other
-    // launches a second one for the K slices costs a little more: 4/3 and the model's 0.9 are 0.5 %
-    // behind the faster one in the mean of 1200 problems timed with both; 48 rows of int4 at 4096 x
-    // 12288, a near draw behind themselves, are 0.9 us ahead of the tile in a decoder layer)
+    // (behind other launches and with cold weights the eight-wave tiles take 1.04-1.11 times their
+    // price at up to 64 rows: 1.1 and the model's 0.9 are 1.4 % behind the fastest kernel in the mean of
+    // 1300 problems and at 4 more than 3 % behind the tile; 1.25 is 0.8 % behind, but at 19 behind the
+    // tile, and further where a call finds its weights in the last-level cache, which helps the tile)
     double pipe_us = tiled_us;
     if (is_pipe_config(c))
       for (const PipeTileCost& t : kPipeTileCosts)
-        if (c.p0 == t.bm && c.p1 == t.bn) pipe_us = 4.0 / 3.0 * pipe_launch_us(p, t, c.p5 > 1 ? c.p5 : 1);
+        if (c.p0 == t.bm && c.p1 == t.bn) pipe_us = 1.1 * pipe_launch_us(p, t, c.p5 > 1 ? c.p5 : 1);
     if (rows_us < g_model.rows_break_even * tiled_us || (whole_ok && whole_us < g_model.rows_break_even * pipe_us)) {
       bool ok = true;
       Route q{64, c, c};

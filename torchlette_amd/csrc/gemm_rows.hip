@@ -394,20 +394,22 @@ bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
   return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
 }
 
-// The cheapest number of column blocks and its time in microseconds, or false.  Fitted at 9165
-// launches of 2811 problems (400..24576 x 512..12288, 17..64 rows, four formats, most of them where
-// another kernel is close): launch, and per round of workgroups a constant, the sums of a block and
-// per 4096 of K the figure of the width, a little more for every row above the middle of its tile.
-// One block a workgroup: a second round overlaps the first (two fit a CU up to 32 rows).  96 % of
-// the launches take 0.87-1.12 times that; the width it picks is 0.08 % slower than the best one in the mean.
+// The cheapest number of column blocks and its time in microseconds, or false.  The time is what it
+// adds to a decoder layer: behind an RMSNorm that writes its activations, cold weights, and the mean
+// of four launches without and three with a residual, as a layer's seven are.  Fitted at 4130 of
+// 1300 problems (500..16384 x 768..12288, 17..64 rows, four formats): launch, and per round of
+// workgroups a constant, the sums of a block and per 4096 of K the figure of the width, a little more
+// for every row above the middle of its tile.  One block a workgroup: a second round overlaps the
+// first (two fit a CU up to 32 rows).  96 % take 0.87-1.15 times that; the width it picks is 0.03 %
+// slower than the best one in the mean.
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
   struct Cost {
     double launch, round, block, walk[kMaxCols];
   };
   static const Cost costs[3][3] = {  // format, row tiles
-      {{1.89, 0.66, 0.42, {5.92, 8.13, 10.83, 12.95}}, {1.22, 1.64, 0.51, {7.53, 10.07, 10.61, 15.13}}, {1.07, 1.90, 0.59, {9.17, 10.59, 14.22, 0.0}}},  // int4
-      {{2.01, 0.77, 0.46, {7.34, 10.67, 14.65, 17.53}}, {1.37, 1.98, 0.32, {8.88, 11.56, 15.96, 0.0}}, {1.33, 1.37, 0.61, {9.83, 14.12, 0.0, 0.0}}},    // int8 in groups
-      {{1.29, 1.04, 0.57, {6.29, 8.79, 11.95, 13.84}}, {0.96, 2.01, 0.47, {8.12, 8.56, 13.30, 0.0}}, {1.03, 1.55, 0.68, {8.60, 11.37, 0.0, 0.0}}}};     // int8 per row
+      {{0.82, 0.99, 0.38, {6.03, 7.60, 10.77, 13.12}}, {0.0, 2.02, 0.53, {8.25, 9.69, 11.03, 16.25}}, {0.0, 2.27, 0.66, {9.66, 10.33, 14.87, 0.0}}},  // int4
+      {{0.96, 0.92, 0.35, {7.60, 10.17, 15.29, 18.46}}, {0.0, 2.52, 0.30, {9.28, 10.92, 16.63, 0.0}}, {0.0, 2.06, 0.42, {10.36, 13.78, 0.0, 0.0}}},    // int8 in groups
+      {{0.53, 1.12, 0.54, {6.49, 7.90, 11.84, 13.96}}, {0.0, 1.81, 0.59, {8.61, 8.87, 13.61, 0.0}}, {0.0, 1.72, 0.71, {9.40, 10.98, 0.0, 0.0}}}};     // int8 per row
   static const double per_row[3] = {0.008, 0.005, 0.004}, second[3] = {0.80, 0.96, 0.96};
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int format = p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1), mt = row_tiles_of(p.m);

@@ -120,20 +120,21 @@ bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& 
   return mfma_applicable(p, (p.n + 15) / 16, c, why);
 }
 
-// What a launch of 17..64 rows costs: fitted at 1980 launches of decode_rows_config's geometries
-// (400..24576 x 512..12288, four formats).  An iteration of a wave, in whole sets of those in flight,
-// takes its time (more where only one is in flight, 0.6 % more a row) once for every one that runs
-// before it, in its round, the rounds of its workgroup and the workgroups that share its CU; K slices
-// add the arrival of the last one and the planes it adds.  96 % of the launches take 0.85-1.25 times
-// that, 80 % 0.93-1.09.
+// What a launch of 17..64 rows adds to a decoder layer (the measure of gemm_rows_default, at the same
+// problems): a residual costs this form 2.4-3.4 us up to 32 rows and 5 beyond, its last arrivals read
+// and store 16 columns a row, against 1.2-1.4 for all of K in one workgroup.  Fitted at 1299 launches
+// of decode_rows_config's geometries.  An iteration of a wave, in whole sets of those in flight, takes
+// its time (more where only one is in flight, 0.6 % more a row) once for every one that runs before
+// it, in its round, the rounds of its workgroup and the workgroups that share its CU; K slices add the
+// arrival of the last one and the planes it adds.  96 % of the launches take 0.84-1.21 times that.
 double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
   struct Cost {
     double base, sliced, iteration, round, plane, alone;
   };
   static const Cost costs[3][2] = {
-      {{4.65, 0.80, 0.64, 0.39, 0.34, 0.03}, {5.58, 1.27, 0.92, 0.43, 0.59, 0.04}},   // int4, up to 32 rows and up to 64
-      {{4.56, 1.57, 0.49, 0.21, 0.17, 0.12}, {5.83, 1.71, 0.49, 0.11, 0.41, 0.11}},   // int8 in groups
-      {{4.51, 1.86, 0.30, 0.47, 0.21, 0.12}, {5.34, 1.76, 0.36, 0.54, 0.53, 0.12}}};  // int8 per row
+      {{4.56, 1.84, 0.64, 0.06, 0.26, 0.07}, {5.46, 1.97, 0.93, 0.69, 0.73, 0.04}},   // int4, up to 32 rows and up to 64
+      {{4.11, 2.26, 0.53, 0.05, 0.24, 0.12}, {5.34, 1.90, 0.56, 0.57, 0.70, 0.13}},   // int8 in groups
+      {{4.59, 2.53, 0.35, 0.14, 0.22, 0.10}, {5.56, 1.98, 0.47, 0.49, 0.64, 0.12}}};  // int8 per row
   const bool few = p.m <= 32;
   const Cost& t = costs[p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)][few ? 0 : 1];
   const int kper = p.format == TLHIP_FMT_INT4_GROUPED ? 128 : 64;
