@@ -429,7 +429,9 @@ bool wave_tile_config(const Problem& p, tlhip_kernel_config_t* out) {
 }
 
 // Up to 16 f32 rows on the matrix cores, three bf16 pieces each, or on the VALU kernel; us, VALU
-// against here, over 13 matrices of 1024 x 768 .. 32768 x 1024 at 3, 4, 5, 8, 9 and 16 rows.
+// against the matrix cores with K slices, over 13 matrices of 1024 x 768 .. 32768 x 1024 at 3, 4, 5, 8,
+// 9 and 16 rows.  (The form that keeps all of K in one workgroup, which gemv_f32_default prefers where
+// it is cheaper, is not weighed here: five rows at 2304 x 2048 would take about 6 us on it.)
 //   From five rows on (five: 28.6 against 16.7 at 2304 x 9216 int8-64), but for small matrices
 //   in groups whose K fills whole passes of the VALU kernel's lanes (five rows of int4: 10.9
 //   against 15.0 at 1024 x 3072, 11.4 against 14.1 at 4096 x 1024; eight rows: level; five of
