@@ -97,6 +97,10 @@ int validate_weight(const tlhip_qweight_t* w, const char* who);
 int launch_dequant(const tlhip_qweight_t& w, float* out, hipStream_t stream);
 bool gemv_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
 int launch_gemv(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
+// The VALU kernel's form for one activation row (p5 = 3, gemv_one.hip).
+bool is_one_config(const tlhip_kernel_config_t& c);
+bool gemv_one_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
+int launch_gemv_one(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 bool gemv_group_compatible(const Problem* ps, int count, const tlhip_kernel_config_t& c, const char** why);
 int launch_gemv_grouped(const Problem* ps, int count, const tlhip_kernel_config_t& c, hipStream_t stream);
 bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
@@ -190,6 +194,7 @@ int launch_kernel(const void* fn, dim3 grid, dim3 block, void** args, size_t lds
 bool prepare_mode();
 int prepare_all_kernels();
 int prepare_gemv_kernels();       // gemv.hip (+ the per-format units)
+int prepare_gemv_one_kernels();   // gemv_one.hip (+ the per-format units)
 int prepare_gemv_mfma_kernels();  // gemv_mfma.hip
 int prepare_gemv_xreg_kernels();  // gemv_mfma_xreg.hip
 int prepare_gemv_wave_kernels();  // gemv_wave.hip

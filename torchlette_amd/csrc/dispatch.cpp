@@ -33,6 +33,7 @@
 #include <dlfcn.h>
 
 #include "common.h"
+#include "gemv_one.h"
 
 namespace tlhip {
 namespace {
@@ -548,6 +549,8 @@ tlhip_kernel_config_t default_config(const Problem& p) {
 // Heuristic default of the VALU kernel (the only one for M <= 4, and the one the
 // prologue entry points use).
 tlhip_kernel_config_t default_valu_config(const Problem& p) {
+  tlhip_kernel_config_t one;
+  if (gemv_one_default(p, p.n, ONE_SINGLE, &one)) return one;
   const int cw = p.format == TLHIP_FMT_INT4_GROUPED ? 32 : 16;
   const int64_t nchunks = p.k / cw;
   if (p.n >= 32768) {
@@ -601,6 +604,17 @@ std::vector<tlhip_kernel_config_t> candidates(const Problem& p) {
               tlhip_kernel_config_t c = gemv_cfg(lpr, r, waves, kw, unroll);
               if (gemv_config_applicable(p, c, nullptr)) out.push_back(c);
             }
+  }
+  if (p.m == 1) {
+    // the one-row form: p4 is its workgroups per CU
+    for (int lpr : {16, 32, 64})
+      for (int waves : {4, 8})
+        for (int kw : {1, 2, 4, 8})
+          for (int resident : {8, 16}) {
+            tlhip_kernel_config_t c = gemv_cfg(lpr, 1, waves, kw, resident / waves);
+            c.p5 = 3;
+            if (gemv_config_applicable(p, c, nullptr)) out.push_back(c);
+          }
   }
   if (p.m <= 4) {
     // the 4x4x4 matrix-core form of the same kernel
@@ -722,6 +736,8 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     there.k = e.k;
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
+    // (one row: the lanes that share it follow from K and the number of rows)
+    if (c.variant == VARIANT_GEMV) (void)gemv_one_default(p, p.n, ONE_SINGLE, &c);
     const double d = dn + 2.0 * dk + dm;  // K decides whether the activations fit LDS: weigh it
     if (d < best && config_applicable(p, c, nullptr)) {
       best = d;
@@ -766,22 +782,24 @@ tlhip_kernel_config_t select_config(const Problem& p) {
   return default_config(p);
 }
 
-// The VALU configuration for launches only that kernel has (grouped, with a prologue):
-// the tuned or selected one if it is of that kernel, else the heuristic.
+// The VALU configuration for launches only that kernel has (with a prologue): one row's own
+// geometry, else the tuned or selected one if it is of that kernel, else the heuristic.
 tlhip_kernel_config_t valu_config(const Problem& p) {
-  tlhip_kernel_config_t c = select_config(p);
+  tlhip_kernel_config_t c;
+  if (p.pro.kind != TLHIP_PRO_NONE && gemv_one_default(p, p.n, ONE_SINGLE, &c)) return c;
+  c = select_config(p);
   if (c.variant != VARIANT_GEMV) c = default_valu_config(p);
   return c;
 }
 
-// The grouped kernel is the dot2 form with two chunks in flight and one or two rows
-// per lane group: the tuned geometry where it is of that form, else the default one.
-tlhip_kernel_config_t grouped_config(const Problem& p) {
-  tlhip_kernel_config_t c = valu_config(p);
-  if (c.p5 != 0) c = default_valu_config(p);
-  c.p4 = 2;
-  if (c.p1 > 2) c.p1 = 2;
-  return c;
+// One launch for up to four problems of one row each, where the one-row kernel takes them.
+bool grouped_config(const Problem* ps, int count, tlhip_kernel_config_t* out) {
+  int big = 0;
+  for (int i = 1; i < count; ++i)
+    if (ps[i].n > ps[big].n) big = i;
+  tlhip_kernel_config_t alone = select_config(ps[big]);
+  if (!is_one_config(alone) && !gemv_one_default(ps[big], ps[big].n, ONE_GROUP, &alone)) return false;
+  return gemv_one_group_config(ps, count, alone, out);
 }
 
 int run_config(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream) {
@@ -1117,6 +1135,13 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
   };
   switch (base.variant) {
     case VARIANT_GEMV:
+      if (is_one_config(base)) {
+        vary(0, {16, 32, 64});
+        vary(2, {4, 8});
+        vary(3, {1, 2, 4, 8});
+        vary(4, {1, 2, 4});
+        break;
+      }
       vary(0, {16, 32, 64});
       vary(1, {1, 2, 4});
       vary(2, {2, 4, 8});
@@ -1588,14 +1613,10 @@ int tlhip_gemv_grouped_rows(const tlhip_gemv_problem_t* problems, int count, int
   if (count == 0 || m == 0) return TLHIP_OK;
   hipStream_t s = resolve_stream(stream);
   if (m == 1 && count > 1) {
-    // one activation row: the configuration of the largest problem, in the VALU kernel's
-    // grouped form (one grouped launch beats separate launches of whichever kernel is
-    // fastest for a single problem: every launch costs 2-3 us)
-    int big = 0;
-    for (int i = 1; i < count; ++i)
-      if (ps[i].n > ps[big].n) big = i;
-    const tlhip_kernel_config_t c = grouped_config(ps[big]);
-    if (gemv_group_compatible(ps, count, c, nullptr)) return launch_gemv_grouped(ps, count, c, s);
+    // one activation row: one launch beats separate launches of whichever kernel is fastest for a
+    // single problem (every launch costs 2-3 us)
+    tlhip_kernel_config_t c;
+    if (grouped_config(ps, count, &c)) return launch_gemv_grouped(ps, count, c, s);
   }
   if (count > 1) {
     // Problems on the SAME activations (q/k/v, gate/up): one launch of a matrix-core
@@ -1683,11 +1704,8 @@ int tlhip_gemv_grouped_prologue(const tlhip_gemv_problem_t* problems, int count,
   }
   if (count == 0) return TLHIP_OK;
   hipStream_t s = resolve_stream(stream);
-  int big = 0;
-  for (int i = 1; i < count; ++i)
-    if (ps[i].n > ps[big].n) big = i;
-  const tlhip_kernel_config_t c = grouped_config(ps[big]);
-  if (gemv_group_compatible(ps, count, c, nullptr)) return launch_gemv_grouped(ps, count, c, s);
+  tlhip_kernel_config_t c;
+  if (grouped_config(ps, count, &c)) return launch_gemv_grouped(ps, count, c, s);
   for (int i = 0; i < count; ++i) {
     int rc = launch_gemv(ps[i], valu_config(ps[i]), s);
     if (rc) return rc;

@@ -1,6 +1,6 @@
 // Host side of the VALU decode GEMV (stands in for dispatchQuantizedGemvNT,
 // src/backend/webgpu/matmul/dispatch.ts:875-931): configuration checks, launch
-// geometry, the single and the grouped launch.  The kernel is in gemv_kernel.h and
+// geometry and the launch.  The kernel is in gemv_kernel.h and
 // is instantiated per weight format in gemv_int4.hip, gemv_int8_grouped.hip and
 // gemv_int8_row.hip.
 #include <cstring>
@@ -33,6 +33,7 @@ bool gemv_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, co
     return false;
   };
   if (c.variant != VARIANT_GEMV) return fail(0);
+  if (is_one_config(c)) return gemv_one_config_applicable(p, c, why);
   if (c.p0 != 16 && c.p0 != 32 && c.p0 != 64) return fail(1);
   if (c.p1 != 1 && c.p1 != 2 && c.p1 != 4) return fail(2);
   if (c.p2 < 1 || c.p2 > 8) return fail(3);
@@ -107,6 +108,7 @@ int launch_gemv(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
   const char* why = nullptr;
   if (!gemv_config_applicable(p, c, &why)) return set_error(TLHIP_ERR_INVALID, "gemv: config not applicable: %s", why);
   if (p.n == 0 || p.m == 0) return TLHIP_OK;
+  if (is_one_config(c)) return launch_gemv_one(p, c, stream);
   const int xbytes = p.x_dtype == TLHIP_F16 ? 2 : 4;
 
   // activation rows per pass: as many (4, 2 or 1) as fit LDS next to the partials
@@ -141,89 +143,10 @@ int launch_gemv(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
   return TLHIP_OK;
 }
 
-// Grouped launch: see gemv_grouped_kernel.  M = 1, f16 activations, and (rows per
-// lane group, chunks in flight) = (1,2) or (2,2) are built.
-bool gemv_group_compatible(const Problem* ps, int count, const tlhip_kernel_config_t& c, const char** why) {
-  static const char* reasons[] = {
-      "a group holds 1..4 problems",
-      "grouped launches are built for M = 1 and f16 activations",
-      "all problems of a group must share format, group size, K and output type",
-      "grouped launches are built for (rows per lane group, chunks in flight) = (1,2) or (2,2)",
-  };
-  auto fail = [&](int i) {
-    if (why) *why = reasons[i];
-    return false;
-  };
-  if (count < 1 || count > kMaxGroup) return fail(0);
-  for (int i = 0; i < count; ++i) {
-    if (ps[i].m != 1 || ps[i].x_dtype != TLHIP_F16) return fail(1);
-    if (ps[i].format != ps[0].format || ps[i].group_size != ps[0].group_size || ps[i].k != ps[0].k ||
-        ps[i].y_dtype != ps[0].y_dtype)
-      return fail(2);
-    if (!gemv_config_applicable(ps[i], c, why)) return false;
-  }
-  const int u = c.p4 == 0 ? 2 : c.p4;
-  if (u != 2 || (c.p1 != 1 && c.p1 != 2)) return fail(3);
-  return true;
-}
-
-int launch_gemv_grouped(const Problem* ps, int count, const tlhip_kernel_config_t& c, hipStream_t stream) {
-  const char* why = nullptr;
-  if (!gemv_group_compatible(ps, count, c, &why))
-    return set_error(TLHIP_ERR_INVALID, "gemv_grouped: %s", why ? why : "?");
-  GroupedGemvArgs g;
-  g.count = 0;
-  g.first[0] = 0;
-  int threads = 0;
-  size_t lds_bytes = 0;
-  // every problem gets the workgroups it would get alone, scaled down together if
-  // the sum exceeds what is resident at once
-  int grids[kMaxGroup], total = 0, resident = 0;
-  for (int i = 0; i < count; ++i) {
-    if (ps[i].n == 0) continue;
-    int mt, grid;
-    size_t lds;
-    fill_args(ps[i], c, 0, 1, g.p[g.count], mt, threads, grid, lds);
-    lds_bytes = lds > lds_bytes ? lds : lds_bytes;
-    const int cus = device_cu_count();
-    int per_cu = 2048 / threads;
-    const int by_lds = (int)((160 * 1024) / (lds ? lds : 1));
-    if (by_lds < per_cu) per_cu = by_lds < 1 ? 1 : by_lds;
-    resident = cus * per_cu;
-    grids[g.count] = grid;
-    total += grid;
-    ++g.count;
-  }
-  if (g.count == 0) return TLHIP_OK;
-  for (int i = 0; i < g.count; ++i) {
-    int grid = grids[i];
-    if (total > resident) {
-      grid = (int)((int64_t)grid * resident / total);
-      if (grid < 1) grid = 1;
-    }
-    g.first[i + 1] = g.first[i] + grid;
-  }
-  int rc;
-  const int r = c.p1;
-  switch (ps[0].format) {
-    case TLHIP_FMT_INT4_GROUPED: rc = launch_gemv_grouped_int4(r, g, threads, lds_bytes, stream); break;
-    case TLHIP_FMT_INT8_GROUPED: rc = launch_gemv_grouped_int8_grouped(r, g, threads, lds_bytes, stream); break;
-    default: rc = launch_gemv_grouped_int8_row(r, g, threads, lds_bytes, stream); break;
-  }
-  if (rc) return rc;
-  TLHIP_CHECK_HIP(hipGetLastError());
-  for (int i = 0; i < g.count; ++i) count_gemv_dispatch();
-  return TLHIP_OK;
-}
-
 // Every instance the launch tables above can reach, in prepare mode (see launch_kernel).
 int prepare_gemv_kernels() {
   GemvArgs a;
   memset(&a, 0, sizeof a);
-  GroupedGemvArgs g;
-  memset(&g, 0, sizeof g);
-  g.count = 1;
-  g.first[1] = 1;
   static const int ru[][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 2}, {2, 4}, {4, 2}};
   for (int xd : {TLHIP_F16, TLHIP_F32})
     for (int mt : {1, 2, 4})
@@ -235,12 +158,6 @@ int prepare_gemv_kernels() {
       }
   for (int u : {2, 4, 8}) {
     const int rc = launch_gemv_mf4_int4(u, a, 64, 1, 0, nullptr);
-    if (rc) return rc;
-  }
-  for (int r : {1, 2}) {
-    int rc = launch_gemv_grouped_int4(r, g, 64, 0, nullptr);
-    if (!rc) rc = launch_gemv_grouped_int8_grouped(r, g, 64, 0, nullptr);
-    if (!rc) rc = launch_gemv_grouped_int8_row(r, g, 64, 0, nullptr);
     if (rc) return rc;
   }
   return TLHIP_OK;

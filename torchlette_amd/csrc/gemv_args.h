@@ -31,21 +31,10 @@ struct GemvArgs {
   DevPrologue pro;
 };
 
-// Several problems of one shape class in one launch: workgroups
-// [first[i], first[i+1]) work on problem i.
-constexpr int kMaxGroup = 4;
-struct GroupedGemvArgs {
-  int count;
-  int first[kMaxGroup + 1];
-  GemvArgs p[kMaxGroup];
-};
-
 // Defined once per weight format (gemv_int4.hip, gemv_int8_grouped.hip, gemv_int8_row.hip).
 #define TLHIP_DECLARE_GEMV_FORMAT(NAME)                                                                  \
   int launch_gemv_##NAME(int x_dtype, int mt, int r, int u, const GemvArgs& a, int threads, int grid,     \
-                         size_t lds_bytes, hipStream_t stream);                                          \
-  int launch_gemv_grouped_##NAME(int r, const GroupedGemvArgs& g, int threads, size_t lds_bytes,          \
-                                 hipStream_t stream);
+                         size_t lds_bytes, hipStream_t stream);
 int launch_gemv_mf4_int4(int u, const GemvArgs& a, int threads, int grid, size_t lds_bytes, hipStream_t stream);
 TLHIP_DECLARE_GEMV_FORMAT(int4)
 TLHIP_DECLARE_GEMV_FORMAT(int8_grouped)

@@ -152,9 +152,6 @@ struct ChunkDot<TLHIP_FMT_INT4_GROUPED, float> {
 // overlaps the staging, the arithmetic and the reductions.  The hot path has no
 // per-lane branches: out-of-range chunks load a clamped address and contribute
 // zero through their scale (or a select).
-// `bid` / `nblk`: this workgroup's index among, and the number of, the workgroups
-// that work on this problem (the whole grid for a single launch; a slice of it
-// when several problems share one launch).
 // MF4 (int4, f16 activations, MT = 4, R = 1): the dot products of up to four activation
 // rows go through v_mfma_f32_4x4x4_16b_f16 instead of one v_dot2 chain per row.  The
 // instruction multiplies 16 independent 4 x 4 blocks: in block b (lanes 4b .. 4b+3) lane
@@ -166,9 +163,10 @@ struct ChunkDot<TLHIP_FMT_INT4_GROUPED, float> {
 // activation row.  Lane mapping: row in the quad = lane % 4, chunk slot = lane / 4 (16
 // chunk slots per wave: "lanes per row" is 16).
 template <int FMT, typename XT, int MT, int R, int U, bool MF4 = false>
-__device__ __forceinline__ void gemv_body(const GemvArgs& a, const int bid, const int nblk) {
+__global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
   static_assert(!MF4 || (FMT == TLHIP_FMT_INT4_GROUPED && sizeof(XT) == 2 && MT == 4 && R == 1),
                 "the 4x4x4 form is built for int4 weights, f16 activations, four rows");
+  const int bid = (int)blockIdx.x, nblk = (int)gridDim.x;
   using Dot = ChunkDot<FMT, XT>;
   constexpr int NQ = Dot::NQ;
   constexpr bool GROUPED = (FMT != TLHIP_FMT_INT8_ROW);
@@ -627,26 +625,6 @@ __device__ __forceinline__ void gemv_body(const GemvArgs& a, const int bid, cons
 }
 
 template <int FMT, typename XT, int MT, int R, int U, bool MF4 = false>
-__global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
-  gemv_body<FMT, XT, MT, R, U, MF4>(a, blockIdx.x, gridDim.x);
-}
-
-// Several problems of one shape class (same format, K, activation type, rows and
-// kernel configuration; N, pointers and epilogues differ) in ONE launch: a decode
-// step issues q/k/v or gate/up on the same activations, each far too small to
-// fill the chip, and every launch costs 2-3 us.  Workgroups
-// [first[i], first[i+1]) work on problem i.
-
-template <int FMT, typename XT, int MT, int R, int U>
-__global__ __launch_bounds__(512) void gemv_grouped_kernel(const GroupedGemvArgs g) {
-  int i = 0;
-#pragma unroll
-  for (int j = 1; j < kMaxGroup; ++j)
-    if (j < g.count && (int)blockIdx.x >= g.first[j]) i = j;
-  gemv_body<FMT, XT, MT, R, U>(g.p[i], (int)blockIdx.x - g.first[i], g.first[i + 1] - g.first[i]);
-}
-
-template <int FMT, typename XT, int MT, int R, int U, bool MF4 = false>
 int launch_t(const GemvArgs& a, int threads, int grid, size_t lds_bytes, hipStream_t stream) {
   const void* fn = (const void*)gemv_kernel<FMT, XT, MT, R, U, MF4>;
   void* args[] = {(void*)&a};
@@ -685,26 +663,13 @@ int launch_x(int x_dtype, int mt, int r, int u, const GemvArgs& a, int threads, 
   return launch_m<FMT, float>(mt, r, u, a, threads, grid, lds_bytes, stream);
 }
 
-template <int FMT, int R>
-int launch_grouped_t(const GroupedGemvArgs& g, int threads, size_t lds_bytes, hipStream_t stream) {
-  const void* fn = (const void*)gemv_grouped_kernel<FMT, _Float16, 1, R, 2>;
-  void* args[] = {(void*)&g};
-  return launch_kernel(fn, dim3(g.first[g.count]), dim3(threads), args, lds_bytes, stream);
-}
-
-
 }  // namespace
 
-// One translation unit per weight format defines these two.
+// One translation unit per weight format defines this.
 #define TLHIP_DEFINE_GEMV_FORMAT(NAME, FMT)                                                                   \
   int launch_gemv_##NAME(int x_dtype, int mt, int r, int u, const GemvArgs& a, int threads, int grid,          \
                          size_t lds_bytes, hipStream_t stream) {                                              \
     return launch_x<FMT>(x_dtype, mt, r, u, a, threads, grid, lds_bytes, stream);                             \
-  }                                                                                                           \
-  int launch_gemv_grouped_##NAME(int r, const GroupedGemvArgs& g, int threads, size_t lds_bytes,               \
-                                 hipStream_t stream) {                                                        \
-    return r == 1 ? launch_grouped_t<FMT, 1>(g, threads, lds_bytes, stream)                                   \
-                  : launch_grouped_t<FMT, 2>(g, threads, lds_bytes, stream);                                  \
   }
 
 }  // namespace tlhip

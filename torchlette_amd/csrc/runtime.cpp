@@ -197,6 +197,7 @@ int prepare_gemv_seq_kernels();  // gemv_seq.hip
 int prepare_all_kernels() {
   t_prepare_mode = true;
   int rc = prepare_gemv_kernels();
+  if (!rc) rc = prepare_gemv_one_kernels();
   if (!rc) rc = prepare_gemv_mfma_kernels();
   if (!rc) rc = prepare_gemv_xreg_kernels();
   if (!rc) rc = prepare_gemv_wave_kernels();
