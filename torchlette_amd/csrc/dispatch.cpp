@@ -33,6 +33,7 @@
 #include <dlfcn.h>
 
 #include "common.h"
+#include "gemv_few.h"
 #include "gemv_one.h"
 
 namespace tlhip {
@@ -454,8 +455,27 @@ bool f32_rows_on_matrix_cores(const Problem& p) {
   return weights >= 8000000;
 }
 
+// 2..16 f16 rows with all of K in a workgroup (gemv_few.hip), wherever it takes them (K a multiple of 128 up to
+// 16384) but for a long matrix (an LM head), which the kernels below stream at the rate of memory, and two
+// rows of a wide short one, on the VALU kernel: 4.4 against 4.6 us at 8476 x 1024 int4.  Us, the kernels below ->
+// here, in the mean of 27 matrices of 1024..18432 x 1024..12288 and four formats 1.37 times faster: 1.2 at
+// two rows, 1.28-1.37 at three, 1.40-1.49 at eight and sixteen; 16 rows of int4 at 1024 x 1024 5.9 -> 3.3,
+// 4096 x 4096 8.0 -> 5.6, 4096 x 12288 14.3 -> 11.5, 12288 x 4096 10.4 -> 9.5; of int8-64 2304 x 9216 14.6 -> 10.3.
+bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
+  double us = 0.0;
+  if (p.n >= 32768 || (p.m == 2 && p.n >= 8 * p.k)) return false;
+  // few columns of a long K: K slices across workgroups are ahead or level (16 rows of int4 at 1024 x 12288
+  // 8.8 against 9.5 us, eight at 528 x 12288 7.8 and 7.8, 16 at 2048 x 12288 9.8 against 9.1; int8 per row at 1024
+  // x 12288 8.3 against 9.1; but eight rows of int8-64 there 8.7 against 7.3)
+  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
+  if (p.k >= 12288 && (int4 ? p.m >= 8 && p.n <= 2048 : p.m > 8 && p.n <= 1024)) return false;
+  return gemv_few_default(&p, 1, FEW_SINGLE, out, &us);
+}
+
 // Heuristic default, used when nothing is tuned.
 tlhip_kernel_config_t default_config(const Problem& p) {
+  tlhip_kernel_config_t few;
+  if (few_rows_config(p, &few)) return few;
   if (p.m > 16 && p.x_dtype == TLHIP_F16) {
     // the eight-wave kernel wherever it takes the problem (K a multiple of 64, groups of 32 or
     // 64 times a power of two): ahead of the kernels below at every one of 196 problems from 64
@@ -627,6 +647,14 @@ std::vector<tlhip_kernel_config_t> candidates(const Problem& p) {
           if (gemv_config_applicable(p, c, nullptr)) out.push_back(c);
         }
   }
+  for (int nb : {1, 2, 3, 4, 6})  // 2..16 rows, all of K in a workgroup: full blocks of columns, or an even share
+    for (int rounds = 0; rounds <= 4; ++rounds) {
+      const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+      tlhip_kernel_config_t c = mfma_cfg(8, 0, 0, 0);
+      c.p4 = nb;
+      c.p2 = rounds ? (int)std::min<int64_t>(((p.n + cus * rounds - 1) / (cus * rounds) + 3) / 4 * 4, 16 * nb) : 16 * nb;
+      if ((rounds == 0 || c.p2 < 16 * nb) && is_few_config(p, c, FEW_SINGLE)) out.push_back(c);
+    }
   for (int cols = 1; cols <= 4 && p.m > 16; ++cols) {  // 17..64 rows, all of K in a workgroup
     tlhip_kernel_config_t c = mfma_cfg(8, 0, 0, 0);
     c.p4 = cols;
@@ -736,7 +764,8 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     there.k = e.k;
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
-    // (one row: the lanes that share it follow from K and the number of rows)
+    if (is_few_config(there, c, FEW_SINGLE) && !few_rows_config(p, &c)) continue;
+    // (one row: the lanes that share it follow from K and the number of columns)
     if (c.variant == VARIANT_GEMV) (void)gemv_one_default(p, p.n, ONE_SINGLE, &c);
     const double d = dn + 2.0 * dk + dm;  // K decides whether the activations fit LDS: weigh it
     if (d < best && config_applicable(p, c, nullptr)) {
@@ -1150,6 +1179,16 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       vary(5, {0, 1});
       break;
     case VARIANT_GEMV_MFMA:
+      if (is_few_config(p, base, FEW_SINGLE)) {  // its columns are its only field
+        for (int nb : {1, 2, 3, 4, 6})
+          for (int cols : {16 * nb, 16 * nb - 4, 16 * nb - 8}) {
+            tlhip_kernel_config_t c = base;
+            c.p4 = nb;
+            c.p2 = cols;
+            push(c);
+          }
+        break;
+      }
       if (is_rows_config(p, base)) {  // its width is its only field
         vary(4, {1, 2, 3, 4});
         tlhip_kernel_config_t sliced;
@@ -1635,7 +1674,9 @@ int tlhip_gemv_grouped_rows(const tlhip_gemv_problem_t* problems, int count, int
       // the per-wave pipelined kernel), the heuristic default of the same problem: one
       // launch of a slightly slower kernel beats `count` launches of the fastest one
       const tlhip_kernel_config_t tries[2] = {select_config(all), default_config(all)};
-      for (const tlhip_kernel_config_t& c : tries) {
+      for (tlhip_kernel_config_t c : tries) {
+        double us = 0.0;  // all of K in a workgroup: each problem ends with a workgroup of its own
+        if (is_few_config(all, c, FEW_GROUP)) (void)gemv_few_default(ps, count, FEW_GROUP, &c, &us);
         if (c.variant == VARIANT_GEMV_MFMA && gemv_mfma_group_applicable(ps, count, c, nullptr))
           return launch_gemv_mfma_group(ps, count, c, s);
         if (c.variant == VARIANT_GEMV_XREG && gemv_xreg_group_applicable(ps, count, c, nullptr))

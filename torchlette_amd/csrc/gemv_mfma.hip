@@ -1,6 +1,7 @@
 // Host side of the skinny matrix-core GEMV (gemv_mfma_kernel.h): configuration checks,
 // launch geometry, the single and the grouped launch, and the single-problem kernel
 // instances.  The instances with a problem table are in gemv_mfma_group.hip.
+#include "gemv_few.h"
 #include "gemv_mfma_kernel.h"
 
 namespace tlhip {
@@ -110,11 +111,12 @@ static bool mfma_applicable(const Problem& p, int64_t nblocks, const tlhip_kerne
 }
 
 bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why) {
-  if (is_rows_config(p, c)) return true;
+  if (is_rows_config(p, c) || is_few_config(p, c, FEW_SINGLE)) return true;
   if (c.variant == VARIANT_GEMV_MFMA && c.p1 == 0 && c.p4 != 0) {  // no geometry of the other form has p1 = 0
     if (why)
       *why = "all of K in one workgroup (p1 = 0, p4 blocks of 16 columns): 17..64 f16 rows, p0 8, p1..p3, p5 and p6 0, K a multiple "
-             "of 128, int4 in groups of 32, int8 in groups of 64 or more or per row, p4 1..4 and no more than its registers hold";
+             "of 128, int4 in groups of 32, int8 in groups of 64 or more or per row, p4 1..4 and no more than its registers hold; "
+             "2..16 rows: also K up to 16384, p2 columns in p4 = 1, 2, 3, 4 or 6 even blocks of at most 16, a multiple of four";
     return false;
   }
   return mfma_applicable(p, (p.n + 15) / 16, c, why);
@@ -166,6 +168,7 @@ bool gemv_mfma_group_applicable(const Problem* ps, int count, const tlhip_kernel
     }
     nblocks += (ps[i].n + 15) / 16;
   }
+  if (is_few_config(ps[0], c, FEW_GROUP)) return true;
   return mfma_applicable(ps[0], nblocks > 0 ? nblocks : 1, c, why);
 }
 
@@ -174,6 +177,7 @@ int launch_gemv_mfma_group(const Problem* ps, int count, const tlhip_kernel_conf
   if (!gemv_mfma_group_applicable(ps, count, c, &why))
     return set_error(TLHIP_ERR_INVALID, "gemv_mfma: config not applicable: %s", why);
   const Problem& p = ps[0];
+  if (is_few_config(p, c, FEW_GROUP)) return launch_gemv_few(ps, count, count > 1 ? FEW_GROUP : FEW_SINGLE, 0, c, stream);
   const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
   const int cw = int4 ? 32 : 16;
   const int waves = c.p0, unroll = c.p1;
@@ -245,6 +249,7 @@ int launch_gemv_mfma(const Problem& p, const tlhip_kernel_config_t& c, hipStream
     return set_error(TLHIP_ERR_INVALID, "gemv_mfma: config not applicable: %s", why);
   if (p.n == 0 || p.m == 0) return TLHIP_OK;
   if (is_rows_config(p, c)) return launch_gemm_rows(p, c, stream);
+  if (is_few_config(p, c, FEW_SINGLE)) return launch_gemv_few(&p, 1, FEW_SINGLE, 0, c, stream);
   return launch_gemv_mfma_group(&p, 1, c, stream);
 }
 

@@ -2,6 +2,7 @@
 // tlhip_mlp_decode, tlhip_sequence_status.
 #include <atomic>
 
+#include "gemv_few.h"
 #include "gemv_one.h"
 #include "gemv_seq_kernel.h"
 
@@ -225,18 +226,20 @@ int tlhip_mlp_decode(const tlhip_qweight_t* gate, const tlhip_qweight_t* up, con
   if (rc) return rc;
   const size_t one = (size_t)m * (size_t)gate->n * sizeof(_Float16);
   if (2 * one > scratch_bytes) return mlp_one_launch(gate, up, down, unary, x, x_dtype, m, h, y, y_dtype, down_epilogue, stream);
-  // one row: both projections of a row and their product in one launch (not where h overlaps x,
-  // which every workgroup reads)
+  // both projections and their product in one launch (not where h overlaps x, which every workgroup reads)
   const char *h0 = (const char*)h, *x0 = (const char*)x;
-  const bool apart = h0 + one <= x0 || x0 + (size_t)gate->k * sizeof(_Float16) <= h0;
-  if (m == 1 && gate->n > 0 && apart && unary >= TLHIP_UNARY_NONE && unary <= TLHIP_UNARY_TANH) {
-    Problem g, u;
-    rc = make_problem(gate, x, x_dtype, m, h, TLHIP_F16, 1.0f, nullptr, &g, "mlp_decode");
-    if (!rc) rc = make_problem(up, x, x_dtype, m, h, TLHIP_F16, 1.0f, nullptr, &u, "mlp_decode");
+  const bool apart = h0 + one <= x0 || x0 + (size_t)m * (size_t)gate->k * sizeof(_Float16) <= h0;
+  if (gate->n > 0 && apart && unary >= TLHIP_UNARY_NONE && unary <= TLHIP_UNARY_TANH) {
+    Problem ps[2];
+    rc = make_problem(gate, x, x_dtype, m, h, TLHIP_F16, 1.0f, nullptr, &ps[0], "mlp_decode");
+    if (!rc) rc = make_problem(up, x, x_dtype, m, h, TLHIP_F16, 1.0f, nullptr, &ps[1], "mlp_decode");
     if (rc) return rc;
     tlhip_kernel_config_t c;
-    if (gemv_one_default(g, g.n, ONE_PAIR, &c) && gemv_pair_applicable(g, u, c)) {
-      rc = launch_gemv_pair(g, u, unary, c, resolve_stream(stream));
+    double us = 0.0;
+    const bool one_row = m == 1 && gemv_one_default(ps[0], gate->n, ONE_PAIR, &c) && gemv_pair_applicable(ps[0], ps[1], c);
+    if (one_row || (m > 1 && gemv_few_default(ps, 1, FEW_PAIR, &c, &us))) {
+      rc = one_row ? launch_gemv_pair(ps[0], ps[1], unary, c, resolve_stream(stream))
+                   : launch_gemv_few(ps, 2, FEW_PAIR, unary, c, resolve_stream(stream));
       return rc ? rc : tlhip_gemv(down, h, TLHIP_F16, m, y, y_dtype, 1.0f, down_epilogue, stream);
     }
   }
