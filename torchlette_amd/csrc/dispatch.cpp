@@ -1206,13 +1206,14 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
       for (int slices : {1, 2, 4, 8, 16, 32}) {
         tlhip_kernel_config_t c = base;
         c.p0 = slices;
-        c.p1 = 0;
+        c.p1 = c.p2 = 0;
         push(c);
       }
       for (int cols : {1, 2, 4}) {
         tlhip_kernel_config_t c = base;
         c.p0 = 8;
         c.p1 = cols;
+        c.p2 = 0;
         push(c);
       }
       break;

@@ -48,6 +48,7 @@ struct F32Args {
   int groups_per_row;
   int blocks;           // K in blocks of one 16-byte chunk on each of four lanes, rounded up
   int slices;
+  int cols, block_cols;  // all of K in a workgroup: its columns, and those of a block
   float* workspace;     // slices > 1: [tile][slice][M][128]
   int* counters;        // one per tile, zero between launches
   float alpha, scale_mul;
@@ -288,16 +289,17 @@ __global__ __launch_bounds__(kThreads, 4) void gemv_f32_kernel(const F32Args a) 
 // ---- all of K in one workgroup ------------------------------------------------------------------
 // The same products where K slices across workgroups cost more than they give (the pieces of a
 // slice behind a barrier, then planes of partial sums through memory and a counter: 4-5 us of 9-17):
-// a workgroup owns 16 NB columns and all of K, which its eight waves take in turn, 128 at a time,
-// each cutting its own rows of X into pieces in a patch of LDS that belongs to it; they meet once.
-// No workspace.  What bounds it: the VALU, in cutting X (45 instructions for 4 values of a row, in
-// every workgroup: more columns share them) and in converting the weights.
-// One launch, us, K slices -> here: 5 rows of int8-64 at 9216 x 2304 13.0 -> 11.2, at 2304 x 9216 16.8 ->
-// 15.3, at 2048 x 2304 10.8 -> 5.8; 10 rows of int4 at 4096 x 4096 16.3 -> 11.3 (0.8 TB/s of weights).
+// a workgroup owns up to 16 NB columns, an even share of them, and all of K.  Each of its eight waves has
+// a range of K: it reads the range's group scales once, cuts its rows of X into pieces in a patch of LDS
+// that belongs to it, 128 of K at a time, and meets the others once.  No workspace.  What bounds it: the
+// VALU, in cutting X in every workgroup (more columns share it) and in converting the weights.  Values
+// that are not finite are cut apart only where a wave finds one.
 constexpr int kWhole = 8;                     // waves; the config's p0, with p1 blocks of 16 columns
 constexpr int kWholeStep = 128;
 constexpr int kWholeRow = kWholeStep * 2 + 16;  // bytes of a piece row in LDS
 constexpr int kWholeMaxCols = 4;
+constexpr int kWholeMaxSteps = 16;              // of a wave
+constexpr int kWholeScaleRow = kWholeMaxSteps * 8 + 16;  // bytes of a column's scales in LDS
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t buffer_of(const void* base, uint32_t bytes) {
@@ -307,83 +309,110 @@ __device__ __forceinline__ u32x4 load16(rsrc_t r, uint32_t at, uint32_t step_at)
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, (int)step_at, 0));
 }
 
-template <int FMT, int T, int NB>
+// x in three pieces, x finite (pieces_of without its selects): each in the upper half of a word
+__device__ __forceinline__ void finite_pieces_of(uint32_t b, uint32_t (&piece)[3]) {
+  const float r1 = as_float(b) - as_float(b & 0xffff0000u);
+  const uint32_t r1b = __builtin_bit_cast(uint32_t, r1);
+  piece[0] = b;
+  piece[1] = r1b;
+  piece[2] = __builtin_bit_cast(uint32_t, r1 - as_float(r1b & 0xffff0000u));
+}
+
+// T: tiles of 16 piece rows; XV: loads of X, two rows each.  WIDE: a group's scales are whole words (int4,
+// int8 in groups of 64)
+template <int FMT, int T, int XV, int NB, bool WIDE>
 __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Args a) {
   constexpr bool INT4 = FMT == TLHIP_FMT_INT4_GROUPED, ROW = FMT == TLHIP_FMT_INT8_ROW;
   constexpr int WV = INT4 ? 1 : 2;         // 16-byte loads of a step, lane and column block
-  constexpr int XV = (16 * T / 3 + 1) / 2; // loads of X: two rows each
+  constexpr int SB = INT4 ? 8 : 4;         // bytes of a step and column in the patch of scales
   extern __shared__ u32x4 lds[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l16 = lane & 15, lg = lane >> 4;
-  const int n0 = (int)blockIdx.x * (16 * NB);
-  const int cols = min(16 * NB, a.n - n0);
+  const int l16 = lane & 15, lg = lane >> 4, m = a.m;
+  const int n0 = (int)blockIdx.x * a.cols, have = min(a.cols, a.n - n0), block_cols = a.block_cols;
   const int steps = a.k / kWholeStep;
   const uint32_t row_bytes = (uint32_t)a.row_chunks * 16u, scale_row_bytes = ROW ? 4u : (uint32_t)a.groups_per_row * 2u;
-  const uint8_t* const packed = (const uint8_t*)a.packed + (int64_t)n0 * row_bytes;
-  const uint8_t* const scales = (const uint8_t*)a.scales + (int64_t)n0 * scale_row_bytes;
 
-  // Buffer loads: rows past M, columns past N and steps past K read zero and cost no traffic, so
-  // that no load stands under a branch.  A lane's place in a step is fixed, the step is a scalar
-  // offset (opaque, or the compiler keeps it in a vector register and loops over the lanes); past
-  // the last step a buffer of no bytes at offset 0.
-  struct Weights {
+  // A lane's place in a step is fixed, the step is a scalar offset.
+  const rsrc_t wb = buffer_of((const uint8_t*)a.packed + (int64_t)n0 * row_bytes, (uint32_t)have * row_bytes);
+  const rsrc_t sb = buffer_of((const uint8_t*)a.scales + (int64_t)n0 * scale_row_bytes, (uint32_t)have * scale_row_bytes);
+  const rsrc_t xb = buffer_of(a.x, (uint32_t)m * (uint32_t)a.k * 4u);
+  uint32_t w_at[NB], s_at[NB], x_at[XV];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {  // columns past the block's or the matrix's: the last one again, not stored
+    const uint32_t col = (uint32_t)min(b * block_cols + min(l16, block_cols - 1), have - 1);
+    w_at[b] = col * row_bytes + (uint32_t)lg * 16u;
+    s_at[b] = col * scale_row_bytes;
+  }
+  const int half = lane >> 5, unit = lane & 31;
+#pragma unroll
+  for (int i = 0; i < XV; ++i) x_at[i] = (uint32_t)min(2 * i + half, m - 1) * (uint32_t)a.k * 4u + (uint32_t)unit * 16u;
+  struct Step {
+    u32x4 x[XV];
     u32x4 w[NB][WV];
-    uint32_t s[NB][2];
   };
-  auto scalar_step = [&](int st) {
-    st = st < steps ? st : -1;
-    asm("" : "+s"(st));
-    return st;
+  auto load_x = [&](Step& v, int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < XV; ++i) v.x[i] = load16(xb, x_at[i], (uint32_t)st * (kWholeStep * 4u));
   };
-  auto load_w = [&](Weights& v, int step) {
-    const int st = scalar_step(step);
-    const uint32_t in = ~(uint32_t)(st >> 31), at = (uint32_t)st & in;
-    const rsrc_t wb = buffer_of(packed, (uint32_t)cols * row_bytes & in), sb = buffer_of(scales, (uint32_t)cols * scale_row_bytes & in);
+  auto load_w = [&](Step& v, int b, int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < WV; ++i) v.w[b][i] = load16(wb, w_at[b] + (uint32_t)i * 64u, (uint32_t)st * (WV * 64u));
+  };
+  auto load = [&](Step& v, int st) __attribute__((always_inline)) {
+    load_x(v, st);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) load_w(v, b, st);
+  };
+
+  // ---- the wave's range of steps and its scales (workgroups of an XCD start at different ranges: all on
+  // the same lines of X at a time is 10-15 % slower)
+  const int range = (wave + ((int)blockIdx.x >> 3)) & (kWhole - 1);
+  const int st0 = steps * range / kWhole, left = steps * (range + 1) / kWhole - st0;
+  constexpr int PER = WIDE ? 64 / SB : 4;  // steps of a load: a quarter of them on each of a column's four lanes
+  constexpr int SL = kWholeMaxSteps / PER;
+  char* const patch = (char*)lds + wave * (16 * T * kWholeRow);
+  char* const scale_patch = (char*)lds + kWhole * (16 * T * kWholeRow) + wave * (NB * 16 * kWholeScaleRow);
+  struct Scales {
+    u32x4 v[NB];
+  };
+  auto load_scales = [&](Scales& v, int from) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const uint32_t row = (uint32_t)(16 * b + l16);
-#pragma unroll
-      for (int i = 0; i < WV; ++i) v.w[b][i] = load16(wb, row * row_bytes + (uint32_t)lg * 16u + (uint32_t)i * 64u, at * (WV * 64u));
-      if constexpr (INT4) {
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-        const u32x2 s = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sb, (int)(row * scale_row_bytes), (int)(at * 8u), 0));
-        v.s[b][0] = s.x;
-        v.s[b][1] = s.y;
-      } else if constexpr (!ROW) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          v.s[b][h] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sb, (int)(row * scale_row_bytes), (int)(((2u * at + (uint32_t)h) >> a.group_shift) * 2u), 0);
-      }
+      if constexpr (WIDE) v.v[b] = load16(sb, s_at[b] + (uint32_t)lg * 16u, (uint32_t)(st0 + from) * SB);
+      else v.v[b].x = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sb, (int)(s_at[b] + ((uint32_t)(2 * (st0 + from + lg)) >> a.group_shift) * 2u), 0, 0);
     }
   };
-  struct Rows {
-    u32x4 v[XV];
+  auto lay_scales = [&](const Scales& v, int from) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      char* const to = scale_patch + (b * 16 + l16) * kWholeScaleRow;
+      if constexpr (WIDE) *(u32x4*)(to + from * SB + lg * 16) = v.v[b];
+      else *(uint32_t*)(to + (from + lg) * 4) = v.v[b].x | v.v[b].x << 16;
+    }
   };
-  const int half = lane >> 5, unit = lane & 31;
-  auto load_x = [&](Rows& r, int step) {
-    const int st = scalar_step(step);
-    const uint32_t in = ~(uint32_t)(st >> 31), at = (uint32_t)st * (kWholeStep * 4u) & in;
+
+  auto cut = [&](const Step& v) __attribute__((always_inline)) {
+    bool odd = false;  // anything not finite
 #pragma unroll
     for (int i = 0; i < XV; ++i)
-      r.v[i] = load16(buffer_of(a.x + (int64_t)(2 * i) * a.k, (uint32_t)max(a.m - 2 * i, 0) * (uint32_t)a.k * 4u & in),
-                      (uint32_t)half * (uint32_t)a.k * 4u + (uint32_t)unit * 16u, at);
-  };
-  char* const patch = (char*)lds + wave * (16 * T * kWholeRow);
-  auto cut = [&](const Rows& r) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd = odd | __builtin_amdgcn_classf(as_float(v.x[i][e]), 0x207);
+    const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
       const int row = 2 * i + half;
       uint32_t p[4][3];
-      pieces_of(r.v[i].x, p[0]);
-      pieces_of(r.v[i].y, p[1]);
-      pieces_of(r.v[i].z, p[2]);
-      pieces_of(r.v[i].w, p[3]);
-      if (row < a.m) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) finite_pieces_of(v.x[i][e], p[e]);
+      if (any)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pieces_of(v.x[i][e], p[e]);
+      if (row < m) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-          const uint64_t v = (uint64_t)upper_halves(p[0][q], p[1][q]) | ((uint64_t)upper_halves(p[2][q], p[3][q]) << 32);
-          *(uint64_t*)(patch + (row * 3 + q) * kWholeRow + unit * 8) = v;
+          const uint64_t w = (uint64_t)upper_halves(p[0][q], p[1][q]) | ((uint64_t)upper_halves(p[2][q], p[3][q]) << 32);
+          *(uint64_t*)(patch + (row * 3 + q) * kWholeRow + unit * 8) = w;
         }
       }
     }
@@ -392,11 +421,14 @@ __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Ar
   const char* arow[T];
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    arow[t] = patch + min(t * 16 + l16, a.m * 3 - 1) * kWholeRow + lg * (INT4 ? 16 : 32);
+    arow[t] = patch + min(t * 16 + l16, m * 3 - 1) * kWholeRow + lg * (INT4 ? 16 : 32);
 #pragma unroll
     for (int b = 0; b < NB; ++b) acc[b][t] = (float4_t){0.f, 0.f, 0.f, 0.f};
   }
-  auto multiply = [&](const Weights& v) __attribute__((always_inline)) {
+  // `next`: the step whose loads take the registers as they become free, or -1
+  auto consume = [&](Step& v, int i_step, int next) __attribute__((always_inline)) {
+    cut(v);
+    if (next >= 0) load_x(v, next);
     bf16x8 xa[4][T];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -412,25 +444,32 @@ __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Ar
         words[4 * i + 2] = v.w[b][i].z;
         words[4 * i + 3] = v.w[b][i].w;
       }
+      if (next >= 0) load_w(v, b, next);
       if constexpr (INT4) transpose4(words[0], words[1], words[2], words[3]);
+      uint32_t sc2[2] = {0u, 0u};  // int4: four group scales; int8: one per half step
+      if constexpr (!ROW) {
+        const char* const from = scale_patch + (b * 16 + l16) * kWholeScaleRow + i_step * SB;
+        sc2[0] = *(const uint32_t*)from;
+        if constexpr (INT4) sc2[1] = *(const uint32_t*)(from + 4);
+      }
       float4_t chain[T], sum[T];  // a step's own sum first: the long one takes a step at a time
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        uint32_t wb[4];
+        uint32_t wq[4];
         if constexpr (INT4) {
-          weight_bf16<FMT>(words[i], wb);
+          weight_bf16<FMT>(words[i], wq);
         } else {
-          weight_bf16<FMT>(words[2 * i], wb);
-          weight_bf16<FMT>(words[2 * i + 1], wb + 2);
+          weight_bf16<FMT>(words[2 * i], wq);
+          weight_bf16<FMT>(words[2 * i + 1], wq + 2);
         }
-        const bf16x8 wv = __builtin_bit_cast(bf16x8, (u32x4){wb[0], wb[1], wb[2], wb[3]});
+        const bf16x8 wv = __builtin_bit_cast(bf16x8, (u32x4){wq[0], wq[1], wq[2], wq[3]});
         constexpr int GROUP = INT4 ? 1 : (ROW ? 4 : 2);  // products of one scale
         const bool first = i % GROUP == 0, last = i % GROUP == GROUP - 1;
 #pragma unroll
         for (int t = 0; t < T; ++t)
           chain[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[i][t], wv, first ? (float4_t){0.f, 0.f, 0.f, 0.f} : chain[t], 0, 0, 0);
         if (last) {
-          const float s = ROW ? 1.f : half_bits_to_float(INT4 ? ((i & 1) ? v.s[b][i >> 1] >> 16 : v.s[b][i >> 1] & 0xffffu) : v.s[b][i >> 1]);
+          const float s = ROW ? 1.f : half_bits_to_float(INT4 ? ((i & 1) ? sc2[i >> 1] >> 16 : sc2[i >> 1] & 0xffffu) : (i >> 1 ? sc2[0] >> 16 : sc2[0] & 0xffffu));
 #pragma unroll
           for (int t = 0; t < T; ++t)
 #pragma unroll
@@ -444,36 +483,65 @@ __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Ar
     }
   };
 
-  Weights w0, w1;
-  Rows x0, x1;
-  load_x(x0, wave);
-  load_w(w0, wave);
-  load_x(x1, wave + kWhole);
-  load_w(w1, wave + kWhole);
-  for (int st = wave; st < steps; st += 2 * kWhole) {
-    cut(x0);
-    load_x(x0, st + 2 * kWhole);
-    multiply(w0);
-    if (st + kWhole >= steps) break;
-    load_w(w0, st + 2 * kWhole);
-    cut(x1);
-    load_x(x1, st + 3 * kWhole);
-    multiply(w1);
-    load_w(w1, st + 3 * kWhole);
+  // ---- one step in flight, or two where a step is short; none past the end, every load unconditional (a
+  // wait at a join would count it as not issued), the scales ahead of them
+  if (left > 0) {
+    Scales sv[SL];
+    if constexpr (!ROW) {
+#pragma unroll
+      for (int q = 0; q < SL; ++q)
+        if (q == 0 || q * PER < left) load_scales(sv[q], q * PER);
+    }
+    auto lay_all = [&]() __attribute__((always_inline)) {
+      if constexpr (!ROW) {
+#pragma unroll
+        for (int q = 0; q < SL; ++q)
+          if (q == 0 || q * PER < left) lay_scales(sv[q], q * PER);
+      }
+    };
+    Step v0;
+    load(v0, st0);
+    int i = 0;
+    if constexpr (NB * T > 2) {
+      lay_all();
+      for (; i + 1 < left; ++i) consume(v0, i, st0 + i + 1);
+      consume(v0, i, -1);
+    } else if (left == 1) {
+      lay_all();
+      consume(v0, 0, -1);
+    } else {
+      Step v1;
+      load(v1, st0 + 1);
+      lay_all();
+      for (; i + 3 < left; i += 2) {
+        consume(v0, i, -1);
+        load(v0, st0 + i + 2);
+        consume(v1, i + 1, -1);
+        load(v1, st0 + i + 3);
+      }
+      if (left & 1) {
+        consume(v0, i, -1);
+        load(v0, st0 + i + 2);
+        consume(v1, i + 1, -1);
+        consume(v0, i + 2, -1);
+      } else {
+        consume(v0, i, -1);
+        consume(v1, i + 1, -1);
+      }
+    }
   }
 
   lds_barrier();  // every wave has read its patch
-  float* const sums = (float*)lds;  // [wave][tile][block][16 x 16]
+  float* const sums = (float*)lds;  // [range][tile][block][16 x 16]
 #pragma unroll
   for (int t = 0; t < T; ++t)
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sums[((wave * T + t) * NB + b) * 256 + (4 * lg + e) * 16 + l16] = acc[b][t][e];
+      for (int e = 0; e < 4; ++e) sums[((range * T + t) * NB + b) * 256 + (4 * lg + e) * 16 + l16] = acc[b][t][e];
   lds_barrier();
-  for (int e = tid; e < a.m * (16 * NB); e += kWhole * 64) {
-    const int row = e / (16 * NB), c = e % (16 * NB), col = n0 + c;
-    if (col >= a.n) continue;
+  for (int e = tid; e < m * have; e += kWhole * 64) {
+    const int row = e / have, oc = e - row * have, col = n0 + oc, ob = oc / block_cols, c = oc - ob * block_cols;
     float part[kWhole];
 #pragma unroll
     for (int w = 0; w < kWhole; ++w) {
@@ -481,7 +549,7 @@ __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Ar
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         const int r = row * 3 + q;
-        p[q] = sums[((w * T + (r >> 4)) * NB + (c >> 4)) * 256 + (r & 15) * 16 + (c & 15)];
+        p[q] = sums[((w * T + (r >> 4)) * NB + ob) * 256 + (r & 15) * 16 + c];
       }
       part[w] = p[0] + (p[1] + p[2]);
     }
@@ -492,22 +560,37 @@ __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Ar
   }
 }
 
-template <int FMT, int T>
-const void* whole_fn(int nb) {
-  return nb == 1   ? (const void*)gemv_f32_whole_kernel<FMT, T, 1>
-         : nb == 2 ? (const void*)gemv_f32_whole_kernel<FMT, T, 2>
-                   : (const void*)gemv_f32_whole_kernel<FMT, T, (T < 3 ? 4 : 2)>;  // three tiles of pieces and four blocks: more registers than a lane has
+template <int FMT, int T, int XV, bool WIDE>
+const void* whole_fn_nb(int nb) {
+  if (nb == 1) return (const void*)gemv_f32_whole_kernel<FMT, T, XV, 1, WIDE>;
+  if (nb == 2) return (const void*)gemv_f32_whole_kernel<FMT, T, XV, 2, WIDE>;
+  if (nb == 3) return (const void*)gemv_f32_whole_kernel<FMT, T, XV, 3, WIDE>;
+  if constexpr (T < 3)  // three tiles of pieces and four blocks: more registers than a lane has
+    if (nb == 4) return (const void*)gemv_f32_whole_kernel<FMT, T, XV, 4, WIDE>;
+  return nullptr;
 }
-template <int FMT>
-const void* whole_fn(int tiles, int nb) {
-  return tiles == 1 ? whole_fn<FMT, 1>(nb) : (tiles == 2 ? whole_fn<FMT, 2>(nb) : whole_fn<FMT, 3>(nb));
+template <int FMT, bool WIDE>
+const void* whole_fn_rows(int64_t m, int nb) {
+  if (m <= 4) return whole_fn_nb<FMT, 1, 2, WIDE>(nb);
+  if (m == 5) return whole_fn_nb<FMT, 1, 3, WIDE>(nb);
+  if (m <= 8) return whole_fn_nb<FMT, 2, 4, WIDE>(nb);
+  if (m <= 10) return whole_fn_nb<FMT, 2, 5, WIDE>(nb);
+  if (m <= 12) return whole_fn_nb<FMT, 3, 6, WIDE>(nb);
+  return whole_fn_nb<FMT, 3, 8, WIDE>(nb);
 }
-const void* whole_fn(int format, int tiles, int nb) {
-  return format == TLHIP_FMT_INT4_GROUPED ? whole_fn<TLHIP_FMT_INT4_GROUPED>(tiles, nb)
-         : format == TLHIP_FMT_INT8_ROW   ? whole_fn<TLHIP_FMT_INT8_ROW>(tiles, nb)
-                                          : whole_fn<TLHIP_FMT_INT8_GROUPED>(tiles, nb);
+const void* whole_fn(const Problem& p, int nb) {
+  if (p.format == TLHIP_FMT_INT4_GROUPED) return whole_fn_rows<TLHIP_FMT_INT4_GROUPED, true>(p.m, nb);
+  if (p.format == TLHIP_FMT_INT8_ROW) return whole_fn_rows<TLHIP_FMT_INT8_ROW, false>(p.m, nb);
+  return p.group_size == 64 ? whole_fn_rows<TLHIP_FMT_INT8_GROUPED, true>(p.m, nb) : whole_fn_rows<TLHIP_FMT_INT8_GROUPED, false>(p.m, nb);
 }
-size_t whole_lds(int tiles, int nb) { return std::max((size_t)kWhole * 16 * tiles * kWholeRow, (size_t)kWhole * tiles * nb * 1024); }
+size_t whole_lds(const Problem& p, int nb) {
+  const size_t tiles = (size_t)((3 * p.m + 15) / 16), scales = p.format == TLHIP_FMT_INT8_ROW ? 0 : (size_t)nb * 16 * kWholeScaleRow;
+  return std::max(kWhole * (16 * tiles * kWholeRow + scales), (size_t)kWhole * tiles * nb * 1024);
+}
+// Columns of a workgroup (p2; 0: 16 p1), its blocks, and the columns of a block.
+int whole_cols(const tlhip_kernel_config_t& c) { return c.p2 ? c.p2 : 16 * c.p1; }
+int whole_blocks(const tlhip_kernel_config_t& c) { return (whole_cols(c) + 15) / 16; }
+int whole_block_cols(const tlhip_kernel_config_t& c) { return (whole_cols(c) + whole_blocks(c) - 1) / whole_blocks(c); }
 
 template <int FMT>
 const void* fn_of(int tiles) {
@@ -535,7 +618,7 @@ bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c
       "not the gemv_f32 variant",
       "built for f32 activations, 1..16 rows, without a prologue",
       "K must be a multiple of 32 (int4) or 16 (int8), groups at least 32 (int4) or 64 (int8)",
-      "K slices (p0) must be 1..64 and no more than K holds blocks of 128 (int4) or 64 (int8), p1..p6 0; or p0 8 and p1 (blocks of 16 columns) 1, 2 or 4: K a multiple of 128 up to 16384, int4 in groups of 32; 4 blocks up to 10 rows",
+      "K slices (p0) must be 1..64 and no more than K holds blocks of 128 (int4) or 64 (int8), p1..p6 0; or p0 8 and p1 (blocks of 16 columns) 1, 2 or 4, or p2 (columns) up to 64: K a multiple of 128 up to 16384, int4 in groups of 32; 4 blocks up to 10 rows",
       "the pieces of a K slice do not fit LDS: more slices",
       "the slices' partial sums do not fit the library's workspace",
   };
@@ -548,8 +631,9 @@ bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c
   const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
   if (p.k <= 0 || p.k % (int4 ? 32 : 16) != 0 || (p.format != TLHIP_FMT_INT8_ROW && p.group_size < (int4 ? 32 : 64))) return fail(2);
   if (c.p1 != 0) {  // chains of at most 2048 in a wave: see gemv_f32_default
-    return c.p0 == kWhole && (c.p1 == 1 || c.p1 == 2 || c.p1 == 4) && p.k % kWholeStep == 0 && p.k <= 2048 * kWhole &&
-                   (!int4 || p.group_size == 32) && (c.p1 < 4 || p.m <= 10) && !c.p2 && !c.p3 && !c.p4 && !c.p5 && !c.p6
+    return c.p0 == kWhole && (c.p1 == 1 || c.p1 == 2 || c.p1 == 4) && p.k % kWholeStep == 0 && p.k <= kWholeStep * kWholeMaxSteps * kWhole &&
+                   (!int4 || p.group_size == 32) && c.p2 >= 0 && c.p2 <= 16 * kWholeMaxCols && whole_fn(p, whole_blocks(c)) &&
+                   whole_block_cols(c) * (whole_blocks(c) - 1) < whole_cols(c) && !c.p3 && !c.p4 && !c.p5 && !c.p6
                ? true
                : fail(3);
   }
@@ -565,36 +649,24 @@ ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c) {
   return ScratchNeed{(size_t)column_tiles(p) * (size_t)c.p0 * (size_t)p.m * kCols, column_tiles(p)};
 }
 
-// All of K in one workgroup at nb blocks of 16 columns: rounds of workgroups, as the VALU feels them.
-// A second workgroup to a CU costs as much as the first (the VALU is what they share), three tiles of
-// pieces fill its LDS alone.
-static double whole_rounds(const Problem& p, int nb) {
-  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  const double x = (double)((p.n + 16 * nb - 1) / (16 * nb)) / cus;
-  return x <= 1.0 ? 1.0 : (p.m > 10 ? 1.15 * (double)(int64_t)(x + 0.999) : (x <= 2.0 ? 2.0 : 0.4 + 0.95 * x));
-}
-// ... what orders the widths of a problem, whatever its format: fitted at 1024..13838 x 768..12288, 3..16
-// rows; the width it picks is 0.4 % behind the best one in the mean (992 problems).
-static double width_us(const Problem& p, int nb) {
-  const double m = (double)p.m, c = nb == 1 ? 0.75 + 0.125 * m : (nb == 2 ? 1.35 + 0.135 * m : 2.7 + 0.16 * m);
-  return 2.9 + (double)p.k / 1000.0 * c * whole_rounds(p, nb);
-}
-// ... and the price of the launch beside that of K slices, in microseconds: fitted at 3182 launches of
-// the one and 1716 of the other (200 matrices of 400..24576 x 512..12288, 3..16 rows, four formats).
-// Per round the sums, 0.27 for every tile of pieces and block, and per 1000 of K the cutting of X and
-// the weights of a block: 96 % of the launches take 0.82-1.13 times that.  K slices: the longest one's
-// pieces and weights, and 0.010-0.017 for every row of every slice that the last arrival adds:
-// 0.85-1.17 times that, int4 (8 % above its fit: its short slices scatter) 0.72-1.2.
+// All of K in one workgroup at `cols` columns of nb blocks, in microseconds: per round of workgroups the
+// sums and the barriers, and per 1000 of K the cutting of X, the weights and the products.  Fitted at 2600
+// launches (34 matrices of 1024..15340 x 1024..12288, 2..16 rows, four formats): 7 % off (rms); the width it picks
+// is 0.5 % behind the best one in the mean, 5 % at worst.
 static int format_index(const Problem& p) { return p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1); }
-static double whole_us(const Problem& p, int nb) {
-  static const double weights[3][3][3] = {  // tiles of pieces, format, 1 / 2 / 4 blocks
-      {{0.61, 1.08, 2.05}, {0.70, 1.24, 2.55}, {0.54, 0.87, 1.84}},
-      {{0.70, 1.25, 2.19}, {0.72, 1.37, 2.49}, {0.50, 0.98, 1.74}},
-      {{0.92, 1.30, 0.0}, {0.91, 1.31, 0.0}, {0.76, 0.90, 0.0}}};
-  const int tiles = tiles_of(p.m);
-  const double m = (double)p.m;
-  return 2.77 + whole_rounds(p, nb) * (0.29 + 0.27 * tiles * nb + (double)p.k / 1000.0 * (0.074 * m + 0.012 * m * nb + weights[tiles - 1][format_index(p)][nb / 2]));
+static double whole_us(const Problem& p, int cols) {
+  static const double weights[3][3][4] = {  // tiles of pieces, format, blocks
+      {{0.404, 0.728, 1.090, 1.388}, {0.314, 0.662, 1.083, 1.376}, {0.162, 0.548, 0.951, 1.217}},
+      {{0.463, 0.842, 1.146, 1.671}, {0.406, 0.922, 1.044, 1.419}, {0.240, 0.550, 0.843, 1.159}},
+      {{0.519, 0.863, 1.315, 0.0}, {0.471, 0.816, 1.163, 0.0}, {0.362, 0.660, 0.915, 0.0}}};
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256, tiles = tiles_of(p.m), nb = (cols + 15) / 16;
+  const int64_t wgs = (p.n + cols - 1) / cols, rounds = (wgs + cus - 1) / cus, steps = p.k / kWholeStep;
+  const double k = (double)((steps + kWhole - 1) / kWhole * kWhole * kWholeStep) / 1000.0;
+  return 2.02 + (double)rounds * (0.88 + 0.186 * tiles * nb + k * (0.09 * (double)p.m + 0.116 * cols / 16.0 + weights[tiles - 1][format_index(p)][nb - 1]));
 }
+// ... and of K slices across workgroups (fitted at 1716 launches, 3..16 rows): the longest one's pieces and
+// weights, and 0.010-0.017 for every row of every slice that the last arrival adds: 0.85-1.17 times that, int4
+// (8 % above its fit: its short slices scatter) 0.72-1.2.
 static double slices_us(const Problem& p, int slices) {
   static const double base[3] = {10.7, 6.2, 6.5}, weights[3] = {5.22, 7.86, 4.98}, cut[3] = {0.471, 0.297, 0.324}, sum[3] = {0.010, 0.017, 0.014};
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256, f = format_index(p);
@@ -602,35 +674,32 @@ static double slices_us(const Problem& p, int slices) {
   return base[f] + (double)(rounds * slice) / 1000.0 * (weights[f] + cut[f] * (double)p.m) + sum[f] * (double)(slices * p.m);
 }
 
-// All of K in one workgroup, at the cheapest number of columns, or false where K slices are ahead.
-// Us, slices against here, over 24 matrices of 512..16246 x 768..12288 at 3..16 rows:
-//   up to five rows at nearly every one (int8-64 9216 x 2304: 13.0 -> 11.2, 2304 x 9216: 16.8 -> 15.3;
-//   int4 at 4096 x 4096 15.4 -> 8.6, at 12288 x 4096 28.8 -> 17.2);
-//   more rows of int4 with K up to 4096 or enough columns for every CU (16 rows at 12288 x 4096 50.8 ->
-//   33.8, at 4096 x 12288 39.7 -> 36.0; but 12 rows at 789 x 9984: 17.9 against 24.0);
-//   more rows of int8 with K up to 4096 where one round of double blocks holds the columns (10 rows
-//   at 2048 x 2304: 12.7 -> 7.1, at 7869 x 768 9.7 -> 6.1; but 16 rows at 9216 x 2304: 16.0 against 21.9).
-// Within these, where the price says so too: of 1174 problems that both forms were timed at nine are
-// more than 3 % behind the slices, by 10 % at most (16 rows of int8-128 at 4114 x 2816: 13.9 against
-// 12.7); without it 5 rows of int8 at 512 x 16384 took 23.2 against 17.1, 16 rows of int4 at 10208 x
-// 3712 32.4 against 26.8.
-static bool whole_default(const Problem& p, tlhip_kernel_config_t* out) {
+// All of K in one workgroup, at the cheapest number of columns (whole blocks, or an even share that
+// leaves no round half empty: 9216 columns in 256 workgroups of 36, not 576 of 16), or false where K slices stay.
+// Us, slices / here: 5 rows of int8-64 at 9216 x 2304 13.0 / 8.5, at 2304 x 9216 16.8 / 10.8; 10 rows at 12288 x
+// 4096 29.4 / 14.1; 16 rows of int4 at 12288 x 4096 46 / 18.5 and at 4096 x 12288 40 / 28.5.  Behind where the
+// price says so: 16 rows of int8 at 1484 x 8320 16-18 / 21-22, at 2304 x 9216 19-22 / 21-22.
+// Three exceptions, where the routes of longer standing are kept though this form has caught up with them:
+// more than 16384 columns; fewer than 1024 of a K beyond 8192 (5 rows at 512 x 16384 17.3 / 15.3); and int4 with
+// more than ten rows, 8192 columns and K an odd number of steps (10208 x 3712, 16 rows 27 / 18; 12748 x 4224, 14
+// rows 26.5 / 30).
+static bool whole_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  if (p.n > 16384) return false;
-  if (p.m > 5) {
-    if (p.format == TLHIP_FMT_INT4_GROUPED ? p.k > 4096 && p.n < (int64_t)cus * 16 : p.k > 4096 || p.n > (int64_t)cus * 32) return false;
-  }
+  if (p.n > 16384 || (p.n < 1024 && p.k > 8192)) return false;
+  if (p.format == TLHIP_FMT_INT4_GROUPED && p.m > 10 && p.n > 8192 && p.k / kWholeStep % 2) return false;
+  memset(out, 0, sizeof *out);
+  out->variant = VARIANT_GEMV_F32;
+  out->p0 = kWhole;
   bool found = false;
-  double best = 0.0;
-  for (int nb = 1; nb <= kWholeMaxCols; nb *= 2) {
-    tlhip_kernel_config_t c;
-    memset(&c, 0, sizeof c);
-    c.variant = VARIANT_GEMV_F32;
-    c.p0 = kWhole;
-    c.p1 = nb;
-    if (!gemv_f32_config_applicable(p, c, nullptr) || (found && width_us(p, nb) >= best)) continue;
+  for (int nb = 1; nb <= kWholeMaxCols; ++nb) {
+    const int64_t rounds = (p.n + (int64_t)cus * 16 * nb - 1) / ((int64_t)cus * 16 * nb);
+    const int even = (int)((p.n + rounds * cus - 1) / (rounds * cus)), cols = even > 16 * (nb - 1) && nb > 1 ? even : 16 * nb;
+    tlhip_kernel_config_t c = *out;
+    c.p2 = cols == 16 * nb && nb != 3 ? 0 : cols;
+    c.p1 = c.p2 ? (cols < 48 ? 1 : 2) : nb;  // beside p2 only the mark of the form
+    if (!gemv_f32_config_applicable(p, c, nullptr) || (found && whole_us(p, cols) >= *us)) continue;
     *out = c;
-    best = width_us(p, nb);
+    *us = whole_us(p, cols);
     found = true;
   }
   return found;
@@ -655,8 +724,9 @@ static bool slices_default(const Problem& p, tlhip_kernel_config_t* out) {
 
 bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out) {
   tlhip_kernel_config_t whole;
+  double us = 0.0;
   const bool found = slices_default(p, out);
-  if (!whole_default(p, &whole) || (found && whole_us(p, whole.p1) >= slices_us(p, out->p0))) return found;
+  if (!whole_default(p, &whole, &us) || (found && us >= slices_us(p, out->p0))) return found;
   *out = whole;
   return true;
 }
@@ -691,8 +761,11 @@ int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_
   a.epi = p.epi;
   void* args[] = {(void*)&a};
   const int tiles = tiles_of(p.m);
-  const int rc = c.p1 ? launch_kernel(whole_fn(p.format, tiles, c.p1), dim3((unsigned)((p.n + 16 * c.p1 - 1) / (16 * c.p1))), dim3(kWhole * 64), args,
-                                      whole_lds(tiles, c.p1), stream)
+  if (c.p1) {
+    a.cols = whole_cols(c);
+    a.block_cols = whole_block_cols(c);
+  }
+  const int rc = c.p1 ? launch_kernel(whole_fn(p, whole_blocks(c)), dim3((unsigned)((p.n + a.cols - 1) / a.cols)), dim3(kWhole * 64), args, whole_lds(p, whole_blocks(c)), stream)
                       : launch_kernel(fn_of(p.format, tiles), dim3((unsigned)(column_tiles(p) * a.slices)), dim3(kThreads), args,
                                       lds_of(p, a.slices), stream);
   if (rc) return rc;
@@ -705,10 +778,18 @@ int prepare_gemv_f32_kernels() {
   for (int format : {TLHIP_FMT_INT4_GROUPED, TLHIP_FMT_INT8_GROUPED, TLHIP_FMT_INT8_ROW})
     for (int tiles = 1; tiles <= 3; ++tiles) {
       int rc = launch_kernel(fn_of(format, tiles), dim3(1), dim3(64), nullptr, 0, nullptr);
-      for (int nb = 1; nb <= kWholeMaxCols && !rc; nb *= 2)
-        if (nb < 4 || tiles < 3) rc = launch_kernel(whole_fn(format, tiles, nb), dim3(1), dim3(64), nullptr, 0, nullptr);
       if (rc) return rc;
     }
+  Problem p;
+  memset(&p, 0, sizeof p);
+  for (p.format = 0; p.format < 3; ++p.format)
+    for (p.group_size = 64; p.group_size <= 128; p.group_size *= 2)
+      for (p.m = 1; p.m <= 16; ++p.m)
+        for (int nb = 1; nb <= kWholeMaxCols; ++nb)
+          if (const void* fn = whole_fn(p, nb)) {
+            const int rc = launch_kernel(fn, dim3(1), dim3(64), nullptr, 0, nullptr);
+            if (rc) return rc;
+          }
   return TLHIP_OK;
 }
 
