@@ -1011,17 +1011,18 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return false;
 }
 
-// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip) unless its price is a
-// twentieth above the former's: 0.5 % behind the faster one in the mean of 1299 problems timed with
-// both (level with no margin; over 66 decoder steps and Linears it lost less where the two are
-// close).  Us of plain launches, K slices against all of K: int8-64 12288 x 4096, 32 rows 28.0 against 22.2,
-// per row 4491 x 6272, 56 rows 31.5 against 20.8, but int8-64 2008 x 8192, 32 rows 12.1 against 18.2; int4
-// 12288 x 4096, 48 rows 27.2 against 18.1, but 2610 x 11520 23.0 against 25.1.
+// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip).  K up to 6144: unless its price
+// is a quarter above the former's; at 84 problems of 400..4000 x 2048..5632 it was the faster one at each, by 23 %
+// at prices alike and still by 20 % at 1.07 (20 rows of int4 at 900 x 3584 7.6 / 6.1 us).  Beyond, where few
+// columns leave most CUs idle: from 0.87 of it on (48 rows of int8-64 at 760 x 10496 14.7 us in K slices, 21.7
+// here; at 2496 x 11008, 32 rows of int4, 15.0 and 13.7); and so from 16384 columns on, where the prices are
+// least sure (17 rows of int4 at 16384 x 4096 16.2 / 14.1, but at 32000 x 4096 24.1 / 28.2).
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
   const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
-  if (!gemm_rows_default(p, &whole, &us) || (found && us >= 1.05 * gemv_mfma_rows_us(p, *out))) return found;
+  const double line = p.k > 6144 || p.n >= 16384 ? 0.87 : 1.25;
+  if (!gemm_rows_default(p, &whole, &us) || (found && us >= line * gemv_mfma_rows_us(p, *out))) return found;
   *out = whole;
   return true;
 }

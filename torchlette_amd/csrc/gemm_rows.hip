@@ -3,24 +3,24 @@
 // Same contract and reference route as gemv.hip (src/backend/webgpu/matmul/gemv.ts:365-466).
 //
 // What bounds it: its own instructions (X into LDS and out of it as operands, the dequantising, the
-// products), then the weights' way from memory, one or two steps ahead of a wave; the activations' way
-// comes last, although every workgroup needs all of X (64 rows of K = 4096 are 512 KB, three times a
-// CU's LDS) from its L2.  Int4, K = 4096, one round of 256 workgroups, us as it is / X from a buffer of no bytes
-// / the weights so / both: 48 rows at one block of columns 11.9 / 10.9 / 9.1 / 8.3, at two 15.5 / 14.4 / 10.6 / 10.2,
-// at three 18.1 / 15.1 / 12.1 / 12.8; 64 rows at three 20.9 / 18.3 / 16.6 / 15.7.  Hence:
+// products), then the weights' way from memory; the activations' way comes last, although every workgroup
+// needs all of X (64 rows of K = 4096 are 512 KB, three times a CU's LDS) from its L2.  Hence:
 //   * A workgroup owns 16 NB columns of Y and all of K, so that nothing is combined between
 //     workgroups: no planes of partial sums, no second launch, no workspace.
-//   * Its eight waves take K in turn, 128 at a time, each alone with its part until one
-//     barrier at the end: the activations of a step (16 MT rows) are loaded into registers
-//     one or two steps ahead, whole lines per row, laid into a patch of LDS that belongs to
-//     the wave, and read back as MFMA operands; every byte of X enters the CU once.
+//   * Each of its eight waves has a range of K, 128 a step, alone until one barrier at the end: the
+//     activations of a step (16 MT rows) are loaded into registers a step ahead, whole lines per row, laid
+//     into a patch of LDS that belongs to the wave, and read back as MFMA operands.
+//   * A range's group scales come once, 16 bytes of a column a lane, into LDS too: a load of 8 bytes of 16
+//     columns with every step cost the memory pipe what the step's weights do.
+//   * Plain loads of the weights: the neighbouring steps of a range share lines, which the nontemporal hint
+//     fetched twice (10-25 % slower).
 //   * An operand of X feeds NB products and a weight, dequantised once, MT.
-// One launch, us, best kernel before -> here: int4-32 12288 x 4096 at 48 / 64 rows 27.2 -> 18.1, 27.6 ->
-// 20.9; 4096 x 4096 at 48 rows 14.9 -> 12.1; int8-64 12288 x 4096 at 17..32 rows 27-28 -> 21-22, 7179 x
-// 896 at 40 rows 13.3 -> 7.0.  18.1 us are 1.5 TB/s of weights and 260 TFLOP/s.
+// Us, steps dealt to the waves in turn with their scales, two in flight and empty loads past the end -> as it is:
+// int4 12288 x 4096 at 48 rows 18.2 -> 14.6, 4096 x 4096 with a residual 13.0 -> 10.8, 1024 x 1024 6.4 -> 5.5; int8-64
+// 12288 x 4096 at 32 rows 21.8 -> 12.6; 1.24 times faster in the mean of 28 matrices of 768..16384 x 768..12288 at
+// 20..64 rows, four formats.  14.6 us are 1.9 TB/s of weights and scales and 330 TFLOP/s.
 // Rearranging X for the cheaper int4 unpacking, or its addresses by lane, moved nothing.
-//   * Buffer loads: rows past M, columns past N and steps past K read zero and cost no traffic,
-//     so that the loop has no branch around a load.
+//   * Buffer loads: rows past M and columns past N read zero, so that the loop has no branch around a load.
 #include <algorithm>
 #include <cstring>
 
@@ -33,6 +33,7 @@ constexpr int kWaves = 8;
 constexpr int kStep = 128;                  // k of a step
 constexpr int kRowBytes = kStep * 2 + 16;   // LDS row of a step: 16 bytes more, so that rows start in other banks
 constexpr int kMaxCols = 4;                 // blocks of 16 columns per workgroup
+constexpr int kMaxScaleSteps = 16;          // steps of a wave whose scales it holds at a time
 
 struct RowsArgs {
   const uint8_t* packed;
@@ -43,6 +44,8 @@ struct RowsArgs {
   int row_bytes;         // packed bytes of a weight row
   int scale_row_bytes;   // bytes of a row's group scales
   int group_shift;       // int8 groups: log2(group size / 64)
+  int scale_steps;       // steps of a wave whose scales its patch holds
+  int scale_stride;      // bytes of a column there
   float alpha, scale_mul;
   int y_dtype;
   int vec_ok;            // N % 4 == 0 and y 16-byte aligned: four columns in one store
@@ -51,17 +54,9 @@ struct RowsArgs {
 
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 
-// A step's number (negative: no such step) as a scalar that the compiler neither keeps in a
-// vector register nor selects with: either puts every load behind it into a loop over the lanes.
-__device__ __forceinline__ int scalar_step(int st, int steps) {
-  st = st < steps ? st : -1;
-  asm("" : "+s"(st));
-  return st;
-}
 __device__ __forceinline__ rsrc_t buffer_of(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00027000);
 }
-constexpr int kNontemporal = 2;  // the load's slc bit
 template <int AUX>
 __device__ __forceinline__ u32x4 load16(rsrc_t r, uint32_t at, uint32_t step_at) {
   return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, (int)step_at, AUX));
@@ -81,8 +76,8 @@ __device__ __forceinline__ half8_t weights_of(uint32_t w) {
   return join8(h);
 }
 
-// MT: tiles of 16 rows (M <= 16 MT); NB: blocks of 16 columns; XD: steps of X in registers (0: one, and one of the weights)
-template <int FMT, int MT, int NB, int XD>
+// MT: tiles of 16 rows (M <= 16 MT); NB: blocks of 16 columns
+template <int FMT, int MT, int NB>
 __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a) {
   constexpr bool INT4 = FMT == TLHIP_FMT_INT4_GROUPED, ROW = FMT == TLHIP_FMT_INT8_ROW;
   constexpr int WV = INT4 ? 1 : 2;      // 16-byte loads of a step, lane and column block
@@ -91,6 +86,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nl = lane & 15, g = lane >> 4;
+  const int a_scale_steps = a.scale_steps, scale_stride = a.scale_stride;
   const int n0 = (int)blockIdx.x * (16 * NB);
   const int cols = min(16 * NB, a.n - n0);
   const int steps = a.k / kStep;
@@ -107,42 +103,72 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
   }
   const uint32_t x_at = (uint32_t)g * (uint32_t)a.k * 2u + (uint32_t)nl * 16u;  // in four rows, a buffer each
 
-  struct Weights {
-    u32x4 w[NB][WV];
-    uint32_t s[NB][2];  // int4: four group scales; int8: one per half step
+  // The wave's range of steps (workgroups of an XCD start at different ones: all on the same lines of X at a
+  // time is slower), and its group scales in a patch of LDS, 16 bytes of a column a lane.
+  const int range = (wave + ((int)blockIdx.x >> 3)) & (kWaves - 1);
+  // (the first ranges are the longer ones: waves four apart share a SIMD, two long ones there are a step more)
+  const int each = steps / kWaves, more = steps % kWaves;
+  const int st0 = range * each + min(range, more), end = st0 + each + (range < more ? 1 : 0);
+  constexpr int SB = INT4 ? 8 : 4;  // bytes of a step and column
+  constexpr bool LATE = INT4 && MT * NB >= 8;  // no registers for the weights of two steps, nor a last step of its own
+  constexpr int SL = INT4 ? 2 : 1;  // 16-byte loads for kMaxScaleSteps steps: 64 bytes of a column each
+  char* const scale_patch = (char*)lds + kWaves * (MT * 16 * kRowBytes) + wave * (16 * NB * scale_stride) + nl * scale_stride;
+  struct Scales {
+    u32x4 v[SL][NB];  // (int8 in wider groups: word q is the scale of step 4 q + g)
   };
-  auto load_w = [&](Weights& v, int step) {
-    const int st = scalar_step(step, steps);
-    const uint32_t in = ~(uint32_t)(st >> 31);
-    const rsrc_t wb = buffer_of(packed, (uint32_t)cols * (uint32_t)a.row_bytes & in);
-    const rsrc_t sb = buffer_of(scales, (uint32_t)cols * (uint32_t)a.scale_row_bytes & in);
-    const uint32_t at = (uint32_t)st & in;
+  const rsrc_t sb = buffer_of(scales, (uint32_t)cols * (uint32_t)a.scale_row_bytes);
+  auto load_scales = [&](Scales& v, int from) __attribute__((always_inline)) {
+    const int count = min(a_scale_steps, end - from);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
+      if (INT4 || a.group_shift == 0) {
 #pragma unroll
-      for (int i = 0; i < WV; ++i) v.w[b][i] = load16<kNontemporal>(wb, w_at[b] + (uint32_t)i * 64u, at * (WV * 64u));
-      if constexpr (INT4) {
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-        const u32x2 s = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sb, (int)s_at[b], (int)(at * 8u), 0));
-        v.s[b][0] = s.x;
-        v.s[b][1] = s.y;
-      } else if constexpr (!ROW) {
+        for (int q = 0; q < SL; ++q) {  // (a lane past the range: what its column's first one reads)
+          const int at = q * 64 + g * 16 < count * SB ? q * 64 + g * 16 : 0;
+          v.v[q][b] = load16<0>(sb, s_at[b] + (uint32_t)at, (uint32_t)from * SB);
+        }
+      } else {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-          v.s[b][h] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sb, (int)s_at[b], (int)(((2u * at + (uint32_t)h) >> a.group_shift) * 2u), 0);
+        for (int q = 0; q < 4; ++q)
+          v.v[0][b][q] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(sb, (int)(s_at[b] + ((uint32_t)(2 * (from + min(4 * q + g, count - 1))) >> a.group_shift) * 2u), 0, 0);
       }
     }
+  };
+  auto lay_scales = [&](const Scales& v, int from) __attribute__((always_inline)) {
+    const int count = min(a_scale_steps, end - from);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      char* const to = scale_patch + 16 * b * scale_stride;
+      if (INT4 || a.group_shift == 0) {
+#pragma unroll
+        for (int q = 0; q < SL; ++q)
+          if (q * 64 + g * 16 < count * SB) *(u32x4*)(to + q * 64 + g * 16) = v.v[q][b];
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (q * 4 + g < count) *(uint32_t*)(to + (q * 4 + g) * 4) = v.v[0][b][q] | v.v[0][b][q] << 16;
+      }
+    }
+  };
+  struct Weights {
+    u32x4 w[NB][WV];
+  };
+  const rsrc_t wb = buffer_of(packed, (uint32_t)cols * (uint32_t)a.row_bytes);
+  auto load_block = [&](Weights& v, int b, int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < WV; ++i) v.w[b][i] = load16<0>(wb, w_at[b] + (uint32_t)i * 64u, (uint32_t)st * (WV * 64u));
+  };
+  auto load_w = [&](Weights& v, int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) load_block(v, b, st);
   };
   struct Rows {
     u32x4 v[XV];
   };
-  auto load_x = [&](Rows& r, int step) {
-    const int st = scalar_step(step, steps);
-    const uint32_t in = ~(uint32_t)(st >> 31);
-    const uint32_t at = (uint32_t)st * (kStep * 2u) & in;
+  auto load_x = [&](Rows& r, int st) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < XV; ++i)
-      r.v[i] = load16<0>(buffer_of(a.x + (int64_t)(4 * i) * a.k, (uint32_t)max(a.m - 4 * i, 0) * (uint32_t)a.k * 2u & in), x_at, at);
+      r.v[i] = load16<0>(buffer_of(a.x + (int64_t)(4 * i) * a.k, (uint32_t)max(a.m - 4 * i, 0) * (uint32_t)a.k * 2u), x_at, (uint32_t)st * (kStep * 2u));
   };
   char* const patch = (char*)lds + wave * (MT * 16 * kRowBytes);
   auto lay_x = [&](const Rows& r) {
@@ -160,7 +186,18 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
     const int unit = INT4 ? 4 * s + g : 8 * (s >> 1) + 2 * g + (s & 1);
     return __builtin_bit_cast(half8_t, *(const u32x4*)(patch + (16 * t + nl) * kRowBytes + unit * 16));
   };
-  auto multiply = [&](const Weights& v) __attribute__((always_inline)) {
+  // `next`: the step whose weights take the registers as they become free, or -1
+  auto multiply = [&](Weights& v, int st_held, int next) __attribute__((always_inline)) {
+    uint32_t scale[NB][2];  // int4: four group scales; int8: one per half step
+    if constexpr (!ROW) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const char* const from = scale_patch + 16 * b * scale_stride + st_held * SB;
+        const uint32_t w = *(const uint32_t*)from;
+        scale[b][0] = INT4 ? w : w & 0xffffu;
+        scale[b][1] = INT4 ? *(const uint32_t*)(from + 4) : w >> 16;
+      }
+    }
     uint32_t word[NB][4 * WV];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -174,6 +211,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
       // a lane holds 32 k of its row, one group; afterwards word i is its eighth of group i
       if constexpr (INT4) transpose4(word[b][0], word[b][1], word[b][2], word[b][3]);
     }
+    if (next >= 0) load_w(v, next);
     // a step's own sum first: the long one takes a step at a time (rel-L2 against 64 bits at K = 8192,
     // int4 / int8-64 / per row: 11.3 / 9.7 / 16.3e-8 one group at a time, 8.4 / 8.9 / 8.8e-8 so, 8.8 / 8.9 / 9.2e-8
     // for the decode kernel with its four to eight K slices)
@@ -184,7 +222,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const half8_t wv = weights_of(word[b][s]);
-          const float sc = half_bits_to_float((s & 1) ? v.s[b][s >> 1] >> 16 : v.s[b][s >> 1] & 0xffffu);
+          const float sc = half_bits_to_float((s & 1) ? scale[b][s >> 1] >> 16 : scale[b][s >> 1] & 0xffffu);
           float4_t d[MT];
 #pragma unroll
           for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(operand(t, s), wv, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -211,7 +249,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
           const half8_t wv = weights_of(word[b][s]);
-          const float sc = half_bits_to_float((s & 1) ? v.s[b][s >> 1] >> 16 : v.s[b][s >> 1] & 0xffffu);
+          const float sc = half_bits_to_float((s & 1) ? scale[b][s >> 1] >> 16 : scale[b][s >> 1] & 0xffffu);
           float4_t d[MT];
 #pragma unroll
           for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[t], wv, (float4_t){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -243,7 +281,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 #pragma unroll
             for (int t = 0; t < MT; ++t) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[i][t], wv, d[t], 0, 0, 0);
           }
-          const float sc = ROW ? 1.f : half_bits_to_float(v.s[b][h]);
+          const float sc = ROW ? 1.f : half_bits_to_float(scale[b][h]);
 #pragma unroll
           for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -262,54 +300,51 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
         for (int r = 0; r < 4; ++r) acc[b][t][r] += sum[b][t][r];
   };
 
-  // Every load below is unconditional (a wait at a join would count it as not issued); the
-  // patch is the wave's own, and a wave's LDS accesses stay in order.
-  if constexpr (XD == 0) {  // one step of either
+  // No load goes past the end, though a buffer would answer it with zeros: at one to four steps a wave those cost
+  // as much as the others (12-20 % at K up to 2304).  The patch is the wave's own, and a
+  // wave's LDS accesses stay in order.  One part, unless the scales of a range do not fit.
+  for (int from = st0; from < end; from += a_scale_steps) {
+    const int upto = min(from + a_scale_steps, end), left = upto - from;
+    Scales v;
+    if constexpr (!ROW) {
+      load_scales(v, from);
+      __builtin_amdgcn_sched_barrier(0);  // ahead of the rest: a wait for them is a wait for nothing else
+    }
     Weights w;
     Rows x;
-    load_x(x, wave);
-    load_w(w, wave);
-    for (int st = wave; st < steps; st += kWaves) {
-      lay_x(x);
-      load_x(x, st + kWaves);
-      multiply(w);
-      load_w(w, st + kWaves);
-    }
-  } else {
-    Weights w0, w1;
-    Rows x0, x1;
-    load_x(x0, wave);
-    load_w(w0, wave);
-    if constexpr (XD == 2) load_x(x1, wave + kWaves);
-    load_w(w1, wave + kWaves);
-    for (int st = wave; st < steps; st += 2 * kWaves) {
-      lay_x(x0);
-      if constexpr (XD == 2) load_x(x0, st + 2 * kWaves);
-      else load_x(x0, st + kWaves);
-      multiply(w0);
-      if (st + kWaves >= steps) break;
-      load_w(w0, st + 2 * kWaves);
-      if constexpr (XD == 2) {
-        lay_x(x1);
-        load_x(x1, st + 3 * kWaves);
-      } else {
-        lay_x(x0);
-        load_x(x0, st + 2 * kWaves);
+    load_x(x, from);
+    load_w(w, from);
+    if constexpr (!ROW) lay_scales(v, from);
+    if constexpr (LATE) {
+      for (int i = 0; i + 1 < left; ++i) {
+        lay_x(x);
+        load_x(x, from + i + 1);
+        multiply(w, i, -1);
+        load_w(w, from + i + 1);
       }
-      multiply(w1);
-      load_w(w1, st + 3 * kWaves);
+      lay_x(x);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(w, left - 1, -1);
+    } else {
+      for (int i = 0; i + 1 < left; ++i) {
+        lay_x(x);
+        load_x(x, from + i + 1);
+        multiply(w, i, from + i + 1);
+      }
+      lay_x(x);
+      multiply(w, left - 1, -1);
     }
   }
 
   // ---- the waves' sums and the epilogue ---------------------------------------
   lds_barrier();  // every wave has read its patch
-  float* const sums = (float*)lds;  // [wave][row tile][block][16 x 16]
+  float* const sums = (float*)lds;  // [range][row tile][block][16 x 16]
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sums[((wave * MT + t) * NB + b) * 256 + (4 * g + r) * 16 + nl] = acc[b][t][r];
+      for (int r = 0; r < 4; ++r) sums[((range * MT + t) * NB + b) * 256 + (4 * g + r) * 16 + nl] = acc[b][t][r];
   lds_barrier();
   float factor = a.scale_mul * a.alpha;
 #pragma unroll
@@ -347,8 +382,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 
 int row_tiles_of(int64_t m) { return (int)((m + 15) / 16); }
 // The column blocks whose instance fits 256 vector registers a lane without spilling one; the fullest
-// (int4, three blocks of 48 rows) uses all of them, three more 249 to 253.  Four row tiles need 16
-// buffer descriptors a step and spill up to 20 scalar registers, to lanes of a vector register.
+// (int4, three blocks of 48 rows and two of 64) use all of them.  Four row tiles need 16 buffer
+// descriptors a step and spill some scalar registers, to lanes of a vector register.
 constexpr int most_columns(int format, int mt) {
   return format == TLHIP_FMT_INT4_GROUPED ? (mt == 4 ? 3 : 4) : (mt == 2 ? 4 : (mt == 3 ? 3 : 2));
 }
@@ -358,10 +393,7 @@ const void* instance() {
   if constexpr (NB > most_columns(FMT, MT)) {
     return nullptr;
   } else {
-    // X two steps ahead where the registers allow it
-    constexpr int used = MT * 32 + NB * MT * 4 + NB * (FMT == TLHIP_FMT_INT4_GROUPED ? 12 : 24) + 40;
-    constexpr bool full = FMT == TLHIP_FMT_INT4_GROUPED && MT * NB >= 9;
-    return (const void*)gemm_rows_kernel<FMT, MT, NB, (full ? 0 : (used <= 200 ? 2 : 1))>;
+    return (const void*)gemm_rows_kernel<FMT, MT, NB>;
   }
 }
 template <int FMT, int MT>
@@ -378,8 +410,21 @@ const void* instance_of(int format, int mt, int nb) {
                                           : instance_of<TLHIP_FMT_INT8_GROUPED>(mt, nb);
 }
 
-size_t lds_of(int mt, int nb) {
-  return std::max((size_t)kWaves * mt * 16 * kRowBytes, (size_t)kWaves * mt * nb * 1024);
+// Steps whose scales a wave's patch holds: all of a range, or as many as fit beside the rows.
+int scale_steps_of(const Problem& p, int mt, int nb) {
+  if (p.format == TLHIP_FMT_INT8_ROW) return (int)(p.k / kStep);
+  const int sb = p.format == TLHIP_FMT_INT4_GROUPED ? 8 : 4, range = (int)((p.k / kStep + kWaves - 1) / kWaves);
+  const int lds = 160 * 1024 - kWaves * mt * 16 * kRowBytes;
+  const int fit = (lds / (kWaves * 16 * nb) / 16 * 16 - 16) / sb;
+  return std::min({range, kMaxScaleSteps, fit});
+}
+int scale_stride_of(const Problem& p, int mt, int nb) {
+  const int steps = scale_steps_of(p, mt, nb);
+  return p.format == TLHIP_FMT_INT8_ROW ? 0 : (steps * (p.format == TLHIP_FMT_INT4_GROUPED ? 8 : 4) + 15) / 16 * 16 + 16;
+}
+size_t lds_of(const Problem& p, int mt, int nb) {
+  const int scales = 16 * nb * scale_stride_of(p, mt, nb);
+  return std::max((size_t)kWaves * (mt * 16 * kRowBytes + scales), (size_t)kWaves * mt * nb * 1024);
 }
 
 }  // namespace
@@ -394,25 +439,23 @@ bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
   return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
 }
 
-// The cheapest number of column blocks and its time in microseconds, or false.  The time is what it
-// adds to a decoder layer: behind an RMSNorm that writes its activations, cold weights, and the mean
-// of four launches without and three with a residual, as a layer's seven are.  Fitted at 4130 of
-// 1300 problems (500..16384 x 768..12288, 17..64 rows, four formats): launch, and per round of
-// workgroups a constant, the sums of a block and per 4096 of K the figure of the width, a little more
-// for every row above the middle of its tile.  One block a workgroup: a second round overlaps the
-// first (two fit a CU up to 32 rows).  96 % take 0.87-1.15 times that; the width it picks is 0.03 %
-// slower than the best one in the mean.
+// The cheapest number of column blocks and its time in microseconds, or false.  Fitted at 3072 launches of
+// 52 matrices of 768..16384 x 768..12288, 17..64 rows, four formats, cold weights, with a residual up to 4608
+// columns: launch, and per round of workgroups a constant, the sums of a block and, per 4096 of K in whole
+// steps of the longest wave, the figure of the width, a little more for every row above the middle of its
+// tile.  One block a workgroup: a second round overlaps the first (two fit a CU up to 32 rows).  8-10 % off
+// (rms); the width it picks is 0.03 % slower than the best one in the mean, 5 % at worst.
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
   struct Cost {
-    double launch, round, block, walk[kMaxCols];
+    double launch, round, block, walk[kMaxCols], second, per_row;
   };
   static const Cost costs[3][3] = {  // format, row tiles
-      {{0.82, 0.99, 0.38, {6.03, 7.60, 10.77, 13.12}}, {0.0, 2.02, 0.53, {8.25, 9.69, 11.03, 16.25}}, {0.0, 2.27, 0.66, {9.66, 10.33, 14.87, 0.0}}},  // int4
-      {{0.96, 0.92, 0.35, {7.60, 10.17, 15.29, 18.46}}, {0.0, 2.52, 0.30, {9.28, 10.92, 16.63, 0.0}}, {0.0, 2.06, 0.42, {10.36, 13.78, 0.0, 0.0}}},    // int8 in groups
-      {{0.53, 1.12, 0.54, {6.49, 7.90, 11.84, 13.96}}, {0.0, 1.81, 0.59, {8.61, 8.87, 13.61, 0.0}}, {0.0, 1.72, 0.71, {9.40, 10.98, 0.0, 0.0}}}};     // int8 per row
-  static const double per_row[3] = {0.008, 0.005, 0.004}, second[3] = {0.80, 0.96, 0.96};
+      {{3.24, 0.0, 0.367, {4.09, 5.39, 6.99, 8.29}, 0.56, 0.004}, {2.70, 0.64, 0.568, {5.64, 6.72, 8.72, 11.71}, 0.83, 0.004}, {2.52, 0.85, 0.584, {7.03, 8.10, 11.91, 0.0}, 0.82, 0.006}},  // int4
+      {{3.37, 0.0, 0.361, {4.54, 5.92, 7.65, 9.23}, 0.64, 0.012}, {3.04, 0.65, 0.507, {6.00, 7.22, 9.62, 0.0}, 0.88, 0.005}, {2.87, 1.27, 0.169, {7.09, 8.70, 0.0, 0.0}, 0.86, 0.006}},    // int8 in groups
+      {{3.62, 0.0, 0.147, {4.26, 5.60, 7.51, 9.12}, 0.73, 0.008}, {2.78, 0.69, 0.495, {5.84, 6.75, 9.22, 0.0}, 0.87, 0.005}, {2.65, 1.44, 0.127, {6.77, 8.13, 0.0, 0.0}, 0.84, 0.009}}};  // int8 per row
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int format = p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1), mt = row_tiles_of(p.m);
+  const double walk = (double)((p.k / kStep + kWaves - 1) / kWaves * kWaves * kStep) / 4096.0;
   bool found = false;
   for (int nb = 1; nb <= kMaxCols; ++nb) {
     tlhip_kernel_config_t c;
@@ -423,9 +466,8 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
     if (!is_rows_config(p, c)) continue;
     const Cost& cost = costs[format][mt - 2];
     const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb);
-    const double rounds = 1.0 + (double)((wgs + cus - 1) / cus - 1) * (nb == 1 ? second[mt - 2] : 1.0);
-    const double t = cost.launch + rounds * (cost.round + cost.block * nb +
-                                             (double)p.k / 4096.0 * cost.walk[nb - 1] * (1.0 + per_row[mt - 2] * (double)(p.m - 16 * mt + 8)));
+    const double rounds = 1.0 + (double)((wgs + cus - 1) / cus - 1) * (nb == 1 ? cost.second : 1.0);
+    const double t = cost.launch + rounds * (cost.round + cost.block * nb + walk * cost.walk[nb - 1] * (1.0 + cost.per_row * (double)(p.m - 16 * mt + 8)));
     if (found && t >= *us) continue;
     *out = c;
     *us = t;
@@ -449,6 +491,8 @@ int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream
   a.row_bytes = (int)(p.format == TLHIP_FMT_INT4_GROUPED ? p.k / 2 : p.k);
   a.scale_row_bytes = p.format == TLHIP_FMT_INT8_ROW ? 4 : (int)(p.k / p.group_size) * 2;
   a.group_shift = p.format == TLHIP_FMT_INT8_GROUPED ? __builtin_ctz((unsigned)(p.group_size / 64)) : 0;
+  a.scale_steps = scale_steps_of(p, row_tiles_of(p.m), c.p4);
+  a.scale_stride = scale_stride_of(p, row_tiles_of(p.m), c.p4);
   a.alpha = p.alpha;
   a.scale_mul = p.format == TLHIP_FMT_INT8_GROUPED ? 1.0f / 127.0f : 1.0f;
   a.y_dtype = p.y_dtype;
@@ -457,7 +501,7 @@ int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream
   void* args[] = {(void*)&a};
   const int mt = row_tiles_of(p.m), nb = c.p4;
   const int rc = launch_kernel(instance_of(p.format, mt, nb), dim3((unsigned)((p.n + 16 * nb - 1) / (16 * nb))), dim3(kWaves * 64), args,
-                               lds_of(mt, nb), stream);
+                               lds_of(p, mt, nb), stream);
   if (rc) return rc;
   count_gemv_dispatch();
   return TLHIP_OK;
