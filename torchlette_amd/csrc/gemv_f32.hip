@@ -368,7 +368,9 @@ __global__ __launch_bounds__(kWhole * 64) void gemv_f32_whole_kernel(const F32Ar
   // ---- the wave's range of steps and its scales (workgroups of an XCD start at different ranges: all on
   // the same lines of X at a time is 10-15 % slower)
   const int range = (wave + ((int)blockIdx.x >> 3)) & (kWhole - 1);
-  const int st0 = steps * range / kWhole, left = steps * (range + 1) / kWhole - st0;
+  // (the first ranges are the longer ones: waves four apart share a SIMD, two long ones there are a step more)
+  const int each = steps / kWhole, more = steps % kWhole;
+  const int st0 = range * each + min(range, more), left = each + (range < more ? 1 : 0);
   constexpr int PER = WIDE ? 64 / SB : 4;  // steps of a load: a quarter of them on each of a column's four lanes
   constexpr int SL = kWholeMaxSteps / PER;
   char* const patch = (char*)lds + wave * (16 * T * kWholeRow);

@@ -136,7 +136,9 @@ __global__ __launch_bounds__(kFewWaves * 64) void gemv_few_kernel(const FewArgs<
   // ---- the wave's range of steps and its scales
   // (workgroups of an XCD start at different ranges: all on the same lines at a time is 10-15 % slower)
   const int range = (wave + (wg >> 3)) & (kFewWaves - 1);
-  const int st0 = steps * range / kFewWaves, left = steps * (range + 1) / kFewWaves - st0;
+  // (the first ranges are the longer ones: waves four apart share a SIMD, two long ones there are a step more)
+  const int each = steps / kFewWaves, more = steps % kFewWaves;
+  const int st0 = range * each + min(range, more), left = each + (range < more ? 1 : 0);
   constexpr int PER = WIDE ? 64 / SB : 4;        // steps of a load: a quarter of them on each of a column's four lanes
   constexpr int SL = WIDE ? kFewMaxSteps / PER : kFewMaxSteps / 4;
   char* const scale_patch = (char*)lds + kFewWaves * (4 * XV * kFewRowBytes) + wave * (NB * 16 * kFewScaleRow);
