@@ -36,6 +36,7 @@
 #include "common.h"
 #include "gemv_few.h"
 #include "gemv_one.h"
+#include "gemv_some.h"
 
 namespace tlhip {
 namespace {
@@ -439,8 +440,10 @@ bool wave_tile_config(const Problem& p, tlhip_kernel_config_t* out) {
 
 // Up to 16 f32 rows on the matrix cores, three bf16 pieces each, or on the VALU kernel; us, VALU
 // against the matrix cores with K slices, over 13 matrices of 1024 x 768 .. 32768 x 1024 at 3, 4, 5, 8,
-// 9 and 16 rows.  (The form that keeps all of K in one workgroup, which gemv_f32_default prefers where
-// it is cheaper, is not weighed here: five rows at 2304 x 2048 would take about 6 us on it.)
+// 9 and 16 rows.  (Both have newer forms: all of K in one workgroup, which gemv_f32_default prefers where it is
+// cheaper, and on the VALU up to five rows in one launch, few_f32_rows_config.  At the line the two are within
+// a third of each other, us, VALU / matrix cores: five rows of int8-64 at 2304 x 2048 5.4 / 5.4, four of int4 at 12288
+// x 4096 14.9 / 11.4.)
 //   From five rows on (five: 28.6 against 16.7 at 2304 x 9216 int8-64), but for small matrices
 //   in groups whose K fills whole passes of the VALU kernel's lanes (five rows of int4: 10.9
 //   against 15.0 at 1024 x 3072, 11.4 against 14.1 at 4096 x 1024; eight rows: level; five of
@@ -479,10 +482,23 @@ bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return gemv_few_default(&p, 1, FEW_SINGLE, out, &us);
 }
 
+// 2 to 5 f32 rows on the VALU in one launch (gemv_some.hip): where they do not go to the matrix cores, and
+// there too where few columns leave the launch to its chain of steps.  Us, four rows and the rest (two and two) in
+// launches of their own -> here / all of K on the matrix cores: 5 rows of int8-64 at 2304 x 2048 10.6 -> 5.4 / 5.4, at
+// 1024 x 4096 10.5 -> 5.0 / 6.8, 3 rows of int4 at 4096 x 4096 14.3 -> 6.8 / 6.7, 2 rows at 4096 x 4096 7.5 -> 6.1 / 6.7,
+// at 1024 x 1024 4.1 -> 3.3 / 3.7.  Two rows of a longer K and more columns: the matrix cores (int4 6376 x 4480
+// 13.8 -> 11.6 / 8.9, 4096 x 12288 18.0 -> - / 11.9, 9216 x 2304 10.9 -> 9.4 / 8.3).
+bool few_f32_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
+  if (p.x_dtype != TLHIP_F32 || p.m < 2 || p.m > 5 || p.n > 16384 || p.pro.kind != TLHIP_PRO_NONE) return false;
+  if (p.m == 2 && (p.k > 8192 || (p.k > 4096 && p.n > 2048) || (p.k > 2048 && p.n > 8192))) return p.k <= 16384 && gemv_f32_default(p, out) && out->p1;
+  const bool few = p.k > 1280 && (p.k <= 4096 ? p.n <= 2048 : p.n <= 1024);
+  return (p.m == 2 || few || !f32_rows_on_matrix_cores(p)) && gemv_some_default(p, out);
+}
+
 // Heuristic default, used when nothing is tuned.
 tlhip_kernel_config_t default_config(const Problem& p) {
   tlhip_kernel_config_t few;
-  if (few_rows_config(p, &few)) return few;
+  if (few_rows_config(p, &few) || few_f32_rows_config(p, &few)) return few;
   if (p.m > 16 && p.x_dtype == TLHIP_F16) {
     // the eight-wave kernel wherever it takes the problem (K a multiple of 64, groups of 32 or
     // 64 times a power of two): ahead of the kernels below at every one of 196 problems from 64
@@ -774,6 +790,7 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     if (is_few_config(there, c, FEW_SINGLE) && !few_rows_config(p, &c)) continue;
     // (one row: the lanes that share it follow from K and the number of columns)
     if (c.variant == VARIANT_GEMV) (void)gemv_one_default(p, p.n, ONE_SINGLE, &c);
+    if (is_some_config(c) && !gemv_some_default(p, &c)) continue;
     const double d = dn + 2.0 * dk + dm;  // K decides whether the activations fit LDS: weigh it
     if (d < best && config_applicable(p, c, nullptr)) {
       best = d;
@@ -1215,6 +1232,10 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
         vary(2, {4, 8});
         vary(3, {1, 2, 4, 8});
         vary(4, {1, 2, 4});
+        break;
+      }
+      if (is_some_config(base)) {  // its columns are its only field
+        vary(4, {4, 8, 12, 16, 24, 32, 48});
         break;
       }
       vary(0, {16, 32, 64});

@@ -6,6 +6,7 @@
 #include <cstring>
 
 #include "gemv_args.h"
+#include "gemv_some.h"
 
 namespace tlhip {
 
@@ -34,6 +35,7 @@ bool gemv_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, co
   };
   if (c.variant != VARIANT_GEMV) return fail(0);
   if (is_one_config(c)) return gemv_one_config_applicable(p, c, why);
+  if (is_some_config(c)) return gemv_some_config_applicable(p, c, why);
   if (c.p0 != 16 && c.p0 != 32 && c.p0 != 64) return fail(1);
   if (c.p1 != 1 && c.p1 != 2 && c.p1 != 4) return fail(2);
   if (c.p2 < 1 || c.p2 > 8) return fail(3);
@@ -109,6 +111,7 @@ int launch_gemv(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t st
   if (!gemv_config_applicable(p, c, &why)) return set_error(TLHIP_ERR_INVALID, "gemv: config not applicable: %s", why);
   if (p.n == 0 || p.m == 0) return TLHIP_OK;
   if (is_one_config(c)) return launch_gemv_one(p, c, stream);
+  if (is_some_config(c)) return launch_gemv_some(p, c, stream);
   const int xbytes = p.x_dtype == TLHIP_F16 ? 2 : 4;
 
   // activation rows per pass: as many (4, 2 or 1) as fit LDS next to the partials

@@ -11,6 +11,7 @@
 #include <unordered_set>
 
 #include "common.h"
+#include "gemv_some.h"
 #include "gemv_few.h"
 
 namespace tlhip {
@@ -199,6 +200,7 @@ int prepare_all_kernels() {
   t_prepare_mode = true;
   int rc = prepare_gemv_kernels();
   if (!rc) rc = prepare_gemv_one_kernels();
+  if (!rc) rc = prepare_gemv_some_kernels();
   if (!rc) rc = prepare_gemv_few_kernels();
   if (!rc) rc = prepare_gemv_mfma_kernels();
   if (!rc) rc = prepare_gemv_xreg_kernels();
