@@ -455,7 +455,9 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
       {{3.62, 0.0, 0.147, {4.26, 5.60, 7.51, 9.12}, 0.73, 0.008}, {2.78, 0.69, 0.495, {5.84, 6.75, 9.22, 0.0}, 0.87, 0.005}, {2.65, 1.44, 0.127, {6.77, 8.13, 0.0, 0.0}, 0.84, 0.009}}};  // int8 per row
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int format = p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1), mt = row_tiles_of(p.m);
-  const double walk = (double)((p.k / kStep + kWaves - 1) / kWaves * kWaves * kStep) / 4096.0;
+  // (up to four steps: on a SIMD each)
+  const int64_t steps = p.k / kStep, walked = steps <= 4 ? steps : (steps + kWaves - 1) / kWaves * kWaves;
+  const double walk = (double)(walked * kStep) / 4096.0;
   bool found = false;
   for (int nb = 1; nb <= kMaxCols; ++nb) {
     tlhip_kernel_config_t c;
