@@ -313,10 +313,10 @@ int tlhip_gemv_sequence(const tlhip_sequence_step_t* steps, int count, int x_dty
 /* The MLP block of a decoder layer from one call:
  * h = unary(x gate^T) * (x up^T)  (f16 [m, gate.N], caller-provided),  y = epilogue(h down^T).
  * f16 activations, 1..16 rows, any weight format.  The library runs the form that measures
- * faster: today three launches (gate and up grouped on the shared activations, the gated
- * multiply, down; gate and up are rounded to f16 in between, as the model's own ops would),
- * with 2 MiB of the stream's workspace between them, so a stream's first call must not be
- * captured.  TLHIP_MLP_ONE_LAUNCH=1 in the environment selects the sequence launch (a gated
+ * faster: two launches (gate, up and their product; down) where a kernel takes the pair, else three
+ * (gate and up grouped on the shared activations, the gated multiply, down); gate and up are rounded
+ * to f16 in between, as the model's own ops would.  It asks for 2 MiB of the stream's workspace
+ * either way, so a stream's first call must not be captured.  TLHIP_MLP_ONE_LAUNCH=1 in the environment selects the sequence launch (a gated
  * step and the down projection waiting for it: int4 g32 only, the product rounded once). */
 int tlhip_mlp_decode(const tlhip_qweight_t* gate, const tlhip_qweight_t* up, const tlhip_qweight_t* down, int unary,
                      const void* x, int x_dtype, int64_t m, void* h, void* y, int y_dtype,
@@ -429,7 +429,9 @@ int tlhip_topk(const float* logits, int64_t offset, int64_t length, int k, float
  * waves per workgroup and, above 32 rows, at most 2 iterations in flight; 17..64 rows with
  * p0 = 8, p4 = 1..4 and every other field 0 keep all of K in one workgroup of 16 p4 columns: K a
  * multiple of 128, int4 in groups of 32, int8 in groups of 64 or more or per row, and few enough
- * columns for its registers: up to 4 / 4 / 3 for int4 and 4 / 3 / 2 for int8 at 32 / 48 / 64 rows),
+ * columns for its registers: up to 4 / 4 / 3 for int4 and 4 / 3 / 2 for int8 at 32 / 48 / 64 rows; 2..16 f16
+ * rows with p0 = 8, p1 = 0, p2 columns, a multiple of 4, in p4 = 1, 2, 3, 4 or 6 blocks keep all of K in one workgroup
+ * of p2 columns: K a multiple of 128 up to 16384, the same formats),
  * 2 = "tiled" (prefill MFMA GEMM, both operands through LDS),
  * 3 = "tiled_direct" (prefill MFMA GEMM whose weights stay packed up to the
  * operand registers; fields as "tiled" with tile K 128; int4-grouped on the tiles
@@ -444,7 +446,8 @@ int tlhip_topk(const float* logits, int64_t offset, int64_t length, int k, float
  * multiple of 64, every format with groups of 32 (int4) or 64 (int8) times a power of two),
  * 6 = "gemv_f32" (f32 activations, 1..16 rows, each value cut into three bf16 pieces on the
  * matrix cores: p0 K slices across workgroups, 1..64; with p0 = 8 and p1 = 1, 2 or 4 all of K in one
- * workgroup of 16 p1 columns, K a multiple of 128 up to 16384, int4 in groups of 32),
+ * workgroup of 16 p1 columns, or of p2 (up to 64; 48 above ten rows) if that is not 0, K a multiple of 128 up
+ * to 16384, int4 in groups of 32),
  * 4 = "gemv_mfma_xreg" (skinny MFMA for int4 g32 with the activations held in
  * registers: p0 waves per workgroup, p1 iterations in flight, p2 workgroups per
  * CU, p3 K slices across workgroups, p4 = 1: every weight load of a wave issued
@@ -459,6 +462,9 @@ typedef struct {
   int32_t p3; /* gemv: K-split waves (LDS combine) gemv_mfma: K slices across workgroups (0/1 = none)  tiled: waves M */
   int32_t p4; /* gemv: chunks in flight (2/4/8)    gemv_mfma, 17..64 rows, p1 = 0: blocks of 16 columns (else not read)  tiled: waves N */
   int32_t p5; /* gemv: 1 = dot products on the 4x4x4 matrix-core instruction (int4, f16 x, m <= 4, p0 = 16, p1 = 1)
+               * gemv: 3 = the kernel for one row (p0 lanes per row, p1 = 1, p2 waves 4 or 8, p3 K-split waves, p4
+               * workgroups per CU); 4 = the kernel for 2..5 f32 rows (p0 lanes of a column, p1 = 1, p2 = 8, p3 = 1,
+               * p4 columns of a workgroup 1..64; K a multiple of 32 up to 64 p0, 8192 for 64 lanes)
                * gemv_mfma: 1 = whole-line weight loads through a wave-private LDS patch (int8 with
                * K % 128 == 0 or int4-g32 with K % 256 == 0; p1 = 2 or 4)
                * tiled, tiled_direct: K slices across workgroups (0/1 = none; 2..16: that many

@@ -649,8 +649,8 @@ class HipBackend:
     def mlpDecode(self, input: HipTensor, gate: HipTensor, up: HipTensor, down: HipTensor,
                   activation: str = "silu", oneLaunch: bool = False) -> HipTensor:
         """down(act(gate(x)) * up(x)) (packages/qwen3-browser/src/model.ts:357-361) from one
-        call: tlhip_mlp_decode, which runs the faster form (today the three launches the model
-        issues); oneLaunch=True asks for the sequence launch (a gated step and the down
+        call: tlhip_mlp_decode, which runs the faster form (gate, up and their product in one
+        launch, then down, or the three launches the model issues); oneLaunch=True asks for the sequence launch (a gated step and the down
         projection waiting for it, int4 weights in groups of 32 only)."""
         qg, qu, qd = (self._qweight(w, transposed=False) for w in (gate, up, down))
         if input.dtype != "f16" or not input.isContiguous or input.shape[-1] != qg.k:
