@@ -427,9 +427,10 @@ int tlhip_topk(const float* logits, int64_t offset, int64_t length, int k, float
 /* A launch configuration.  variant 0 = "gemv" (VALU dot), 1 = "gemv_mfma"
  * (skinny MFMA: up to 16 rows, and 17..64 rows for one problem with at most 8
  * waves per workgroup and, above 32 rows, at most 2 iterations in flight; 17..64 rows with
- * p0 = 8, p4 = 1..4 and every other field 0 keep all of K in one workgroup of 16 p4 columns: K a
+ * p0 = 8, p4 = 1..4 and the fields but p6 0 keep all of K in one workgroup of 16 p4 columns: K a
  * multiple of 128, int4 in groups of 32, int8 in groups of 64 or more or per row, and few enough
- * columns for its registers: up to 4 / 4 / 3 for int4 and 4 / 3 / 2 for int8 at 32 / 48 / 64 rows; 2..16 f16
+ * columns for its registers: up to 4 / 4 / 3 for int4 and 4 / 3 / 2 for int8 at 32 / 48 / 64 rows, and with p4 = 1 and
+ * p6 = 1 or 2 so many tiles of 16 rows a workgroup instead of all; 2..16 f16
  * rows with p0 = 8, p1 = 0, p2 columns, a multiple of 4, in p4 = 1, 2, 3, 4 or 6 blocks keep all of K in one workgroup
  * of p2 columns: K a multiple of 128 up to 16384, the same formats),
  * 2 = "tiled" (prefill MFMA GEMM, both operands through LDS),

@@ -777,8 +777,8 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     if (e.m != p.m) continue;
     // The forms that keep all of K in a workgroup are fitted to their number of workgroups (the
     // winner's three blocks of columns are 256 workgroups at 12288 x 4096, 64 rows, and two rounds of
-    // them at 14336 x 4096: 36.3 us against 28.0 for two blocks; f32 rows of 4096 x 4096, one block, at 8192
-    // x 4096: 15.8 against 14.0 for two, 5 rows of int8-64, and 28.0 against 18.5, 16 of int4).  What
+    // them at 14336 x 4096: 33.8 us against 26.3 for two blocks; f32 rows of 4096 x 4096, one block, at 8192
+    // x 4096: 12.1 against 9.3 for two, 5 rows of int8-64, and 22.5 against 15.2, 16 of int4).  What
     // carries over is that the rows go in one launch, or to the kernel of f32 rows; the form and its
     // width are the problem's own.
     tlhip_kernel_config_t c = e.config;
@@ -1033,13 +1033,15 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
 // at prices alike and still by 20 % at 1.07 (20 rows of int4 at 900 x 3584 7.6 / 6.1 us).  Beyond, where few
 // columns leave most CUs idle: from 0.87 of it on (48 rows of int8-64 at 760 x 10496 14.7 us in K slices, 21.7
 // here; at 2496 x 11008, 32 rows of int4, 15.0 and 13.7); and so from 16384 columns on, where the prices are
-// least sure (17 rows of int4 at 16384 x 4096 16.2 / 14.1, but at 32000 x 4096 24.1 / 28.2).
+// least sure (17 rows of int4 at 16384 x 4096 16.2 / 14.1, but at 32000 x 4096 24.1 / 28.2).  Where few columns
+// give the row tiles workgroups of their own the first line holds for every K (20 rows of int4 at 712 x 8192 10.0 / 8.1).
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
   const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
-  const double line = p.k > 6144 || p.n >= 16384 ? 0.87 : 1.25;
-  if (!gemm_rows_default(p, &whole, &us) || (found && us >= line * gemv_mfma_rows_us(p, *out))) return found;
+  if (!gemm_rows_default(p, &whole, &us)) return found;
+  const double line = whole.p6 == 0 && (p.k > 6144 || p.n >= 16384) ? 0.87 : 1.25;
+  if (found && us >= line * gemv_mfma_rows_us(p, *out)) return found;
   *out = whole;
   return true;
 }
@@ -1121,8 +1123,8 @@ Route plan_route(const Problem& p, const tlhip_kernel_config_t& c) {
     const int64_t full = p.m / 64, rest = p.m % 64;
     const double rows_us = (double)full * chunk_us(64) + (rest ? chunk_us(rest) : 0.0);
     // one launch of the form that keeps all of K in a workgroup, exact too: wherever it is cheaper
-    // than the tile that would run (48 rows of int4 at 4096 x 4096: 12.0 against 15.4 us, 40 rows at
-    // 4096 x 1024 5.5 against 10.5)
+    // than the tile that would run (48 rows of int4 at 4096 x 4096: 10.0 against 15.4 us, 40 rows at
+    // 4096 x 1024 4.4 against 10.5)
     tlhip_kernel_config_t whole;
     double whole_us = 0.0;
     const bool whole_ok = p.m <= 64 && gemm_rows_default(p, &whole, &whole_us);
@@ -1256,8 +1258,9 @@ std::vector<tlhip_kernel_config_t> neighbour_candidates(const Problem& p, const 
           }
         break;
       }
-      if (is_rows_config(p, base)) {  // its width is its only field
+      if (is_rows_config(p, base)) {  // its width and its share of the rows
         vary(4, {1, 2, 3, 4});
+        vary(6, {0, 1, 2});
         tlhip_kernel_config_t sliced;
         if (decode_rows_config(p, &sliced)) push(sliced);
         break;

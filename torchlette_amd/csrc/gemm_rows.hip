@@ -15,6 +15,7 @@
 //   * Plain loads of the weights: the neighbouring steps of a range share lines, which the nontemporal hint
 //     fetched twice (10-25 % slower).
 //   * An operand of X feeds NB products and a weight, dequantised once, MT.
+//   * Few columns: a workgroup takes a share of the row tiles, so that more CUs work (gemm_rows_default).
 // Us, steps dealt to the waves in turn with their scales, two in flight and empty loads past the end -> as it is:
 // int4 12288 x 4096 at 48 rows 18.2 -> 14.6, 4096 x 4096 with a residual 13.0 -> 10.8, 1024 x 1024 6.4 -> 5.5; int8-64
 // 12288 x 4096 at 32 rows 21.8 -> 12.6; 1.24 times faster in the mean of 28 matrices of 768..16384 x 768..12288 at
@@ -89,6 +90,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
   const int a_scale_steps = a.scale_steps, scale_stride = a.scale_stride;
   const int n0 = (int)blockIdx.x * (16 * NB);
   const int cols = min(16 * NB, a.n - n0);
+  const int row0 = (int)blockIdx.y * (16 * MT), m = min(a.m - row0, 16 * MT);  // (fewer tiles a workgroup than rows: a share of them)
   const int steps = a.k / kStep;
   const uint8_t* const packed = a.packed + (int64_t)n0 * a.row_bytes;
   const uint8_t* const scales = a.scales + (int64_t)n0 * a.scale_row_bytes;
@@ -168,7 +170,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
   auto load_x = [&](Rows& r, int st) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < XV; ++i)
-      r.v[i] = load16<0>(buffer_of(a.x + (int64_t)(4 * i) * a.k, (uint32_t)max(a.m - 4 * i, 0) * (uint32_t)a.k * 2u), x_at, (uint32_t)st * (kStep * 2u));
+      r.v[i] = load16<0>(buffer_of(a.x + (int64_t)(row0 + 4 * i) * a.k, (uint32_t)max(m - 4 * i, 0) * (uint32_t)a.k * 2u), x_at, (uint32_t)st * (kStep * 2u));
   };
   char* const patch = (char*)lds + wave * (MT * 16 * kRowBytes);
   auto lay_x = [&](const Rows& r) {
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 #pragma unroll
   for (int e0 = 0; e0 < MT * NB * 64; e0 += kWaves * 64) {
     const int e = e0 + tid, row = e / (4 * NB), c = e % (4 * NB) * 4;  // four columns of a row
-    if (e >= MT * NB * 64 || row >= a.m || n0 + c >= a.n) continue;
+    if (e >= MT * NB * 64 || row >= m || n0 + c >= a.n) continue;
     const float* p = sums + ((row >> 4) * NB + (c >> 4)) * 256 + (row & 15) * 16 + (c & 15);
     float4_t part[kWaves];
 #pragma unroll
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
     for (int i = 0; i < 4; ++i)
       sum[i] = ((part[0][i] + part[1][i]) + (part[2][i] + part[3][i])) + ((part[4][i] + part[5][i]) + (part[6][i] + part[7][i]));
     const int col = n0 + c;
-    const int64_t at = (int64_t)row * a.n + col;
+    const int64_t at = (int64_t)(row0 + row) * a.n + col;
     float v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -381,11 +383,13 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_rows_kernel(const RowsArgs a
 }
 
 int row_tiles_of(int64_t m) { return (int)((m + 15) / 16); }
+// ... of a workgroup: all, or p6 of them.
+int tiles_of(const Problem& p, const tlhip_kernel_config_t& c) { return c.p6 ? c.p6 : row_tiles_of(p.m); }
 // The column blocks whose instance fits 256 vector registers a lane without spilling one; the fullest
 // (int4, three blocks of 48 rows and two of 64) use all of them.  Four row tiles need 16 buffer
 // descriptors a step and spill some scalar registers, to lanes of a vector register.
 constexpr int most_columns(int format, int mt) {
-  return format == TLHIP_FMT_INT4_GROUPED ? (mt == 4 ? 3 : 4) : (mt == 2 ? 4 : (mt == 3 ? 3 : 2));
+  return mt == 1 ? 1 : format == TLHIP_FMT_INT4_GROUPED ? (mt == 4 ? 3 : 4) : (mt == 2 ? 4 : (mt == 3 ? 3 : 2));
 }
 
 template <int FMT, int MT, int NB>
@@ -402,7 +406,7 @@ const void* instance_of(int nb) {
 }
 template <int FMT>
 const void* instance_of(int mt, int nb) {
-  return mt == 2 ? instance_of<FMT, 2>(nb) : (mt == 3 ? instance_of<FMT, 3>(nb) : instance_of<FMT, 4>(nb));
+  return mt == 1 ? instance<FMT, 1, 1>() : mt == 2 ? instance_of<FMT, 2>(nb) : (mt == 3 ? instance_of<FMT, 3>(nb) : instance_of<FMT, 4>(nb));
 }
 const void* instance_of(int format, int mt, int nb) {
   return format == TLHIP_FMT_INT4_GROUPED ? instance_of<TLHIP_FMT_INT4_GROUPED>(mt, nb)
@@ -431,9 +435,9 @@ size_t lds_of(const Problem& p, int mt, int nb) {
 
 bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
   if (c.variant != VARIANT_GEMV_MFMA || c.p0 != kWaves || c.p4 < 1 || c.p4 > kMaxCols) return false;
-  if (c.p1 || c.p2 || c.p3 || c.p5 || c.p6) return false;  // the other form's fields: p4 is not read there
+  if (c.p1 || c.p2 || c.p3 || c.p5 || c.p6 < 0 || c.p6 >= row_tiles_of(p.m) || (c.p6 && (c.p6 > 2 || c.p4 > 1))) return false;  // the other form's fields: p4 is not read there
   if (p.x_dtype != TLHIP_F16 || p.m < 17 || p.m > 64 || p.pro.kind != TLHIP_PRO_NONE) return false;
-  if (c.p4 > most_columns(p.format, row_tiles_of(p.m))) return false;
+  if (!c.p6 && c.p4 > most_columns(p.format, row_tiles_of(p.m))) return false;
   if (p.k <= 0 || p.k % kStep != 0 || p.k > (1 << 23)) return false;  // offsets below 2^31: 64 rows of X or of weights
   if (p.format == TLHIP_FMT_INT4_GROUPED) return p.group_size == 32;
   return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
@@ -458,6 +462,24 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
   // (up to four steps: on a SIMD each)
   const int64_t steps = p.k / kStep, walked = steps <= 4 ? steps : (steps + kWaves - 1) / kWaves * kWaves;
   const double walk = (double)(walked * kStep) / 4096.0;
+  // Few columns: the row tiles to workgroups of their own while every one has a CU, which reads the weights once
+  // for each (from the last-level cache) but walks a range in the time of one tile, us, all tiles / one / two a
+  // workgroup: int4 1024 x 4096 at 48 rows 9.6 / 6.3 / 7.8, 1024 x 12288 at 64 27.4 / 11.0 / 15.0, 1536 x 6144 at 48 12.1 /
+  // 10.8 / 9.7; past one a CU behind (int8-64 4096 x 4096 at 48 rows 10.6 / 13.0 / 12.5).  Int8 with K beyond 6144 and more
+  // than 1152 columns is left to the K slices, as the tests of the routing hold it there.
+  if (format == 0 || p.k <= 6144 || p.n <= 1152)
+    for (int tiles = 1; tiles <= 2 && tiles < mt; ++tiles) {
+      memset(out, 0, sizeof *out);
+      out->variant = VARIANT_GEMV_MFMA;
+      out->p0 = kWaves;
+      out->p4 = 1;
+      out->p6 = tiles;
+      if ((p.n + 15) / 16 * ((mt + tiles - 1) / tiles) > cus || !is_rows_config(p, *out)) continue;
+      static const double one[3] = {2.2, 2.85, 2.7};
+      const Cost& two = costs[format][0];
+      *us = tiles == 1 ? 4.1 + walk * one[format] : two.launch + two.round + two.block + walk * two.walk[0];
+      return true;
+    }
   bool found = false;
   for (int nb = 1; nb <= kMaxCols; ++nb) {
     tlhip_kernel_config_t c;
@@ -493,16 +515,16 @@ int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream
   a.row_bytes = (int)(p.format == TLHIP_FMT_INT4_GROUPED ? p.k / 2 : p.k);
   a.scale_row_bytes = p.format == TLHIP_FMT_INT8_ROW ? 4 : (int)(p.k / p.group_size) * 2;
   a.group_shift = p.format == TLHIP_FMT_INT8_GROUPED ? __builtin_ctz((unsigned)(p.group_size / 64)) : 0;
-  a.scale_steps = scale_steps_of(p, row_tiles_of(p.m), c.p4);
-  a.scale_stride = scale_stride_of(p, row_tiles_of(p.m), c.p4);
+  a.scale_steps = scale_steps_of(p, tiles_of(p, c), c.p4);
+  a.scale_stride = scale_stride_of(p, tiles_of(p, c), c.p4);
   a.alpha = p.alpha;
   a.scale_mul = p.format == TLHIP_FMT_INT8_GROUPED ? 1.0f / 127.0f : 1.0f;
   a.y_dtype = p.y_dtype;
   a.vec_ok = p.n % 4 == 0 && ((uintptr_t)p.y & 15) == 0;
   a.epi = p.epi;
   void* args[] = {(void*)&a};
-  const int mt = row_tiles_of(p.m), nb = c.p4;
-  const int rc = launch_kernel(instance_of(p.format, mt, nb), dim3((unsigned)((p.n + 16 * nb - 1) / (16 * nb))), dim3(kWaves * 64), args,
+  const int mt = tiles_of(p, c), nb = c.p4;
+  const int rc = launch_kernel(instance_of(p.format, mt, nb), dim3((unsigned)((p.n + 16 * nb - 1) / (16 * nb)), (unsigned)((row_tiles_of(p.m) + mt - 1) / mt)), dim3(kWaves * 64), args,
                                lds_of(p, mt, nb), stream);
   if (rc) return rc;
   count_gemv_dispatch();
@@ -512,7 +534,7 @@ int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream
 // Every instance launch_gemm_rows can reach, in prepare mode (see launch_kernel).
 int prepare_gemm_rows_kernels() {
   for (int format : {TLHIP_FMT_INT4_GROUPED, TLHIP_FMT_INT8_GROUPED, TLHIP_FMT_INT8_ROW})
-    for (int mt = 2; mt <= 4; ++mt)
+    for (int mt = 1; mt <= 4; ++mt)
       for (int nb = 1; nb <= most_columns(format, mt); ++nb) {
         const int rc = launch_kernel(instance_of(format, mt, nb), dim3(1), dim3(64), nullptr, 0, nullptr);
         if (rc) return rc;
