@@ -208,7 +208,7 @@ __global__ __launch_bounds__(512) void gemv_one_kernel(const OneArgs<KIND> a) {
   int cc[P];
   bool in[P];
 #pragma unroll
-  for (int j = 0; j < P; ++j) {  // past the row's end: its last chunk again, scaled by zero
+  for (int j = 0; j < P; ++j) {  // past the row's end: its last chunk again, not added
     const int c = (kwi * P + j) * lpr + lj;
     in[j] = c < nchunks;
     cc[j] = min(c, nchunks - 1);
@@ -345,7 +345,8 @@ __global__ __launch_bounds__(512) void gemv_one_kernel(const OneArgs<KIND> a) {
 #pragma unroll
       for (int j = 0; j < P; ++j) {
         const float d = Dot::of(b.w[i][j], x[j]);
-        if constexpr (GROUPED) acc[i] = fmaf(in[j] ? half_bits_to_float(b.s[i][j]) : 0.f, d, acc[i]);
+        // (a select, not a scale of zero: the last chunk's sum may be infinite)
+        if constexpr (GROUPED) acc[i] = in[j] ? fmaf(half_bits_to_float(b.s[i][j]), d, acc[i]) : acc[i];
         else acc[i] += in[j] ? d : 0.f;
         if constexpr (sizeof(XT) == 4) __builtin_amdgcn_sched_barrier(0);  // one chunk's 32 floats at a time
       }
