@@ -205,13 +205,14 @@ __global__ __launch_bounds__(512) void gemv_one_kernel(const OneArgs<KIND> a) {
   const int sub = lane >> lpr_shift, lj = lane & (lpr - 1);
   const int kwi = wave & (kw - 1);
   const int row_in_wg = (wave >> kw_shift) * (64 >> lpr_shift) + sub;
-  int cc[P];
+  int cc[P], xc[P];
   bool in[P];
 #pragma unroll
-  for (int j = 0; j < P; ++j) {  // past the row's end: its last chunk again, not added
+  for (int j = 0; j < P; ++j) {  // past the row's end: its last chunk again, times activations of zero (and a scale of zero)
     const int c = (kwi * P + j) * lpr + lj;
     in[j] = c < nchunks;
     cc[j] = min(c, nchunks - 1);
+    xc[j] = min(c, nchunks);
   }
   struct Batch {
     u32x4 w[NA][P];
@@ -240,9 +241,11 @@ __global__ __launch_bounds__(512) void gemv_one_kernel(const OneArgs<KIND> a) {
   load_batch(cur, rb);
 
   // ---- staging: unit q of chunk c at q * stride + c, so that lanes on consecutive chunks read
-  // consecutive units (one unit of padding: a thread's neighbours write to other banks).  A thread past
-  // the last unit writes it again, the same value.
+  // consecutive units (a thread's neighbours write to other banks).  A thread past the last unit writes it
+  // again, the same value.  Behind the last chunk one of zeros for the lanes past the row's end: a scale of zero alone
+  // leaves NaN where the last chunk's sum is infinite, and a select behind every sum is up to 10 % of a launch.
   const uint32_t stride = (uint32_t)nchunks + 1;
+  if (tid < NQ) lds[tid * stride + (uint32_t)nchunks] = (u32x4){0u, 0u, 0u, 0u};
   auto place = [&](int u) {
     const uint32_t c = (uint32_t)u / NQ, q = (uint32_t)u % NQ;
     return lds + q * stride + c;
@@ -334,7 +337,7 @@ __global__ __launch_bounds__(512) void gemv_one_kernel(const OneArgs<KIND> a) {
 #pragma unroll
   for (int j = 0; j < P; ++j)
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) x[j][q] = lds[q * stride + (uint32_t)cc[j]];
+    for (int q = 0; q < NQ; ++q) x[j][q] = lds[q * stride + (uint32_t)xc[j]];
   float* const partial = (float*)(lds + stride * NQ);  // [kw][row][NA]
 
   auto consume = [&](const Batch& b, int rb) {
@@ -345,9 +348,8 @@ __global__ __launch_bounds__(512) void gemv_one_kernel(const OneArgs<KIND> a) {
 #pragma unroll
       for (int j = 0; j < P; ++j) {
         const float d = Dot::of(b.w[i][j], x[j]);
-        // (a select, not a scale of zero: the last chunk's sum may be infinite)
-        if constexpr (GROUPED) acc[i] = in[j] ? fmaf(half_bits_to_float(b.s[i][j]), d, acc[i]) : acc[i];
-        else acc[i] += in[j] ? d : 0.f;
+        if constexpr (GROUPED) acc[i] = fmaf(in[j] ? half_bits_to_float(b.s[i][j]) : 0.f, d, acc[i]);
+        else acc[i] += d;
         if constexpr (sizeof(XT) == 4) __builtin_amdgcn_sched_barrier(0);  // one chunk's 32 floats at a time
       }
       acc[i] = lanes_sum(acc[i], lpr_shift);
