@@ -15,10 +15,10 @@ int chunk_weights(int format) { return format == TLHIP_FMT_INT4_GROUPED ? 32 : 1
 int x_units(const Problem& p) { return chunk_weights(p.format) * (p.x_dtype == TLHIP_F16 ? 2 : 4) / 16; }  // of a chunk
 int64_t chunks_of(const Problem& p) { return p.k / chunk_weights(p.format); }
 
-// Chunks a lane holds, as built: five run as six.
+// Chunks a lane holds (seven: more than any instance is built for).
 int positions(const Problem& p, const tlhip_kernel_config_t& c) {
   const int64_t lanes = (int64_t)c.p0 * c.p3, n = (chunks_of(p) + lanes - 1) / lanes;
-  return n > 6 ? 7 : (n == 5 ? 6 : (int)n);
+  return (int)std::min<int64_t>(n, 7);
 }
 // Units of activations a thread stages: one, two, or four at a time.
 int units(const Problem& p, const tlhip_kernel_config_t& c) {
@@ -191,11 +191,11 @@ bool gemv_one_group_config(const Problem* ps, int count, const tlhip_kernel_conf
 // them past the row's end and give the chip 1024 waves, but not many more; a wave less in the row
 // where a workgroup pays for a prologue, or the lanes can be few because a group has many rows.
 // Against the best of 60 geometries at 19 matrices of 1024..151936 x 1024..12288, five pairs of format
-// and type: 1.8 % behind it in the mean.  What it does not take is left to gemv_kernel.h, which stays
-// ahead on long f32 rows (11.0 against 11.1 us at 4096 x 12288 int8-64, 9.2 against 9.7 for int4); behind
-// it elsewhere, us: one f16 row of int4 1024 x 1024 2.72 -> 2.26, 9216 x
-// 2304 6.5 -> 5.1, 12288 x 4096 7.8 -> 7.2, 151936 x 2048 39.3 -> 30.0; int8-64 1024 x 3072 3.7 -> 2.9,
-// 12288 x 4096 10.4 -> 10.0, 4096 x 12288 10.7 -> 10.1.  The rows of a long matrix (an LM head) go to
+// and type: 1.8 % behind it in the mean.  What it does not take, and long rows of many (one_row_config in dispatch.cpp), are
+// left to gemv_kernel.h; us, that kernel -> here, cold weights, one f16 row of int4 1024 x 1024 2.8 -> 2.3, 12288 x 4096 7.8 -> 7.2,
+// 65536 x 2048 22.0 -> 16.3; int8-64 1024 x 3072 3.7 -> 2.9, 12288 x 4096 11.2 -> 10.7, level at 4096 x 12288 (10.8-11.0); per
+// row 2048 x 5120 4.9 -> 3.9; one f32 row of int8-64 1024 x 9728 7.4 -> 5.1.  Five chunks have an instance of their own: run
+// as six they took 8 % more at 5120 and 9728 of int8 (2048 x 5120 4.4 us).  The rows of a long matrix (an LM head) go to
 // fewer lanes: 256000 x 2304 per row 95 us on 64 lanes, 88 on 32.
 bool gemv_one_default(const Problem& p, int64_t rows, int kind, tlhip_kernel_config_t* out) {
   if (p.m != 1) return false;
@@ -238,7 +238,7 @@ int prepare_gemv_one_kernels() {
     for (p.x_dtype = 0; p.x_dtype < 2; ++p.x_dtype)
       for (int kind : {ONE_SINGLE, ONE_GROUP, ONE_PAIR})
         for (int pro : {TLHIP_PRO_NONE, TLHIP_PRO_RMSNORM, TLHIP_PRO_GATED_MUL})
-          for (int pos : {1, 2, 3, 4, 6})
+          for (int pos = 1; pos <= 6; ++pos)
             for (int units : {1, 2, 4})
               if (const void* fn = instance(p, pos, units, pro, kind)) {
                 const int rc = launch_kernel(fn, dim3(1), dim3(64), nullptr, 0, nullptr);

@@ -423,8 +423,10 @@ const void* one_instance_p(int p) {
   if (p == 3) return (const void*)gemv_one_kernel<FMT, XT, 3, XS, PRO, KIND>;
   if constexpr (NQ <= 4) {
     if (p == 4) return (const void*)gemv_one_kernel<FMT, XT, 4, XS, PRO, KIND>;
-    if constexpr (KIND != ONE_PAIR)  // (two weights' batches as well: spills)
-      if (p <= 6 && p > 4) return (const void*)gemv_one_kernel<FMT, XT, 6, XS, PRO, KIND>;
+    if constexpr (KIND != ONE_PAIR) {  // (two weights' batches as well: spills)
+      if (p == 5) return (const void*)gemv_one_kernel<FMT, XT, 5, XS, PRO, KIND>;
+      if (p == 6) return (const void*)gemv_one_kernel<FMT, XT, 6, XS, PRO, KIND>;
+    }
   }
   return nullptr;
 }
