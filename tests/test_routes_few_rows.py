@@ -1,0 +1,62 @@
+"""Which kernel a few rows take with nothing tuned: the one that measured faster (cold weights, us)."""
+import ctypes
+import os
+
+import pytest
+
+import torchlette_amd as T
+from torchlette_amd import _lib as L
+
+INT4, INT8, ROW = (L.FMT_INT4_GROUPED, 32), (L.FMT_INT8_GROUPED, 64), (L.FMT_INT8_ROW, 0)
+
+
+def chosen(fmt, n, k, m, x, cache=None):
+    lib = L.load()
+    before = T.exportTuningCache()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    w, c = L.QWeight(*fmt, n, k, ptr, ptr), L.KernelConfig()
+    try:
+        T.clearTuningCache()
+        if cache is not None:
+            T.importTuningCache(cache)
+        assert lib.tlhip_selected_config(ctypes.byref(w), x, m, x, ctypes.byref(c)) == 0
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(before)
+    return c.as_tuple()
+
+
+def whole(c):  # all of K in a workgroup
+    return c[0] == L.VARIANT_GEMV_MFMA and c[2] == 0 and c[5] > 0
+
+
+@pytest.mark.parametrize("fmt,n,k,m,all_of_k", [
+    # K slices or the VALU kernel / all of K in a workgroup
+    (INT4, 4096, 12288, 16, False),   # 12.0 / 13.5
+    (INT8, 2048, 12288, 16, False),   # 10.1 / 13.0
+    (ROW, 2048, 12288, 16, False),    # 10.1 / 12.9
+    (INT8, 4096, 12288, 16, False),   # 14.2 / 16.9
+    (INT4, 24576, 4096, 8, False),    # 16.1 / 18.9
+    (INT4, 768, 16384, 16, False),    # 9.8 / 12.1
+    (INT4, 1024, 4096, 2, False),     # 3.7 / 4.2
+    (INT4, 24576, 4096, 3, False),    # 15.1 / 17.4
+    (ROW, 14336, 3072, 2, False),     # 9.9 / 11.2
+    (INT4, 4096, 4096, 16, True),     # 6.7 / 6.6, with a residual 7.6 / 6.5
+    (INT4, 1024, 4096, 8, True),      # 6.1 / 4.5
+    (INT8, 4096, 4096, 8, True),      # 7.3 / 6.3
+    (INT8, 1024, 12288, 8, True),     # 11.0 / 8.1
+    (INT8, 12288, 4096, 2, True),     # 13.0 / 11.7
+])
+def test_up_to_sixteen_f16_rows(fmt, n, k, m, all_of_k):
+    assert whole(chosen(fmt, n, k, m, L.F16)) == all_of_k
+
+
+@pytest.mark.parametrize("n,k,all_of_k", [(4096, 12288, False), (4096, 8192, True), (2048, 12288, False)])
+def test_a_neighbours_k_slices_are_weighed_at_a_problems_own_prices(n, k, all_of_k):
+    """Sixteen rows of int4 beside the shipped winners."""
+    cache = open(os.path.join(os.path.dirname(T.__file__), "tuning", "mi355x.json")).read()
+    c = chosen(INT4, n, k, 16, L.F16, cache)
+    assert whole(c) == all_of_k, c
+    if (n, k) == (2048, 12288):  # those of the winner at 4096 x 12288: 12.0, its own 9.4
+        assert c == chosen(INT4, n, k, 16, L.F16)

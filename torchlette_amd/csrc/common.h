@@ -91,6 +91,12 @@ struct Problem {
 int make_problem(const tlhip_qweight_t* w, const void* x, int x_dtype, int64_t m, void* y,
                  int y_dtype, float alpha, const tlhip_epilogue_t* epilogue, Problem* p,
                  const char* who);
+// Whether p's epilogue has an input of p's rows: what it costs differs between the kernels.
+inline bool has_residual(const Problem& p) {
+  for (int i = 0; i < p.epi.n_ops; ++i)
+    if (p.epi.kind[i] == TLHIP_EPI_BINARY) return true;
+  return false;
+}
 int validate_weight(const tlhip_qweight_t* w, const char* who);
 
 // Launchers (each returns a TLHIP_* code; launch errors are reported).
@@ -130,7 +136,8 @@ ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c);
 bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c);
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us);
 int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
-// Time of a launch of the decode kernel at 17..64 rows, in microseconds (gemv_mfma.hip); c applicable.
+// Time of a launch of the decode kernel at up to 16 and at 17..64 rows, in microseconds (gemv_mfma.hip); c applicable.
+double gemv_mfma_us(const Problem& p, const tlhip_kernel_config_t& c);
 double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c);
 // elementwise.hip: the steps of `ep` over a finished [M,N] output, in place, 8 columns a lane
 bool epilogue_tail_applicable(const void* y, int64_t n);

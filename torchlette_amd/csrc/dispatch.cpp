@@ -211,6 +211,7 @@ bool config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const c
 }
 
 tlhip_kernel_config_t default_valu_config(const Problem& p);
+tlhip_kernel_config_t default_below_few(const Problem& p);
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out);
 
 // The numbers the default routing was fitted with on MI355X: measurements, not structure.
@@ -465,21 +466,37 @@ bool f32_rows_on_matrix_cores(const Problem& p) {
   return weights >= 8000000;
 }
 
-// 2..16 f16 rows with all of K in a workgroup (gemv_few.hip), wherever it takes them (K a multiple of 128 up to
-// 16384) but for a long matrix (an LM head), which the kernels below stream at the rate of memory, and two
-// rows of a wide short one, on the VALU kernel: 4.4 against 4.6 us at 8476 x 1024 int4.  Us, the kernels below ->
-// here, in the mean of 27 matrices of 1024..18432 x 1024..12288 and four formats 1.37 times faster: 1.2 at
-// two rows, 1.28-1.37 at three, 1.40-1.49 at eight and sixteen; 16 rows of int4 at 1024 x 1024 5.9 -> 3.3,
-// 4096 x 4096 8.0 -> 5.6, 4096 x 12288 14.3 -> 11.5, 12288 x 4096 10.4 -> 9.5; of int8-64 2304 x 9216 14.6 -> 10.3.
-bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
+// 2..16 f16 rows with all of K in a workgroup (gemv_few.hip), where it takes them (K a multiple of 128 up to 16384):
+// not a long matrix (an LM head), which the kernels below stream at the rate of memory, nor two rows of a wide
+// short one, on the VALU kernel (4.4 against 4.6 us at 8476 x 1024 int4).
+bool few_rows_possible(const Problem& p, tlhip_kernel_config_t* out) {
   double us = 0.0;
-  if (p.n >= 32768 || (p.m == 2 && p.n >= 8 * p.k)) return false;
-  // few columns of a long K: K slices across workgroups are ahead or level (16 rows of int4 at 1024 x 12288
-  // 8.8 against 9.5 us, eight at 528 x 12288 7.8 and 7.8, 16 at 2048 x 12288 9.8 against 9.1; int8 per row at 1024
-  // x 12288 8.3 against 9.1; but eight rows of int8-64 there 8.7 against 7.3)
-  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
-  if (p.k >= 12288 && (int4 ? p.m >= 8 && p.n <= 2048 : p.m > 8 && p.n <= 1024)) return false;
-  return gemv_few_default(&p, 1, FEW_SINGLE, out, &us);
+  return p.n < 32768 && !(p.m == 2 && p.n >= 8 * p.k) && gemv_few_default(&p, 1, FEW_SINGLE, out, &us);
+}
+
+// ... and where it is ahead of what would run without it: over 8554 problems of 768..28672 x 1024..16384 (2..16 rows, three
+// formats, with and without a residual, cold weights) 1.15-1.21 times faster than that in the mean and more than 3 % behind
+// it at 2-3 %, where it is at 5-11 %, by up to 39 %, if it is taken wherever it is possible.  Us, without / here:
+//   beside the skinny kernel the cheaper price, up to K = 14336 (16 rows of int4 at 4096 x 4096 with a residual 7.6 / 6.5,
+//   but plain at 4096 x 12288 12.0 / 13.5; of int8-64 at 2048 x 12288 10.1 / 13.0); longer, where the launches are 10 % above
+//   the price, all but 9 to 16 rows of few columns (16 of int4 at 768 x 16384 9.8 / 12.1, at 6144 x 16384 17.8 / 21.9);
+//   beside the VALU kernel all but two rows of int4 with up to 1024 columns and K from 3072 to 12288 (1024 x 4096 3.7 / 4.2),
+//   and three or four rows of int4 on the 4 x 4 x 4 form with 14336 columns or more (24576 x 4096, three 15.1 / 17.4; four
+//   15.8 / 17.3, with a residual 18.0 / 17.1) or, three of them without a residual, 5120 to 8192 columns of K from 5120 (8192 x
+//   8192 11.4 / 12.0).
+bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
+  if (!few_rows_possible(p, out)) return false;
+  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED, plain = !has_residual(p);
+  const tlhip_kernel_config_t below = default_below_few(p);
+  if (below.variant == VARIANT_GEMV) {
+    if (p.m == 2) return !(int4 && p.n <= 1024 && p.k >= 3072 && p.k < 12288);
+    const bool wide = p.n >= 14336, level = p.n >= 5120 && p.n <= 8192 && p.k >= 5120;
+    return !(p.m == 3 ? (wide && p.k >= 2048) || (level && plain) : wide && plain && p.k >= 4096);
+  }
+  if (below.variant != VARIANT_GEMV_MFMA) return true;
+  if (p.m == 2) return false;
+  if (p.k > 14336) return !(p.m > 8 && (p.n <= 1024 || (plain && p.n <= (int4 ? 6144 : 2048))));
+  return gemv_few_us(p, *out) <= gemv_mfma_us(p, below);
 }
 
 // 2 to 5 f32 rows on the VALU in one launch (gemv_some.hip): where they do not go to the matrix cores, and
@@ -499,6 +516,19 @@ bool few_f32_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
 tlhip_kernel_config_t default_config(const Problem& p) {
   tlhip_kernel_config_t few;
   if (few_rows_config(p, &few) || few_f32_rows_config(p, &few)) return few;
+  return default_below_few(p);
+}
+
+// ... without the kernels for a few rows in one launch of all of K.
+tlhip_kernel_config_t default_below_few(const Problem& p) {
+  // two rows of int8 per row on a wide matrix: the skinny kernel, two waves to a row block (14336 x 3072 9.9 us against 12.0 on
+  // the VALU kernel and 11.2 with all of K in a workgroup, 16384 x 6144 20.5 / 21.0 / 22.9)
+  if (p.m == 2 && p.x_dtype == TLHIP_F16 && p.pro.kind == TLHIP_PRO_NONE && p.format == TLHIP_FMT_INT8_ROW && p.n >= 12288 && p.n < 32768 &&
+      p.k >= 2048 && p.k <= 6144) {
+    tlhip_kernel_config_t c = mfma_cfg(8, 4, 2, 1);
+    c.p5 = 1;
+    if (gemv_mfma_config_applicable(p, c, nullptr)) return c;
+  }
   if (p.m > 16 && p.x_dtype == TLHIP_F16) {
     // the eight-wave kernel wherever it takes the problem (K a multiple of 64, groups of 32 or
     // 64 times a power of two): ahead of the kernels below at every one of 196 problems from 64
@@ -787,7 +817,19 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     there.k = e.k;
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
-    if (is_few_config(there, c, FEW_SINGLE) && !few_rows_config(p, &c)) continue;
+    // (where a neighbour of 2..16 rows is on the matrix cores, the problem's own prices tell which of their two forms it has, and
+    // whether the neighbour's K slices are cheaper than its own: 16 rows of int4 at 2048 x 12288 12.0 us in those of the winner at
+    // 4096 x 12288, 9.4 in its own)
+    tlhip_kernel_config_t few;
+    const bool whole_there = is_few_config(there, c, FEW_SINGLE);
+    if ((whole_there || (c.variant == VARIANT_GEMV_MFMA && p.m <= 16)) && few_rows_config(p, &few)) {
+      c = few;
+    } else if (whole_there) {
+      continue;
+    } else if (c.variant == VARIANT_GEMV_MFMA && p.m > 1 && p.m <= 16 && p.n < 32768) {
+      const tlhip_kernel_config_t own = default_below_few(p);
+      if (own.variant == VARIANT_GEMV_MFMA && config_applicable(p, c, nullptr) && gemv_mfma_us(p, own) < gemv_mfma_us(p, c)) c = own;
+    }
     // (one row: the lanes that share it follow from K and the number of columns)
     if (c.variant == VARIANT_GEMV) (void)gemv_one_default(p, p.n, ONE_SINGLE, &c);
     if (is_some_config(c) && !gemv_some_default(p, &c)) continue;
@@ -835,14 +877,14 @@ tlhip_kernel_config_t choose_config(const Problem& p) {
   return default_config(p);
 }
 
-// ... and what a thread chose last for such sizes and types (the choice depends on nothing else of a problem
-// with the library's own workspace), while neither the tuning cache nor the model has changed since: the two
+// ... and what a thread chose last for such sizes and types, with or without a residual (the choice depends on
+// nothing else of a problem with the library's own workspace), while neither the tuning cache nor the model has changed since: the two
 // text keys, their lookups and the prices took 1.5 us of a call (one
 // row of int8-64 at 1024 x 3072, call after call: 4.7 -> 4.1 us, the launch itself the rest).
 tlhip_kernel_config_t select_config(const Problem& p) {
   struct Key {
     int64_t n, k, m;
-    int format, group_size, x_dtype, y_dtype, prologue, cus;
+    int format, group_size, x_dtype, y_dtype, prologue, residual, cus;
   };
   struct Entry {
     Key key;
@@ -862,8 +904,9 @@ tlhip_kernel_config_t select_config(const Problem& p) {
   key.x_dtype = p.x_dtype;
   key.y_dtype = p.y_dtype;
   key.prologue = p.pro.kind;
+  key.residual = has_residual(p);
   key.cus = device_cu_count();
-  const uint64_t mixed = ((uint64_t)p.n * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)p.k * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)(p.m * 8 + p.format * 2 + p.y_dtype) * 0x165667b19e3779f9ull);
+  const uint64_t mixed = ((uint64_t)p.n * 0x9e3779b97f4a7c15ull) ^ ((uint64_t)p.k * 0xc2b2ae3d27d4eb4full) ^ ((uint64_t)(p.m * 16 + p.format * 4 + p.y_dtype * 2 + key.residual) * 0x165667b19e3779f9ull);
   Entry& e = entries[(mixed >> 40) % kEntries];
   const uint64_t now = g_tune_generation.load(std::memory_order_acquire);
   if (e.generation == now && !memcmp(&e.key, &key, sizeof key)) return e.config;
@@ -1753,6 +1796,11 @@ int tlhip_gemv_grouped_rows(const tlhip_gemv_problem_t* problems, int count, int
         if (c.variant == VARIANT_GEMV_XREG && gemv_xreg_group_applicable(ps, count, c, nullptr))
           return launch_gemv_xreg_group(ps, count, c, s);
       }
+      // ... and where that is a kernel without one too (three rows of int4 on the 4x4x4 form), all of K in a workgroup
+      tlhip_kernel_config_t few;
+      double us = 0.0;
+      if (few_rows_possible(all, &few) && gemv_few_default(ps, count, FEW_GROUP, &few, &us) && gemv_mfma_group_applicable(ps, count, few, nullptr))
+        return launch_gemv_mfma_group(ps, count, few, s);
     }
   }
   for (int i = 0; i < count; ++i) {

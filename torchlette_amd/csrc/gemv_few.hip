@@ -92,10 +92,11 @@ bool is_few_config(const Problem& p, const tlhip_kernel_config_t& c, int kind) {
   return instance(p, x_loads(p), c.p4, kind) && lds_of(p, c.p4) <= kLds;
 }
 
-// Time of a launch in microseconds: per round of workgroups a constant, a little more for more rows, and per
-// 1000 of K the step, the rows and the width of the blocks.  Fitted at 27 matrices of 1024..18432 x
-// 1024..12288, 2..16 rows, four formats (3600 launches, 3.6-7.1 % rms each); the geometry it picks is 0.8 %
-// behind the best one in the mean.
+// What orders the geometries of a problem: per round of workgroups a constant, a little more for more rows, and
+// per 1000 of K the step, the rows and the width of the blocks.  Fitted at 27 matrices of 1024..18432 x
+// 1024..12288, 2..16 rows, four formats (3600 launches, 3.6-7.1 % rms each, warm); the geometry it picks is 0.6-1.2 %
+// behind the best one in the mean of 1700 problems (18084 launches on cold weights, where it is 15 % too low: what a
+// launch takes beside another kernel's is gemv_few_us).
 static double few_us(const Problem* ps, int count, int kind, const tlhip_kernel_config_t& c) {
   const Problem& p = ps[0];
   struct Cost {
@@ -111,6 +112,29 @@ static double few_us(const Problem* ps, int count, int kind, const tlhip_kernel_
   for (int i = 0; i < count; ++i) wgs += (ps[i].n + c.p2 - 1) / c.p2;
   const double rows = 0.25 * x_loads(p), width = (double)c.p2 * (kind == FEW_PAIR ? 2 : 1) / (16.0 * c.p4);
   return t.launch + (double)((wgs + cus - 1) / cus) * (t.round + t.rows * rows + (double)p.k / 1000.0 * (t.k + t.k_rows * rows + t.k_width * width));
+}
+
+// Beside other kernels, behind each other and on cold weights: the weights' way from memory, the activations' into every
+// workgroup (16 rows of K = 12288 are 100 MB at 256 workgroups, four times the int4 weights of 4096 columns), and per
+// round the blocks' sums and, per 1000 of K, the blocks, the rows and the columns.
+// A residual costs next to nothing: it is loaded ahead of the sums.  Fitted at 7919 launches of the geometries it
+// is asked for (17 x 13 matrices of 768..28672 x 1024..14336, 2..16 rows, with and without a residual): 4.3-4.6 % rms.
+double gemv_few_us(const Problem& p, const tlhip_kernel_config_t& c) {
+  struct Cost {
+    double launch, mb, x, sums, sums_rows, k_blocks, k_rows, k_both, k_cols, residual, residual_out;
+  };
+  static const Cost costs[3] = {{2.583, 0.0801, 0.0382, 0.226, 0.104, 0.273, 0.106, 0.030, 0.049, 0.067, 0.034},   // int4
+                                {2.602, 0.0564, 0.0592, 0.224, 0.071, 0.126, 0.173, 0.0, 0.306, 0.118, 0.001},    // int8 in groups
+                                {2.628, 0.0633, 0.0526, 0.232, 0.065, 0.125, 0.187, 0.0, 0.261, 0.045, 0.015}};   // int8 per row
+  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
+  const Cost& t = costs[int4 ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)];
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int64_t wgs = (p.n + c.p2 - 1) / c.p2;
+  const double rounds = (double)((wgs + cus - 1) / cus), rows = 0.25 * x_loads(p), nb = c.p4, k = (double)p.k / 1000.0;
+  const double mb = (double)p.n * (double)p.k * (int4 ? 0.5 : 1.0) / 1e6;
+  return t.launch + t.mb * mb + t.x * (double)(wgs * p.m) * (double)p.k / 1e6 +
+         rounds * (nb * (t.sums + t.sums_rows * rows) + k * (t.k_blocks * nb + t.k_rows * rows + t.k_both * rows * nb + t.k_cols * c.p2 / 16.0)) +
+         (has_residual(p) ? t.residual + t.residual_out * (double)p.m * (double)p.n / 1e5 : 0.0);
 }
 
 // Full blocks, or the columns dealt evenly over one to six rounds of workgroups (several problems: the

@@ -152,6 +152,34 @@ double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
          (ks > 1 ? t.sliced + t.plane * (double)ks * (double)wgblocks / (double)sets : 0.0);
 }
 
+// Up to 16 rows, beside all of K in a workgroup (gemv_few_us), the same way: the weights' way from memory, an iteration
+// of a wave, in whole sets of those in flight (more where none is behind it), in its round and the workgroups that
+// share its CU, what a workgroup stages of the activations, and with K slices the arrival of the last one and the
+// planes it adds.  A residual is read behind the sums.  Fitted at 6527 launches of the geometries of default_below_few:
+// 6.6-7.7 % rms, 4.2-5.0 % where the two are within a quarter of each other.
+double gemv_mfma_us(const Problem& p, const tlhip_kernel_config_t& c) {
+  struct Cost {
+    double launch, sliced, mb, iteration, alone, pair, round, plane, staged, residual, residual_out;
+  };
+  static const Cost costs[3] = {{3.254, 1.056, 0.0495, 0.371, 0.171, 0.0, 0.082, 0.119, 27.2, 0.861, 0.157},     // int4
+                                {2.934, 1.219, 0.0921, 0.144, 0.333, 0.075, 0.255, 0.066, 29.5, 0.862, 0.051},   // int8 in groups
+                                {3.180, 1.327, 0.1025, 0.104, 0.164, 0.033, 0.084, 0.064, 30.8, 0.661, 0.307}};  // int8 per row
+  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
+  const Cost& t = costs[int4 ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)];
+  const int kper = int4 ? 128 : 64, kw = c.p2 == 0 ? c.p0 : c.p2, ks = c.p3 < 1 ? 1 : c.p3, per_wg = c.p0 / kw;
+  const int64_t wgblocks = ((p.n + 15) / 16 + per_wg - 1) / per_wg, slice = (p.k / kper + ks - 1) / ks;
+  MfmaGeometry geo;
+  if (!mfma_geometry((p.n + 15) / 16, slice * kper, p.m, c.p0, kw, ks, line_patch_bytes(c), &geo)) return 1e9;
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int64_t sets = geo.grid / ks, rounds = (wgblocks + sets - 1) / sets, shared = (geo.grid + cus - 1) / cus;
+  const int64_t own = (slice + kw - 1) / kw, in_flight = c.p1 < 1 ? 1 : c.p1;
+  const double walk = (double)(rounds * shared * ((own + in_flight - 1) / in_flight * in_flight));
+  return t.launch + t.mb * (double)p.n * (double)p.k * (int4 ? 0.5 : 1.0) / 1e6 +
+         walk * (t.iteration + (in_flight == 1 ? t.alone : (in_flight == 2 ? t.pair : 0.0))) + t.round * (double)(rounds * shared) +
+         t.staged * (double)(shared * p.m * slice * kper) / 1e6 + (ks > 1 ? t.sliced + t.plane * (double)ks * (double)wgblocks / (double)sets : 0.0) +
+         (has_residual(p) ? t.residual + t.residual_out * (double)p.m * (double)p.n / 1e5 : 0.0);
+}
+
 // The problems of a group: same activations and rows, one shape class; N, pointers and
 // epilogues per problem.  The configuration is checked against the group's total rows.
 bool gemv_mfma_group_applicable(const Problem* ps, int count, const tlhip_kernel_config_t& c, const char** why) {

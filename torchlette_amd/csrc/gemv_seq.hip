@@ -198,11 +198,28 @@ static int mlp_one_launch(const tlhip_qweight_t* gate, const tlhip_qweight_t* up
   return tlhip_gemv_sequence(steps, 2, x_dtype, m, 1.0f, stream);
 }
 
-// One call for the block, whichever way is faster.  Measured on MI355X at 1..16 rows the
-// three launches the model issues (gate and up grouped on the shared activations, the gated
-// multiply, down) take 23-33 us at 4096 -> 12288 -> 4096 and the sequence launch 42-50 us,
-// so the three launches are what runs; TLHIP_MLP_ONE_LAUNCH=1 selects the sequence launch.
-// Between its launches the gate and up outputs live in 2 MiB of the stream's workspace.
+// Gate, up and their product of 2..16 rows in one launch: not three and more rows of int8 per row above the line from
+// which the kernels below stream a long matrix (32768 x 1024, six rows 31.5 us the block in three launches, 35.7 so),
+// nor int8 where one launch of both and the gated multiply (2.6 us) are cheaper by the prices, which hold up to that line
+// (12 and 16 rows of int8-64 at 14336 x 2048 30.1 and 29.7 / 31.2 and 33.6).
+static bool pair_of_few_rows(const Problem& gate) {
+  if (gate.format == TLHIP_FMT_INT4_GROUPED) return true;
+  if (gate.n >= 32768) return gate.format != TLHIP_FMT_INT8_ROW || gate.m == 2;
+  if (gate.n >= 16384) return true;
+  Problem both = gate;
+  both.n = 2 * gate.n;
+  const tlhip_kernel_config_t c = select_gemv_config(both);
+  if (c.variant != VARIANT_GEMV_MFMA || is_few_config(both, c, FEW_SINGLE)) return true;
+  tlhip_kernel_config_t few;
+  double us = 0.0;
+  return !gemv_few_default(&both, 1, FEW_SINGLE, &few, &us) || gemv_few_us(both, few) <= gemv_mfma_us(both, c) + 2.6;
+}
+
+// One call for the block, whichever way is faster: gate, up and their product in one launch and down behind it
+// where a kernel takes the pair, else the three launches the model issues (gate and up grouped on the shared
+// activations, the gated multiply, down).  Measured on MI355X at 4096 -> 12288 -> 4096 of int4: 20.3-32.3 us at 1..16 rows
+// the former, 28.2-34.3 us the latter (cold weights), and 42-50 us the sequence launch, which TLHIP_MLP_ONE_LAUNCH=1 selects.
+// Between the three launches the gate and up outputs live in 2 MiB of the stream's workspace.
 int tlhip_mlp_decode(const tlhip_qweight_t* gate, const tlhip_qweight_t* up, const tlhip_qweight_t* down, int unary,
                      const void* x, int x_dtype, int64_t m, void* h, void* y, int y_dtype,
                      const tlhip_epilogue_t* down_epilogue, tlhip_stream_t stream) {
@@ -237,7 +254,7 @@ int tlhip_mlp_decode(const tlhip_qweight_t* gate, const tlhip_qweight_t* up, con
     tlhip_kernel_config_t c;
     double us = 0.0;
     const bool one_row = m == 1 && gemv_one_default(ps[0], gate->n, ONE_PAIR, &c) && gemv_pair_applicable(ps[0], ps[1], c);
-    if (one_row || (m > 1 && gemv_few_default(ps, 1, FEW_PAIR, &c, &us))) {
+    if (one_row || (m > 1 && pair_of_few_rows(ps[0]) && gemv_few_default(ps, 1, FEW_PAIR, &c, &us))) {
       rc = one_row ? launch_gemv_pair(ps[0], ps[1], unary, c, resolve_stream(stream))
                    : launch_gemv_few(ps, 2, FEW_PAIR, unary, c, resolve_stream(stream));
       return rc ? rc : tlhip_gemv(down, h, TLHIP_F16, m, y, y_dtype, 1.0f, down_epilogue, stream);
