@@ -60,3 +60,19 @@ def test_a_neighbours_k_slices_are_weighed_at_a_problems_own_prices(n, k, all_of
     assert whole(c) == all_of_k, c
     if (n, k) == (2048, 12288):  # those of the winner at 4096 x 12288: 12.0, its own 9.4
         assert c == chosen(INT4, n, k, 16, L.F16)
+
+
+@pytest.mark.parametrize("fmt,n,k,x,own_kernel", [
+    # the VALU kernel / the kernel for one row
+    (INT4, 16384, 14336, L.F16, False),   # 28.2 / 32.7
+    (INT4, 6144, 14336, L.F16, True),     # 14.9 / 14.1
+    (INT4, 12288, 9728, L.F32, False),    # 19.7 / 24.1
+    (INT4, 4096, 9728, L.F32, True),      # 9.6 / 9.8
+    (INT8, 16384, 7168, L.F32, False),    # 22.6 / 25.5
+    (INT8, 8192, 8192, L.F32, True),      # 15.2 / 14.9
+    (ROW, 12288, 7168, L.F16, True),      # 17.0 / 16.6
+    (INT4, 12288, 4096, L.F16, True),
+])
+def test_one_row(fmt, n, k, x, own_kernel):
+    c = chosen(fmt, n, k, 1, x)
+    assert c[0] == L.VARIANT_GEMV and (c[6] == 3) == own_kernel, c

@@ -212,6 +212,8 @@ bool config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const c
 
 tlhip_kernel_config_t default_valu_config(const Problem& p);
 tlhip_kernel_config_t default_below_few(const Problem& p);
+bool one_row_config(const Problem& p, tlhip_kernel_config_t* out);
+bool prologue_rows_config(const Problem& p, tlhip_kernel_config_t* out);
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out);
 
 // The numbers the default routing was fitted with on MI355X: measurements, not structure.
@@ -619,11 +621,54 @@ tlhip_kernel_config_t default_below_few(const Problem& p) {
   return default_valu_config(p);
 }
 
+// One row on its own kernel (gemv_one.hip), where it takes it and the VALU kernel is not ahead of it: long rows whose
+// chunks take more lanes than a wave has, on matrices of 3073..4096 or at least 8192 rows.  Us, the VALU kernel / this one:
+// f16 int4 with K beyond 12288 at 16384 x 14336 24.2 / 28.1 (6144 x 14336 13.2 / 12.5); f32 int4 with K beyond 8192 at 12288 x
+// 9728 20.1 / 24.7 (4096 rows: level); f32 int8 with K beyond 6144 of which a lane in 25 has none, at 16384 x 7168 22.2 / 24.9 (K = 8192,
+// 128 lanes with four chunks each: level).  A gated multiply in front of int8 rows beyond 12288 (8192 x 14336 23.5 / 29.0),
+// an RMSNorm in front of rows of 10241 to 12288 in groups and few columns (2048 x 12288 8.9 / 10.4).
+bool one_row_config(const Problem& p, tlhip_kernel_config_t* out) {
+  if (p.m != 1 || !gemv_one_default(p, p.n, ONE_SINGLE, out)) return false;
+  const bool f16 = p.x_dtype == TLHIP_F16, int4 = p.format == TLHIP_FMT_INT4_GROUPED;
+  const bool many = p.n < 32768 && (p.n >= 8192 || (p.n > 3072 && p.n <= 4096));
+  if (p.pro.kind == TLHIP_PRO_GATED_MUL) return int4 || p.k <= 12288 || !many;
+  if (p.pro.kind == TLHIP_PRO_RMSNORM) return p.format != TLHIP_FMT_INT8_GROUPED || p.k <= 10240 || p.k > 12288 || p.n < 2048 || p.n > 4096;
+  if (int4) return f16 ? p.k <= 12288 || !many : p.k <= 8192 || p.n < 6144 || p.n >= 32768;
+  const int64_t lanes = (int64_t)out->p0 * out->p3, chunks = p.k / 16, held = (chunks + lanes - 1) / lanes * lanes;
+  return f16 || p.k <= 6144 || !many || lanes <= 64 || 25 * held <= 26 * chunks;
+}
+
+// One or two f16 rows with a prologue on the VALU kernel: the lanes that share a row by the number of columns and, for
+// int4, the 4x4x4 form on wide matrices.  Us, the geometry below / here, two rows, gated multiply / RMSNorm: int4 2048 x 9728
+// 16.2 -> 11.7 / 15.0 -> 12.2, 4096 x 9728 17.9 -> 13.4 / 14.4 -> 12.7, 8192 x 14336 35.3 -> 22.3 / 29.2 -> 20.4; int8-64 2048 x 4096
+// 8.5 -> 6.8 / 7.5 -> 6.9, 2048 x 12288 15.3 -> 13.2 / 13.0 -> 11.2.
+bool prologue_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
+  if (p.pro.kind == TLHIP_PRO_NONE || p.x_dtype != TLHIP_F16 || p.m > 2 || p.n >= 32768) return false;
+  const bool gated = p.pro.kind == TLHIP_PRO_GATED_MUL;
+  if (p.m == 1) {  // (the rows that one_row_config leaves)
+    *out = p.n <= 4096 ? gemv_cfg(64, 1, 8, 1, 4) : gemv_cfg(32, 1, 8, 1, 8);
+  } else if (p.format == TLHIP_FMT_INT4_GROUPED) {
+    if (p.k < (p.n > 1024 && p.n <= 2048 ? 2048 : 3072) || (p.n >= 12288 && p.k < 6144)) return false;
+    if (p.n <= 2048) {
+      *out = gemv_cfg(64, 1, 8, 1, 2);
+    } else if (p.n <= 4096 && !(gated && p.k > 8192)) {
+      *out = gemv_cfg(32, 1, 8, 1, 4);
+    } else {
+      *out = gemv_cfg(16, 1, 8, p.n <= 4096 ? 2 : 1, 2);
+      out->p5 = 1;
+    }
+  } else {
+    if (p.k < (p.n <= 1024 ? 3072 : 2048) || p.n > (p.k <= 4096 ? 4096 : 2048)) return false;
+    *out = p.n <= 2048 ? gemv_cfg(64, 1, 8, 1, p.k >= 8192 ? 4 : 2) : gemv_cfg(32, 1, 8, 1, 4);
+  }
+  return gemv_config_applicable(p, *out, nullptr);
+}
+
 // Heuristic default of the VALU kernel (the only one for M <= 4, and the one the
 // prologue entry points use).
 tlhip_kernel_config_t default_valu_config(const Problem& p) {
   tlhip_kernel_config_t one;
-  if (gemv_one_default(p, p.n, ONE_SINGLE, &one)) return one;
+  if (one_row_config(p, &one) || prologue_rows_config(p, &one)) return one;
   const int cw = p.format == TLHIP_FMT_INT4_GROUPED ? 32 : 16;
   const int64_t nchunks = p.k / cw;
   if (p.n >= 32768) {
@@ -830,8 +875,9 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
       const tlhip_kernel_config_t own = default_below_few(p);
       if (own.variant == VARIANT_GEMV_MFMA && config_applicable(p, c, nullptr) && gemv_mfma_us(p, own) < gemv_mfma_us(p, c)) c = own;
     }
-    // (one row: the lanes that share it follow from K and the number of columns)
-    if (c.variant == VARIANT_GEMV) (void)gemv_one_default(p, p.n, ONE_SINGLE, &c);
+    // (one row: the kernel and the lanes that share it follow from K and the number of columns; the VALU kernel's winner
+    // at 4096 x 12288 int8 is 10-15 % behind them at 2560 x 9728 and 3072 x 11008)
+    if (p.m == 1 && c.variant == VARIANT_GEMV && !one_row_config(p, &c)) continue;
     if (is_some_config(c) && !gemv_some_default(p, &c)) continue;
     const double d = dn + 2.0 * dk + dm;  // K decides whether the activations fit LDS: weigh it
     if (d < best && config_applicable(p, c, nullptr)) {
@@ -916,12 +962,12 @@ tlhip_kernel_config_t select_config(const Problem& p) {
   return e.config;
 }
 
-// The VALU configuration for launches only that kernel has (with a prologue): one row's own
-// geometry, else the tuned or selected one if it is of that kernel, else the heuristic.
+// The VALU configuration for launches only that kernel has (with a prologue): one row's by the rules of default_valu_config
+// (a winner of the plain launch is fitted to a workgroup that has no prologue to make), more rows' the tuned or selected
+// one if it is of that kernel, else by the rules.
 tlhip_kernel_config_t valu_config(const Problem& p) {
-  tlhip_kernel_config_t c;
-  if (p.pro.kind != TLHIP_PRO_NONE && gemv_one_default(p, p.n, ONE_SINGLE, &c)) return c;
-  c = select_config(p);
+  if (p.pro.kind != TLHIP_PRO_NONE && p.m == 1) return default_valu_config(p);
+  tlhip_kernel_config_t c = select_config(p);
   if (c.variant != VARIANT_GEMV) c = default_valu_config(p);
   return c;
 }
