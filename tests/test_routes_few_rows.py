@@ -76,3 +76,22 @@ def test_a_neighbours_k_slices_are_weighed_at_a_problems_own_prices(n, k, all_of
 def test_one_row(fmt, n, k, x, own_kernel):
     c = chosen(fmt, n, k, 1, x)
     assert c[0] == L.VARIANT_GEMV and (c[6] == 3) == own_kernel, c
+
+
+@pytest.mark.parametrize("fmt,n,k,m,form", [
+    # all of K in a workgroup on the matrix cores / K slices there / the VALU
+    (ROW, 5120, 12288, 6, "slices"),    # 30.1 / 21.4
+    (ROW, 4096, 14336, 12, "slices"),   # 31.9 / 24.7
+    (INT8, 4096, 8192, 10, "whole"),    # 15.1 / 19.3
+    (ROW, 4096, 8192, 8, "whole"),      # 13.3 / 14.1
+    (INT4, 768, 9728, 4, "whole"),      # 10.4 / 19.0
+    (INT4, 1024, 9728, 2, "valu"),      # 10.0 / - / 8.0
+    (INT4, 8192, 3072, 2, "valu"),      # 8.9 in one launch of all of K on the VALU, 7.7
+    (INT8, 10240, 1536, 2, "valu"),     # 7.6, 6.0
+    (INT8, 4096, 1024, 2, "some"),      # 4.4, 4.4
+    (ROW, 1024, 16384, 2, "whole"),     # 13.1 / - / 18.7
+])
+def test_a_few_f32_rows(fmt, n, k, m, form):
+    c = chosen(fmt, n, k, m, L.F32)
+    got = ("whole" if c[2] else "slices") if c[0] == L.VARIANT_GEMV_F32 else ("some" if c[6] == 4 else "valu")
+    assert got == form, c

@@ -129,6 +129,8 @@ struct ScratchNeed {
 // gemv_f32.hip: f32 activations in three bf16 pieces on the matrix cores
 bool gemv_f32_config_applicable(const Problem& p, const tlhip_kernel_config_t& c, const char** why);
 bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out);
+// ... all of K in a workgroup, K slices or not.
+bool gemv_f32_whole_default(const Problem& p, tlhip_kernel_config_t* out);
 int launch_gemv_f32(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c);
 // The gemv_mfma variant's form for 17..64 rows (gemm_rows.hip; p4: blocks of 16 columns per

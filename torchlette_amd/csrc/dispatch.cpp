@@ -501,6 +501,15 @@ bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return gemv_few_us(p, *out) <= gemv_mfma_us(p, below);
 }
 
+// Two f32 rows that stay on the VALU kernel of gemv_kernel.h, us, there / where they would go: int4, up to 1536 columns of a K
+// between 8192 and 12288 (1024 x 9728 8.0 / 10.0 with all of K on the matrix cores), and 7169..8192 columns, its workgroups two to a CU
+// (8192 x 3072 7.7 / 8.9 on gemv_some); int8 with K up to 1536 on wide matrices (10240 x 1536 6.0 / 7.6) and up to 2048 on
+// 4097..6144 columns (6144 x 1536 5.1 / 5.7).
+bool two_f32_rows_on_valu(const Problem& p) {
+  if (p.format == TLHIP_FMT_INT4_GROUPED) return (p.n <= 1536 && p.k > 8192 && p.k < 12288) || (p.n > 7168 && p.n <= 8192 && p.k <= 4096);
+  return (p.n > 6144 && p.k <= 1536) || (p.n > 4096 && p.n <= 6144 && p.k > 1024 && p.k <= 2048);
+}
+
 // 2 to 5 f32 rows on the VALU in one launch (gemv_some.hip): where they do not go to the matrix cores, and
 // there too where few columns leave the launch to its chain of steps.  Us, four rows and the rest (two and two) in
 // launches of their own -> here / all of K on the matrix cores: 5 rows of int8-64 at 2304 x 2048 10.6 -> 5.4 / 5.4, at
@@ -509,7 +518,8 @@ bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
 // 13.8 -> 11.6 / 8.9, 4096 x 12288 18.0 -> - / 11.9, 9216 x 2304 10.9 -> 9.4 / 8.3).
 bool few_f32_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   if (p.x_dtype != TLHIP_F32 || p.m < 2 || p.m > 5 || p.n > 16384 || p.pro.kind != TLHIP_PRO_NONE) return false;
-  if (p.m == 2 && (p.k > 8192 || (p.k > 4096 && p.n > 2048) || (p.k > 2048 && p.n > 8192))) return p.k <= 16384 && gemv_f32_default(p, out) && out->p1;
+  if (p.m == 2 && two_f32_rows_on_valu(p)) return false;
+  if (p.m == 2 && (p.k > 8192 || (p.k > 4096 && p.n > 2048) || (p.k > 2048 && p.n > 8192))) return gemv_f32_whole_default(p, out);
   const bool few = p.k > 1280 && (p.k <= 4096 ? p.n <= 2048 : p.n <= 1024);
   return (p.m == 2 || few || !f32_rows_on_matrix_cores(p)) && gemv_some_default(p, out);
 }

@@ -651,10 +651,12 @@ ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c) {
   return ScratchNeed{(size_t)column_tiles(p) * (size_t)c.p0 * (size_t)p.m * kCols, column_tiles(p)};
 }
 
-// All of K in one workgroup at `cols` columns of nb blocks, in microseconds: per round of workgroups the
+// What orders the widths of all of K in one workgroup, `cols` columns of nb blocks: per round of workgroups the
 // sums and the barriers, and per 1000 of K the cutting of X, the weights and the products.  Fitted at 2600
-// launches (34 matrices of 1024..15340 x 1024..12288, 2..16 rows, four formats): 7 % off (rms); the width it picks
-// is 0.5 % behind the best one in the mean, 5 % at worst.
+// launches (34 matrices of 1024..15340 x 1024..12288, 2..16 rows, four formats, warm): 7 % off (rms); the width it picks
+// is 0.5 % behind the best one in the mean, 5 % at worst.  On cold weights it is 5-11 % too low: what the launch takes
+// beside K slices is whole_beside_us.
+static double packed_mb(const Problem& p) { return (double)p.n * (double)p.k * (p.format == TLHIP_FMT_INT4_GROUPED ? 0.5 : 1.0) / 1e6; }
 static int format_index(const Problem& p) { return p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1); }
 static double whole_us(const Problem& p, int cols) {
   static const double weights[3][3][4] = {  // tiles of pieces, format, blocks
@@ -666,28 +668,49 @@ static double whole_us(const Problem& p, int cols) {
   const double k = (double)((steps + kWhole - 1) / kWhole * kWhole * kWholeStep) / 1000.0;
   return 2.02 + (double)rounds * (0.88 + 0.186 * tiles * nb + k * (0.09 * (double)p.m + 0.116 * cols / 16.0 + weights[tiles - 1][format_index(p)][nb - 1]));
 }
-// ... and of K slices across workgroups (fitted at 1716 launches, 3..16 rows): the longest one's pieces and
-// weights, and 0.010-0.017 for every row of every slice that the last arrival adds: 0.85-1.17 times that, int4
-// (8 % above its fit: its short slices scatter) 0.72-1.2.
+// Behind each other and on cold weights, the picked width and K slices across workgroups: the weights' way from memory,
+// per round the sums and, per 1000 of K, the cutting of X and the blocks' products; of slices the longest one's pieces
+// and weights and, for every row of every slice, what the last arrival adds.  Fitted at 2287 launches of either (106
+// matrices of 768..16384 x 1024..16384, 3..16 rows, three formats): 2-7 % and 4-9 % rms; the cheaper one is 0.05-0.3 % behind the faster
+// in the mean and more than 3 % at 1-4 % of the problems (2-7 % by warm prices: five rows of int8 per row at
+// 5120 x 12288 21.4 us in slices, 30.1 so).
+static double whole_beside_us(const Problem& p, int cols) {
+  struct Cost {
+    double launch, mb, round, sums, k, k_rows, k_blocks;
+  };
+  static const Cost costs[3][3] = {  // format, tiles of pieces
+      {{0.0, 0.073, 2.511, 0.415, 0.0, 0.080, 0.446}, {2.925, 0.084, 0.0, 0.343, 0.084, 0.057, 0.617}, {1.159, 0.091, 0.883, 0.985, 0.335, 0.079, 0.458}},
+      {{0.0, 0.063, 2.817, 0.348, 0.0, 0.071, 0.374}, {3.447, 0.079, 0.0, 0.043, 0.0, 0.045, 0.644}, {1.246, 0.068, 1.205, 0.701, 0.587, 0.070, 0.392}},
+      {{2.604, 0.059, 0.0, 0.348, 0.0, 0.063, 0.407}, {3.179, 0.081, 0.0, 0.080, 0.0, 0.045, 0.587}, {1.157, 0.080, 0.861, 0.687, 0.672, 0.068, 0.293}}};
+  const Cost& t = costs[format_index(p)][tiles_of(p.m) - 1];
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256, nb = (cols + 15) / 16;
+  const int64_t wgs = (p.n + cols - 1) / cols, steps = p.k / kWholeStep;
+  const double rounds = (double)((wgs + cus - 1) / cus), k = (double)((steps + kWhole - 1) / kWhole * kWhole * kWholeStep) / 1000.0;
+  return t.launch + t.mb * packed_mb(p) + rounds * (t.round + t.sums * nb + k * (t.k + t.k_rows * (double)p.m + t.k_blocks * nb));
+}
 static double slices_us(const Problem& p, int slices) {
-  static const double base[3] = {10.7, 6.2, 6.5}, weights[3] = {5.22, 7.86, 4.98}, cut[3] = {0.471, 0.297, 0.324}, sum[3] = {0.010, 0.017, 0.014};
-  const int cus = device_cu_count() > 0 ? device_cu_count() : 256, f = format_index(p);
+  struct Cost {
+    double launch, mb, weights, cut, slice, sum, out;
+  };
+  static const Cost costs[3] = {{10.40, 0.103, 6.152, 0.256, 0.022, 0.010, 0.064}, {5.73, 0.096, 6.809, 0.113, 0.097, 0.012, 0.057}, {5.06, 0.091, 3.680, 0.113, 0.093, 0.010, 0.065}};
+  const Cost& t = costs[format_index(p)];
+  const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int64_t wgs = column_tiles(p) * slices, rounds = (wgs + cus - 1) / cus, slice = (blocks_of(p) + slices - 1) / slices * block_k(p);
-  return base[f] + (double)(rounds * slice) / 1000.0 * (weights[f] + cut[f] * (double)p.m) + sum[f] * (double)(slices * p.m);
+  const double rows = (double)(slices * p.m);
+  return t.launch + t.mb * packed_mb(p) + (double)(rounds * slice) / 1000.0 * (t.weights + t.cut * (double)p.m) + t.slice * slices + t.sum * rows +
+         t.out * (double)column_tiles(p) * rows / 100.0;
 }
 
 // All of K in one workgroup, at the cheapest number of columns (whole blocks, or an even share that
 // leaves no round half empty: 9216 columns in 256 workgroups of 36, not 576 of 16), or false where K slices stay.
-// Us, slices / here: 5 rows of int8-64 at 9216 x 2304 13.0 / 8.5, at 2304 x 9216 16.8 / 10.8; 10 rows at 12288 x
-// 4096 29.4 / 14.1; 16 rows of int4 at 12288 x 4096 46 / 18.5 and at 4096 x 12288 40 / 28.5.  Behind where the
-// price says so: 16 rows of int8 at 1484 x 8320 16-18 / 21-22, at 2304 x 9216 19-22 / 21-22.
+// Us, slices / here, cold weights: ten rows of int8-64 at 3072 x 8192 19.9 / 16.3; 16 rows of int4 at 12288 x 4096 45 / 20.
 // Three exceptions, where the routes of longer standing are kept though this form has caught up with them:
-// more than 16384 columns; fewer than 1024 of a K beyond 8192 (5 rows at 512 x 16384 17.3 / 15.3); and int4 with
-// more than ten rows, 8192 columns and K an odd number of steps (10208 x 3712, 16 rows 27 / 18; 12748 x 4224, 14
-// rows 26.5 / 30).
+// more than 16384 columns; fewer than 1024 of a K beyond 8192 of int8 (5 rows at 512 x 16384 17.3 / 15.3; of int4 at 768 x 9728
+// 18.9 / 12.7, which goes by the price); and int4 with more than ten rows, 8192 columns and K an odd number of steps (10208 x
+// 3712, 16 rows 27 / 18; 12748 x 4224, 14 rows 26.5 / 30).
 static bool whole_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  if (p.n > 16384 || (p.n < 1024 && p.k > 8192)) return false;
+  if (p.n > 16384 || (p.n < 1024 && p.k > 8192 && p.format != TLHIP_FMT_INT4_GROUPED)) return false;
   if (p.format == TLHIP_FMT_INT4_GROUPED && p.m > 10 && p.n > 8192 && p.k / kWholeStep % 2) return false;
   memset(out, 0, sizeof *out);
   out->variant = VARIANT_GEMV_F32;
@@ -724,11 +747,16 @@ static bool slices_default(const Problem& p, tlhip_kernel_config_t* out) {
   return false;
 }
 
+bool gemv_f32_whole_default(const Problem& p, tlhip_kernel_config_t* out) {
+  double us = 0.0;
+  return whole_default(p, out, &us);
+}
+
 bool gemv_f32_default(const Problem& p, tlhip_kernel_config_t* out) {
   tlhip_kernel_config_t whole;
   double us = 0.0;
   const bool found = slices_default(p, out);
-  if (!whole_default(p, &whole, &us) || (found && us >= slices_us(p, out->p0))) return found;
+  if (!whole_default(p, &whole, &us) || (found && whole_beside_us(p, whole_cols(whole)) >= slices_us(p, out->p0))) return found;
   *out = whole;
   return true;
 }
