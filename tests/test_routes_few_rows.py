@@ -95,3 +95,32 @@ def test_a_few_f32_rows(fmt, n, k, m, form):
     c = chosen(fmt, n, k, m, L.F32)
     got = ("whole" if c[2] else "slices") if c[0] == L.VARIANT_GEMV_F32 else ("some" if c[6] == 4 else "valu")
     assert got == form, c
+
+
+@pytest.mark.parametrize("fmt,n,k,m,all_of_k", [
+    # K slices (or none) of the skinny kernel / all of K in a workgroup
+    (INT4, 24576, 2048, 32, False),   # 14.0 / 20.9
+    (ROW, 768, 16384, 32, False),     # 12.2 / 16.4
+    (INT4, 20480, 1024, 32, False),   # 9.8 / 12.6
+    (INT8, 28672, 1024, 24, False),   # 13.0 / 16.5
+    (INT8, 1024, 16384, 32, False),   # 13.8 / 16.9
+    (INT4, 20480, 11008, 24, True),   # three blocks of columns 50.5, one 69.3
+    (INT4, 4096, 8192, 17, True),     # 13.2 / 10.6
+    (ROW, 5120, 1536, 40, True),      # 9.3 / 7.4
+    (INT4, 14336, 1536, 17, True),    # 9.8 / 8.3
+])
+def test_17_to_64_f16_rows(fmt, n, k, m, all_of_k):
+    lib = L.load()
+    before = T.exportTuningCache()
+    buf = ctypes.create_string_buffer(64)
+    ptr = ctypes.cast(buf, ctypes.c_void_p).value
+    w, rows, first, last = L.QWeight(*fmt, n, k, ptr, ptr), ctypes.c_int64(), L.KernelConfig(), L.KernelConfig()
+    try:
+        T.clearTuningCache()
+        assert lib.tlhip_selected_route(ctypes.byref(w), L.F16, m, L.F16, ctypes.byref(rows), ctypes.byref(first), ctypes.byref(last)) == 0
+    finally:
+        T.clearTuningCache()
+        T.importTuningCache(before)
+    c = last.as_tuple()
+    assert c[0] == L.VARIANT_GEMV_MFMA and whole(c) == all_of_k, c
+    assert (n, k) != (20480, 11008) or c[5] == 3, c

@@ -137,6 +137,8 @@ ScratchNeed gemv_f32_scratch(const Problem& p, const tlhip_kernel_config_t& c);
 // workgroup): all of K in one workgroup, no workspace.  What it does not take runs the other form.
 bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c);
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us);
+// Time of such a launch behind others, in microseconds; c applicable.
+double gemm_rows_us(const Problem& p, const tlhip_kernel_config_t& c);
 int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
 // Time of a launch of the decode kernel at up to 16 and at 17..64 rows, in microseconds (gemv_mfma.hip); c applicable.
 double gemv_mfma_us(const Problem& p, const tlhip_kernel_config_t& c);

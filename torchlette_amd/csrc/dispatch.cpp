@@ -1127,20 +1127,18 @@ bool decode_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   return false;
 }
 
-// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip).  K up to 6144: unless its price
-// is a quarter above the former's; at 84 problems of 400..4000 x 2048..5632 it was the faster one at each, by 23 %
-// at prices alike and still by 20 % at 1.07 (20 rows of int4 at 900 x 3584 7.6 / 6.1 us).  Beyond, where few
-// columns leave most CUs idle: from 0.87 of it on (48 rows of int8-64 at 760 x 10496 14.7 us in K slices, 21.7
-// here; at 2496 x 11008, 32 rows of int4, 15.0 and 13.7); and so from 16384 columns on, where the prices are
-// least sure (17 rows of int4 at 16384 x 4096 16.2 / 14.1, but at 32000 x 4096 24.1 / 28.2).  Where few columns
-// give the row tiles workgroups of their own the first line holds for every K (20 rows of int4 at 712 x 8192 10.0 / 8.1).
+// That form, or the one that keeps all of K in one workgroup (gemm_rows.hip) where it is the cheaper one: over 3946
+// problems 0.2-0.3 % behind the faster one in the mean, more than 3 % at 2-3 % of them (by warm prices and lines between them
+// 0.9-2.5 %, at 6-12 %: 24 rows of int4 at 24576 x 2048 14.3 us in K slices, 18.7 so).  Four tiles of int4 rows without a
+// residual and K beyond 6144 keep the K slices unless they are a ninth dearer, the route of longer standing (64 rows at 3312 x 8960
+// 21.6 / 21.0, at prices of 22.4 and 20.5).
 bool rows_in_one_launch_config(const Problem& p, tlhip_kernel_config_t* out) {
   const bool found = decode_rows_config(p, out);
   tlhip_kernel_config_t whole;
   double us = 0.0;
   if (!gemm_rows_default(p, &whole, &us)) return found;
-  const double line = whole.p6 == 0 && (p.k > 6144 || p.n >= 16384) ? 0.87 : 1.25;
-  if (found && us >= line * gemv_mfma_rows_us(p, *out)) return found;
+  const double line = p.format == TLHIP_FMT_INT4_GROUPED && p.m > 48 && p.k > 6144 && whole.p6 == 0 && !has_residual(p) ? 0.9 : 1.0;
+  if (found && gemm_rows_us(p, whole) >= line * gemv_mfma_rows_us(p, *out)) return found;
   *out = whole;
   return true;
 }

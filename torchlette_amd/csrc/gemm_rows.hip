@@ -443,12 +443,46 @@ bool is_rows_config(const Problem& p, const tlhip_kernel_config_t& c) {
   return p.format == TLHIP_FMT_INT8_ROW || p.group_size >= 64;
 }
 
-// The cheapest number of column blocks and its time in microseconds, or false.  Fitted at 3072 launches of
-// 52 matrices of 768..16384 x 768..12288, 17..64 rows, four formats, cold weights, with a residual up to 4608
-// columns: launch, and per round of workgroups a constant, the sums of a block and, per 4096 of K in whole
-// steps of the longest wave, the figure of the width, a little more for every row above the middle of its
-// tile.  One block a workgroup: a second round overlaps the first (two fit a CU up to 32 rows).  8-10 % off
-// (rms); the width it picks is 0.03 % slower than the best one in the mean, 5 % at worst.
+// What a launch takes behind others and on cold weights, beside K slices across workgroups (gemv_mfma_rows_us): the
+// weights' way from memory, per round of workgroups the blocks' sums and, per 4096 of K, a step, its blocks and its
+// rows; a share of the row tiles, of which every workgroup has a CU, the walk of a range.
+// Fitted at 4968 launches of the geometries that gemm_rows_default weighs (13 x 11 matrices of 768..28672 x 1024..16384,
+// 17..64 rows, three formats, with and without a residual): 3-5 % rms, two tiles of int8 8 %.
+double gemm_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
+  struct Whole {
+    double launch, mb, round, sums, k, k_blocks, k_rows, residual, residual_out;
+  };
+  struct Share {
+    double launch, k, mb, residual, residual_out;
+  };
+  static const Whole whole[3][3] = {  // format, row tiles
+      {{2.035, 0.089, 0.0, 0.876, 1.163, 1.220, 1.005, 0.990, 0.140}, {1.401, 0.121, 0.464, 1.145, 2.486, 1.195, 0.686, 0.916, 0.165}, {1.627, 0.104, 0.253, 1.290, 0.0, 2.078, 1.285, 0.830, 0.158}},
+      {{1.878, 0.061, 0.394, 0.587, 0.718, 1.677, 1.555, 1.062, 0.124}, {1.182, 0.069, 1.001, 0.848, 2.336, 1.383, 1.132, 0.868, 0.202}, {1.415, 0.077, 0.475, 1.299, 0.0, 0.978, 1.863, 0.855, 0.165}},
+      {{1.682, 0.068, 0.518, 0.631, 0.907, 1.445, 1.500, 1.000, 0.099}, {1.586, 0.081, 0.272, 0.996, 2.676, 1.101, 1.028, 0.833, 0.183}, {1.477, 0.082, 0.498, 1.019, 0.0, 1.118, 1.766, 0.808, 0.163}}};
+  static const Share share[3][2] = {  // format, one or two tiles a workgroup
+      {{2.699, 2.401, 0.115, 0.771, 0.804}, {2.899, 3.771, 0.108, 0.816, 0.438}},
+      {{2.786, 3.127, 0.045, 0.816, 0.812}, {2.899, 4.408, 0.047, 0.702, 0.805}},
+      {{2.710, 3.085, 0.045, 0.795, 0.775}, {2.828, 4.293, 0.043, 0.662, 0.781}}};
+  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED, residual = has_residual(p);
+  const int format = int4 ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1), cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  const double mb = (double)p.n * (double)p.k * (int4 ? 0.5 : 1.0) / 1e6, out = (double)p.m * (double)p.n / 1e5, walk = (double)p.k / 4096.0;
+  if (c.p6) {
+    const Share& t = share[format][c.p6 - 1];
+    return t.launch + t.k * walk + t.mb * mb + (residual ? t.residual + t.residual_out * out : 0.0);
+  }
+  const Whole& t = whole[format][row_tiles_of(p.m) - 2];
+  const int64_t wgs = (p.n + 16 * c.p4 - 1) / (16 * c.p4);
+  const double rounds = (double)((wgs + cus - 1) / cus);
+  return t.launch + t.mb * mb + rounds * (t.round + t.sums * c.p4 + walk * (t.k + t.k_blocks * c.p4 + t.k_rows * (double)p.m / 16.0)) +
+         (residual ? t.residual + t.residual_out * out : 0.0);
+}
+
+// The number of column blocks or the share of the row tiles, and its time in microseconds where the launch is not behind
+// others (beside the tiles, which were priced so), or false.  Fitted at 3072 launches of 52 matrices of 768..16384 x
+// 768..12288, 17..64 rows, four formats: launch, and per round of workgroups a constant, the sums of a block and, per
+// 4096 of K in whole steps of the longest wave, the figure of the width, a little more for every row above the middle of
+// its tile.  One block a workgroup: up to four rounds overlap (two fit a CU up to 32 rows).  8-10 % off (rms); the width
+// it picks is 0.0-0.4 % behind the best one in the mean of 2624 problems on cold weights.
 bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us) {
   struct Cost {
     double launch, round, block, walk[kMaxCols], second, per_row;
@@ -462,24 +496,6 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
   // (up to four steps: on a SIMD each)
   const int64_t steps = p.k / kStep, walked = steps <= 4 ? steps : (steps + kWaves - 1) / kWaves * kWaves;
   const double walk = (double)(walked * kStep) / 4096.0;
-  // Few columns: the row tiles to workgroups of their own while every one has a CU, which reads the weights once
-  // for each (from the last-level cache) but walks a range in the time of one tile, us, all tiles / one / two a
-  // workgroup: int4 1024 x 4096 at 48 rows 9.6 / 6.3 / 7.8, 1024 x 12288 at 64 27.4 / 11.0 / 15.0, 1536 x 6144 at 48 12.1 /
-  // 10.8 / 9.7; past one a CU behind (int8-64 4096 x 4096 at 48 rows 10.6 / 13.0 / 12.5).  Int8 with K beyond 6144 and more
-  // than 1152 columns is left to the K slices, as the tests of the routing hold it there.
-  if (format == 0 || p.k <= 6144 || p.n <= 1152)
-    for (int tiles = 1; tiles <= 2 && tiles < mt; ++tiles) {
-      memset(out, 0, sizeof *out);
-      out->variant = VARIANT_GEMV_MFMA;
-      out->p0 = kWaves;
-      out->p4 = 1;
-      out->p6 = tiles;
-      if ((p.n + 15) / 16 * ((mt + tiles - 1) / tiles) > cus || !is_rows_config(p, *out)) continue;
-      static const double one[3] = {2.2, 2.85, 2.7};
-      const Cost& two = costs[format][0];
-      *us = tiles == 1 ? 4.1 + walk * one[format] : two.launch + two.round + two.block + walk * two.walk[0];
-      return true;
-    }
   bool found = false;
   for (int nb = 1; nb <= kMaxCols; ++nb) {
     tlhip_kernel_config_t c;
@@ -489,14 +505,30 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
     c.p4 = nb;
     if (!is_rows_config(p, c)) continue;
     const Cost& cost = costs[format][mt - 2];
-    const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb);
-    const double rounds = 1.0 + (double)((wgs + cus - 1) / cus - 1) * (nb == 1 ? cost.second : 1.0);
+    const int64_t wgs = (p.n + 16 * nb - 1) / (16 * nb), turns = (wgs + cus - 1) / cus;
+    const double rounds = 1.0 + (nb == 1 ? cost.second * (double)(std::min<int64_t>(turns, 4) - 1) + (double)std::max<int64_t>(turns - 4, 0) : (double)(turns - 1));
     const double t = cost.launch + rounds * (cost.round + cost.block * nb + walk * cost.walk[nb - 1] * (1.0 + cost.per_row * (double)(p.m - 16 * mt + 8)));
     if (found && t >= *us) continue;
     *out = c;
     *us = t;
     found = true;
   }
+  // Few columns: the row tiles to workgroups of their own while every one has a CU, which reads the weights once
+  // for each (from the last-level cache) but walks a range in the time of one tile, us, all tiles / one / two a
+  // workgroup: int4 1024 x 4096 at 48 rows 9.6 / 6.3 / 7.8, 1024 x 12288 at 64 27.4 / 11.0 / 15.0, 1536 x 6144 at 48 12.1 /
+  // 10.8 / 9.7; past one a CU behind (int8-64 4096 x 4096 at 48 rows 10.6 / 13.0 / 12.5).  Int8 with K beyond 6144 and more
+  // than 1152 columns is left to the K slices, as the tests of the routing hold it there.
+  if (found && (format == 0 || p.k <= 6144 || p.n <= 1152))
+    for (int tiles = 1; tiles <= 2 && tiles < mt; ++tiles) {
+      tlhip_kernel_config_t c = *out;
+      c.p4 = 1;
+      c.p6 = tiles;
+      if ((p.n + 15) / 16 * ((mt + tiles - 1) / tiles) > cus || !is_rows_config(p, c) || gemm_rows_us(p, c) >= gemm_rows_us(p, *out)) continue;
+      static const double one[3] = {2.2, 2.85, 2.7};
+      const Cost& two = costs[format][0];
+      *out = c;
+      *us = tiles == 1 ? 4.1 + walk * one[format] : two.launch + two.round + two.block + walk * two.walk[0];
+    }
   return found;
 }
 

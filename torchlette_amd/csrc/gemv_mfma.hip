@@ -122,34 +122,33 @@ bool gemv_mfma_config_applicable(const Problem& p, const tlhip_kernel_config_t& 
   return mfma_applicable(p, (p.n + 15) / 16, c, why);
 }
 
-// What a launch of 17..64 rows adds to a decoder layer (the measure of gemm_rows_default, at the same
-// problems): a residual costs this form 2.4-3.4 us up to 32 rows and 5 beyond, its last arrivals read
-// and store 16 columns a row, against 1.2-1.4 for all of K in one workgroup.  Fitted at 1299 launches
-// of decode_rows_config's geometries.  An iteration of a wave, in whole sets of those in flight, takes
-// its time (more where only one is in flight, 0.6 % more a row) once for every one that runs before
-// it, in its round, the rounds of its workgroup and the workgroups that share its CU; K slices add the
-// arrival of the last one and the planes it adds.  96 % of the launches take 0.84-1.21 times that.
+// What a launch of 17..64 rows takes behind others and on cold weights (the measure of gemm_rows_us, at the same
+// problems): the weights' way from memory, an iteration of a wave, in whole sets of those in flight (more where only one
+// is, and for more rows) once for every one that runs before it, in its round, the rounds of its workgroup and the
+// workgroups that share its CU; K slices add the arrival of the last one and the planes it adds.  A residual costs this
+// form more, its last arrivals read and store 16 columns a row.  Fitted at 4072 launches of decode_rows_config's
+// geometries: 6 % rms up to 32 rows, 8 % beyond.
 double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c) {
   struct Cost {
-    double base, sliced, iteration, round, plane, alone;
+    double launch, mb, iteration, alone, rows, round, sliced, plane, residual, residual_out, residual_sliced;
   };
-  static const Cost costs[3][2] = {
-      {{4.56, 1.84, 0.64, 0.06, 0.26, 0.07}, {5.46, 1.97, 0.93, 0.69, 0.73, 0.04}},   // int4, up to 32 rows and up to 64
-      {{4.11, 2.26, 0.53, 0.05, 0.24, 0.12}, {5.34, 1.90, 0.56, 0.57, 0.70, 0.13}},   // int8 in groups
-      {{4.59, 2.53, 0.35, 0.14, 0.22, 0.10}, {5.56, 1.98, 0.47, 0.49, 0.64, 0.12}}};  // int8 per row
-  const bool few = p.m <= 32;
-  const Cost& t = costs[p.format == TLHIP_FMT_INT4_GROUPED ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)][few ? 0 : 1];
-  const int kper = p.format == TLHIP_FMT_INT4_GROUPED ? 128 : 64;
-  const int kw = c.p2 == 0 ? c.p0 : c.p2, ks = c.p3 < 1 ? 1 : c.p3, per_wg = c.p0 / kw;
-  const int64_t nblocks = (p.n + 15) / 16, wgblocks = (nblocks + per_wg - 1) / per_wg, slice = (p.k / kper + ks - 1) / ks;
+  static const Cost costs[3][2] = {  // format, up to 32 rows and up to 64
+      {{5.126, 0.054, 0.385, 0.104, 0.110, 0.0, 1.081, 0.274, 1.267, 0.055, 0.779}, {4.818, 0.103, 0.444, 0.129, 0.120, 0.758, 1.388, 0.560, 1.765, 0.267, 2.407}},
+      {{4.663, 0.031, 0.426, 0.135, 0.062, 0.0, 1.682, 0.202, 1.365, 0.0, 0.466}, {4.555, 0.132, 0.341, 0.072, 0.061, 0.087, 1.333, 0.552, 2.768, 0.074, 1.599}},
+      {{5.338, 0.075, 0.193, 0.111, 0.040, 0.0, 1.657, 0.233, 1.328, 0.178, 0.979}, {4.129, 0.166, 0.039, 0.071, 0.083, 1.009, 1.499, 0.564, 2.659, 0.231, 2.019}}};
+  const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED;
+  const Cost& t = costs[int4 ? 0 : (p.format == TLHIP_FMT_INT8_ROW ? 2 : 1)][p.m <= 32 ? 0 : 1];
+  const int kper = int4 ? 128 : 64, kw = c.p2 == 0 ? c.p0 : c.p2, ks = c.p3 < 1 ? 1 : c.p3, per_wg = c.p0 / kw;
+  const int64_t wgblocks = ((p.n + 15) / 16 + per_wg - 1) / per_wg, slice = (p.k / kper + ks - 1) / ks;
   MfmaGeometry geo;
-  if (!mfma_geometry(nblocks, slice * kper, p.m, c.p0, kw, ks, line_patch_bytes(c), &geo)) return 1e9;
+  if (!mfma_geometry((p.n + 15) / 16, slice * kper, p.m, c.p0, kw, ks, line_patch_bytes(c), &geo)) return 1e9;
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int64_t sets = geo.grid / ks, rounds = (wgblocks + sets - 1) / sets, shared = (geo.grid + cus - 1) / cus;
   const int64_t own = (slice + kw - 1) / kw, in_flight = c.p1 < 1 ? 1 : c.p1;
-  const double iterations = (double)((own + in_flight - 1) / in_flight * in_flight) * (1.0 + 0.006 * (double)(p.m - (few ? 24 : 48)));
-  return t.base + (double)(rounds * shared) * (iterations * (t.iteration + (c.p1 == 1 ? t.alone : 0.0)) + t.round) +
-         (ks > 1 ? t.sliced + t.plane * (double)ks * (double)wgblocks / (double)sets : 0.0);
+  const double turns = (double)(rounds * shared), walk = turns * (double)((own + in_flight - 1) / in_flight * in_flight), rows = (double)p.m / 16.0;
+  return t.launch + t.mb * (double)p.n * (double)p.k * (int4 ? 0.5 : 1.0) / 1e6 + walk * (t.iteration + (in_flight == 1 ? t.alone : 0.0) + t.rows * rows) +
+         t.round * turns + (ks > 1 ? t.sliced + t.plane * (double)ks * (double)wgblocks / (double)sets : 0.0) +
+         (has_residual(p) ? t.residual + t.residual_out * (double)p.m * (double)p.n / 1e5 + (ks > 1 ? t.residual_sliced : 0.0) : 0.0);
 }
 
 // Up to 16 rows, beside all of K in a workgroup (gemv_few_us), the same way: the weights' way from memory, an iteration
