@@ -1,6 +1,5 @@
 """Which kernel a few rows take with nothing tuned: the one that measured faster (cold weights, us)."""
 import ctypes
-import os
 
 import pytest
 
@@ -52,14 +51,13 @@ def test_up_to_sixteen_f16_rows(fmt, n, k, m, all_of_k):
     assert whole(chosen(fmt, n, k, m, L.F16)) == all_of_k
 
 
-@pytest.mark.parametrize("n,k,all_of_k", [(4096, 12288, False), (4096, 8192, True), (2048, 12288, False)])
+@pytest.mark.parametrize("n,k,all_of_k", [(4096, 8192, True), (2048, 12288, False)])
 def test_a_neighbours_k_slices_are_weighed_at_a_problems_own_prices(n, k, all_of_k):
-    """Sixteen rows of int4 beside the shipped winners."""
-    cache = open(os.path.join(os.path.dirname(T.__file__), "tuning", "mi355x.json")).read()
+    """Sixteen rows of int4 beside a winner in K slices at 4096 x 12288 (2048 x 12288: 12.0 us in those, 9.4 in its own)."""
+    cache = '{"version":1,"entries":{"16_4096_12288_int4-grouped_g32_f16_f16":[1,8,2,2,4,0,1,0]}}'
+    assert chosen(INT4, 4096, 12288, 16, L.F16, cache) == (1, 8, 2, 2, 4, 0, 1, 0)
     c = chosen(INT4, n, k, 16, L.F16, cache)
-    assert whole(c) == all_of_k, c
-    if (n, k) == (2048, 12288):  # those of the winner at 4096 x 12288: 12.0, its own 9.4
-        assert c == chosen(INT4, n, k, 16, L.F16)
+    assert whole(c) == all_of_k and c == chosen(INT4, n, k, 16, L.F16), c
 
 
 @pytest.mark.parametrize("fmt,n,k,x,own_kernel", [

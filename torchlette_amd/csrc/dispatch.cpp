@@ -873,7 +873,7 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
     // (where a neighbour of 2..16 rows is on the matrix cores, the problem's own prices tell which of their two forms it has, and
-    // whether the neighbour's K slices are cheaper than its own: 16 rows of int4 at 2048 x 12288 12.0 us in those of the winner at
+    // whether the neighbour's K slices are cheaper than its own: 16 rows of int4 at 2048 x 12288 12.0 us in those of a winner at
     // 4096 x 12288, 9.4 in its own)
     tlhip_kernel_config_t few;
     const bool whole_there = is_few_config(there, c, FEW_SINGLE);
