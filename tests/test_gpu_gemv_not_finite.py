@@ -50,3 +50,26 @@ def test_one_row_with_its_last_chunk_not_finite(be, fmt, g, n, k, xdt, value):
         ran += 1
         assert same_kind(got, want), (lpr, kw)
     assert ran >= 2
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("xdt", ["f16", "f32"])
+@pytest.mark.parametrize("fmt,g,n,k", [
+    ("int4-grouped", 32, 67, 1312),
+    ("int8-grouped", 64, 130, 5248),
+    ("int8-row", 0, 70, 6128),
+])
+def test_one_to_five_rows_with_a_last_chunk_not_finite(be, fmt, g, n, k, xdt, value):
+    """The kernel whose lanes hold several chunks of several rows at a time, and its 4 x 4 x 4 form."""
+    rng = np.random.default_rng(zlib.crc32(repr((fmt, k, xdt)).encode()))
+    packed, scales, deq = make_weight(fmt, n, k, g, rng)
+    for m in (1, 2, 3, 5):
+        x = make_x(m, k, xdt, rng)
+        x[m // 2, k - 3] = value
+        want = product(x, deq)
+        configs = [(16, 1, 4, 1, 2, 0), (32, 2, 8, 2, 2, 0), (64, 1, 4, 4, 8, 0), (64, 4, 8, 1, 2, 0)]
+        if fmt == "int4-grouped" and xdt == "f16" and m <= 4:
+            configs += [(16, 1, 4, 1, 2, 1), (16, 1, 8, 2, 8, 1)]
+        for c in configs:
+            got = run_linear(be, fmt, packed, scales, n, k, g, x, "f32", config=L.KernelConfig.of(L.VARIANT_GEMV, *c))
+            assert same_kind(got, want), (m, c)

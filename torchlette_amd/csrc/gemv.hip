@@ -89,10 +89,10 @@ static void fill_args(const Problem& p, const tlhip_kernel_config_t& c, int64_t 
   a.epi = epilogue_from_row(p.epi, m0, p.n);  // this pass starts at row m0, like y
   a.pro = p.pro;
   if (a.pro.kind == TLHIP_PRO_GATED_MUL) a.pro.operand = (const char*)p.pro.operand + m0 * p.k * xbytes;
-  // LDS: staged x (mt rows) + split-K partials
+  // LDS: staged x (mt rows, a chunk of zeros behind each) + split-K partials
   const int chunk_x_bytes = cw * xbytes;
   const size_t partial_bytes = a.kw > 1 ? (size_t)a.kw * a.rows_per_wg * mt * sizeof(float) : 0;
-  lds_bytes = (size_t)mt * chunk_x_bytes * a.nchunks + partial_bytes + (c.p5 == 1 ? 4 * 16 * 16 : 0);  // + the row skew
+  lds_bytes = (size_t)mt * chunk_x_bytes * (a.nchunks + 1) + partial_bytes + (c.p5 == 1 ? 4 * 16 * 16 : 0);  // + the row skew
   threads = waves * 64;
   const int cus = device_cu_count();
   // resident workgroups per CU: bounded by 2048 lanes and by LDS

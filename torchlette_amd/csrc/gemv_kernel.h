@@ -141,8 +141,9 @@ struct ChunkDot<TLHIP_FMT_INT4_GROUPED, float> {
 };
 
 // LDS layout of the staged activations: 16-byte unit (row m, quarter qd of
-// chunk c) lives at unit index (m*NQ + qd)*nchunks + c, so the lanes of a row
-// group, which hold consecutive c, read consecutive units.
+// chunk c) lives at unit index (m*NQ + qd)*stride + c, so the lanes of a row
+// group, which hold consecutive c, read consecutive units.  stride = nchunks + 1:
+// the chunk behind a row's last is zero.
 //
 // Work of one lane is a sequence of batches: U chunks x R rows of 16-byte
 // weight loads (plus their scales).  The batches of all row blocks of the
@@ -150,8 +151,11 @@ struct ChunkDot<TLHIP_FMT_INT4_GROUPED, float> {
 // before batch i is consumed, and the very first batch is issued right after
 // the activation loads and before the LDS store and barrier, so HBM latency
 // overlaps the staging, the arithmetic and the reductions.  The hot path has no
-// per-lane branches: out-of-range chunks load a clamped address and contribute
-// zero through their scale (or a select).
+// per-lane branches: out-of-range chunks load a clamped address, multiply by the
+// chunk of zeros (a scale of zero alone leaves NaN where the last chunk's sum is
+// infinite) and have a scale of zero.  Without the zeros -> with them, 10 matrices, cold:
+// one to four f32 rows of int4 0.96 times the time, one and two f16 rows of int4 1.01
+// (two in the 4x4x4 form 1.02), the others level.
 // MF4 (int4, f16 activations, MT = 4, R = 1): the dot products of up to four activation
 // rows go through v_mfma_f32_4x4x4_16b_f16 instead of one v_dot2 chain per row.  The
 // instruction multiplies 16 independent 4 x 4 blocks: in block b (lanes 4b .. 4b+3) lane
@@ -183,11 +187,12 @@ __global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
   const int cfirst = kw_idx * a.lpr + lj;
   const int x_units_per_row = a.k * (int)sizeof(XT) / 16;  // 16-byte units per activation row
   const u32x4* xg = (const u32x4*)a.x;
+  const int stride = a.nchunks + 1;
   // MF4: the four lanes of a block read four different activation rows at the same
   // chunk; a skew of 16 units per row keeps them (and the 16 blocks) on 64 different
   // 16-byte units instead of 4 lanes on each bank.
   constexpr int XSKEW = MF4 ? 16 : 0;
-  float* partial = (float*)(lds + (size_t)MT * NQ * a.nchunks + MT * XSKEW);  // kw x rows_per_wg x MT, if kw > 1
+  float* partial = (float*)(lds + (size_t)MT * NQ * stride + MT * XSKEW);  // kw x rows_per_wg x MT, if kw > 1
   const int row_in_wg = rg * a.rows_per_wave + sub * R;
   const int last_chunk = a.nchunks - 1;
 
@@ -232,12 +237,12 @@ __global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int c = cb + u * cstride;
-        const int cc = min(c, last_chunk);
+        const int xc = min(c, a.nchunks);
         // this lane's operand row: activation row `sub` of the chunk (rows past M read the last one)
         const int xrow = min(sub, a.m - 1);
         u32x4 xq[NQ];
 #pragma unroll
-        for (int qd = 0; qd < NQ; ++qd) xq[qd] = lds[(xrow * NQ + qd) * a.nchunks + xrow * XSKEW + cc];
+        for (int qd = 0; qd < NQ; ++qd) xq[qd] = lds[(xrow * NQ + qd) * stride + xrow * XSKEW + xc];
         Dot d;
         d.unpack(b.w[u][0]);
         float4_t dd = {0.f, 0.f, 0.f, 0.f};
@@ -261,12 +266,12 @@ __global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = cb + u * cstride;
-      const int cc = min(c, last_chunk);
+      const int xc = min(c, a.nchunks);
       u32x4 xv[MT][NQ];
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int qd = 0; qd < NQ; ++qd) xv[m][qd] = lds[(m * NQ + qd) * a.nchunks + cc];
+        for (int qd = 0; qd < NQ; ++qd) xv[m][qd] = lds[(m * NQ + qd) * stride + xc];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         Dot d;
@@ -276,7 +281,7 @@ __global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
         for (int m = 0; m < MT; ++m) {
           const float part = d.dot(xv[m]);
           if (GROUPED) acc[r][m] = fmaf(sc, part, acc[r][m]);
-          else acc[r][m] += (c <= last_chunk ? part : 0.f);
+          else acc[r][m] += part;
         }
       }
     }
@@ -378,8 +383,9 @@ __global__ __launch_bounds__(512) void gemv_kernel(const GemvArgs a) {
     int m, u;
     split(idx, m, u);
     const int c = u / NQ, qd = u - c * NQ;
-    return lds + (m * NQ + qd) * a.nchunks + m * XSKEW + c;
+    return lds + (m * NQ + qd) * stride + m * XSKEW + c;
   };
+  if (tid < MT * NQ) lds[tid * stride + (tid / NQ) * XSKEW + a.nchunks] = (u32x4){0u, 0u, 0u, 0u};
   if (a.pro.kind != TLHIP_PRO_NONE) {
     // What is staged is f(x): see stage_with_prologue.
     constexpr int E = 16 / (int)sizeof(XT);  // elements per 16-byte unit
