@@ -140,6 +140,11 @@ bool gemm_rows_default(const Problem& p, tlhip_kernel_config_t* out, double* us)
 // Time of such a launch behind others, in microseconds; c applicable.
 double gemm_rows_us(const Problem& p, const tlhip_kernel_config_t& c);
 int launch_gemm_rows(const Problem& p, const tlhip_kernel_config_t& c, hipStream_t stream);
+// What a launch of the skinny kernel or the VALU kernel (40 KB of code an instance, 90 to 230) costs more, in microseconds, where
+// other kernels ran since its last, than one with all of K in a workgroup (6 to 15): two CUs share 64 KB of instruction cache.
+// Behind three other kernels and 64 MB of weights the former took 1.7-2.0 us longer than in a row of their own, the latter 0.1
+// (2 to 16 f16 rows, 1600 problems, medians); half the difference, as a launch meets both.
+constexpr double kColdCodeUs = 0.85;
 // Time of a launch of the decode kernel at up to 16 and at 17..64 rows, in microseconds (gemv_mfma.hip); c applicable.
 double gemv_mfma_us(const Problem& p, const tlhip_kernel_config_t& c);
 double gemv_mfma_rows_us(const Problem& p, const tlhip_kernel_config_t& c);

@@ -481,24 +481,27 @@ bool few_rows_possible(const Problem& p, tlhip_kernel_config_t* out) {
 // it at 2-3 %, where it is at 5-11 %, by up to 39 %, if it is taken wherever it is possible.  Us, without / here:
 //   beside the skinny kernel the cheaper price, up to K = 14336 (16 rows of int4 at 4096 x 4096 with a residual 7.6 / 6.5,
 //   but plain at 4096 x 12288 12.0 / 13.5; of int8-64 at 2048 x 12288 10.1 / 13.0); longer, where the launches are 10 % above
-//   the price, all but 9 to 16 rows of few columns (16 of int4 at 768 x 16384 9.8 / 12.1, at 6144 x 16384 17.8 / 21.9);
-//   beside the VALU kernel all but two rows of int4 with up to 1024 columns and K from 3072 to 12288 (1024 x 4096 3.7 / 4.2),
-//   and three or four rows of int4 on the 4 x 4 x 4 form with 14336 columns or more (24576 x 4096, three 15.1 / 17.4; four
-//   15.8 / 17.3, with a residual 18.0 / 17.1) or, three of them without a residual, 5120 to 8192 columns of K from 5120 (8192 x
-//   8192 11.4 / 12.0).
+//   the price, all but 9 to 16 rows of few columns (16 of int4 at 768 x 16384 9.8 / 12.1, at 6144 x 16384 17.8 / 21.9); fewer columns
+//   than were measured stay in slices from K = 12288 on (16 rows at 768 x 12288 8.9 / 10.5, eight 10.7 / 8.8);
+//   beside the VALU kernel all but three or four rows of int4 on the 4 x 4 x 4 form with 14336 columns or more (24576 x 4096,
+//   three 15.1 / 17.4; four 15.8 / 17.3, with a residual 18.0 / 17.1).
+// Those are launches in a row of their own; the kernels without all of K are ahead only by more than what their code costs
+// behind others (kColdCodeUs: two rows of int4 at 1024 x 4096 3.7 / 4.2, three at 8192 x 8192 11.4 / 12.0 go here).  Fifteen calls,
+// 1 to 16 rows of int4 at the three matrices of a 4096 x 12288 layer in turn, take 106.3 us with all but the one row here,
+// 108.3 with 16 rows of 4096 x 12288 in K slices (12.3 / 13.8 by themselves), 110.3 with four rows of 12288 x 4096 in K slices (9.6 /
+// 9.8) and 110.4 with two rows there on the 4 x 4 x 4 form (8.9 / 9.9).
 bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   if (!few_rows_possible(p, out)) return false;
   const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED, plain = !has_residual(p);
   const tlhip_kernel_config_t below = default_below_few(p);
   if (below.variant == VARIANT_GEMV) {
-    if (p.m == 2) return !(int4 && p.n <= 1024 && p.k >= 3072 && p.k < 12288);
-    const bool wide = p.n >= 14336, level = p.n >= 5120 && p.n <= 8192 && p.k >= 5120;
-    return !(p.m == 3 ? (wide && p.k >= 2048) || (level && plain) : wide && plain && p.k >= 4096);
+    if (p.m == 2) return true;
+    return !(p.n >= 14336 && (p.m == 3 ? p.k >= 2048 : plain && p.k >= 4096));
   }
   if (below.variant != VARIANT_GEMV_MFMA) return true;
-  if (p.m == 2) return false;
+  if (p.m == 2 || (p.n < 768 && p.k >= 12288)) return false;
   if (p.k > 14336) return !(p.m > 8 && (p.n <= 1024 || (plain && p.n <= (int4 ? 6144 : 2048))));
-  return gemv_few_us(p, *out) <= gemv_mfma_us(p, below);
+  return gemv_few_us(p, *out) <= gemv_mfma_us(p, below) + kColdCodeUs;
 }
 
 // Two f32 rows that stay on the VALU kernel of gemv_kernel.h, us, there / where they would go: int4, up to 1536 columns of a K
@@ -872,16 +875,17 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     there.k = e.k;
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
-    // (where a neighbour of 2..16 rows is on the matrix cores, the problem's own prices tell which of their two forms it has, and
-    // whether the neighbour's K slices are cheaper than its own: 16 rows of int4 at 2048 x 12288 12.0 us in those of a winner at
+    // (where a neighbour of 2..16 rows keeps all of K in a workgroup or has K slices across workgroups, the problem's own prices tell
+    // which of the two it has, and whether the neighbour's slices are cheaper than its own: 16 rows of int4 at 2048 x 12288 12.0 us in those of a winner at
     // 4096 x 12288, 9.4 in its own)
     tlhip_kernel_config_t few;
     const bool whole_there = is_few_config(there, c, FEW_SINGLE);
-    if ((whole_there || (c.variant == VARIANT_GEMV_MFMA && p.m <= 16)) && few_rows_config(p, &few)) {
+    const bool slices_there = !whole_there && c.variant == VARIANT_GEMV_MFMA && p.m > 1 && p.m <= 16 && c.p3 > 1;
+    if ((whole_there || slices_there) && few_rows_config(p, &few)) {
       c = few;
     } else if (whole_there) {
       continue;
-    } else if (c.variant == VARIANT_GEMV_MFMA && p.m > 1 && p.m <= 16 && p.n < 32768) {
+    } else if (slices_there && p.n < 32768) {
       const tlhip_kernel_config_t own = default_below_few(p);
       if (own.variant == VARIANT_GEMV_MFMA && config_applicable(p, c, nullptr) && gemv_mfma_us(p, own) < gemv_mfma_us(p, c)) c = own;
     }
@@ -921,7 +925,16 @@ tlhip_kernel_config_t choose_config(const Problem& p) {
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     auto it = g_tuned.find(problem_key(p));
-    if (it != g_tuned.end() && config_applicable(p, it->second, nullptr)) return it->second;
+    if (it != g_tuned.end() && config_applicable(p, it->second, nullptr)) {
+      // (a key does not tell whether a residual was added when its winner was timed, and K slices read it behind the
+      // sums: 16 rows of int4 at 4096 x 12288 12.3 / 13.8 us with all of K in a workgroup, with a residual 13.7 / 13.8, and a
+      // decode step of 8 billion weights, its code cold, 216.5 us with them there and 211.6 without)
+      tlhip_kernel_config_t few;
+      if (has_residual(p) && it->second.variant == VARIANT_GEMV_MFMA && p.m <= 16 && !is_few_config(p, it->second, FEW_SINGLE) && few_rows_possible(p, &few) &&
+          gemv_few_us(p, few) <= gemv_mfma_us(p, it->second) + kColdCodeUs)
+        return few;
+      return it->second;
+    }
   }
   tlhip_kernel_config_t c;
   // Above 64 rows a neighbour's winner knows less than the launch model of the eight-wave
