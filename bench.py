@@ -206,7 +206,15 @@ class Bench:
 
 
 def kernel_name_of(cfg) -> str:
-    return {0: "gemv_kernel (VALU dot2)", 1: "gemv_mfma_kernel (16x16x32 f16)", 2: "gemm_prefill_kernel (32x32x16 f16)",
+    """The kernel a configuration runs, by all its fields (a variant holds several)."""
+    if cfg.variant == 0:
+        return {1: "gemv_kernel (4x4x4 f16)", 3: "gemv_one_kernel (VALU dot2, one row)",
+                4: "gemv_some_kernel (VALU, 2 to 5 f32 rows)"}.get(cfg.p5, "gemv_kernel (VALU dot2)")
+    if cfg.variant == 1 and cfg.p1 == 0:
+        return "gemv_few_kernel (16x16x32 f16, all of K in a workgroup)" if cfg.p2 > 0 else "gemm_rows_kernel (16x16x32 f16, all of K in a workgroup)"
+    if cfg.variant == 6:
+        return "gemv_f32_whole_kernel (16x16x32 bf16, all of K in a workgroup)" if cfg.p1 else "gemv_f32_kernel (16x16x32 bf16, K slices)"
+    return {1: "gemv_mfma_kernel (16x16x32 f16)", 2: "gemm_prefill_kernel (32x32x16 f16)",
             3: "gemm_direct_kernel (32x32x16 f16, weights dequantised in registers)",
             4: "gemv_xreg_kernel (16x16x32 f16, activations in registers)",
             5: "gemv_wave_kernel (16x16x32 f16, every wave its own K range)"}.get(cfg.variant, f"variant {cfg.variant}")
