@@ -3,8 +3,9 @@
 // Same contract and reference route as gemv.hip (src/backend/webgpu/matmul/gemv.ts:365-466).
 //
 // What bounds it: its own instructions (X into LDS and out of it as operands, the dequantising, the
-// products), then the weights' way from memory; the activations' way comes last, although every workgroup
-// needs all of X (64 rows of K = 4096 are 512 KB, three times a CU's LDS) from its L2.  Hence:
+// products), then the weights' way from memory.  Every workgroup needs all of X (64 rows of K = 4096 are 512 KB,
+// three times a CU's LDS) from its L2: little beside the instructions at that K, the largest part at long K on few columns
+// (48 rows at 4096 x 12288: 302 MB of X for 28 MB of weights).  Hence:
 //   * A workgroup owns 16 NB columns of Y and all of K, so that nothing is combined between
 //     workgroups: no planes of partial sums, no second launch, no workspace.
 //   * Each of its eight waves has a range of K, 128 a step, alone until one barrier at the end: the
@@ -16,10 +17,11 @@
 //     fetched twice (10-25 % slower).
 //   * An operand of X feeds NB products and a weight, dequantised once, MT.
 //   * Few columns: a workgroup takes a share of the row tiles, so that more CUs work (gemm_rows_default).
-// Us, steps dealt to the waves in turn with their scales, two in flight and empty loads past the end -> as it is:
-// int4 12288 x 4096 at 48 rows 18.2 -> 14.6, 4096 x 4096 with a residual 13.0 -> 10.8, 1024 x 1024 6.4 -> 5.5; int8-64
-// 12288 x 4096 at 32 rows 21.8 -> 12.6; 1.24 times faster in the mean of 28 matrices of 768..16384 x 768..12288 at
-// 20..64 rows, four formats.  14.6 us are 1.9 TB/s of weights and scales and 330 TFLOP/s.
+// Us on cold weights, steps dealt to the waves in turn with their scales, two in flight and empty loads past the end -> as it
+// is: int4 12288 x 4096 at 48 rows 18.1 -> 16.5, with a residual 19.9 -> 18.6, 4096 x 4096 with a residual 12.7 -> 11.3,
+// 4096 x 12288 25.7 -> 22.6, 1024 x 1024 5.4 -> 3.5; int8-64 12288 x 4096 at 32 rows 22.3 -> 15.7; 1.22 times faster in the mean
+// of 6588 problems of up to 16384 columns at 17..64 rows, three formats.  16.5 us are 1.7 TB/s of weights and scales and
+// 293 TFLOP/s.
 // Rearranging X for the cheaper int4 unpacking, or its addresses by lane, moved nothing.
 //   * Buffer loads: rows past M and columns past N read zero, so that the loop has no branch around a load.
 #include <algorithm>
