@@ -481,8 +481,9 @@ bool few_rows_possible(const Problem& p, tlhip_kernel_config_t* out) {
 // it at 2-3 %, where it is at 5-11 %, by up to 39 %, if it is taken wherever it is possible.  Us, without / here:
 //   beside the skinny kernel the cheaper price, up to K = 14336 (16 rows of int4 at 4096 x 4096 with a residual 7.6 / 6.5,
 //   but plain at 4096 x 12288 12.0 / 13.5; of int8-64 at 2048 x 12288 10.1 / 13.0); longer, where the launches are 10 % above
-//   the price, all but 9 to 16 rows of few columns (16 of int4 at 768 x 16384 9.8 / 12.1, at 6144 x 16384 17.8 / 21.9); fewer columns
-//   than were measured stay in slices from K = 12288 on (16 rows at 768 x 12288 8.9 / 10.5, eight 10.7 / 8.8);
+//   the price, all but 9 to 16 rows of few columns (16 of int4 at 768 x 16384 9.8 / 12.1, at 6144 x 16384 17.8 / 21.9); from
+//   K = 12288 on 13 to 16 rows of up to 2048 columns are in slices too, which the price sees 1-2 us dearer than they are (int8-64 at
+//   768 x 12288 with a residual 10.0 / 11.2), and fewer columns than were measured (eight at 768 x 12288 10.7 / 8.8);
 //   beside the VALU kernel all but three or four rows of int4 on the 4 x 4 x 4 form with 14336 columns or more (24576 x 4096,
 //   three 15.1 / 17.4; four 15.8 / 17.3, with a residual 18.0 / 17.1).
 // Those are launches in a row of their own; the kernels without all of K are ahead only by more than what their code costs
@@ -499,17 +500,17 @@ bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
     return !(p.n >= 14336 && (p.m == 3 ? p.k >= 2048 : plain && p.k >= 4096));
   }
   if (below.variant != VARIANT_GEMV_MFMA) return true;
-  if (p.m == 2 || (p.n < 768 && p.k >= 12288)) return false;
-  if (p.k > 14336) return !(p.m > 8 && (p.n <= 1024 || (plain && p.n <= (int4 ? 6144 : 2048))));
+  if (p.m == 2 || (p.k >= 12288 && (p.n < 768 || (p.m > 12 && p.n <= 2048)))) return false;
+  if (p.k > 14336) return !(p.m > 8 && (p.n <= 2048 || (plain && p.n <= (int4 ? 6144 : 2048))));
   return gemv_few_us(p, *out) <= gemv_mfma_us(p, below) + kColdCodeUs;
 }
 
 // Two f32 rows that stay on the VALU kernel of gemv_kernel.h, us, there / where they would go: int4, up to 1536 columns of a K
 // between 8192 and 12288 (1024 x 9728 8.0 / 10.0 with all of K on the matrix cores), and 7169..8192 columns, its workgroups two to a CU
-// (8192 x 3072 7.7 / 8.9 on gemv_some); int8 with K up to 1536 on wide matrices (10240 x 1536 6.0 / 7.6) and up to 2048 on
+// (8192 x 3072 7.7 / 8.9 on gemv_some, but 7664 x 1152 7.5 / 5.8); int8 with K up to 1536 on wide matrices (10240 x 1536 6.0 / 7.6) and up to 2048 on
 // 4097..6144 columns (6144 x 1536 5.1 / 5.7).
 bool two_f32_rows_on_valu(const Problem& p) {
-  if (p.format == TLHIP_FMT_INT4_GROUPED) return (p.n <= 1536 && p.k > 8192 && p.k < 12288) || (p.n > 7168 && p.n <= 8192 && p.k <= 4096);
+  if (p.format == TLHIP_FMT_INT4_GROUPED) return (p.n <= 1536 && p.k > 8192 && p.k < 12288) || (p.n > 7168 && p.n <= 8192 && p.k >= 2048 && p.k <= 4096);
   return (p.n > 6144 && p.k <= 1536) || (p.n > 4096 && p.n <= 6144 && p.k > 1024 && p.k <= 2048);
 }
 
@@ -875,12 +876,13 @@ bool nearest_in_class(const Problem& p, const std::vector<ClassEntry>& list, tlh
     there.k = e.k;
     if (is_rows_config(there, c) && !rows_in_one_launch_config(p, &c)) continue;
     if (c.variant == VARIANT_GEMV_F32 && c.p1 && !gemv_f32_default(p, &c)) continue;
-    // (where a neighbour of 2..16 rows keeps all of K in a workgroup or has K slices across workgroups, the problem's own prices tell
-    // which of the two it has, and whether the neighbour's slices are cheaper than its own: 16 rows of int4 at 2048 x 12288 12.0 us in those of a winner at
+    // (where a neighbour of 2..16 rows keeps all of K in a workgroup, or is on the skinny kernel with K slices across workgroups or
+    // another K, for which it was staged, the problem's own prices tell which of the two it has, and whether the neighbour's
+    // geometry is cheaper than its own: eight of int4 with a residual at 20480 x 2048 13.5 us in that of 24576 x 4096, 10.4 here; 16 rows of int4 at 2048 x 12288 12.0 us in those of a winner at
     // 4096 x 12288, 9.4 in its own)
     tlhip_kernel_config_t few;
     const bool whole_there = is_few_config(there, c, FEW_SINGLE);
-    const bool slices_there = !whole_there && c.variant == VARIANT_GEMV_MFMA && p.m > 1 && p.m <= 16 && c.p3 > 1;
+    const bool slices_there = !whole_there && c.variant == VARIANT_GEMV_MFMA && p.m > 1 && p.m <= 16 && (c.p3 > 1 || e.k != p.k);
     if ((whole_there || slices_there) && few_rows_config(p, &few)) {
       c = few;
     } else if (whole_there) {
@@ -925,16 +927,7 @@ tlhip_kernel_config_t choose_config(const Problem& p) {
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
     auto it = g_tuned.find(problem_key(p));
-    if (it != g_tuned.end() && config_applicable(p, it->second, nullptr)) {
-      // (a key does not tell whether a residual was added when its winner was timed, and K slices read it behind the
-      // sums: 16 rows of int4 at 4096 x 12288 12.3 / 13.8 us with all of K in a workgroup, with a residual 13.7 / 13.8, and a
-      // decode step of 8 billion weights, its code cold, 216.5 us with them there and 211.6 without)
-      tlhip_kernel_config_t few;
-      if (has_residual(p) && it->second.variant == VARIANT_GEMV_MFMA && p.m <= 16 && !is_few_config(p, it->second, FEW_SINGLE) && few_rows_possible(p, &few) &&
-          gemv_few_us(p, few) <= gemv_mfma_us(p, it->second) + kColdCodeUs)
-        return few;
-      return it->second;
-    }
+    if (it != g_tuned.end() && config_applicable(p, it->second, nullptr)) return it->second;
   }
   tlhip_kernel_config_t c;
   // Above 64 rows a neighbour's winner knows less than the launch model of the eight-wave

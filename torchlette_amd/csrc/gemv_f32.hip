@@ -673,7 +673,9 @@ static double whole_us(const Problem& p, int cols) {
 // and weights and, for every row of every slice, what the last arrival adds.  Fitted at 2287 launches of either (106
 // matrices of 768..16384 x 1024..16384, 3..16 rows, three formats): 2-7 % and 4-9 % rms; the cheaper one is 0.05-0.3 % behind the faster
 // in the mean and more than 3 % at 1-4 % of the problems (2-7 % by warm prices: five rows of int8 per row at
-// 5120 x 12288 21.4 us in slices, 30.1 so).
+// 5120 x 12288 21.4 us in slices, 30.1 so).  Most of those K are multiples of 1024, whose rows crowd onto a part of the memory's channels:
+// at others slices of int4 take 0.86 of it for an odd number of steps (16 rows at 1712 x 8064 16.9 us, 20.9 so), and up to
+// eight rows of int8 per row in one workgroup 0.83-0.93 (five at 4384 x 7424 15.0 us in slices, 12.3 so).
 static double whole_beside_us(const Problem& p, int cols) {
   struct Cost {
     double launch, mb, round, sums, k, k_rows, k_blocks;
@@ -686,7 +688,8 @@ static double whole_beside_us(const Problem& p, int cols) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256, nb = (cols + 15) / 16;
   const int64_t wgs = (p.n + cols - 1) / cols, steps = p.k / kWholeStep;
   const double rounds = (double)((wgs + cus - 1) / cus), k = (double)((steps + kWhole - 1) / kWhole * kWhole * kWholeStep) / 1000.0;
-  return t.launch + t.mb * packed_mb(p) + rounds * (t.round + t.sums * nb + k * (t.k + t.k_rows * (double)p.m + t.k_blocks * nb));
+  const double spread = p.format == TLHIP_FMT_INT8_ROW && p.m <= 8 && p.k % 1024 ? 0.93 : 1.0;
+  return spread * (t.launch + t.mb * packed_mb(p) + rounds * (t.round + t.sums * nb + k * (t.k + t.k_rows * (double)p.m + t.k_blocks * nb)));
 }
 static double slices_us(const Problem& p, int slices) {
   struct Cost {
@@ -697,8 +700,9 @@ static double slices_us(const Problem& p, int slices) {
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const int64_t wgs = column_tiles(p) * slices, rounds = (wgs + cus - 1) / cus, slice = (blocks_of(p) + slices - 1) / slices * block_k(p);
   const double rows = (double)(slices * p.m);
-  return t.launch + t.mb * packed_mb(p) + (double)(rounds * slice) / 1000.0 * (t.weights + t.cut * (double)p.m) + t.slice * slices + t.sum * rows +
-         t.out * (double)column_tiles(p) * rows / 100.0;
+  const double spread = p.format == TLHIP_FMT_INT4_GROUPED && p.k % 256 ? 0.87 : 1.0;
+  return spread * (t.launch + t.mb * packed_mb(p) + (double)(rounds * slice) / 1000.0 * (t.weights + t.cut * (double)p.m) + t.slice * slices + t.sum * rows +
+                   t.out * (double)column_tiles(p) * rows / 100.0);
 }
 
 // All of K in one workgroup, at the cheapest number of columns (whole blocks, or an even share that
