@@ -488,9 +488,9 @@ bool few_rows_possible(const Problem& p, tlhip_kernel_config_t* out) {
 //   three 15.1 / 17.4; four 15.8 / 17.3, with a residual 18.0 / 17.1).
 // Those are launches in a row of their own; the kernels without all of K are ahead only by more than what their code costs
 // behind others (kColdCodeUs: two rows of int4 at 1024 x 4096 3.7 / 4.2, three at 8192 x 8192 11.4 / 12.0 go here).  Fifteen calls,
-// 1 to 16 rows of int4 at the three matrices of a 4096 x 12288 layer in turn, take 106.3 us with all but the one row here,
-// 108.3 with 16 rows of 4096 x 12288 in K slices (12.3 / 13.8 by themselves), 110.3 with four rows of 12288 x 4096 in K slices (9.6 /
-// 9.8) and 110.4 with two rows there on the 4 x 4 x 4 form (8.9 / 9.9).
+// 1 to 16 rows of int4 at the three matrices of a 4096 x 12288 layer in turn, take 109 us with the stored winners, 112 with 16
+// rows of 4096 x 12288 in K slices (12.0 / 13.4 by themselves; the seven launches of a layer of 16 rows, few kinds of kernels,
+// 59.2 / 60.2) and 112 with four rows of 12288 x 4096 in K slices (8.9 / 9.5), 114 with both.
 bool few_rows_config(const Problem& p, tlhip_kernel_config_t* out) {
   if (!few_rows_possible(p, out)) return false;
   const bool int4 = p.format == TLHIP_FMT_INT4_GROUPED, plain = !has_residual(p);
