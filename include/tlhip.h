@@ -491,8 +491,9 @@ int tlhip_candidate_get(const tlhip_qweight_t* w, int x_dtype, int64_t m, int y_
  * exact problem if cached, else the winner of the nearest tuned problem of the same
  * shape class (autotune.ts:269-300), else the heuristic default — selectMatmulChoice,
  * dispatch.ts:171-192.  Every level is re-gated on applicability.  A neighbour's winner
- * carries over as it is only where its geometry does not follow from the sizes: one row, and
- * the forms that keep all of K in a workgroup, have the problem's own kernel and geometry.
+ * carries over as it is only where its geometry does not follow from the sizes: one row, the
+ * forms that keep all of K in a workgroup and, of 2..16 rows, K slices across workgroups and a
+ * winner timed at another K have the problem's own kernel and geometry.
  * The epilogue counts too: a binary step moves 2..16 rows to the form it costs less
  * (this query has none).  A launch of ONE row with a prologue (tlhip_gemv_prologue) goes by
  * the heuristic default whatever is tuned: winners are timed without a prologue.  Where the
